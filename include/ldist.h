@@ -210,6 +210,21 @@ LDIST_API int ldist_adamw_lp_step(float* param, const float* grad, float* exp_av
                         double p_norm, double lr, double beta1, double beta2, double eps, double weight_decay,
                         int step, ldist_stream_t stream);
 
+/* Evaluation-mode shift of a layer's output, a contiguous (B, C, L) tensor: y = (x - mean[c]) + bias[c], in this order;
+ * mean and bias are (C) each and may be NULL; y may be x.  No native counterpart in the reference: it is the torch code
+ * of its MeanNorm and of its layer's bias (model/norm_dist.py:96-97,136-139), two kernels per output there. */
+LDIST_API int ldist_channel_shift(const float* x, int B, int C, int L, const float* mean, const float* bias, float* y,
+                                  ldist_stream_t stream);
+/* margins[b,j] = upper[b,j] - lower[b,targets[b]] and 0 at j = targets[b]: the certified margins of the reference's
+ * BoundFinalIdentity (model/bound_module.py:95-103, four torch kernels there).  lower, upper, margins (B, J); a target
+ * outside [0, J) fills its row with NaN. */
+LDIST_API int ldist_certified_margins(const float* lower, const float* upper, const int64_t* targets, int B, int J,
+                                      float* margins, ldist_stream_t stream);
+/* One step of the projected-gradient attack on n values (reference attack.py:26-33, nine torch kernels there):
+ *   next = clip(clip(adv + step * sign(grad), centre - eps, centre + eps), down, up). */
+LDIST_API int ldist_pgd_step(const float* adv, const float* grad, const float* centre, long long n, float step, float eps,
+                             float down, float up, float* next, ldist_stream_t stream);
+
 /* Patch extraction for the convolution-shaped layer, with torch's F.unfold layout, which the
  * reference uses to turn an image into the layer's input (model/norm_dist.py:132,144-145):
  *   cols[b, (c*KH + i)*KW + j, h*WO + w] = img[b, c, h*stride + i*dilation - padding, w*stride + j*dilation - padding]

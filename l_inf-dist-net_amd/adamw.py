@@ -18,7 +18,7 @@ import torch
 from torch.optim import Optimizer
 
 from . import norm_dist_cpp
-from .norm_dist import get_p_norm
+from .norm_dist import NormDistConv, get_p_norm
 
 
 def lp_weight_decay_(param, p_norm, lr, weight_decay, eps):
@@ -72,8 +72,11 @@ class AdamW(Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
+        fused, hyper = ([], [], [], []), []   # tensors and hyper-parameters of the native call
+        ops = norm_dist_cpp.layer_ops
         for group in self.param_groups:
-            p_norm = get_p_norm(group["module"])
+            module = group["module"]
+            p_norm = module.p if isinstance(module, NormDistConv) else get_p_norm(module)
             beta1, beta2 = group["betas"]
             lr, eps, wd = group["lr"], group["eps"], group["weight_decay"]
             for prm in group["params"]:
@@ -89,9 +92,15 @@ class AdamW(Optimizer):
                     state["exp_avg_sq"] = torch.zeros_like(prm, memory_format=torch.preserve_format)
                 state["step"] += 1
                 m, v = state["exp_avg"], state["exp_avg_sq"]
-                if _fused_ok(prm, grad, m, v):
+                if ops is not None and _fused_ok(prm, grad, m, v):
+                    for tensors, t in zip(fused, (prm, grad, m, v)):
+                        tensors.append(t)
+                    hyper.append((-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd, state["step"]))
+                elif _fused_ok(prm, grad, m, v):
                     norm_dist_cpp.adamw_lp_step(prm, grad, m, v, p_norm, lr, beta1, beta2, eps, wd, state["step"])
                 else:
                     lp_weight_decay_(prm, p_norm, lr, wd, eps)
                     _adam_(prm, grad, m, v, lr, beta1, beta2, eps, state["step"])
+        if hyper:
+            ops.adamw_step(*fused, hyper)
         return loss

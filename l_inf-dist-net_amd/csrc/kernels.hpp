@@ -113,6 +113,14 @@ hipError_t adamw_lp_step(float* param, const float* grad, float* exp_avg, float*
                          double p_norm, double lr, double beta1, double beta2, double eps, double weight_decay, int step,
                          hipStream_t stream);
 
+// The small elementwise operations around the layers (elementwise.hip).
+hipError_t channel_shift(const float* x, const float* mean, const float* bias, float* y, int B, int C, int L, int num_cu,
+                         hipStream_t stream);
+hipError_t certified_margins(const float* lower, const float* upper, const int64_t* targets, float* margins, int B, int J,
+                             hipStream_t stream);
+hipError_t pgd_step(const float* adv, const float* grad, const float* centre, float* next, long long n, float step, float eps,
+                    float down, float up, int num_cu, hipStream_t stream);
+
 // Geometry of a convolution-shaped layer working on an image tensor (B, C, H, W).
 struct ConvGeom {
     int B, C, H, W;        // image

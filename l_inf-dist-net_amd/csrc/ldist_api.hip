@@ -258,6 +258,33 @@ int ldist_adamw_lp_step(float* param, const float* grad, float* exp_avg, float* 
                                        weight_decay, step, (hipStream_t)stream));
 }
 
+int ldist_channel_shift(const float* x, int B, int C, int L, const float* mean, const float* bias, float* y,
+                        ldist_stream_t stream) {
+    if (!x || !y || B <= 0 || C <= 0 || L <= 0) return LDIST_EINVAL;
+    if ((long long)B * C * L >= (1LL << 31)) return LDIST_ERANGE;
+    ldist::Problem pr{};
+    if (int rc = current_device(pr)) return rc;
+    return finish(ldist::channel_shift(x, mean, bias, y, B, C, L, pr.num_cu, (hipStream_t)stream));
+}
+
+int ldist_certified_margins(const float* lower, const float* upper, const int64_t* targets, int B, int J, float* margins,
+                            ldist_stream_t stream) {
+    if (!lower || !upper || !targets || !margins || B <= 0 || J <= 0) return LDIST_EINVAL;
+    if ((long long)B * J >= (1LL << 31)) return LDIST_ERANGE;
+    ldist::Problem pr{};
+    if (int rc = current_device(pr)) return rc;
+    return finish(ldist::certified_margins(lower, upper, targets, margins, B, J, (hipStream_t)stream));
+}
+
+int ldist_pgd_step(const float* adv, const float* grad, const float* centre, long long n, float step, float eps, float down,
+                   float up, float* next, ldist_stream_t stream) {
+    if (!adv || !grad || !centre || !next || n <= 0) return LDIST_EINVAL;
+    if (n >= (1LL << 31)) return LDIST_ERANGE;
+    ldist::Problem pr{};
+    if (int rc = current_device(pr)) return rc;
+    return finish(ldist::pgd_step(adv, grad, centre, next, n, step, eps, down, up, pr.num_cu, (hipStream_t)stream));
+}
+
 int ldist_unfold(const float* img, int B, int C, int H, int W, int KH, int KW, int stride, int padding, int dilation,
                  float* cols, ldist_stream_t stream) {
     ldist::ConvGeom q{};

@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import norm_dist_cpp
 from .norm_dist import get_p_norm, set_p_norm
 
 
@@ -67,7 +68,10 @@ def train_step(net, loss_fun, optimizer, inputs, targets):
     optimizer.zero_grad()
     loss.backward()
     optimizer.step()
-    return loss.item(), cal_acc(outputs.detach(), targets).mean().item()
+    accuracy = cal_acc(outputs.detach(), targets).mean()
+    if loss.dim() == 0 and loss.dtype == accuracy.dtype and loss.device == accuracy.device:
+        return tuple(torch.stack((loss.detach(), accuracy)).tolist())   # one wait for the device instead of two
+    return loss.item(), accuracy.item()
 
 
 @contextlib.contextmanager
@@ -96,6 +100,15 @@ class AttackPGD:
             x = _box(x, centre - self.eps, centre + self.eps)
         return _box(x, self.down, self.up)
 
+    def _ascend(self, adv, grad, inputs):
+        """One signed-gradient step and its projections."""
+        ops = norm_dist_cpp.layer_ops
+        if (ops is not None and type(self)._project is AttackPGD._project and adv.is_cuda and
+                adv.dtype == grad.dtype == inputs.dtype == torch.float32 and adv.shape == inputs.shape and
+                not any(isinstance(v, torch.Tensor) for v in (self.eps, self.step_size, self.up, self.down))):
+            return ops.pgd_step(adv, grad, inputs, self.step_size, self.eps, self.down, self.up)   # one kernel
+        return self._project(adv + self.step_size * grad.sign(), centre=inputs)
+
     def find(self, inputs, targets):
         start = inputs.detach()
         if self.rand:
@@ -106,7 +119,7 @@ class AttackPGD:
             for _ in range(self.num_steps):
                 adv = adv.detach().requires_grad_(True)
                 F.cross_entropy(self.net(adv), targets, reduction="sum").backward()
-                adv = self._project(adv.detach() + self.step_size * adv.grad.sign(), centre=inputs)
+                adv = self._ascend(adv.detach(), adv.grad, inputs)
         return adv.detach()
 
 

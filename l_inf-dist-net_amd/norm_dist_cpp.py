@@ -483,25 +483,30 @@ def inf_dist_bound_conv_forward(lower_img, upper_img, weight, output_lower, outp
 REFERENCE_NAMES = ("norm_dist_forward", "norm_dist_backward_input", "norm_dist_backward_weight", "inf_dist_forward",
                    "inf_dist_bound_forward", "inf_dist_backward_input", "inf_dist_backward_weight")
 ctypes_binding = {name: globals()[name] for name in REFERENCE_NAMES}
-_extension = None
+_modules = {}
 BINDING = "ctypes"     # or "torch_extension": what the seven reference names are bound to right now
 
 
-def torch_extension():
-    """The compiled module (torch_ext/norm_dist_cpp*.so), or None when it has not been built."""
-    global _extension
-    if _extension is None:
+def _compiled(name):
+    """The compiled module torch_ext/<name>*.so, or None when it has not been built."""
+    if name not in _modules:
         import glob
         import importlib.util
         import os
-        hits = glob.glob(os.path.join(os.path.dirname(os.path.abspath(__file__)), "torch_ext", "norm_dist_cpp*.so"))
+        hits = glob.glob(os.path.join(os.path.dirname(os.path.abspath(__file__)), "torch_ext", name + "*.so"))
         if not hits:
             return None
         _lib.lib()     # libldist_hip.so first: a missing library should be reported by its own message
-        spec = importlib.util.spec_from_file_location("norm_dist_cpp", hits[0])
-        _extension = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(_extension)
-    return _extension
+        spec = importlib.util.spec_from_file_location(name, hits[0])
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _modules[name] = module
+    return _modules[name]
+
+
+def torch_extension():
+    """The compiled module norm_dist_cpp, or None when it has not been built."""
+    return _compiled("norm_dist_cpp")
 
 
 def use_torch_extension(on=True):
@@ -521,8 +526,24 @@ def use_torch_extension(on=True):
     return BINDING
 
 
+# The layers' host path in native code (csrc/torch_ext/ldist_layers.cpp: routes, autograd nodes, optimizer loop), over
+# the same library with the same results; None: the Python route of norm_dist.py, which also serves CPU tensors, other
+# types and modules with hooks inside.
+layer_ops = None
+
+
+def use_native_layers(on=True):
+    """Switches the native host path of the layers on (RuntimeError when it has not been built) or off."""
+    global layer_ops
+    layer_ops = _compiled("ldist_layers") if on else None
+    if on and layer_ops is None:
+        raise RuntimeError("torch_ext/ldist_layers*.so is missing: build it with `make -C csrc torch_ext`")
+    return layer_ops
+
+
 try:
     if torch_extension() is not None:
         use_torch_extension(True)
+        use_native_layers(True)
 except (RuntimeError, ImportError, OSError):   # no library yet (the first call reports it), or built for another torch
     pass

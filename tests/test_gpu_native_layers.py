@@ -1,0 +1,144 @@
+"""The native host path of the layers (csrc/torch_ext/ldist_layers.cpp) against the Python route: both make the same
+calls of the same library, so outputs, gradients, running means and parameters must agree bit for bit (one-pass p-norm
+weight gradients, which collect float atomics, to float32 rounding)."""
+import math
+
+import pytest
+import torch
+
+import __graft_entry__ as entry
+from helpers import gen
+
+pkg = entry.load_package()
+cpp = pkg.norm_dist_cpp
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+INF = float("inf")
+
+
+@pytest.fixture()
+def both_routes():
+    """Runs a function on the native path and on the Python route and returns both results."""
+    def run(fn):
+        try:
+            cpp.use_native_layers(True)
+            native = fn()
+            cpp.use_native_layers(False)
+            return native, fn()
+        finally:
+            cpp.use_native_layers(True)
+    return run
+
+
+def _same(a, b, exact=True):
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert (x is None) == (y is None)
+        if x is not None:
+            assert x.shape == y.shape
+            assert torch.equal(x, y) if exact else torch.allclose(x, y, rtol=1e-5, atol=1e-5)
+
+
+# fully connected 2-D, 1x1 image, 3x3 image (image kernels), 5x5 (columns), 3x3 with two positions per row, groups
+LAYERS = [dict(kind="fc", cin=37, cout=22), dict(kind="fc", cin=64, cout=9), dict(kind="conv", cin=6, cout=10, k=1, hw=5),
+          dict(kind="conv", cin=8, cout=40, k=3, hw=9, group=2), dict(kind="conv", cin=3, cout=32, k=5, hw=8, stride=2)]
+
+
+@pytest.mark.parametrize("p", [INF, 8.0, 37.3])
+@pytest.mark.parametrize("shift,bias", [(True, False), (False, True), (True, True), (False, False)])
+@pytest.mark.parametrize("case", range(len(LAYERS)))
+def test_layer_routes_agree(both_routes, case, shift, bias, p):
+    c = LAYERS[case]
+    g = gen(500 + case)
+    if c["kind"] == "fc":
+        layer = pkg.NormDist(c["cin"], c["cout"], p=p, bias=bias, mean_normalize=shift)
+        x = torch.rand(13, c["cin"], generator=g)
+    else:
+        layer = pkg.NormDistConv(c["cin"], c["cout"], c["k"], stride=c.get("stride", 1), padding=c["k"] // 2, p=p,
+                                 group=c.get("group", 1), bias=bias, mean_normalize=shift)
+        x = torch.rand(5, c["cin"], c["hw"], c["hw"] + 1, generator=g)
+    with torch.no_grad():
+        layer.weight.copy_(torch.randn(layer.weight.shape, generator=g) * 0.3)
+        if bias:
+            layer.bias.copy_(torch.randn(c["cout"], generator=g))
+    layer = layer.to(DEV)
+    x = x.to(DEV)
+
+    def step(train, grad):
+        if shift:
+            layer.normalize.running_mean.copy_(torch.linspace(-1, 1, c["cout"], device=DEV))
+        layer.train(train)
+        for prm in layer.parameters():
+            prm.grad = None
+        xi = x.clone().requires_grad_(grad)
+        with torch.set_grad_enabled(grad):
+            y = layer(xi)[0]
+        if grad:
+            y.backward(torch.sin(torch.arange(y.numel(), device=DEV, dtype=torch.float32)).view_as(y))
+        extra = [prm.grad for prm in layer.parameters()] if grad else []
+        return [y.detach(), xi.grad, layer.normalize.running_mean.clone() if shift else None] + extra, dict(layer.last_route)
+
+    for train, grad in ((True, True), (False, True), (False, False)):
+        (a, ra), (b, rb) = both_routes(lambda: step(train, grad))
+        _same(a, b, exact=math.isinf(p))
+        assert ra == rb
+    if math.isinf(p):
+        with torch.no_grad():
+            layer.eval()
+            (a, ra), (b, rb) = both_routes(lambda: (layer(x, x - 0.1, x + 0.1), dict(layer.last_route)))
+        _same(a, b)
+        assert ra == rb
+
+
+def test_a_hooked_mean_shift_is_still_called():
+    layer = pkg.NormDist(12, 8, p=INF, bias=False, mean_normalize=True).to(DEV).train()
+    seen = []
+    handle = layer.normalize.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+    x = torch.rand(4, 12, device=DEV)
+    hooked = layer(x)[0]
+    handle.remove()
+    assert len(seen) == 1 and torch.equal(hooked, layer(x)[0]) and len(seen) == 1
+
+
+@pytest.mark.parametrize("shape,L", [((3, 5), 1), ((7, 8), 1), ((2, 3), 6), ((2, 3), 7), ((1, 1), 4), ((65, 260), 1)])
+def test_evaluation_shift_against_torch(shape, L):
+    B, C = shape
+    x = torch.randn(B, C, L, generator=gen(3)).to(DEV)
+    mean, bias = torch.randn(C, generator=gen(4)).to(DEV), torch.randn(C, generator=gen(5)).to(DEV)
+    layer = pkg.NormDistConv(4, C, 1, p=INF, bias=True, mean_normalize=True).to(DEV).eval()
+    with torch.no_grad():
+        layer.bias.copy_(bias)
+        layer.normalize.running_mean.copy_(mean)
+        img = torch.rand(B, 4, 1, L, generator=gen(6)).to(DEV)
+        y = layer(img)[0]
+        raw = pkg.norm_dist(img.view(B, 4, L), layer.weight.view(C, 4), 1, INF)
+    assert torch.equal(y.view(B, C, L), (raw - mean.view(1, -1, 1)) + bias.view(1, -1, 1))
+
+
+def test_margins_and_their_gradients(both_routes):
+    lo, up = torch.randn(7, 10, generator=gen(8)).to(DEV), torch.randn(7, 10, generator=gen(9)).to(DEV)
+    t = torch.randint(0, 10, (7,), generator=gen(10)).to(DEV)
+
+    def run():
+        a, b = lo.clone().requires_grad_(), up.clone().requires_grad_()
+        m = pkg.BoundFinalIdentity()(lo, a, b, t)[1]
+        m.backward(torch.cos(torch.arange(70, device=DEV, dtype=torch.float32)).view(7, 10))
+        return [m.detach(), b.grad], a.grad
+    (x, ga), (y, gb) = both_routes(run)
+    _same(x, y)
+    torch.testing.assert_close(ga, gb, rtol=1e-6, atol=1e-6)
+
+
+def test_attack_and_optimizer_agree(both_routes):
+    def run():
+        torch.manual_seed(0)
+        net = pkg.Model(pkg.MLP(depth=3, width=1, input_dim=(1, 9, 7)), pkg.BoundFinalIdentity(), 0.1)
+        pkg.set_p_norm(net, INF)
+        net = net.to(DEV)
+        x, t = torch.rand(6, 1, 9, 7, generator=gen(11)).to(DEV), torch.arange(6, device=DEV)
+        adv = pkg.AttackPGD(net.eval(), 0.1, 0.03, 3, 1.0, 0.0, random_start=False).find(x, t)
+        opt = pkg.AdamW(net, lr=1e-2, weight_decay=1e-2)
+        got = [pkg.train_step(net, lambda o, w, t: torch.nn.functional.cross_entropy(o, t), opt, x, t) for _ in range(2)]
+        return [adv, torch.tensor(got)] + [prm.detach() for prm in net.parameters()] + list(net.buffers())
+    a, b = both_routes(run)
+    _same(a, b)
