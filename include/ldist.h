@@ -63,7 +63,9 @@ LDIST_API int ldist_last_hip_error(void);
  * (128x80 / 128x64 tiles), the one-pass kernel of ldist_norm_dist_backward included,
  * 2 / 3 / 4 keep them off; 5 forces that one-pass kernel on with 128x48 tiles (its third
  * width, which it otherwise takes where the wider ones leave CUs idle) and is like 2
- * for every other kernel.  Process-wide; not thread safe. */
+ * for every other kernel.  10..16 force the seven small tiles (32x80, 32x40, 16x40, 32x64, 32x32, 16x32, 64x80) and 30 the
+ * few-rows kernel of the fully connected forward passes with more than 16 outputs per group and at least 4 inputs, which
+ * otherwise are chosen by an estimate of their time.  Process-wide; not thread safe. */
 LDIST_API int ldist_set_tile_override(int choice);
 /* Tuning knob, no counterpart in the reference: 1 (default) orders the tiles of
  * the forward kernels so that each of the 8 XCDs works on one contiguous run of
@@ -132,6 +134,12 @@ LDIST_API int ldist_inf_dist_backward_weight(const float* grad_output, const int
  * stabilisation and seeds (norm_dist_cuda.cu:232-233,253-264,289). */
 LDIST_API int ldist_norm_dist_forward(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
                             float* output, float p, ldist_stream_t stream);
+/* The same for a forward pass that no gradient follows (evaluation, torch.no_grad()): same accuracy, but free to sum in
+ * the order of whichever kernel is fastest for the size, so the last bits may differ from ldist_norm_dist_forward's.
+ * No counterpart in the reference. */
+LDIST_API int ldist_norm_dist_forward_values(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
+                                             float* output, float p, ldist_stream_t stream);
+
 
 /* p-norm backward w.r.t. input.  Replaces norm_dist_backward_input_cuda
  * (model/norm_dist.cpp:9-10, model/norm_dist_cuda.cu:438-448).

@@ -208,6 +208,8 @@ hipError_t bound_forward(const float* lower, const float* upper, const float* we
 #undef LDIST_LAUNCH_RW
         return hipGetLastError();
     }
+    if (const int tile = small_forward_tile(pr, ForwardKind::kBounds, 0.f); tile >= 0)
+        return bound_forward_small(lower, upper, weight, out_lower, out_upper, pr, tile, stream);
     return dispatch_forward<BoundForward>(pr, can_vec4(pr, lower, upper, weight),
                                           can_vec4_out(pr, out_lower, out_upper), stream, lower, upper, weight,
                                           out_lower, out_upper);

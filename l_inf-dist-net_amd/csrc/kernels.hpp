@@ -72,6 +72,25 @@ hipError_t inf_forward(const float* input, const float* weight, float* output, i
 bool inf_forward_values_applicable(const Problem& pr, const void* input, const void* weight);
 hipError_t inf_forward_values(const float* input, const float* weight, float* output, const Problem& pr,
                               hipStream_t stream);
+// Small tiles with the reduction split over many k-groups, for fully connected layers whose outputs are too few to fill
+// the device with the tiles above, and the kernel for a handful of rows (small_forward.hip, which also estimates which of
+// them is fastest; -1: the larger tiles).
+enum class ForwardKind { kInf, kValues, kBounds, kNorm };
+int small_forward_tile(const Problem& pr, ForwardKind kind, float p);
+// pos == nullptr: values only
+hipError_t inf_forward_small(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr, int tile,
+                             hipStream_t stream);
+hipError_t bound_forward_small(const float* lower, const float* upper, const float* weight, float* out_lower, float* out_upper,
+                               const Problem& pr, int tile, hipStream_t stream);
+hipError_t norm_forward_small(const float* input, const float* weight, float* output, float p, const Problem& pr, int tile,
+                              hipStream_t stream);
+// A handful of rows: lanes along k, weights straight into registers (few_rows_forward.hip).
+hipError_t inf_forward_few_rows(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr,
+                                hipStream_t stream);
+hipError_t bound_forward_few_rows(const float* lower, const float* upper, const float* weight, float* out_lower, float* out_upper,
+                                  const Problem& pr, hipStream_t stream);
+hipError_t norm_forward_few_rows(const float* input, const float* weight, float* output, float p, const Problem& pr,
+                                 hipStream_t stream);
 bool inf_forward_shortk_applicable(const Problem& pr, const void* input, const void* output, const void* pos);
 hipError_t inf_forward_shortk(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr,
                               hipStream_t stream);
@@ -88,7 +107,7 @@ hipError_t inf_backward_input(const float* grad_output, const int32_t* pos, floa
 hipError_t inf_backward_weight(const float* grad_output, const int32_t* pos, float* grad_weight, const Problem& pr,
                                bool overwrite, hipStream_t stream);
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
-                        hipStream_t stream);
+                        bool values_only, hipStream_t stream);
 hipError_t norm_backward_input(const float* grad_output, const float* input, const float* weight,
                                const float* output, float* grad_input, float p, const Problem& pr,
                                hipStream_t stream);

@@ -99,7 +99,7 @@ int ldist_set_xcd_remap(int on) {
 }
 
 int ldist_set_tile_override(int choice) {
-    if (choice < -1 || choice > 5) return LDIST_EINVAL;
+    if (choice < -1 || (choice > 5 && choice < 10) || (choice > 16 && choice != 30)) return LDIST_EINVAL;
     ldist::g_tile_override = choice;
     return LDIST_OK;
 }
@@ -187,12 +187,22 @@ int ldist_inf_dist_backward_overwrite(const float* grad_output, const int32_t* p
     return finish(ldist::inf_backward_both(grad_output, pos, grad_input, grad_weight, pr, (hipStream_t)stream));
 }
 
-int ldist_norm_dist_forward(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
-                            float* output, float p, ldist_stream_t stream) {
+static int norm_forward_entry(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output,
+                              float p, bool values_only, ldist_stream_t stream) {
     if (!input || !weight || !output || !valid_p(p)) return LDIST_EINVAL;
     ldist::Problem pr{};
     if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
-    return finish(ldist::norm_forward(input, weight, output, p, pr, (hipStream_t)stream));
+    return finish(ldist::norm_forward(input, weight, output, p, pr, values_only, (hipStream_t)stream));
+}
+
+int ldist_norm_dist_forward(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
+                            float* output, float p, ldist_stream_t stream) {
+    return norm_forward_entry(input, weight, B, CO, CI, G, HW, output, p, false, stream);
+}
+
+int ldist_norm_dist_forward_values(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
+                                   float* output, float p, ldist_stream_t stream) {
+    return norm_forward_entry(input, weight, B, CO, CI, G, HW, output, p, true, stream);
 }
 
 int ldist_norm_dist_backward_input(const float* grad_output, const float* input, const float* weight,

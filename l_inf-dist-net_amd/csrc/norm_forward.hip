@@ -87,8 +87,13 @@ struct NormForward {
     }
 };
 
+// `values_only`: no gradient follows.  Such a pass may sum in any order and takes whichever kernel is fastest for the
+// size.  A forward pass that trains keeps the order of summation it has always had (chunks of 32 k, alternating between
+// the k-groups of the tile that fits the size): the batch-mean shift behind a layer of nearly equal distances leaves small
+// differences of large numbers, and one unit in the last place of the distances was seen a thousand times as large in the
+// gradients of a five-layer net.
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
-                        hipStream_t stream) {
+                        bool values_only, hipStream_t stream) {
     if (pr.NG <= kSkinnyMaxNG) {
         const Dims d = make_dims(pr);
         const bool vec = pr.HW == 1 && pr.K % 4 == 0 && aligned16(input) && aligned16(weight);
@@ -105,6 +110,8 @@ hipError_t norm_forward(const float* input, const float* weight, float* output, 
 #undef LDIST_LAUNCH_RW
         return hipGetLastError();
     }
+    if (const int tile = values_only || g_tile_override >= 10 ? small_forward_tile(pr, ForwardKind::kNorm, p) : -1; tile >= 0)
+        return norm_forward_small(input, weight, output, p, pr, tile, stream);
     return dispatch_forward<NormForward>(pr, can_vec4(pr, input, weight), can_vec4_out(pr, output), stream, input,
                                          weight, output, p);
 }

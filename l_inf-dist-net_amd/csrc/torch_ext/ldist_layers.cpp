@@ -113,7 +113,8 @@ Sizes sizes_of(const Tensor& x, const Tensor& w, int64_t G) {
 }
 Tensor sum_per_channel(const Tensor& g) { return g.dim() == 2 ? g.sum(0) : g.sum(at::IntArrayRef{0, 2}); }
 
-// No gradient follows: the argmax that the forward with gradients records has no reader.
+// No gradient follows: the argmax that the forward with gradients records has no reader, and p-norm sums may be taken in
+// any order.
 Tensor distances(const On& on, const Tensor& x, const Tensor& w, int64_t G, double p) {
     const Sizes s = sizes_of(x, w, G);
     Tensor y = torch::empty(s.output(), x.options());
@@ -127,8 +128,8 @@ Tensor distances(const On& on, const Tensor& x, const Tensor& w, int64_t G, doub
                                                             pos.data_ptr<int32_t>(), on.stream));
         }
     } else {
-        done("norm_dist_forward", ldist_norm_dist_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y), (float)p,
-                                                          on.stream));
+        done("norm_dist_forward_values", ldist_norm_dist_forward_values(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y),
+                                                                        (float)p, on.stream));
     }
     return y;
 }

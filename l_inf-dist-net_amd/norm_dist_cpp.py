@@ -62,6 +62,19 @@ def norm_dist_forward(input, weight, output, G, p):
     _call("ldist_norm_dist_forward", dev, _p(input), _p(weight), B, CO, CI, G, HW, _p(output), float(p))
 
 
+def norm_dist_forward_values(input, weight, output, G, p):
+    """norm_dist_forward for a forward pass that no gradient follows: free to sum in the order of whichever kernel is
+    fastest for the size (no counterpart in the reference)."""
+    for t, n in ((input, "input"), (weight, "weight"), (output, "output")):
+        _check_input(t, n)
+    dev = _same_device(input, weight, output)
+    B, CO, CI, HW = input.size(0), output.size(1), input.size(1), input.size(2)
+    _expect(input.dim() == 3 and output.dim() == 3 and weight.dim() == 2, "input/output must be 3-D, weight 2-D")
+    _expect(weight.size(0) == CO and weight.size(1) * G == CI, "weight must be (CO, CI/G)")
+    _expect(output.size(0) == B and output.size(2) == HW, "output must be (B, CO, HW)")
+    _call("ldist_norm_dist_forward_values", dev, _p(input), _p(weight), B, CO, CI, G, HW, _p(output), float(p))
+
+
 def norm_dist_backward_input(grad_output, input, weight, output, grad_input, G, p):
     """model/norm_dist.cpp:30-40."""
     for t, n in ((grad_output, "grad_output"), (input, "input"), (weight, "weight"), (output, "output"),
