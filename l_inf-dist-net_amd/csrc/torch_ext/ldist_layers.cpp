@@ -359,6 +359,7 @@ struct NormImageLayer : public Function<NormImageLayer> {
 // ---- what Python calls -------------------------------------------------------------------------------------------
 // Tensors arrive contiguous or are made so where the Python route does the same; p is checked there too.
 Tensor norm_dist(const Tensor& x, const Tensor& w, int64_t G, double p) {
+    TORCH_CHECK(x.dim() == 3 && w.dim() == 2, "input must be 3-D, weight 2-D");
     check(x, "input", x.device());
     check(w, "weight", x.device());
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w)))
@@ -371,6 +372,7 @@ std::tuple<Tensor, Tensor> inf_dist_bound(const Tensor& lower, const Tensor& upp
     check(upper, "input_upper", lower.device());
     check(w, "weight", lower.device());
     TORCH_CHECK(lower.sizes() == upper.sizes(), "input_upper must match input_lower");
+    TORCH_CHECK(w.dim() == 2 || w.dim() == 4, "weight must be (CO, CI/G)");
     const On on(lower);
     const Sizes s = sizes_of(lower, w, G);
     Tensor lo = torch::empty(s.output(), lower.options()), hi = torch::empty_like(lo);
@@ -402,14 +404,30 @@ Tensor as_output(const Tensor& y, const Tensor& x, const Window& win) {
     return y.view({y.size(0), y.size(1), ho, wo});
 }
 
+// The weight of a layer on x (B, CI, H, W) or (B, CI) is (CO, CI/G, k, k): the kernels that read the image take its
+// channels from the image and the reduction's length from the window, so both have to agree with what the weight holds.
+void check_weight(const Tensor& w, const Tensor& x, int64_t G, const Window& win) {
+    check(w, "weight", x.device());
+    TORCH_CHECK(x.dim() == 4 || (x.dim() == 2 && win.trivial()), "input must be (B, C, H, W), or (B, C) without a window");
+    TORCH_CHECK(G > 0 && w.dim() == 4 && w.size(1) * G == x.size(1) && w.size(2) == win.k && w.size(3) == win.k,
+                "weight must be (CO, CI/G, k, k) with as many input channels as the input has");
+}
+
+void check_per_channel(const OptTensor& t, const char* name, const Tensor& w) {
+    if (!t.has_value()) return;
+    check(*t, name, w.device());
+    TORCH_CHECK(t->numel() == w.size(0), name, " must hold one value per output channel");
+}
+
 // Values of a layer: x (B, CI, H, W) or, fully connected, (B, CI); weight (CO, CI/G, k, k).  Returns (y, whether it came straight from the image).
 std::tuple<Tensor, bool> layer(const Tensor& x, const Tensor& weight, const OptTensor& bias, const OptTensor& running,
                                double momentum, bool training, int64_t G, double p, int64_t k, int64_t stride, int64_t pad,
                                int64_t dil, bool finite_p_from_image, int64_t folded_max_row) {
     const Window win{k, stride, pad, dil};
     const Tensor w = weight.contiguous();
-    check(w, "weight", x.device());
-    if (bias.has_value()) check(*bias, "bias", x.device());
+    check_weight(w, x, G, win);
+    check_per_channel(bias, "bias", w);
+    check_per_channel(running, "running_mean", w);
     const Shift shift = make_shift(running, momentum, training, x.device());
     const bool inf = std::isinf(p), grad = at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w) || wants_grad(bias));
     bool from_image = false;
@@ -454,7 +472,9 @@ std::tuple<Tensor, Tensor, bool> layer_bounds(const Tensor& lower, const Tensor&
     at::NoGradGuard no_grad;
     const Window win{k, stride, pad, dil};
     const Tensor w = weight.contiguous();
-    if (bias.has_value()) check(*bias, "bias", lower.device());
+    check_weight(w, lower, G, win);
+    check_per_channel(bias, "bias", w);
+    check_per_channel(running, "running_mean", w);
     const Shift shift = make_shift(running, 0.0, false, lower.device());
     const On on(lower);
     Tensor lo, hi;
@@ -493,8 +513,9 @@ std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Ten
     check(cx, "input", w.device());
     check(cl, "input_lower", w.device());
     check(cu, "input_upper", w.device());
-    if (bias.has_value()) check(*bias, "bias", w.device());
-    if (running.has_value()) check(*running, "mean", w.device());
+    check_weight(w, x, G, Window{1, 1, 0, 1});
+    check_per_channel(bias, "bias", w);
+    check_per_channel(running, "mean", w);
     TORCH_CHECK(cl.sizes() == cx.sizes() && cu.sizes() == cx.sizes(), "input_lower and input_upper must match input");
     const On on(cx);
     const Sizes s = sizes_of(cx, w, G);

@@ -40,10 +40,11 @@ class BoundFinalIdentity(nn.Module):
     def forward(self, x, lower=None, upper=None, targets=None):
         if lower is None or upper is None or targets is None:
             return x
-        if (norm_dist_cpp.layer_ops is not None and upper.is_cuda and upper.dim() == 2 and
+        ops = norm_dist_cpp.native_ops()
+        if (ops is not None and upper.is_cuda and upper.dim() == 2 and upper.numel() > 0 and
                 lower.dtype == upper.dtype == torch.float32 and targets.dtype == torch.int64 and
                 lower.shape == upper.shape and targets.numel() == upper.size(0)):
-            return x, norm_dist_cpp.layer_ops.margins(lower, upper, targets)   # one kernel instead of four
+            return x, ops.margins(lower, upper, targets)   # one kernel instead of four
         at = targets.view(-1, 1)
         margins = upper - lower.gather(1, at)          # every class's upper bound against the label's lower bound
         return x, margins.scatter(1, at, 0.0)

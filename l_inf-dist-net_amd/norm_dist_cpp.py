@@ -554,6 +554,16 @@ def use_native_layers(on=True):
     return layer_ops
 
 
+def native_ops():
+    """`layer_ops`, or None where a transformation has to see every operation of a call: forward-mode differentiation,
+    tracing, functorch.  The native path makes its library calls behind torch's back; the Python route's autograd
+    functions and torch expressions take part in these or refuse them."""
+    if (layer_ops is None or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None or
+            torch._C._are_functorch_transforms_active()):
+        return None
+    return layer_ops
+
+
 try:
     if torch_extension() is not None:
         use_torch_extension(True)

@@ -142,3 +142,64 @@ def test_attack_and_optimizer_agree(both_routes):
         return [adv, torch.tensor(got)] + [prm.detach() for prm in net.parameters()] + list(net.buffers())
     a, b = both_routes(run)
     _same(a, b)
+
+
+def test_a_layer_refuses_an_input_of_other_channels_than_its_weight():
+    for k, c in ((3, 12), (3, 4), (1, 12), (1, 4)):
+        layer = pkg.NormDistConv(8, 8, k, padding=k // 2, p=INF, bias=False).to(DEV).eval()
+        x = torch.rand(2, c, 6, 6, device=DEV)
+        for p in (INF, 8.0):
+            layer.p = p
+            with pytest.raises((RuntimeError, AssertionError)):
+                layer(x)
+        layer.p = INF
+        with torch.no_grad(), pytest.raises((RuntimeError, AssertionError)):
+            layer(x, x, x)
+
+
+def test_vectors_that_are_not_one_value_per_channel_take_the_python_route(both_routes):
+    layer = pkg.NormDist(12, 8, p=INF, bias=True, mean_normalize=True).to(DEV).eval()
+    layer.bias = torch.nn.Parameter(torch.tensor([0.75], device=DEV))            # broadcasts over the channels
+    layer.normalize.running_mean = torch.arange(16.0, device=DEV)[::2]          # strided
+    x = torch.rand(4, 12, generator=gen(12)).to(DEV)
+    a, b = both_routes(lambda: [t.detach() for t in layer(x, x - 0.1, x + 0.1)])
+    _same(a, b)
+
+
+def test_bounds_carry_the_gradient_of_the_bias(both_routes):
+    layer = pkg.NormDist(12, 8, p=INF, bias=True).to(DEV).eval()
+    x = torch.rand(4, 12, generator=gen(13)).to(DEV)
+
+    def run():
+        layer.bias.grad = None
+        y, lo, hi = layer(x, x - 0.1, x + 0.1)
+        (2 * lo.sum() + 3 * hi.sum()).backward()
+        return [y.detach(), lo.detach(), hi.detach(), layer.bias.grad]
+    a, b = both_routes(run)
+    _same(a, b)
+    assert torch.equal(a[3], torch.full((8,), 20.0, device=DEV))
+
+
+def test_transformations_see_every_operation():
+    import torch.autograd.forward_ad as fwd
+    layer = pkg.NormDist(12, 8, p=8.0, bias=False).to(DEV)
+    for prm in layer.parameters():
+        prm.requires_grad_(False)
+    x = torch.rand(4, 12, device=DEV)
+    with fwd.dual_level(), pytest.raises(RuntimeError):        # no forward derivative: refused, not dropped
+        layer(fwd.make_dual(x, torch.ones_like(x)))
+    lo, up = torch.rand(3, 5, 10, device=DEV), torch.rand(3, 5, 10, device=DEV)
+    t = torch.randint(0, 10, (5,), device=DEV)
+    margins = pkg.BoundFinalIdentity()
+    got = torch.func.vmap(lambda a, b: margins(a, a, b, t)[1])(lo, up)
+    assert torch.equal(got, torch.stack([margins(a, a, b, t)[1] for a, b in zip(lo, up)]))
+
+
+def test_empty_batches_and_other_dimensions():
+    none = torch.empty(0, 10, device=DEV)
+    assert pkg.BoundFinalIdentity()(none, none, none, torch.empty(0, dtype=torch.int64, device=DEV))[1].shape == (0, 10)
+    x, w = torch.rand(4, 12, device=DEV), torch.rand(8, 12, device=DEV)
+    with pytest.raises((RuntimeError, IndexError)):
+        pkg.norm_dist(x, w, 1, INF)
+    with pytest.raises((RuntimeError, IndexError)):
+        pkg.norm_dist(x.view(4, 12, 1), w.view(8, 12, 1, 1), 1, INF)
