@@ -60,10 +60,9 @@ LDIST_API int ldist_last_hip_error(void);
  * 0..4 also keep the L_inf forward of an unfolded-conv layout on the tiled kernels
  * where it would otherwise take the kernel that holds a tile's whole reduction axis
  * in LDS (K up to 320), and 0 / 1 force the register-tiled p-norm backward kernels
- * (128x80 / 128x64 tiles), the one-pass kernel of ldist_norm_dist_backward included,
- * 2 / 3 / 4 keep them off; 5 forces that one-pass kernel on with 128x48 tiles (its third
- * width, which it otherwise takes where the wider ones leave CUs idle) and is like 2
- * for every other kernel.  10..16 force the seven small tiles (32x80, 32x40, 16x40, 32x64, 32x32, 16x32, 64x80) and 30 the
+ * (128x80 / 128x64 tiles), the one-pass kernel of ldist_norm_dist_backward (which has
+ * one width) included, 2 / 3 / 4 keep them off; 5 forces that one-pass kernel on and is
+ * like 2 for every other kernel.  10..16 force the seven small tiles (32x80, 32x40, 16x40, 32x64, 32x32, 16x32, 64x80) and 30 the
  * few-rows kernel of the fully connected forward passes with more than 16 outputs per group and at least 4 inputs, which
  * otherwise are chosen by an estimate of their time.  Process-wide; not thread safe. */
 LDIST_API int ldist_set_tile_override(int choice);

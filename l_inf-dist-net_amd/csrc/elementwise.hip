@@ -44,6 +44,20 @@ static unsigned lanes_grid(unsigned total, int num_cu) {
     return blocks < most ? blocks : most;
 }
 
+__global__ void __launch_bounds__(256) zero_fill_kernel(float* __restrict__ p, size_t n, bool vec) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (vec && i + 3 < n) {
+        *reinterpret_cast<float4*>(p + i) = make_float4(0.f, 0.f, 0.f, 0.f);
+    } else {
+        for (size_t j = i; j < n && j < i + 4; j++) p[j] = 0.f;
+    }
+}
+
+hipError_t zero_fill(float* p, size_t n, hipStream_t stream) {
+    hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, stream, p, n, aligned16(p));
+    return hipGetLastError();
+}
+
 hipError_t channel_shift(const float* x, const float* mean, const float* bias, float* y, int B, int C, int L, int num_cu,
                          hipStream_t stream) {
     const unsigned n = (unsigned)B * C * L;

@@ -133,6 +133,7 @@ hipError_t adamw_lp_step(float* param, const float* grad, float* exp_avg, float*
                          hipStream_t stream);
 
 // The small elementwise operations around the layers (elementwise.hip).
+hipError_t zero_fill(float* p, size_t n, hipStream_t stream);   // a kernel, so that the call can be captured in a graph
 hipError_t channel_shift(const float* x, const float* mean, const float* bias, float* y, int B, int C, int L, int num_cu,
                          hipStream_t stream);
 hipError_t certified_margins(const float* lower, const float* upper, const int64_t* targets, float* margins, int B, int J,

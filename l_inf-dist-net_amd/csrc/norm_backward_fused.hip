@@ -6,18 +6,28 @@
 // the other instructions), and that is what bounds either gradient; sharing the term between the two sums takes
 // 4.2 ms on 512 x 5120 -> 5120 at p = 20.5 where the two separate kernels take 3.6 + 3.1 ms.
 //
-// The kernel has the shape of the register-tiled grad_input kernel: a workgroup owns 128 rows m x BN inputs k and
-// walks the outputs n; a lane keeps an 8 x TN patch of x and of the grad_input sums (BN x TN = 80 x 5, 64 x 4 or
-// 48 x 3: the host takes the width whose tiles fill the device best).  For grad_weight the lane
-// also adds, per output n, its eight rows' terms of each of its TN columns (one more fused multiply-add per term),
-// the sixteen lanes that share those columns (one DPP row: the lane index runs along m first here) add their
-// partial sums over each half of the row with three row shifts, the halves' last lanes park the two totals of the
-// tile's 128 rows in two LDS tiles [stage's outputs][BN], and once per stage the whole workgroup adds the tiles'
-// sum onto grad_weight with float atomics
-// (64 consecutive columns per instruction).  grad_weight therefore collects one addend per tile of 128 rows, in no
+// The kernel has the shape of the register-tiled grad_input kernel: a workgroup owns 64 rows m x 64 inputs k and
+// walks its share of the outputs n; a lane keeps an 8 x 4 patch of x and of the grad_input sums.  For grad_weight the
+// lane also adds, per output n, its eight rows' terms of each of its four columns (one more fused multiply-add per
+// term), the eight lanes that share those columns (half a DPP row: the lane index runs along m first here) add their
+// partial sums with three row shifts, the last of them parks the total of the tile's 64 rows in an LDS tile
+// [stage's outputs][64], and once per stage the whole workgroup adds the tile onto grad_weight with float atomics
+// (64 consecutive columns per instruction).  grad_weight therefore collects one addend per tile of 64 rows, in no
 // fixed order, and must be zero-filled (or hold the values to accumulate onto) by the caller, as with the separate
 // call.  IE = 0: any p > 2; the power is taken of the normalised difference (x - w) / out, which never leaves the
 // float range.
+//
+// Tiles of 64 x 64, two workgroups of 256 lanes per CU, outputs shared out.  A CU does 8.2 k differences of a stage
+// in 22 us (p = 8; p = 37.3: 36) with two workgroups on it and needs 20 (24) for half of them with a single one, so a
+// launch should put an even number on every CU: the tiles of a problem are multiplied by splitting the outputs over
+// `splits` workgroups, whose grad_input sums meet by float atomics in a zero-filled grad_input.  Against tiles of
+// 128 x 80, 128 x 64 and 128 x 48 with one 512-lane workgroup per CU that walked all outputs, and the two separate
+// kernels where those did not fill the device (rows x inputs -> outputs, us, both gradients):
+//   512 x 5120 -> 5120   p = 8 2250 -> 2270, p = 37.3 3930 -> 3660, p = 300 4450 -> 4170, p = 4 1890 -> 1870
+//   512 x 3072 -> 5120   p = 8 1500 -> 1380, p = 37.3 2490 -> 2240
+//   64 x 5120 -> 5120    p = 8 520 -> 333, p = 37.3 906 -> 517 (both separate ones split as well; 2140 before that)
+//   200 x 2048 -> 2048   p = 8 298 -> 202, p = 37.3 538 -> 321;   100 x 1024 -> 1024  60 -> 39, 92 -> 54
+// Tiles of 64 x 80 spill (104 bytes of scratch; 2370 at p = 8 on the first), 64 x 48 pay for fewer terms per LDS word (2520).
 //
 // IE = p - 1 for the multiply-only exponents (1, 2, 3, 7).  There the two register-tiled kernels of
 // norm_backward_tiled.hip each spend a subtraction and the multiplications of the power on every term before their
@@ -25,11 +35,8 @@
 // instructions per term for both sums, counted in the loop, instead of 7.1 + 6.5), and x, w, g and out are staged
 // once.  As in those kernels the power is taken of the raw difference with F = g / out^(p-1) staged in place of g,
 // and a stage that holds an output outside [2^-12, 2^12] is reduced the careful way from g and 1/out.  The loop does
-// not fetch the next row's operands ahead: with a second fragment in flight the kernel spills, and what it spills it
-// reloads behind the stage's global loads, so that every wait for a reloaded value waits for those as well (measured:
-// no faster than this form).  What keeps it from the rate its instruction count promises (1.6 ms at p = 8) is the
-// time its waves do not issue arithmetic: 20 % of it at waits (each row's LDS fetch, the stage's loads), as much again
-// at the stage's barriers, the conversion and the flush, which nothing overlaps with one workgroup per CU.
+// not fetch the next row's operands ahead: the other workgroup on the CU covers the LDS fetch, the barriers, the
+// conversion and the flush.
 #include "fwd_engine.hpp"
 #include "pow.hpp"
 #include "wave_reduce.hpp"
@@ -40,11 +47,11 @@ template <class GEO, int IE>
 __global__ void __launch_bounds__(GEO::NT, 2)
 norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* __restrict__ input,
                            const float* __restrict__ weight, const float* __restrict__ output,
-                           float* __restrict__ grad_input, float* __restrict__ grad_weight, float e, Dims d) {
+                           float* __restrict__ grad_input, float* __restrict__ grad_weight, float e, Dims d, int n_per_wg, int logs) {
     constexpr int BM = GEO::BM, BN = GEO::BN, TM = GEO::TM, TN = GEO::TN, KS = GEO::KS, KK = GEO::KK;
     constexpr int NGRP = GEO::NGRP, NT = GEO::NT, XS = GEO::XS, WS = GEO::WS;
     constexpr int STAGE = 2 * XS + WS;     // [F or g][1/out][w]
-    static_assert(GEO::TY == 16, "the lanes that share a column fill one DPP row");
+    static_assert(GEO::TY == 8, "the lanes that share a column fill half a DPP row");
     using RowLoad = RowsK<BM, GEO::SM, NT, KK, 4>;   // outputs are contiguous in g and out
     using ColLoad = RowsT<BN, GEO::SN, NT, KK, 4>;
     static_assert((KS - 1) * TM * TN * NGRP <= STAGE, "merge area fits in the panels");
@@ -55,8 +62,9 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
     const int m0 = tm * BM, k0 = tk * BN;
     const int tid = threadIdx.x;
     const int grp = tid / NGRP, t = tid % NGRP;
-    const int ty = t % GEO::TY, tx = t / GEO::TY;    // m first: the 16 lanes of a column group are neighbours
+    const int ty = t % GEO::TY, tx = t / GEO::TY;    // m first: the 8 lanes of a column group are neighbours
     const int K = d.K, NG = d.NG;
+    const int n_begin = blockIdx.y * n_per_wg, n_end = min(NG, n_begin + n_per_wg);   // this workgroup's outputs
 
     // sign(u) * |u|^(p-1).  IE == 0: as u * |u|^(p-2) (the host sends exponents p <= 2 to the separate kernels);
     // u == 0 gives 0
@@ -87,36 +95,30 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
         }
     }
     float* const gw_group = grad_weight + (size_t)g * NG * K;
-    // The lane's column sums of output n (already summed over its rows) are summed over each half of the 16 lanes
-    // that share the columns (three DPP row shifts; lanes 7 and 15 of the row hold the halves' totals) and parked in
-    // two LDS tiles [stage's outputs][BN columns], one per half; the sign: d/dw of |x - w| is minus d/dx.  The fourth
-    // shift, which would join the halves, costs more than the second tile: a DPP instruction takes 4.4 clocks, the
-    // twenty-five of a step (five sums) were a quarter of the p = 8 launch, and without the last level 2.51 -> 2.28 ms
-    // on 512 x 5120 -> 5120.  (LDS float atomics from the four quarter totals instead: 3.13 ms.)  The tiles go
-    // onto grad_weight once per stage (flush_weight_tile): straight from here an atomic instruction had four active
-    // lanes (the last lane of each row of sixteen), and the float atomics of a 5120-wide layer, 105 M in 26 M
-    // instructions, took 1.7 ms of the launch's 4.2.
-    float* const Gs = lds + 2 * XS + GEO::WS;   // 2 x [KK][BN], all zero between stages
+    // The lane's column sums of output n (already summed over its rows) are summed over the eight lanes that share the
+    // columns (three DPP row shifts of 4.4 clocks each, 12 per 32 terms) and parked by the last of them; the sign: d/dw
+    // of |x - w| is minus d/dx.  The tile goes onto grad_weight once per stage (flush_weight_tile): straight from here
+    // an atomic instruction had four active lanes, and the float atomics of a 5120-wide layer, 105 M in 26 M
+    // instructions, took 1.7 ms of a launch of 4.2.
+    float* const Gs = lds + 2 * XS + GEO::WS;   // [KK][BN], all zero between stages
     auto add_weight_row = [&](int n_local, const float (&s)[TN]) {
         float tot[TN];
 #pragma unroll
         for (int j = 0; j < TN; j++) tot[j] = dpp_lanes_total<8>(s[j]);
-        if ((ty & 7) == 7) {
-            float* half = Gs + (ty >> 3) * (KK * BN);
+        if (ty == 7) {
 #pragma unroll
-            for (int j = 0; j < TN; j++) half[n_local * BN + GEO::col(tx, j)] = -tot[j];
+            for (int j = 0; j < TN; j++) Gs[n_local * BN + GEO::col(tx, j)] = -tot[j];
         }
     };
-    // All lanes of the workgroup: 64 consecutive columns of one output per wave instruction; two parked zeros (nothing
-    // added: padding, or a row the large-exponent path passed over) cost no atomic.  Leaves the tiles zero.
+    // All lanes of the workgroup: 64 consecutive columns of one output per wave instruction; a parked zero (nothing
+    // added: padding, or a row the large-exponent path passed over) costs no atomic.  Leaves the tile zero.
     auto flush_weight_tile = [&](int n_first) {
         for (int i = tid; i < KK * BN; i += GEO::NT) {
-            const float a = Gs[i], b = Gs[i + KK * BN];
-            if (a != 0.f || b != 0.f) {
+            const float a = Gs[i];
+            if (a != 0.f) {
                 Gs[i] = 0.f;
-                Gs[i + KK * BN] = 0.f;
                 const int nl = i / BN, c = i - nl * BN;
-                if (n_first + nl < NG && k0 + c < K) atomicAdd(gw_group + (size_t)(n_first + nl) * K + k0 + c, a + b);
+                if (n_first + nl < n_end && k0 + c < K) atomicAdd(gw_group + (size_t)(n_first + nl) * K + k0 + c, a);
             }
         }
     };
@@ -144,7 +146,7 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
             static_assert(RowLoad::PER_ROW == 16 && NT % RowLoad::PER_ROW == 0, "a lane keeps its outputs over the rounds");
             const int row0 = lane / RowLoad::PER_ROW, nq = (lane % RowLoad::PER_ROW) * 4;
             const unsigned ldb = 4u * (unsigned)(d.G * NG);
-            const bool n_ok = n_first + nq < NG;                      // NG % 4 == 0: a vector is inside or outside
+            const bool n_ok = n_first + nq < n_end;                   // NG % 4 == 0: a vector is inside or outside
             const int rows_valid = d.M - m0;
 #pragma unroll
             for (int i = 0; i < RowLoad::N; i++) {
@@ -163,7 +165,7 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
             for (int i = 0; i < ColLoad::N; i++) {
                 const int id = lane + i * NT;
                 const int rr = id / ColLoad::PER_ROW, cq = id - rr * ColLoad::PER_ROW;
-                const bool ok = (ColLoad::TOTAL % NT == 0 || id < ColLoad::TOTAL) && n_first + rr < NG && k0 + cq * 4 < K;
+                const bool ok = (ColLoad::TOTAL % NT == 0 || id < ColLoad::TOTAL) && n_first + rr < n_end && k0 + cq * 4 < K;
                 const unsigned o = ok ? 4u * ((unsigned)rr * (unsigned)K + (unsigned)cq * 4u) : ~0u;
                 const F4 t = __builtin_bit_cast(F4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, o, 0, 0));
                 wl.v[i][0] = t.x; wl.v[i][1] = t.y; wl.v[i][2] = t.z; wl.v[i][3] = t.w;
@@ -171,7 +173,7 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
         }
     };
     // every (row, output) pair has its own largest term among its K differences, and a row of the test holds
-    // 16 pairs x 4 TN columns per wave: with a short K most rows hold one and the tests only cost
+    // 8 pairs x 8 TN columns per wave: with a short K most rows hold one and the tests only cost
     const bool sparse = e >= 63.0f && K >= 1024;
     const float cut = __builtin_exp2f(-36.0f / e);
     // General exponent without the tests: the term g * u * |u|^(p-2), u = (x - w) / out, can be taken as
@@ -190,7 +192,7 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
     // the largest and the smallest output of the first stage, the lane's patch of x and every stage's weights are taken in that unit
     // (exact: powers of two), and so are the outputs, so that data of any overall magnitude takes the logarithmic
     // form; a layer whose outputs differ by more than the window does not.
-    const bool logscale = IE == 0 && !sparse;
+    const bool logscale = IE == 0 && logs;
     float unit_inv = 1.0f;   // 1 / unit
     // Turns the parked out values into what the panel holds: 1/out, and 0 where nothing was loaded (padding loads g
     // and out as 0; a real 0 output gives inf like the reference), so that padding multiplies by 0, not by infinity.
@@ -245,29 +247,12 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
     auto store = [&]() {
         gk.store(lds, tid);
         ok_.store(lds + XS, tid);
-        if constexpr (TN == 3) {
-            // three columns per lane at a pitch of four in the panel, so that the sweep's 128-bit reads stay as they
-            // are: column c of the tile lives at word (c / 3) * 4 + c % 3 of its panel row
-            float* panel = lds + 2 * XS;
-#pragma unroll
-            for (int i = 0; i < ColLoad::N; i++) {
-                const int id = tid + i * NT;
-                if (ColLoad::TOTAL % NT != 0 && id >= ColLoad::TOTAL) continue;
-                const int rr = id / ColLoad::PER_ROW, cq = id - rr * ColLoad::PER_ROW;
-#pragma unroll
-                for (int c4 = 0; c4 < 4; c4++) {
-                    const int c = cq * 4 + c4, third = c / 3;
-                    panel[rr * GEO::SN + ((third * 4 + (c - third * 3)) ^ swz(rr))] = wl.v[i][c4];
-                }
-            }
-        } else {
-            wl.store(lds + 2 * XS, tid);
-        }
+        wl.store(lds + 2 * XS, tid);
     };
 
-    const int nstage = (NG + KK - 1) / KK;
-    for (int i = tid; i < 2 * KK * BN; i += GEO::NT) Gs[i] = 0.f;
-    load(0);
+    const int nstage = (n_end - n_begin + KK - 1) / KK;
+    for (int i = tid; i < KK * BN; i += GEO::NT) Gs[i] = 0.f;
+    load(n_begin);
     if (logscale) {
         float top = 0.f, nbot = -__builtin_inff();   // the largest and minus the smallest output this lane loaded
 #pragma unroll
@@ -312,7 +297,7 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
     store();
     __syncthreads();
     for (int s = 0; s < nstage; s++) {
-        if (s + 1 < nstage) load((s + 1) * KK);
+        if (s + 1 < nstage) load(n_begin + (s + 1) * KK);
         const float* fp = lds + grp * kChunk * GEO::SM;
         const float* wp = lds + 2 * XS + grp * kChunk * GEO::SN;
         // No operand prefetch: a second fragment in flight does not fit next to the patch, the sums and the weight
@@ -419,7 +404,7 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
         // stage's outputs rides on the same barrier
         if (IE > 0 || logscale) factored = !__syncthreads_or(s + 1 < nstage ? out_of_range() : false);
         else __syncthreads();
-        flush_weight_tile(s * KK);
+        flush_weight_tile(n_begin + s * KK);
         if (s + 1 < nstage) {
             convert(factored);
             scale_weights();
@@ -447,27 +432,68 @@ norm_backward_fused_kernel(const float* __restrict__ grad_output, const float* _
         }
         __syncthreads();
     }
-    if (grp == 0) {
+    if (gridDim.y > 1) {   // several workgroups hold parts of the tile's sums: added up in grad_input, which was zero-filled
+        if (grp == 0) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) lds[GEO::row(ty, i) * BN + GEO::col(tx, j)] = acc[i][j];
+        }
+        __syncthreads();
+        for (int i = tid; i < BM * BN; i += NT) {   // a wave instruction covers consecutive columns
+            const int r = i / BN, c = i - r * BN;
+            if (m0 + r < d.M && k0 + c < K) atomicAdd(grad_input + ((size_t)(m0 + r) * d.G + g) * K + k0 + c, lds[i]);
+        }
+    } else if (grp == 0) {
         Dims od = d;
         od.NG = K;   // the result has the input's shape: K columns per group
         store_patch<GEO, false>(grad_input, acc, od, m0, k0, g, tx, ty, d.ovec != 0);
     }
 }
 
-template <class GEO, int IE>
+using FusedGeo = Geo<64, 64, 8, 4, 2>;
+
+// Whether the general exponent may take the logarithmic form, which is 8 % faster and whose error against 64 bits is up
+// to 6 % larger than that of the divided difference (64 x 1024 -> 1024: 2.84e-6 and 2.89e-6 at p = 37.3; 33 x 3072 -> 640:
+// 4.65e-6 and 4.95e-6 at p = 62): layers large enough to count, below the exponents at which a term carries too much
+// of the logarithms' rounding.
+static bool logarithmic_form(const Problem& pr, float p) {
+    const long columns = (long)((pr.B + 127) / 128) * ((pr.K + 47) / 48) * pr.G;   // of 48 inputs, per 128 rows
+    return p < 64.0f && columns * 10 >= 7L * pr.num_cu && pr.NG >= 256;
+}
+
+template <int IE>
 static hipError_t launch_fused(const Problem& pr, hipStream_t stream, const float* grad_output, const float* input,
                                const float* weight, const float* output, float* grad_input, float* grad_weight, float p) {
+    using GEO = FusedGeo;
     Dims d = make_dims(pr);
     d.ovec = 1;   // the result has the input's shape: K % 4 == 0, aligned
     d.tiles_m = (d.M + GEO::BM - 1) / GEO::BM;
     d.tiles_n = (d.K + GEO::BN - 1) / GEO::BN;
-    const unsigned grid = (unsigned)d.tiles_m * d.tiles_n * d.G;
-    constexpr size_t lds = (size_t)(2 * GEO::XS + GEO::WS + 2 * GEO::KK * GEO::BN) * sizeof(float);   // panels, the two grad_weight tiles
+    const long tiles = (long)d.tiles_m * d.tiles_n * d.G;
+    // How many workgroups share a tile's outputs: the number with the shortest estimate of the busiest CU's time, which
+    // takes its workgroups in pairs and a last one alone at half the rate and less (`alone`: its share of a pair's time),
+    // each with about a third of a stage for what it does once.
+    const int stages = (d.NG + GEO::KK - 1) / GEO::KK;
+    const double alone = IE == 0 ? 0.65 : 0.87;
+    int splits = 1;
+    double best = 1e300;
+    for (int s = 1; s <= stages && s <= 64; s++) {
+        const int per_wg = (stages + s - 1) / s;
+        if (s > 1 && (stages + per_wg - 1) / per_wg != s) continue;   // the same shares as a smaller number gives
+        const long on_cu = (tiles * s + pr.num_cu - 1) / pr.num_cu;
+        const double cost = (per_wg + 0.35) * ((double)(on_cu / 2) + (on_cu % 2) * alone);
+        if (cost < best) { best = cost; splits = s; }
+    }
+    const int per_wg = (stages + splits - 1) / splits;
+    constexpr size_t lds = (size_t)(2 * GEO::XS + GEO::WS + GEO::KK * GEO::BN) * sizeof(float);   // panels, the grad_weight tile
     auto kern = norm_backward_fused_kernel<GEO, IE>;
     static LdsRecord lds_allowed = {};
     if (hipError_t e = allow_lds(kern, lds, pr.device, lds_allowed); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(GEO::NT), lds, stream, grad_output, input, weight, output, grad_input,
-                       grad_weight, p - 1.0f, d);
+    if (splits > 1)
+        if (hipError_t e = zero_fill(grad_input, (size_t)d.M * d.G * d.K, stream); e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)splits), dim3(GEO::NT), lds, stream, grad_output, input, weight,
+                       output, grad_input, grad_weight, p - 1.0f, d, per_wg * GEO::KK, logarithmic_form(pr, p));
     return hipGetLastError();
 }
 
@@ -478,59 +504,41 @@ static int fused_int_power(float p) {
 }
 
 // Whether the one-pass kernel takes the problem: the fc layout, every panel loadable with 128-bit loads, and a shape
-// that fills the device with 128-row tiles (the rest stays with the two separate kernels).
+// whose tiles are not mostly padding (the rest stays with the two separate kernels).
 bool norm_backward_fused_applicable(const Problem& pr, float p, const void* grad_output, const void* input,
                                     const void* weight, const void* output, const void* grad_input,
                                     const void* grad_weight) {
-    if (fused_int_power(p) == 0 && !(p > 2.0f)) return false;   // the general kernel takes sign(u) |u|^(p-1) as u |u|^(p-2)
+    const int ie = fused_int_power(p);
+    if (ie == 0 && !(p > 2.0f)) return false;   // the general kernel takes sign(u) |u|^(p-1) as u |u|^(p-2)
     if (pr.HW != 1 || pr.K % 4 != 0 || pr.NG % 4 != 0) return false;
-    // a lane addresses its vectors by 32-bit byte offsets from its tile's first row: 128 rows of G * NG elements of g
+    // a lane addresses its vectors by 32-bit byte offsets from its tile's first row: 64 rows of G * NG elements of g
     // and out, 64 rows of K weights
     if (4LL * 130 * pr.G * pr.NG >= (1LL << 31) || 4LL * 66 * pr.K >= (1LL << 31)) return false;
     if (!(aligned16(grad_output) && aligned16(input) && aligned16(weight) && aligned16(output) && aligned16(grad_input) &&
           aligned16(grad_weight)))
         return false;
-    if (g_tile_override == 0 || g_tile_override == 1 || g_tile_override == 5) return true;   // tests and tuning: forced on (128 x 80, 128 x 64, 128 x 48)
-    if (g_tile_override >= 2) return false;                          // forced off
+    if (g_tile_override == 0 || g_tile_override == 1 || g_tile_override == 5) return true;   // tests and tuning: forced on
+    if (g_tile_override >= 2) return false;                                                // forced off
     // p = 2: a term is one instruction and sharing it saves less than the row sums of grad_weight cost (512 x 5120 ->
-    // 5120: 1.44 against 1.42 ms).  p = 3: 1.65 against 1.83 ms where the tiles fill the device (10240 inputs: 3.30
-    // against 3.71 ms), a tie at 192 tiles of 256 (3072 inputs), a loss at 128.  p = 4: 1.88 against 2.22 ms, p = 8:
-    // 2.27 against 3.06 ms.
-    const int ie = fused_int_power(p);
+    // 5120: 1.44 against 1.42 ms on the two).
     if (ie == 1) return false;
-    const long M = (long)pr.B * pr.HW;
-    const long t48 = ((M + 127) / 128) * ((pr.K + 47) / 48) * pr.G;   // the narrowest tiles: the most workgroups
-    return t48 * 10 >= (ie == 2 ? 9L : 7L) * pr.num_cu && pr.NG >= 256;
-}
-
-template <class GEO>
-static hipError_t launch_fused_for(const Problem& pr, hipStream_t stream, const float* grad_output, const float* input,
-                                   const float* weight, const float* output, float* grad_input, float* grad_weight,
-                                   float p) {
-    switch (fused_int_power(p)) {
-        case 1: return launch_fused<GEO, 1>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-        case 2: return launch_fused<GEO, 2>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-        case 3: return launch_fused<GEO, 3>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-        case 7: return launch_fused<GEO, 7>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-        default: return launch_fused<GEO, 0>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-    }
+    // Few outputs: a stage is 64 of them and takes 20 us at the least, the separate kernels walk 32 in 8.
+    if (pr.NG < 128) return false;
+    // Up to 32 rows fill half a tile here and all of one there.  That shows where the terms and not the latency of a
+    // launch count: 5 x 5120 -> 5120 517 against 462 us at p = 37.3, 331 against 330 at p = 8; 20 x 1024 -> 1024 37
+    // against 76 us.
+    return !(ie == 0 && pr.B <= 32 && (long long)pr.G * pr.NG * pr.K >= (1LL << 23));
 }
 
 hipError_t norm_backward_fused(const float* grad_output, const float* input, const float* weight, const float* output,
                                float* grad_input, float* grad_weight, float p, const Problem& pr, hipStream_t stream) {
-    const long rows = (long)pr.B * pr.HW;
-    // Rounds of workgroups (one per CU) times columns per tile, the narrower tiles charged for what a term costs more
-    // in them (more LDS words and cross-lane steps per term).  3072 inputs at batch 512: 156 tiles of 80 columns, 192
-    // of 64 or 256 of 48 -- only the last fill the 256 CUs.
-    const long rt = (rows + 127) / 128;
-    const long t80 = rt * ((pr.K + 79) / 80) * pr.G, t64 = rt * ((pr.K + 63) / 64) * pr.G, t48 = rt * ((pr.K + 47) / 48) * pr.G;
-    const double c80 = (double)((t80 + pr.num_cu - 1) / pr.num_cu) * 80, c64 = (double)((t64 + pr.num_cu - 1) / pr.num_cu) * 64 * 1.1,
-                 c48 = (double)((t48 + pr.num_cu - 1) / pr.num_cu) * 48 * 1.2;
-    if (g_tile_override == 0 || (g_tile_override != 1 && g_tile_override != 5 && c80 <= c64 && c80 <= c48))
-        return launch_fused_for<Geo<128, 80, 8, 5, 2>>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-    if (g_tile_override == 1 || (g_tile_override != 5 && c64 <= c48))
-        return launch_fused_for<Geo<128, 64, 8, 4, 2>>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
-    return launch_fused_for<Geo<128, 48, 8, 3, 2>>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
+    switch (fused_int_power(p)) {
+        case 1: return launch_fused<1>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
+        case 2: return launch_fused<2>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
+        case 3: return launch_fused<3>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
+        case 7: return launch_fused<7>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
+        default: return launch_fused<0>(pr, stream, grad_output, input, weight, output, grad_input, grad_weight, p);
+    }
 }
 
 }  // namespace ldist

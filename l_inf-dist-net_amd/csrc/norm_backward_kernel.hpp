@@ -277,7 +277,9 @@ norm_backward_kernel(const float* __restrict__ grad_output, const float* __restr
                     size_t off;
                     if (v.x_tap(a, k, off)) atomicAdd(grad + off, acc[i][j]);
                 } else {
-                    grad[v.x_at(a, k)] = acc[i][j];
+                    float* dst = grad + v.x_at(a, k);
+                    if (SPLIT) atomicAdd(dst, acc[i][j]);
+                    else *dst = acc[i][j];
                 }
             }
         }
@@ -293,7 +295,7 @@ static hipError_t launch_norm_backward_ba(const float* grad_output, const float*
     const int tiles_a = (A + BA - 1) / BA, tiles_k = (d.K + BKO - 1) / BKO;
     const long tiles = (long)tiles_a * tiles_k * d.G;
     int splits = 1;
-    if (WEIGHT && tiles < 2L * pr.num_cu) {  // few output tiles, long reduction over the rows: share it out
+    if (tiles < 2L * pr.num_cu) {  // few output tiles, long reduction (over the rows, or the outputs): share it out
         const long want = (4L * pr.num_cu + tiles - 1) / tiles;
         const long most = max(1L, (long)R / (4 * RB));
         splits = (int)min(want, most);
@@ -301,6 +303,8 @@ static hipError_t launch_norm_backward_ba(const float* grad_output, const float*
     int r_per_wg = (R + splits - 1) / splits;
     r_per_wg = (r_per_wg + RB - 1) / RB * RB;
     splits = (R + r_per_wg - 1) / r_per_wg;
+    if (!WEIGHT && !IMG && splits > 1)
+        if (hipError_t e = zero_fill(grad, (size_t)d.M * d.G * d.K, stream); e != hipSuccess) return e;
     const dim3 grid((unsigned)tiles, (unsigned)splits);
     const bool conv = pr.HW != 1;
 #define LDIST_LAUNCH(W, C, S)                                                                                      \
@@ -309,11 +313,9 @@ static hipError_t launch_norm_backward_ba(const float* grad_output, const float*
     if constexpr (IMG) {   // an image always has the conv layout (a single position included)
         (void)conv;
         if (WEIGHT && splits > 1) LDIST_LAUNCH(WEIGHT, true, true); else LDIST_LAUNCH(WEIGHT, true, false);
-    } else if (WEIGHT) {
+    } else {
         if (splits > 1) { if (conv) LDIST_LAUNCH(WEIGHT, true, true); else LDIST_LAUNCH(WEIGHT, false, true); }
         else { if (conv) LDIST_LAUNCH(WEIGHT, true, false); else LDIST_LAUNCH(WEIGHT, false, false); }
-    } else {
-        if (conv) LDIST_LAUNCH(WEIGHT, true, false); else LDIST_LAUNCH(WEIGHT, false, false);
     }
 #undef LDIST_LAUNCH
     return hipGetLastError();

@@ -33,15 +33,6 @@ Problem problem_of(const ConvGeom& q, int G, int CO, int num_cu, int device) {
     return Problem{q.B, G, q.C / G * 9, CO / G, q.HO * q.WO, num_cu, device};
 }
 
-__global__ void __launch_bounds__(256) zero_fill_kernel(float* __restrict__ p, size_t n, bool vec) {
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (vec && i + 3 < n) {
-        *reinterpret_cast<float4*>(p + i) = make_float4(0.f, 0.f, 0.f, 0.f);
-    } else {
-        for (size_t j = i; j < n && j < i + 4; j++) p[j] = 0.f;
-    }
-}
-
 }  // namespace
 
 // 3x3 windows (any stride, padding, dilation) with more than one output position.  Layers with few outputs per
@@ -66,9 +57,7 @@ hipError_t norm_conv_backward_input(const float* grad_output, const float* img, 
                                     int num_cu, int device, hipStream_t stream) {
     const Problem pr = problem_of(q, G, CO, num_cu, device);
     const size_t n = (size_t)q.B * q.C * q.H * q.W;
-    hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, stream, grad_img, n,
-                       aligned16(grad_img));
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    if (hipError_t e = zero_fill(grad_img, n, stream); e != hipSuccess) return e;
     return launch_norm_backward<false, true>(grad_output, img, weight, output, grad_img, p, pr, stream, window_of(q, G));
 }
 

@@ -1,0 +1,51 @@
+"""p-norm gradients whose reduction is shared out over workgroups: the one-pass kernel (csrc/norm_backward_fused.hip) and the
+separate grad_input (csrc/norm_backward_kernel.hpp) at the edges of their tiles and shares, against the oracle: one row to one
+past a tile, outputs that end inside a stage and inside a share, four inputs to one vector past a tile, groups."""
+import pytest
+import torch
+
+import oracle
+from helpers import assert_sum_close, gen, make_inputs
+
+pytestmark = pytest.mark.gpu
+# B, CO, CI, G
+ONE_PASS = [(1, 128, 4, 1), (8, 132, 60, 1), (33, 260, 68, 1), (64, 1028, 64, 1), (65, 196, 132, 1), (7, 280, 128, 2),
+            (129, 644, 4, 1), (2, 4100, 12, 1)]
+SEPARATE = [(1, 300, 5, 1), (33, 1000, 63, 1), (40, 390, 130, 2), (65, 1100, 31, 1), (100, 513, 67, 1)]
+
+
+@pytest.mark.parametrize("p", [3.0, 4.0, 8.0, 37.3, 62.0, 300.0])
+@pytest.mark.parametrize("shape", ONE_PASS + SEPARATE)
+def test_shared_reductions(shape, p):
+    from gpu_common import DEV, cpp, say
+    B, CO, CI, G = shape
+    say("split backward", shape, "p", p)
+    x, w = make_inputs(B, CO, CI, G, 1, seed=sum(shape))
+    go = torch.randn(B, CO, 1, generator=gen(7))
+    out = oracle.norm_dist_forward(x, w, G, p)
+    ex, mx = oracle.norm_dist_backward_input(go, x, w, out, G, p, with_abs_terms=True)
+    ew, mw = oracle.norm_dist_backward_weight(go, x, w, out, G, p, with_abs_terms=True)
+    args = [t.to(DEV) for t in (go, x, w, out)]
+    for both in (True, False):
+        gx = torch.full((B, CI, 1), float("nan"), device=DEV)   # overwritten, whatever it held
+        gw = torch.full((CO, CI // G), 0.125, device=DEV)       # added to
+        if both:
+            cpp.norm_dist_backward(*args, gx, gw, G, p)
+        else:
+            cpp.norm_dist_backward_input(*args, gx, G, p)
+            cpp.norm_dist_backward_weight(*args, gw, G, p)
+        torch.cuda.synchronize()
+        assert_sum_close(gx.cpu(), ex, mx, p, 1e-5, 1e-6)
+        assert_sum_close(gw.cpu() - 0.125, ew, mw, p, 1e-5, 1e-6)
+
+
+# 16 x 32 tiles, 32 x 40 tiles (their busiest CU has least to do there), ragged ends of both
+@pytest.mark.parametrize("p", [2.0, 8.0, 37.3, 200.0])
+@pytest.mark.parametrize("shape", [(17, 33, 260, 1), (100, 1001, 513, 1), (30, 66, 1000, 2), (64, 5117, 300, 1), (61, 5120, 2052, 1)])
+def test_forward_tiles_of_eight_groups(shape, p):
+    from gpu_common import gpu_norm_forward, say
+    B, CO, CI, G = shape
+    say("eight groups", shape, "p", p)
+    x, w = make_inputs(B, CO, CI, G, 1, seed=sum(shape))
+    got = gpu_norm_forward(x, w, G, p)
+    torch.testing.assert_close(got, oracle.norm_dist_forward(x, w, G, p), rtol=1e-5, atol=1e-6)
