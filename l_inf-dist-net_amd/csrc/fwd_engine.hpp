@@ -171,19 +171,20 @@ struct RowAddr {
     }
 };
 
-// Writes one run of four consecutive rows (global rows m_first .. m_first+3) times the
+// Writes one run of R consecutive rows (four, or two in the fc layout; global rows m_first .. m_first+R-1) times the
 // lane's TN columns of a result tensor.  When `vec` is set (base pointer 16-byte aligned,
 // NG % 4 == 0 in the fc layout, HW % 4 == 0 in the conv layout) every group of four values
 // along the contiguous axis (n for fc, the row index for conv) that lies fully inside the
 // tensor goes out as one 128-bit store; everything else falls back to single stores.
-template <class GEO, bool CONV, class T>
-__device__ __forceinline__ void store_run(T* __restrict__ dst, const T (&val)[4][GEO::TN], const Dims& d, int m_first,
+template <class GEO, bool CONV, int R, class T>
+__device__ __forceinline__ void store_run(T* __restrict__ dst, const T (&val)[R][GEO::TN], const Dims& d, int m_first,
                                           int n0, int g, int tx, bool vec) {
+    static_assert(R == 4 || !CONV, "the conv layout stores four rows at a time");
     constexpr int TN = GEO::TN;
     using V4 = typename std::conditional<std::is_same<T, float>::value, float4, int4>::type;
     if constexpr (!CONV) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
+        for (int e = 0; e < R; e++) {
             const int m = m_first + e;
             if (m >= d.M) continue;
             T* row = dst + ((size_t)m * d.G + g) * d.NG;
@@ -236,14 +237,15 @@ __device__ __forceinline__ void store_run(T* __restrict__ dst, const T (&val)[4]
 template <class GEO, bool CONV, class T>
 __device__ __forceinline__ void store_patch(T* __restrict__ dst, const T (&val)[GEO::TM][GEO::TN], const Dims& d,
                                             int m0, int n0, int g, int tx, int ty, bool vec) {
+    constexpr int R = GEO::TM < 4 ? GEO::TM : 4;
 #pragma unroll
-    for (int r = 0; r < GEO::TM / 4; r++) {
-        T run[4][GEO::TN];
+    for (int r = 0; r < GEO::TM / R; r++) {
+        T run[R][GEO::TN];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
+        for (int e = 0; e < R; e++)
 #pragma unroll
-            for (int j = 0; j < GEO::TN; j++) run[e][j] = val[4 * r + e][j];
-        store_run<GEO, CONV>(dst, run, d, m0 + GEO::row(ty, 4 * r), n0, g, tx, vec);
+            for (int j = 0; j < GEO::TN; j++) run[e][j] = val[R * r + e][j];
+        store_run<GEO, CONV, R>(dst, run, d, m0 + GEO::row(ty, R * r), n0, g, tx, vec);
     }
 }
 

@@ -79,6 +79,16 @@ norm_forward_skinny_kernel(const float* __restrict__ input, const float* __restr
     }
 }
 
+// The fc layout alone (launch_forward names both layouts).
+template <class GEO, bool CONV, int VEC>
+struct NormForwardColumns {
+    static hipError_t launch(unsigned grid, const Dims& d, int device, hipStream_t stream, const float* input,
+                             const float* weight, float* output, float p) {
+        if constexpr (!CONV) return NormForwardLaunch<GEO, false, VEC, false>::launch(grid, d, device, stream, input, weight, output, p, ImgWin{});
+        else return hipErrorInvalidValue;
+    }
+};
+
 template <class GEO, bool CONV, int VEC>
 struct NormForward {
     static hipError_t launch(unsigned grid, const Dims& d, int device, hipStream_t stream, const float* input,
@@ -86,6 +96,31 @@ struct NormForward {
         return NormForwardLaunch<GEO, CONV, VEC, false>::launch(grid, d, device, stream, input, weight, output, p, ImgWin{});
     }
 };
+
+// Fully connected layers that choose_tile gives tiles of 32 x 32 with eight k-groups (the 128-row tiles would leave the
+// device idle): the same eight k-groups, hence the same order of summation, on the tile whose shares load the busiest CU
+// least; a CU runs one workgroup of eight waves at a time.  32 x 40: 64 x 5120 -> 5120 is 256 tiles instead of 320, 280 ->
+// 189 us at p = 8, 602 -> 386 at p = 37.3.  16 x 32 with two rows per lane: 128 x 12288 -> 512 is 128 tiles instead of 64,
+// 290 -> 184 us and 684 -> 369; 100 x 1024 -> 1024 43 -> 27 and 84 -> 48.  A lane of the latter reads six LDS words for
+// eight differences instead of eight for sixteen, hence the surcharge.
+template <class GEO>
+static hipError_t launch_eight_groups(const Problem& pr, hipStream_t stream, const float* input, const float* weight,
+                                      float* output, float p) {
+    return launch_forward<NormForwardColumns, GEO>(pr, can_vec4(pr, input, weight), can_vec4_out(pr, output), stream, input,
+                                                   weight, output, p);
+}
+
+static hipError_t norm_forward_eight_groups(const float* input, const float* weight, float* output, float p, const Problem& pr,
+                                            hipStream_t stream) {
+    auto cost = [&](int bm, int bn, double price) {
+        const long tiles = (long)((pr.B + bm - 1) / bm) * ((pr.NG + bn - 1) / bn) * pr.G;
+        return (double)((tiles + pr.num_cu - 1) / pr.num_cu) * bm * bn * price;
+    };
+    const double square = cost(32, 32, 1.0), wide = cost(32, 40, 1.0), flat = cost(16, 32, 1.1);
+    if (wide < square && wide <= flat) return launch_eight_groups<Geo<32, 40, 4, 5, 8>>(pr, stream, input, weight, output, p);
+    if (flat < square) return launch_eight_groups<Geo<16, 32, 2, 4, 8>>(pr, stream, input, weight, output, p);
+    return launch_eight_groups<Geo<32, 32, 4, 4, 8>>(pr, stream, input, weight, output, p);
+}
 
 // `values_only`: no gradient follows.  Such a pass may sum in any order and takes whichever kernel is fastest for the
 // size.  A forward pass that trains keeps the order of summation it has always had (chunks of 32 k, alternating between
@@ -112,6 +147,8 @@ hipError_t norm_forward(const float* input, const float* weight, float* output, 
     }
     if (const int tile = values_only || g_tile_override >= 10 ? small_forward_tile(pr, ForwardKind::kNorm, p) : -1; tile >= 0)
         return norm_forward_small(input, weight, output, p, pr, tile, stream);
+    if (pr.HW == 1 && g_tile_override < 0 && choose_tile(pr.B, pr.NG, pr.G, pr.num_cu) == TileChoice::M32N32K8)
+        return norm_forward_eight_groups(input, weight, output, p, pr, stream);
     return dispatch_forward<NormForward>(pr, can_vec4(pr, input, weight), can_vec4_out(pr, output), stream, input,
                                          weight, output, p);
 }

@@ -54,20 +54,19 @@ struct Geo {
     static constexpr int SN = (BN + 31) / 32 * 32;
     static constexpr int XS = KK * SM;           // floats of one x panel
     static constexpr int WS = KK * SN;
-    static_assert(TM == 4 || TM == 8, "TM");
-    static_assert(TN == 3 || TN == 4 || TN == 5 || TN == 8, "TN");   // 3: columns tx*3 + j of the tile, kept at a pitch of four in the w panel
+    static_assert(TM == 2 || TM == 4 || TM == 8, "TM");
+    static_assert(TN == 4 || TN == 5 || TN == 8, "TN");
     static_assert(BM % TM == 0 && BN % TN == 0, "tile");
     static_assert(NT % 64 == 0, "whole waves");
 
     // Tile-local row of the i-th value a lane owns.  Eight values are two runs
     // of four, BM/2 apart, so that neighbouring lanes read neighbouring 16 bytes.
     __device__ static constexpr int row(int ty, int i) {
-        return TM == 8 ? (i < 4 ? ty * 4 + i : BM / 2 + ty * 4 + (i - 4)) : ty * 4 + i;
+        return TM == 8 ? (i < 4 ? ty * 4 + i : BM / 2 + ty * 4 + (i - 4)) : ty * TM + i;
     }
     __device__ static constexpr int col(int tx, int j) {
         return TN == 8 ? (j < 4 ? tx * 4 + j : BN / 2 + tx * 4 + (j - 4))
              : TN == 5 ? (j < 4 ? tx * 4 + j : TX * 4 + tx)
-             : TN == 3 ? tx * 3 + j
                        : tx * 4 + j;
     }
 };
@@ -83,7 +82,7 @@ struct LanePtr {
     const float* w5;  // w panel, row kk, the lane's fifth column (TN == 5 only)
     __device__ __forceinline__ void set(const float* xp, const float* wp, int kk, int tx, int ty) {
         const int s = swz(kk);
-        x = xp + kk * GEO::SM + ((ty * 4) ^ s);
+        x = xp + kk * GEO::SM + ((ty * (GEO::TM == 2 ? 2 : 4)) ^ s);
         w = wp + kk * GEO::SN + ((tx * 4) ^ s);
         if constexpr (GEO::TN == 5) w5 = wp + kk * GEO::SN + ((GEO::TX * 4 + tx) ^ s);
     }
@@ -91,19 +90,24 @@ struct LanePtr {
 
 template <class GEO>
 __device__ __forceinline__ void read_x(const float* __restrict__ p, int r, float (&xf)[GEO::TM]) {
+    if constexpr (GEO::TM == 2) {
+        float2 a = *reinterpret_cast<const float2*>(p + r * GEO::SM);
+        xf[0] = a.x; xf[1] = a.y;
+        return;
+    } else {
     float4 a = *reinterpret_cast<const float4*>(p + r * GEO::SM);
     xf[0] = a.x; xf[1] = a.y; xf[2] = a.z; xf[3] = a.w;
     if constexpr (GEO::TM == 8) {
         float4 b = *reinterpret_cast<const float4*>(p + r * GEO::SM + GEO::BM / 2);
         xf[4] = b.x; xf[5] = b.y; xf[6] = b.z; xf[7] = b.w;
     }
+    }
 }
 
 template <class GEO>
 __device__ __forceinline__ void read_w(const LanePtr<GEO>& lp, int r, float (&wf)[GEO::TN]) {
     float4 a = *reinterpret_cast<const float4*>(lp.w + r * GEO::SN);
-    wf[0] = a.x; wf[1] = a.y; wf[2] = a.z;
-    if constexpr (GEO::TN > 3) wf[3] = a.w;   // TN == 3: the fourth word of the lane's pitch is not a column
+    wf[0] = a.x; wf[1] = a.y; wf[2] = a.z; wf[3] = a.w;
     if constexpr (GEO::TN == 8) {
         float4 b = *reinterpret_cast<const float4*>(lp.w + r * GEO::SN + GEO::BN / 2);
         wf[4] = b.x; wf[5] = b.y; wf[6] = b.z; wf[7] = b.w;
