@@ -45,7 +45,7 @@ namespace {
 
 constexpr int TR = 64;              // rows of a tile
 constexpr int TCP = 64;             // columns a tile has lanes for
-constexpr int WLD = TCP + 4;        // row length of the weight and grad_weight tiles (rows 16-byte aligned)
+constexpr int WLD = TCP;            // row length of the weight and grad_weight tiles (a wave reads one row at a time: no padding)
 constexpr int TI = 8, TJ = 2;       // a lane's patch: rows x columns; 64 / TI lanes share a column pair, inside one DPP row
 constexpr int kPlanes = 7;          // IMG: channels per tile (63 columns)
 constexpr size_t kMaxLds = 159 * 1024;   // all of LDS less the kernel's own static words
@@ -54,7 +54,7 @@ struct ConvBwd {
     int B, G, K, NG, HW, M;          // the unfolded problem: K = 9 channels per group (image) or CI / G
     int tiles_k;                     // column tiles per group
     int units, units_per_wg;         // what a workgroup walks: tiles of 64 rows (columns), whole images (image)
-    int ring_rows;                   // IMG: image rows per channel plane held in LDS, a power of two
+    int ring_rows;                   // IMG: image rows per channel plane held in LDS
     int park_extra;                  // IMG: floats between the 1/out panel and the ring that the parked tile runs into
     int slices;                      // workgroups per (group, column tile): units / units_per_wg, rounded up
 };
@@ -91,7 +91,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     float* Fp = Rs + NG * TR + (IMG ? d.park_extra : 0);   // IMG: [kPlanes][ring_rows][W] gradient of the image rows still being added to
     const int tid = threadIdx.x;
     constexpr int TYN = TR / TI;             // lanes along the rows
-    const int ty = tid % TYN, tx = tid / TYN;   // rows first: the lanes of a column group are neighbours in a DPP row
+    const int ty = tid % TYN;                // rows first: the lanes of a column group are neighbours in a DPP row
     // Consecutive workgroup ids go to different XCDs (8 per device, each with its own L2).  The grid is padded to a
     // multiple of 8 and remapped so that every XCD gets one contiguous run of (slice, group, column tile) with the
     // column tile fastest: the workgroups of one (slice, group) stage the same g and out, walk their units in step,
@@ -102,6 +102,13 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     const int slice = remapped / pairs, pair = remapped - slice * pairs;
     const int tk = pair % d.tiles_k, g = pair / d.tiles_k;
     const int k0 = tk * TC;
+    // A tile of at most 32 columns (three channels: the first layer of a net; the last tile of 64) would leave two of the
+    // four waves without columns: they take the same ones and the second half of the outputs instead, and the halves'
+    // grad_input sums meet where they are parked (128 images of 3 x 32 x 32 to 32 channels, p = 8: 248 -> 182 us).
+    const bool halved = IMG && min(TC, K - k0) <= TCP / 2;
+    const int second = halved ? tid >> 7 : 0;   // this wave's half
+    const int tx = halved ? (tid / TYN) & 15 : tid / TYN;
+    const int n_lo = second * ((NG + 1) / 2), n_hi = halved && !second ? (NG + 1) / 2 : NG;
     const int u_begin = slice * d.units_per_wg, u_end = min(d.units, u_begin + d.units_per_wg);
 
     auto spower = [&](float u) {   // sign(u) * |u|^(p-1); by reference: the integer-exponent instantiations do not use e
@@ -305,7 +312,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             __syncthreads();
         }
         auto reduce = [&](auto term) {   // term(x - w, 1/out): the power that g (or g / out^IE) multiplies
-            for (int n = 0; n < NG; n++) {
+            for (int n = n_lo; n < n_hi; n++) {
                 float cv[TI], rv[TI], wv[TJ];
 #pragma unroll
                 for (int i = 0; i < TI; i += 4) {
@@ -378,7 +385,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             const bool ok = hh >= 0 && o * win.S == hh && o < lim;
             HT[i] = ok ? (row ? o * win.WO : o) : kNone;   // WT follows HT
         }
-        const float inv_w = 1.0f / (float)W;
+        const float inv_w = 1.0f / (float)W, inv_r = 1.0f / (float)R;
+        auto ring_row = [&](int h) { return h - R * (int)(((float)h + 0.5f) * inv_r); };   // h modulo R
         for (int b = u_begin; b < u_end; b++) {
             float* dst = grad_input + ((size_t)b * win.C + g * win.CG + first_ch) * H * W;
             // Writes image rows h_from .. h_to - 1 of the planes to memory and clears their ring rows.  Rows more than
@@ -389,7 +397,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                     const int w = i % W, rest = i / W, hr = rest % nrow, c = rest / nrow, h = h_from + hr;
                     float v = 0.f;
                     if (hr < R) {
-                        float* cell = Fp + (c * R + (h & (R - 1))) * W + w;
+                        float* cell = Fp + (c * R + ring_row(h)) * W + w;
                         v = *cell;
                         *cell = 0.f;
                     }
@@ -435,13 +443,23 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 // The tile's sums join the planes.  They are parked by (column, position) over the two panels, and
                 // every pixel that a window of this tile can reach fetches its up to nine (position, tap) entries
                 // and adds them to its ring word: one owner per pixel, a fixed order of the nine, no rounds.
+                auto park = [&](bool add) {
 #pragma unroll
-                for (int j = 0; j < TJ; j++)
+                    for (int j = 0; j < TJ; j++)
 #pragma unroll
-                    for (int i = 0; i < TI; i += 4)
-                        *reinterpret_cast<float4*>(Pk + (tx * TJ + j) * TR + ty * TI + i) =
-                            make_float4(acc[i][j], acc[i + 1][j], acc[i + 2][j], acc[i + 3][j]);
+                        for (int i = 0; i < TI; i += 4) {
+                            float4* at = reinterpret_cast<float4*>(Pk + (tx * TJ + j) * TR + ty * TI + i);
+                            float4 v = make_float4(acc[i][j], acc[i + 1][j], acc[i + 2][j], acc[i + 3][j]);
+                            if (add) { const float4 o = *at; v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w; }
+                            *at = v;
+                        }
+                };
+                if (second == 0) park(false);
                 __syncthreads();
+                if (halved) {   // the same in every lane of the workgroup
+                    if (second == 1) park(true);
+                    __syncthreads();
+                }
                 const int last = pos0 + rows - 1;
                 const int h_first = max(0, (pos0 / win.WO) * win.S - win.P);
                 const int h_last = min(H - 1, (last / win.WO) * win.S - win.P + 2 * win.D);
@@ -467,7 +485,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                             const bool in = (unsigned)(pos - pos0) < (unsigned)rows;
                             sum += *(in ? col + (th * 3 + tw) * TR + pos : zero_word);
                         }
-                    Fp[(c * R + (h & (R - 1))) * W + w] += sum;
+                    Fp[(c * R + ring_row(h)) * W + w] += sum;
                 }
                 __syncthreads();   // the next tile stages over the parked sums; its flush reads the ring
             }
@@ -496,7 +514,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
 namespace {
 
 // Image rows per plane the ring must hold: the most that the windows of one tile of 64 positions cover (tiles start
-// at multiples of 64 inside an image), rounded up to a power of two.
+// at multiples of 64 inside an image).  Not more: 32 -> 64 channels at stride 2 on 32 x 32 need nine rows, and with
+// sixteen (the next power of two) a CU held one workgroup instead of two (128 images, p = 8: 386 -> 270 us).
 int ring_rows_for(const ImgWin& win, int HW) {
     int out_rows = 1;
     for (int pos0 = 0; pos0 < HW; pos0 += TR) {
@@ -504,10 +523,7 @@ int ring_rows_for(const ImgWin& win, int HW) {
         out_rows = std::max(out_rows, last / win.WO - pos0 / win.WO + 1);
         if (pos0 / TR >= win.WO) break;   // the pattern of starts inside an output row repeats by then
     }
-    const int rows = (out_rows - 1) * win.S + 2 * win.D + 1;
-    int ring = 1;
-    while (ring < rows) ring *= 2;
-    return ring;
+    return (out_rows - 1) * win.S + 2 * win.D + 1;
 }
 
 template <bool IMG, int IE>
