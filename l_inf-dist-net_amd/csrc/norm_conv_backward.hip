@@ -57,15 +57,23 @@ struct ConvBwd {
     int ring_rows;                   // IMG: image rows per channel plane held in LDS
     int park_extra;                  // IMG: floats between the 1/out panel and the ring that the parked tile runs into
     int slices;                      // workgroups per (group, column tile): units / units_per_wg, rounded up
+    int chunk;                       // outputs whose g and 1/out are staged at a time
 };
 
+// A tile's g and 1/out are staged for up to 32 outputs at a time, in equal shares of a group's outputs: staged whole, the
+// panels of 64 outputs let a CU hold two workgroups, in halves three.
+inline int outputs_staged(int NG) {
+    const int shares = (NG + 31) / 32;
+    return (NG + shares - 1) / shares;
+}
+
 inline size_t lds_bytes(int NG, size_t plane_floats) {
-    return ((size_t)2 * NG * WLD + (size_t)2 * NG * TR + plane_floats) * sizeof(float);
+    return ((size_t)2 * NG * WLD + (size_t)2 * outputs_staged(NG) * TR + plane_floats) * sizeof(float);
 }
 
 // IMG: a tile's grad_input sums are parked as [64 columns][64 positions] over the g and 1/out panels; what that
 // takes beyond the panels' 2 * NG * 64 floats
-inline int park_extra(int NG) { return std::max(0, TCP * TR - 2 * NG * TR); }
+inline int park_extra(int NG) { return std::max(0, TCP * TR - 2 * outputs_staged(NG) * TR); }
 
 // IMG: the floats behind the panels: the parked tile's overhang, the ring of image rows, a word that stays zero,
 // and the two tables (image row, tap row) -> output row and (image column, tap column) -> output column
@@ -86,9 +94,9 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     const int NG = d.NG, K = d.K;
     float* Ws = lds;                     // [NG][WLD]  w[n][k0 + c]
     float* Gw = Ws + NG * WLD;           // [NG][WLD]  sums for grad_weight[n][k0 + c]
-    float* Cs = Gw + NG * WLD;           // [NG][TR]   g, or g / out^IE
-    float* Rs = Cs + NG * TR;            // [NG][TR]   1 / out
-    float* Fp = Rs + NG * TR + (IMG ? d.park_extra : 0);   // IMG: [kPlanes][ring_rows][W] gradient of the image rows still being added to
+    float* Cs = Gw + NG * WLD;           // [chunk][TR]   g, or g / out^IE, of the staged outputs
+    float* Rs = Cs + d.chunk * TR;       // [chunk][TR]   1 / out
+    float* Fp = Rs + d.chunk * TR + (IMG ? d.park_extra : 0);   // IMG: [kPlanes][ring_rows][W] gradient of the image rows still being added to
     const int tid = threadIdx.x;
     constexpr int TYN = TR / TI;             // lanes along the rows
     const int ty = tid % TYN;                // rows first: the lanes of a column group are neighbours in a DPP row
@@ -108,7 +116,6 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     const bool halved = IMG && min(TC, K - k0) <= TCP / 2;
     const int second = halved ? tid >> 7 : 0;   // this wave's half
     const int tx = halved ? (tid / TYN) & 15 : tid / TYN;
-    const int n_lo = second * ((NG + 1) / 2), n_hi = halved && !second ? (NG + 1) / 2 : NG;
     const int u_begin = slice * d.units_per_wg, u_end = min(d.units, u_begin + d.units_per_wg);
 
     auto spower = [&](float u) {   // sign(u) * |u|^(p-1); by reference: the integer-exponent instantiations do not use e
@@ -223,7 +230,11 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 }
             }
         }
-        // g and out of the tile's rows for every output of the group; rows are contiguous in memory
+        // g and out of the tile's rows for outputs nc .. nc + cnt - 1 of the group; rows are contiguous in memory
+        for (int nc = 0; nc < NG; nc += d.chunk) {
+        const int cnt = min(d.chunk, NG - nc);
+        const int n_lo = second * ((cnt + 1) / 2), n_hi = halved && !second ? (cnt + 1) / 2 : cnt;   // this wave's
+        if (nc > 0) __syncthreads();   // everyone has left the outputs before
         bool unsafe = false;
         if constexpr (IMG) {
             // A lane takes row r = tid % 64 of outputs tid / 64, + 4, + 8, ...: four outputs per pass, their eight
@@ -232,19 +243,19 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             const int r = tid & (TR - 1);
             const unsigned row_off = 4u * (unsigned)(pos0 + r), out_stride = 4u * (unsigned)d.HW;
 #pragma unroll 1
-            for (int n0 = tid / TR; n0 < NG; n0 += 16) {
+            for (int n0 = tid / TR; n0 < cnt; n0 += 16) {
                 float gv[4], ov[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int n = n0 + 4 * u;
-                    const unsigned o = ((r < rows) & (n < NG)) ? row_off + (unsigned)n * out_stride : ~0u;
+                    const unsigned o = ((r < rows) & (n < cnt)) ? row_off + (unsigned)(nc + n) * out_stride : ~0u;
                     gv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(g_rsrc, o, 0, 0));
                     ov[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(o_rsrc, o, 0, 0));
                 }
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int n = n0 + 4 * u;
-                    if (n < NG) {
+                    if (n < cnt) {
                         const float out = ov[u] * unit_inv;
                         float ri = 0.f;   // IE == 0: ri holds the output itself until the vote is in
                         if (r < rows) {
@@ -264,18 +275,18 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             const int m = first_row + min(r, rows - 1), bi = m / d.HW;
             const size_t row0 = ((size_t)(bi * d.G + g) * NG) * d.HW + (m - bi * d.HW);
 #pragma unroll 1
-            for (int n0 = tid / TR; n0 < NG; n0 += 16) {
+            for (int n0 = tid / TR; n0 < cnt; n0 += 16) {
                 float gv[4], ov[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    const int n = min(n0 + 4 * u, NG - 1);   // past the last output: a valid address, the value is not used
+                    const int n = nc + min(n0 + 4 * u, cnt - 1);   // past the last output: a valid address, the value is not used
                     gv[u] = grad_output[row0 + (size_t)n * d.HW];
                     ov[u] = output[row0 + (size_t)n * d.HW];
                 }
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int n = n0 + 4 * u;
-                    if (n < NG) {
+                    if (n < cnt) {
                         const float out = ov[u] * unit_inv;
                         float c = 0.f, ri = 0.f;   // IE == 0: ri holds the output itself until the vote is in
                         if (r < rows) {
@@ -291,11 +302,11 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         }
         const bool factored = !__syncthreads_or(unsafe);   // also: the panels are written
         if (IE > 0 && factored) {
-            for (int i = tid; i < NG * TR; i += 256) Cs[i] *= pow_int<(IE > 0 ? IE : 1)>(Rs[i]);   // each lane its own elements
+            for (int i = tid; i < cnt * TR; i += 256) Cs[i] *= pow_int<(IE > 0 ? IE : 1)>(Rs[i]);   // each lane its own elements
             __syncthreads();
         }
         if constexpr (IE == 0) {   // each lane its own elements: out -> 1/out, or the logarithmic form's summand
-            for (int i = tid; i < NG * TR; i += 256) {
+            for (int i = tid; i < cnt * TR; i += 256) {
                 const float out = Rs[i];
                 if (i % TR >= rows) {
                     Rs[i] = factored ? -__builtin_inff() : 0.f;   // rows that do not exist: a power of 0, a factor 0
@@ -322,10 +333,10 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                     rv[i] = r4.x; rv[i + 1] = r4.y; rv[i + 2] = r4.z; rv[i + 3] = r4.w;
                 }
                 if constexpr (TJ == 4) {
-                    const float4 w4 = *reinterpret_cast<const float4*>(Ws + n * WLD + tx * 4);
+                    const float4 w4 = *reinterpret_cast<const float4*>(Ws + (nc + n) * WLD + tx * 4);
                     wv[0] = w4.x; wv[1] = w4.y; wv[2] = w4.z; wv[3] = w4.w;
                 } else {
-                    const float2 w2 = *reinterpret_cast<const float2*>(Ws + n * WLD + tx * 2);
+                    const float2 w2 = *reinterpret_cast<const float2*>(Ws + (nc + n) * WLD + tx * 2);
                     wv[0] = w2.x; wv[1] = w2.y;
                 }
                 float s[TJ];
@@ -343,7 +354,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
 #pragma unroll
                 for (int j = 0; j < TJ; j++) tot[j] = dpp_lanes_total<TYN>(s[j]);
                 if (ty == TYN - 1) {   // d/dw of |x - w| is minus d/dx
-                    float* gp = Gw + n * WLD + tx * TJ;
+                    float* gp = Gw + (nc + n) * WLD + tx * TJ;
                     if constexpr (TJ == 4) {
                         float4 v = *reinterpret_cast<float4*>(gp);
                         v.x -= tot[0]; v.y -= tot[1]; v.z -= tot[2]; v.w -= tot[3];
@@ -360,6 +371,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         else if (IE == 0 && factored)
             reduce([&](float df, float c4) { return df * __builtin_amdgcn_exp2f(__builtin_fmaf(__builtin_amdgcn_logf(__builtin_fabsf(df)), em1, c4)); });
         else reduce([&](float df, float ri) { return spower(df * ri); });
+        }
     };
 
     float acc[TI][TJ];
@@ -530,7 +542,7 @@ template <bool IMG, int IE>
 hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
-    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0};
+    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, outputs_staged(pr.NG)};
     d.tiles_k = IMG ? (win.CG + kPlanes - 1) / kPlanes : (d.K + TCP - 1) / TCP;
     d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
     const long pairs = (long)d.tiles_k * d.G;
