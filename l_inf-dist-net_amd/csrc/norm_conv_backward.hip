@@ -6,7 +6,7 @@
 // with m = (image, output position), n the outputs of one group, k = (channel, tap) of the group's window.
 //
 // A layer of this shape has few outputs per group and very many rows, so a workgroup keeps the weights of its
-// columns k for ALL outputs of the group in LDS, next to a tile of grad_weight sums of the same shape, and walks
+// columns k for ALL outputs of the group (or of a block of up to 64) in LDS, next to a tile of grad_weight sums of the same shape, and walks
 // tiles of 64 rows.  Per tile it stages g and 1/out (NG x 64 each), and every lane reduces an 8 x 2 patch of
 // (row, column) over n: a term is evaluated once, added to the lane's grad_input sum and to the column's partial sum
 // over the lane's eight rows; the eight lanes that share the columns (half a DPP row) add those with three row
@@ -57,23 +57,35 @@ struct ConvBwd {
     int ring_rows;                   // IMG: image rows per channel plane held in LDS
     int park_extra;                  // IMG: floats between the 1/out panel and the ring that the parked tile runs into
     int slices;                      // workgroups per (group, column tile): units / units_per_wg, rounded up
-    int chunk;                       // outputs whose g and 1/out are staged at a time
+    int block;                       // outputs whose weights and grad_weight sums are in LDS at a time
+    int chunk;                       // of which g and 1/out are staged at a time
 };
+
+// A group's outputs are taken in equal blocks of up to 64, one after the other over the same units: the two tiles of 128
+// outputs would leave room for one workgroup per CU.  grad_input has one owner all along, who writes it for the first
+// block and adds to it for the others.  128 images of 64 x 16 x 16 (us, both gradients; in brackets the two separate
+// kernels): 128 outputs, p = 8, 1109 -> 604 (811); 192 outputs 902 (1398), at p = 37.3 1345 (2222), which the separate kernels
+// took before; 128 channels to 128 outputs, p = 37.3, 2874 -> 1586 (2810), to 256, p = 8, 2173 (3388).
+inline int outputs_in_block(int NG) {
+    const int blocks = (NG + 63) / 64;
+    return (NG + blocks - 1) / blocks;
+}
 
 // A tile's g and 1/out are staged for up to 32 outputs at a time, in equal shares of a group's outputs: staged whole, the
 // panels of 64 outputs let a CU hold two workgroups, in halves three.
-inline int outputs_staged(int NG) {
-    const int shares = (NG + 31) / 32;
-    return (NG + shares - 1) / shares;
+inline int outputs_staged(int block) {
+    const int shares = (block + 31) / 32;
+    return (block + shares - 1) / shares;
 }
 
 inline size_t lds_bytes(int NG, size_t plane_floats) {
-    return ((size_t)2 * NG * WLD + (size_t)2 * outputs_staged(NG) * TR + plane_floats) * sizeof(float);
+    const int block = outputs_in_block(NG);
+    return ((size_t)2 * block * WLD + (size_t)2 * outputs_staged(block) * TR + plane_floats) * sizeof(float);
 }
 
 // IMG: a tile's grad_input sums are parked as [64 columns][64 positions] over the g and 1/out panels; what that
-// takes beyond the panels' 2 * NG * 64 floats
-inline int park_extra(int NG) { return std::max(0, TCP * TR - 2 * outputs_staged(NG) * TR); }
+// takes beyond the panels' 128 floats per staged output
+inline int park_extra(int NG) { return std::max(0, TCP * TR - 2 * outputs_staged(outputs_in_block(NG)) * TR); }
 
 // IMG: the floats behind the panels: the parked tile's overhang, the ring of image rows, a word that stays zero,
 // and the two tables (image row, tap row) -> output row and (image column, tap column) -> output column
@@ -83,7 +95,9 @@ inline size_t image_floats(int NG, int ring_rows, int H, int W) {
 
 }  // namespace
 
-template <bool IMG, int IE>
+// BLOCKS: more outputs per group than one block holds (its own instantiation: the loop around everything costs registers,
+// 3 % on 32 and 64 outputs).
+template <bool IMG, int IE, bool BLOCKS>
 __global__ void __launch_bounds__(256, 4)   // four workgroups per CU is what LDS allows at 32 outputs per group: 128 registers
 norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __restrict__ input,
                           const float* __restrict__ weight, const float* __restrict__ output,
@@ -91,10 +105,10 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                           ImgWin win) {
     constexpr int TC = IMG ? 9 * kPlanes : TCP;   // columns per tile
     extern __shared__ __align__(16) float lds[];
-    const int NG = d.NG, K = d.K;
-    float* Ws = lds;                     // [NG][WLD]  w[n][k0 + c]
-    float* Gw = Ws + NG * WLD;           // [NG][WLD]  sums for grad_weight[n][k0 + c]
-    float* Cs = Gw + NG * WLD;           // [chunk][TR]   g, or g / out^IE, of the staged outputs
+    const int K = d.K;
+    float* Ws = lds;                     // [block][WLD]  w[n][k0 + c]
+    float* Gw = Ws + d.block * WLD;      // [block][WLD]  sums for grad_weight[n][k0 + c]
+    float* Cs = Gw + d.block * WLD;           // [chunk][TR]   g, or g / out^IE, of the staged outputs
     float* Rs = Cs + d.chunk * TR;       // [chunk][TR]   1 / out
     float* Fp = Rs + d.chunk * TR + (IMG ? d.park_extra : 0);   // IMG: [kPlanes][ring_rows][W] gradient of the image rows still being added to
     const int tid = threadIdx.x;
@@ -125,9 +139,12 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         else return pow_int<IE>(u);
     };
 
+    float unit_inv = 1.0f;   // 1 / unit (below)
+    for (int nb = 0; nb < (BLOCKS ? d.NG : 1); nb += BLOCKS ? d.block : 1) {   // outputs nb .. nb + NG - 1 of the group
+    const int NG = BLOCKS ? min(d.block, d.NG - nb) : d.NG;
     for (int i = tid; i < NG * TCP; i += 256) {
         const int n = i / TCP, c = i % TCP;
-        Ws[n * WLD + c] = (c < TC && k0 + c < K) ? weight[((size_t)g * NG + n) * K + k0 + c] : 0.f;
+        Ws[n * WLD + c] = (c < TC && k0 + c < K) ? weight[((size_t)g * d.NG + nb + n) * K + k0 + c] : 0.f;
         Gw[n * WLD + c] = 0.f;
     }
     // General exponent (IE == 0): the term g * u * |u|^(p-2), u = (x - w) / out, is taken as
@@ -141,9 +158,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     // outputs of the workgroup's first tile (exact scalings of x, the weights and the outputs; the one nearest to the
     // geometric mean of the largest and the smallest of them), and a tile takes the form only if all its outputs lie within [1/2, 2] units
     // (voted on the barrier that follows the staging); other tiles divide first.
-    float unit_inv = 1.0f;   // 1 / unit
     const float em1 = e - 1.0f;   // p - 2
-    if constexpr (IE == 0) {
+    if (IE == 0 && nb == 0) {
         float top = 0.f, nbot = -__builtin_inff();   // the largest and minus the smallest output of the first tile
         if (u_begin < u_end) {
             const int rows = IMG ? min(TR, d.HW) : min(TR, d.M - u_begin * TR);
@@ -152,10 +168,10 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 if (r < rows) {
                     size_t o;
                     if constexpr (IMG) {
-                        o = ((size_t)(u_begin * d.G + g) * NG + n) * d.HW + r;
+                        o = ((size_t)(u_begin * d.G + g) * d.NG + n) * d.HW + r;
                     } else {
                         const int m = u_begin * TR + r, bi = m / d.HW;
-                        o = ((size_t)(bi * d.G + g) * NG + n) * d.HW + (m - bi * d.HW);
+                        o = ((size_t)(bi * d.G + g) * d.NG + n) * d.HW + (m - bi * d.HW);
                     }
                     const float ov = output[o];
                     if (ov > 0.f && ov < __builtin_inff()) {   // a NaN is not taken either
@@ -178,8 +194,9 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         const float mid = __builtin_sqrtf(top) * __builtin_sqrtf(-nbot) * 1.41421356f;
         const int ex = min(100, max(-100, (int)((__float_as_uint(mid) >> 23) & 0xff) - 127));
         unit_inv = top > 0.f ? __uint_as_float((unsigned)(127 - ex) << 23) : 1.0f;
-        for (int i = tid; i < NG * TCP; i += 256) Ws[(i / TCP) * WLD + i % TCP] *= unit_inv;   // each lane the words it wrote
     }
+    if constexpr (IE == 0)
+        for (int i = tid; i < NG * TCP; i += 256) Ws[(i / TCP) * WLD + i % TCP] *= unit_inv;   // each lane the words it wrote
     // the lane's four columns: whether they exist, and for the image their channel plane and tap
     bool col_ok[TJ];
     int col_plane[TJ], col_tap[TJ], col_dh[TJ], col_dw[TJ];   // IMG: the column's channel plane inside the tile, its tap and the tap's offsets
@@ -273,7 +290,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             // element offset of its row in output 0 and steps by HW per output
             const int r = tid & (TR - 1);
             const int m = first_row + min(r, rows - 1), bi = m / d.HW;
-            const size_t row0 = ((size_t)(bi * d.G + g) * NG) * d.HW + (m - bi * d.HW);
+            const size_t row0 = ((size_t)(bi * d.G + g) * d.NG + nb) * d.HW + (m - bi * d.HW);
 #pragma unroll 1
             for (int n0 = tid / TR; n0 < cnt; n0 += 16) {
                 float gv[4], ov[4];
@@ -413,16 +430,17 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                         v = *cell;
                         *cell = 0.f;
                     }
-                    dst[(c * H + h) * W + w] = v;
+                    float* const at = dst + (c * H + h) * W + w;
+                    *at = nb == 0 ? v : *at + v;
                 }
             };
             for (int i = tid; i < kPlanes * R * W; i += 256) Fp[i] = 0.f;   // the first tile's barriers come before its use
             x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<float*>(input + ((size_t)b * win.C + g * win.CG + first_ch) * H * W), 0, (int)0x80000000u, 0x00020000);
             g_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float*>(grad_output + (size_t)(b * d.G + g) * NG * d.HW), 0, (int)0x80000000u, 0x00020000);
+                const_cast<float*>(grad_output + ((size_t)(b * d.G + g) * d.NG + nb) * d.HW), 0, (int)0x80000000u, 0x00020000);
             o_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float*>(output + (size_t)(b * d.G + g) * NG * d.HW), 0, (int)0x80000000u, 0x00020000);
+                const_cast<float*>(output + ((size_t)(b * d.G + g) * d.NG + nb) * d.HW), 0, (int)0x80000000u, 0x00020000);
             // the corners of the windows of the lane's positions, moved on by 64 positions per tile (positions past
             // the image's last one are never used: every use asks for i < rows)
 #pragma unroll
@@ -512,14 +530,18 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             for (int i = 0; i < TI; i++)
 #pragma unroll
                 for (int j = 0; j < TJ; j++)
-                    if (ty * TI + i < rows && col_ok[j]) grad_input[xoff[i] + (size_t)(k0 + tx * TJ + j) * d.HW] = acc[i][j];
+                    if (ty * TI + i < rows && col_ok[j]) {
+                        float* const at = grad_input + xoff[i] + (size_t)(k0 + tx * TJ + j) * d.HW;
+                        *at = nb == 0 ? acc[i][j] : *at + acc[i][j];
+                    }
             __syncthreads();   // the next tile overwrites the panels
         }
     }
     __syncthreads();
     for (int i = tid; i < NG * TCP; i += 256) {
         const int n = i / TCP, c = i % TCP;
-        if (c < TC && k0 + c < K) atomicAdd(grad_weight + ((size_t)g * NG + n) * K + k0 + c, Gw[n * WLD + c]);
+        if (c < TC && k0 + c < K) atomicAdd(grad_weight + ((size_t)g * d.NG + nb + n) * K + k0 + c, Gw[n * WLD + c]);
+    }
     }
 }
 
@@ -538,11 +560,12 @@ int ring_rows_for(const ImgWin& win, int HW) {
     return (out_rows - 1) * win.S + 2 * win.D + 1;
 }
 
-template <bool IMG, int IE>
-hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
+template <bool IMG, int IE, bool BLOCKS>
+hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
-    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, outputs_staged(pr.NG)};
+    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, outputs_in_block(pr.NG),
+              outputs_staged(outputs_in_block(pr.NG))};
     d.tiles_k = IMG ? (win.CG + kPlanes - 1) / kPlanes : (d.K + TCP - 1) / TCP;
     d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
     const long pairs = (long)d.tiles_k * d.G;
@@ -575,13 +598,22 @@ hipError_t launch_conv_backward(const float* grad_output, const float* input, co
     const long slices = (d.units + d.units_per_wg - 1) / d.units_per_wg;
     d.slices = (int)slices;
     const long grid = (pairs * slices + 7) / 8 * 8;   // whole rounds of the eight XCDs; the padding exits at once
-    auto kern = norm_conv_backward_kernel<IMG, IE>;
+    auto kern = norm_conv_backward_kernel<IMG, IE, BLOCKS>;
     static LdsRecord lds_allowed = {};
     // the limit is raised once, to the most any layer may ask for
     if (hipError_t e = allow_lds(kern, kMaxLds, pr.device, lds_allowed); e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, grad_output, input, weight,
                        output, grad_input, grad_weight, p - 1.0f, d, win);
     return hipGetLastError();
+}
+
+template <bool IMG, int IE>
+hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
+                                float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
+                                hipStream_t stream) {
+    return outputs_in_block(pr.NG) < pr.NG
+        ? launch_conv_backward_blocks<IMG, IE, true>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream)
+        : launch_conv_backward_blocks<IMG, IE, false>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream);
 }
 
 template <bool IMG>
@@ -602,10 +634,9 @@ bool forced_on() { return g_tile_override == 0 || g_tile_override == 1; }   // t
 }  // namespace
 
 // Whether the one-pass kernel takes a layer given as unfolded columns: the conv layout with enough rows to give
-// every CU work, and few enough outputs per group for the four LDS tiles (NG KB).
+// every CU work.
 bool norm_conv_backward_fused_applicable(const Problem& pr) {
     if (pr.HW == 1 || g_tile_override >= 2) return false;
-    if (lds_bytes(pr.NG, 0) > kMaxLds) return false;
     return forced_on() || (long)pr.B * pr.HW >= 64L * pr.num_cu;
 }
 

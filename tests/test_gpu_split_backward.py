@@ -1,5 +1,5 @@
 """p-norm gradients whose reduction is shared out over workgroups: the one-pass kernel (csrc/norm_backward_fused.hip) and the
-separate grad_input (csrc/norm_backward_kernel.hpp) at the edges of their tiles and shares, against the oracle: one row to one
+grad_input of the general kernel (csrc/norm_backward_kernel.hpp) at the edges of their tiles and shares, against the oracle: one row to one
 past a tile, outputs that end inside a stage and inside a share, four inputs to one vector past a tile, groups."""
 import pytest
 import torch
@@ -49,3 +49,28 @@ def test_forward_tiles_of_eight_groups(shape, p):
     x, w = make_inputs(B, CO, CI, G, 1, seed=sum(shape))
     got = gpu_norm_forward(x, w, G, p)
     torch.testing.assert_close(got, oracle.norm_dist_forward(x, w, G, p), rtol=1e-5, atol=1e-6)
+
+
+# More outputs per group than one block of 64 holds: just over it, equal blocks, a short last one.
+@pytest.mark.parametrize("p", [8.0, 5.5, 37.3])
+@pytest.mark.parametrize("outputs", [65, 96, 257])
+def test_conv_backward_in_blocks_of_outputs(outputs, p):
+    from gpu_common import DEV, cpp, say, set_tile
+    from test_gpu_parity import test_norm_conv_backward_both_gradients_in_one_pass_from_the_image as from_the_image
+    try:
+        from_the_image((2, 10, 11, 9, outputs, 1, 2 if outputs == 96 else 1, 1, 1), p)
+        B, CI, HW = 3, 70, 50
+        say("blocks, columns", outputs, "p", p)
+        x, w = make_inputs(B, CI=CI, CO=outputs, G=1, HW=HW, seed=outputs)
+        go = torch.randn(B, outputs, HW, generator=gen(3))
+        out = oracle.norm_dist_forward(x, w, 1, p)
+        ex, mx = oracle.norm_dist_backward_input(go, x, w, out, 1, p, with_abs_terms=True)
+        ew, mw = oracle.norm_dist_backward_weight(go, x, w, out, 1, p, with_abs_terms=True)
+        set_tile(0)
+        gx, gw = torch.full((B, CI, HW), float("nan"), device=DEV), torch.zeros((outputs, CI), device=DEV)
+        cpp.norm_dist_backward(*(t.to(DEV) for t in (go, x, w, out)), gx, gw, 1, p)
+        torch.cuda.synchronize()
+        assert_sum_close(gx.cpu(), ex, mx, p, 1e-5, 1e-6)
+        assert_sum_close(gw.cpu(), ew, mw, p, 1e-5, 1e-6)
+    finally:
+        set_tile(-1)
