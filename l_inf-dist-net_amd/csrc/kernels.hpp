@@ -108,8 +108,9 @@ hipError_t inf_backward_weight(const float* grad_output, const int32_t* pos, flo
                                bool overwrite, hipStream_t stream);
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
                         bool values_only, hipStream_t stream);
+// `shared`: a small problem's outputs may be shared out over workgroups whose sums meet by float atomics, in no fixed order.
 hipError_t norm_backward_input(const float* grad_output, const float* input, const float* weight,
-                               const float* output, float* grad_input, float p, const Problem& pr,
+                               const float* output, float* grad_input, float p, const Problem& pr, bool shared,
                                hipStream_t stream);
 bool norm_backward_input_tiled_applicable(const Problem& pr, float p, const void* grad_output, const void* input,
                                           const void* weight, const void* output, const void* grad_input);

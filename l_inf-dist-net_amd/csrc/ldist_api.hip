@@ -211,7 +211,7 @@ int ldist_norm_dist_backward_input(const float* grad_output, const float* input,
     if (!grad_output || !input || !weight || !output || !grad_input || !valid_p(p)) return LDIST_EINVAL;
     ldist::Problem pr{};
     if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
-    return finish(ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr,
+    return finish(ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, false,
                                              (hipStream_t)stream));
 }
 
@@ -237,7 +237,7 @@ int ldist_norm_dist_backward(const float* grad_output, const float* input, const
     if (ldist::norm_conv_backward_fused_applicable(pr))
         return finish(ldist::norm_conv_backward_fused_columns(grad_output, input, weight, output, grad_input, grad_weight,
                                                               p, pr, (hipStream_t)stream));
-    if (hipError_t e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, (hipStream_t)stream);
+    if (hipError_t e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, true, (hipStream_t)stream);
         e != hipSuccess)
         return finish(e);
     return finish(ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr,

@@ -287,7 +287,7 @@ norm_backward_kernel(const float* __restrict__ grad_output, const float* __restr
 
 template <bool WEIGHT, int BA, int BKO, bool IMG>
 static hipError_t launch_norm_backward_ba(const float* grad_output, const float* input, const float* weight,
-                                          const float* output, float* grad, float p, const Problem& pr,
+                                          const float* output, float* grad, float p, const Problem& pr, bool shared,
                                           hipStream_t stream, const ImgWin& win) {
     const NbDims d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW};
     const int A = WEIGHT ? d.NG : d.M;
@@ -295,7 +295,9 @@ static hipError_t launch_norm_backward_ba(const float* grad_output, const float*
     const int tiles_a = (A + BA - 1) / BA, tiles_k = (d.K + BKO - 1) / BKO;
     const long tiles = (long)tiles_a * tiles_k * d.G;
     int splits = 1;
-    if (tiles < 2L * pr.num_cu) {  // few output tiles, long reduction (over the rows, or the outputs): share it out
+    // few output tiles, long reduction (over the rows, or the outputs): share it out.  grad_input only where the caller
+    // does not promise the same bits in every run (64 x 5120 -> 5120 at p = 37.3: 1744 -> 506 us)
+    if (shared && tiles < 2L * pr.num_cu) {
         const long want = (4L * pr.num_cu + tiles - 1) / tiles;
         const long most = max(1L, (long)R / (4 * RB));
         splits = (int)min(want, most);
@@ -323,17 +325,17 @@ static hipError_t launch_norm_backward_ba(const float* grad_output, const float*
 
 template <bool WEIGHT, bool IMG>
 static hipError_t launch_norm_backward(const float* grad_output, const float* input, const float* weight,
-                                       const float* output, float* grad, float p, const Problem& pr,
+                                       const float* output, float* grad, float p, const Problem& pr, bool shared,
                                        hipStream_t stream, const ImgWin& win) {
     // 64-row tiles unless they would give fewer than four workgroups per CU (and the rows allow halving);
     // P with at most 32 rows (grad_weight of a grouped layer with few outputs per group): 32 x 128 tiles
     const int A = WEIGHT ? pr.NG : pr.B * pr.HW;
     if (A <= 32 && pr.K > 64)
-        return launch_norm_backward_ba<WEIGHT, 32, 128, IMG>(grad_output, input, weight, output, grad, p, pr, stream, win);
+        return launch_norm_backward_ba<WEIGHT, 32, 128, IMG>(grad_output, input, weight, output, grad, p, pr, shared, stream, win);
     const long tiles64 = (long)((A + 63) / 64) * ((pr.K + 63) / 64) * pr.G;
     if (tiles64 < 4L * pr.num_cu && A > 32)
-        return launch_norm_backward_ba<WEIGHT, 32, 64, IMG>(grad_output, input, weight, output, grad, p, pr, stream, win);
-    return launch_norm_backward_ba<WEIGHT, 64, 64, IMG>(grad_output, input, weight, output, grad, p, pr, stream, win);
+        return launch_norm_backward_ba<WEIGHT, 32, 64, IMG>(grad_output, input, weight, output, grad, p, pr, shared, stream, win);
+    return launch_norm_backward_ba<WEIGHT, 64, 64, IMG>(grad_output, input, weight, output, grad, p, pr, shared, stream, win);
 }
 
 }  // namespace ldist

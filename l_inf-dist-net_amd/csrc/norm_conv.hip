@@ -58,7 +58,7 @@ hipError_t norm_conv_backward_input(const float* grad_output, const float* img, 
     const Problem pr = problem_of(q, G, CO, num_cu, device);
     const size_t n = (size_t)q.B * q.C * q.H * q.W;
     if (hipError_t e = zero_fill(grad_img, n, stream); e != hipSuccess) return e;
-    return launch_norm_backward<false, true>(grad_output, img, weight, output, grad_img, p, pr, stream, window_of(q, G));
+    return launch_norm_backward<false, true>(grad_output, img, weight, output, grad_img, p, pr, true, stream, window_of(q, G));
 }
 
 // grad_weight is added to, as in the column entry point.
@@ -66,7 +66,7 @@ hipError_t norm_conv_backward_weight(const float* grad_output, const float* img,
                                      const float* output, float* grad_weight, float p, const ConvGeom& q, int G, int CO,
                                      int num_cu, int device, hipStream_t stream) {
     const Problem pr = problem_of(q, G, CO, num_cu, device);
-    return launch_norm_backward<true, true>(grad_output, img, weight, output, grad_weight, p, pr, stream, window_of(q, G));
+    return launch_norm_backward<true, true>(grad_output, img, weight, output, grad_weight, p, pr, true, stream, window_of(q, G));
 }
 
 }  // namespace ldist
