@@ -64,8 +64,8 @@ struct ConvBwd {
 // A group's outputs are taken in equal blocks of up to 64, one after the other over the same units: the two tiles of 128
 // outputs would leave room for one workgroup per CU.  grad_input has one owner all along, who writes it for the first
 // block and adds to it for the others.  128 images of 64 x 16 x 16 (us, both gradients; in brackets the two separate
-// kernels): 128 outputs, p = 8, 1109 -> 604 (811); 192 outputs 902 (1398), at p = 37.3 1345 (2222), which the separate kernels
-// took before; 128 channels to 128 outputs, p = 37.3, 2874 -> 1586 (2810), to 256, p = 8, 2173 (3388).
+// kernels): 128 outputs, p = 8, 1109 -> 556 (811); 192 outputs 834 (1398), at p = 37.3 1301 (2222), which the separate kernels
+// took before; 128 channels to 128 outputs, p = 37.3, 2874 -> 1533 (2810), to 256, p = 8, 2003 (3388).
 inline int outputs_in_block(int NG) {
     const int blocks = (NG + 63) / 64;
     return (NG + blocks - 1) / blocks;
@@ -97,8 +97,10 @@ inline size_t image_floats(int NG, int ring_rows, int H, int W) {
 
 // BLOCKS: more outputs per group than one block holds (its own instantiation: the loop around everything costs registers,
 // 3 % on 32 and 64 outputs).
-template <bool IMG, int IE, bool BLOCKS>
-__global__ void __launch_bounds__(256, 4)   // four workgroups per CU is what LDS allows at 32 outputs per group: 128 registers
+// WAVES: what LDS allows per SIMD, four workgroups per CU (128 registers, some spilled) up to 32 outputs per group, three
+// (168) above (64 -> 64 channels on 128 images of 16 x 16, p = 8: 326 -> 299 us; to 128 outputs 604 -> 556).
+template <bool IMG, int IE, bool BLOCKS, int WAVES>
+__global__ void __launch_bounds__(256, WAVES)
 norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __restrict__ input,
                           const float* __restrict__ weight, const float* __restrict__ output,
                           float* __restrict__ grad_input, float* __restrict__ grad_weight, float e, ConvBwd d,
@@ -108,7 +110,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     const int K = d.K;
     float* Ws = lds;                     // [block][WLD]  w[n][k0 + c]
     float* Gw = Ws + d.block * WLD;      // [block][WLD]  sums for grad_weight[n][k0 + c]
-    float* Cs = Gw + d.block * WLD;           // [chunk][TR]   g, or g / out^IE, of the staged outputs
+    float* Cs = Gw + d.block * WLD;        // [chunk][TR]   g, or g / out^IE, of the staged outputs
     float* Rs = Cs + d.chunk * TR;       // [chunk][TR]   1 / out
     float* Fp = Rs + d.chunk * TR + (IMG ? d.park_extra : 0);   // IMG: [kPlanes][ring_rows][W] gradient of the image rows still being added to
     const int tid = threadIdx.x;
@@ -560,7 +562,7 @@ int ring_rows_for(const ImgWin& win, int HW) {
     return (out_rows - 1) * win.S + 2 * win.D + 1;
 }
 
-template <bool IMG, int IE, bool BLOCKS>
+template <bool IMG, int IE, bool BLOCKS, int WAVES>
 hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
@@ -598,7 +600,7 @@ hipError_t launch_conv_backward_blocks(const float* grad_output, const float* in
     const long slices = (d.units + d.units_per_wg - 1) / d.units_per_wg;
     d.slices = (int)slices;
     const long grid = (pairs * slices + 7) / 8 * 8;   // whole rounds of the eight XCDs; the padding exits at once
-    auto kern = norm_conv_backward_kernel<IMG, IE, BLOCKS>;
+    auto kern = norm_conv_backward_kernel<IMG, IE, BLOCKS, WAVES>;
     static LdsRecord lds_allowed = {};
     // the limit is raised once, to the most any layer may ask for
     if (hipError_t e = allow_lds(kern, kMaxLds, pr.device, lds_allowed); e != hipSuccess) return e;
@@ -611,9 +613,11 @@ template <bool IMG, int IE>
 hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
-    return outputs_in_block(pr.NG) < pr.NG
-        ? launch_conv_backward_blocks<IMG, IE, true>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream)
-        : launch_conv_backward_blocks<IMG, IE, false>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream);
+#define LDIST_LAUNCH(BLOCKS, WAVES) \
+    launch_conv_backward_blocks<IMG, IE, BLOCKS, WAVES>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream)
+    if (outputs_in_block(pr.NG) < pr.NG) return LDIST_LAUNCH(true, 3);
+    return pr.NG > 32 ? LDIST_LAUNCH(false, 3) : LDIST_LAUNCH(false, 4);
+#undef LDIST_LAUNCH
 }
 
 template <bool IMG>
