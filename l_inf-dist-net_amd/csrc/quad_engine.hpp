@@ -67,9 +67,11 @@ struct QPanel {
 #pragma unroll
         for (int i = 0; i < N; i++) {
             if (TOTAL % GEO::NT != 0 && (i * GEO::NT + wave * 64) >= TOTAL) continue;
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+            // A load that takes its LDS address from M0 needs one wait state behind a scalar write of M0, which nobody
+            // adds inside inline assembly.
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                          :: "s"(panel + (unsigned)(i * GEO::NT + wave * 64) * 16u), "v"(off[i] + (4u * (unsigned)k0 - back)), "s"(rsrc), "s"(0)
-                                                  : "memory");
+                         : "memory", "m0");
         }
     }
     // Zeros over what does not belong to the stage in the row's last vectors: the values before the vector that ends
