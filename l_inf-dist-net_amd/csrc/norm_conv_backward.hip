@@ -158,8 +158,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     // carries (p - 1) times as large: inside the tolerance of a gradient whose terms cancel (1e-6 * p / 8 of the sum
     // of their magnitudes) only while |log2 out| < 1.  So everything is taken in units of a power of two read off the
     // outputs of the workgroup's first tile (exact scalings of x, the weights and the outputs; the one nearest to the
-    // geometric mean of the largest and the smallest of them), and a tile takes the form only if all its outputs lie within [1/2, 2] units
-    // (voted on the barrier that follows the staging); other tiles divide first.
+    // geometric mean of the largest and the smallest of them), and a tile takes the form only if p > 2 and all its outputs lie
+    // within [1/2, 2] units (voted on the barrier that follows the staging); other tiles divide first.
     const float em1 = e - 1.0f;   // p - 2
     if (IE == 0 && nb == 0) {
         float top = 0.f, nbot = -__builtin_inff();   // the largest and minus the smallest output of the first tile
@@ -254,7 +254,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         const int cnt = min(d.chunk, NG - nc);
         const int n_lo = second * ((cnt + 1) / 2), n_hi = halved && !second ? (cnt + 1) / 2 : cnt;   // this wave's
         if (nc > 0) __syncthreads();   // everyone has left the outputs before
-        bool unsafe = false;
+        bool unsafe = IE == 0 && !(em1 > 0.f);   // p < 2: the logarithmic form would take x == w for 0 * infinity
         if constexpr (IMG) {
             // A lane takes row r = tid % 64 of outputs tid / 64, + 4, + 8, ...: four outputs per pass, their eight
             // loads in flight together (one output at a time, every load is waited for on its own).  Rows and outputs

@@ -74,3 +74,37 @@ def test_conv_backward_in_blocks_of_outputs(outputs, p):
         assert_sum_close(gw.cpu(), ew, mw, p, 1e-5, 1e-6)
     finally:
         set_tile(-1)
+
+
+# Exponents below 2: a term whose x equals its w is 0 whatever form the kernel takes.  Quantised inputs and weights meet in
+# many elements; a zero row of weights meets the zeros of the padding and the rows past a ragged last tile.
+@pytest.mark.parametrize("p", [1.25, 1.5, 1.9])
+@pytest.mark.parametrize("outputs", [9, 33, 70, 150])
+def test_conv_backward_below_two(outputs, p):
+    import torch.nn.functional as F
+    from gpu_common import DEV, cpp, say, set_tile
+    B, C, H, W = 3, 10, 9, 11
+    say("conv backward below 2", outputs, "p", p)
+    img, w = torch.round(torch.rand(B, C, H, W, generator=gen(outputs)) * 8) / 8, torch.randn(outputs, C * 9, generator=gen(8))
+    w = torch.round(w * 4) / 8
+    w[outputs // 2] = 0.0
+    cols = F.unfold(img, 3, 1, 1, 1).contiguous()
+    go = torch.randn(B, outputs, cols.size(2), generator=gen(9))
+    out = oracle.norm_dist_forward(cols, w, 1, p)
+    ex, mx = oracle.norm_dist_backward_input(go, cols, w, out, 1, p, with_abs_terms=True)
+    ew, mw = oracle.norm_dist_backward_weight(go, cols, w, out, 1, p, with_abs_terms=True)
+    fold = lambda t: F.fold(t.double(), (H, W), 3, 1, 1, 1)
+    g, x, xc, wd, o = (t.to(DEV) for t in (go, img, cols, w, out))
+    try:
+        set_tile(0)
+        gi, gw = torch.full_like(x, float("nan")), torch.zeros_like(wd)
+        cpp.norm_dist_conv_backward(g, x, wd, o, gi, gw, 1, p, 3, 1, 1, 1)
+        gx, gc = torch.full_like(xc, float("nan")), torch.zeros_like(wd)
+        cpp.norm_dist_backward(g, xc, wd, o, gx, gc, 1, p)
+        torch.cuda.synchronize()
+    finally:
+        set_tile(-1)
+    assert_sum_close(gi.cpu(), fold(ex), fold(mx), p, 1e-5, 1e-6)
+    assert_sum_close(gx.cpu(), ex, mx, p, 1e-5, 1e-6)
+    for got in (gw, gc):
+        assert_sum_close(got.cpu(), ew, mw, p, 1e-5, 1e-6)
