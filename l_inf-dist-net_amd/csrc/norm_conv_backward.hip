@@ -97,15 +97,21 @@ inline size_t image_floats(int NG, int ring_rows, int H, int W) {
 
 // BLOCKS: more outputs per group than one block holds (its own instantiation: the loop around everything costs registers,
 // 3 % on 32 and 64 outputs).
-// WAVES: what LDS allows per SIMD, four workgroups per CU (128 registers, some spilled) up to 32 outputs per group, three
-// (168) above (64 -> 64 channels on 128 images of 16 x 16, p = 8: 326 -> 299 us; to 128 outputs 604 -> 556).
-template <bool IMG, int IE, bool BLOCKS, int WAVES>
+// WAVES: what LDS allows per SIMD, four workgroups per CU (128 registers) up to 32 outputs per group, three (168) above
+// (64 -> 64 channels on 128 images of 16 x 16, p = 8: 326 -> 299 us; to 128 outputs 604 -> 556).  With four, nothing that
+// only larger groups need may cost a register: outputs are staged whole (ONE_CHUNK: the loop over chunks around it had the
+// instance for columns spill 108 bytes and the one for images 172, against 0 and 60 without it; 64 images of 71 inputs x
+// 1024 positions to 20 outputs, p = 4, 61 us against 50, 46 images of 14 x 29 x 21 to 6 outputs, p = 62, 90 against 77),
+// and there is no halving where not every tile can be halved.
+// HALF: column tiles of at most half the width are shared by two halves of the workgroup (below).
+template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
 __global__ void __launch_bounds__(256, WAVES)
 norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __restrict__ input,
                           const float* __restrict__ weight, const float* __restrict__ output,
                           float* __restrict__ grad_input, float* __restrict__ grad_weight, float e, ConvBwd d,
                           ImgWin win) {
     constexpr int TC = IMG ? 9 * kPlanes : TCP;   // columns per tile
+    constexpr bool ONE_CHUNK = WAVES == 4;        // up to 32 outputs are staged whole
     extern __shared__ __align__(16) float lds[];
     const int K = d.K;
     float* Ws = lds;                     // [block][WLD]  w[n][k0 + c]
@@ -129,7 +135,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     // A tile of at most 32 columns (three channels: the first layer of a net; the last tile of 64) would leave two of the
     // four waves without columns: they take the same ones and the second half of the outputs instead, and the halves'
     // grad_input sums meet where they are parked (128 images of 3 x 32 x 32 to 32 channels, p = 8: 248 -> 182 us).
-    const bool halved = IMG && min(TC, K - k0) <= TCP / 2;
+    const bool halved = HALF && min(TC, K - k0) <= TCP / 2;
     const int second = halved ? tid >> 7 : 0;   // this wave's half
     const int tx = halved ? (tid / TYN) & 15 : tid / TYN;
     const int u_begin = slice * d.units_per_wg, u_end = min(d.units, u_begin + d.units_per_wg);
@@ -250,8 +256,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
             }
         }
         // g and out of the tile's rows for outputs nc .. nc + cnt - 1 of the group; rows are contiguous in memory
-        for (int nc = 0; nc < NG; nc += d.chunk) {
-        const int cnt = min(d.chunk, NG - nc);
+        for (int nc = 0; nc < (ONE_CHUNK ? 1 : NG); nc += ONE_CHUNK ? 1 : d.chunk) {
+        const int cnt = ONE_CHUNK ? NG : min(d.chunk, NG - nc);
         const int n_lo = second * ((cnt + 1) / 2), n_hi = halved && !second ? (cnt + 1) / 2 : cnt;   // this wave's
         if (nc > 0) __syncthreads();   // everyone has left the outputs before
         bool unsafe = IE == 0 && !(em1 > 0.f);   // p < 2: the logarithmic form would take x == w for 0 * infinity
@@ -562,7 +568,7 @@ int ring_rows_for(const ImgWin& win, int HW) {
     return (out_rows - 1) * win.S + 2 * win.D + 1;
 }
 
-template <bool IMG, int IE, bool BLOCKS, int WAVES>
+template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
 hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
@@ -600,7 +606,7 @@ hipError_t launch_conv_backward_blocks(const float* grad_output, const float* in
     const long slices = (d.units + d.units_per_wg - 1) / d.units_per_wg;
     d.slices = (int)slices;
     const long grid = (pairs * slices + 7) / 8 * 8;   // whole rounds of the eight XCDs; the padding exits at once
-    auto kern = norm_conv_backward_kernel<IMG, IE, BLOCKS, WAVES>;
+    auto kern = norm_conv_backward_kernel<IMG, IE, BLOCKS, WAVES, HALF>;
     static LdsRecord lds_allowed = {};
     // the limit is raised once, to the most any layer may ask for
     if (hipError_t e = allow_lds(kern, kMaxLds, pr.device, lds_allowed); e != hipSuccess) return e;
@@ -613,10 +619,14 @@ template <bool IMG, int IE>
 hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
-#define LDIST_LAUNCH(BLOCKS, WAVES) \
-    launch_conv_backward_blocks<IMG, IE, BLOCKS, WAVES>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream)
-    if (outputs_in_block(pr.NG) < pr.NG) return LDIST_LAUNCH(true, 3);
-    return pr.NG > 32 ? LDIST_LAUNCH(false, 3) : LDIST_LAUNCH(false, 4);
+#define LDIST_LAUNCH(BLOCKS, WAVES, HALF) \
+    launch_conv_backward_blocks<IMG, IE, BLOCKS, WAVES, HALF>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream)
+    if (outputs_in_block(pr.NG) < pr.NG) return LDIST_LAUNCH(true, 3, IMG);
+    if (pr.NG > 32) return LDIST_LAUNCH(false, 3, IMG);
+    // Halving shortens the launch where every column tile is halved; beside whole tiles, which take as long as before, it only
+    // costs its registers (6 % of four-output layers, nothing gained by any with 2 to 17 column tiles).
+    if (IMG && win.CG * 9 <= TCP / 2) return LDIST_LAUNCH(false, 4, IMG);
+    return LDIST_LAUNCH(false, 4, false);
 #undef LDIST_LAUNCH
 }
 
