@@ -61,9 +61,9 @@ struct ConvBwd {
     int chunk;                       // of which g and 1/out are staged at a time
 };
 
-// A group's outputs are taken in equal blocks of up to 64, one after the other over the same units: the two tiles of 128
-// outputs would leave room for one workgroup per CU.  grad_input has one owner all along, who writes it for the first
-// block and adds to it for the others.  128 images of 64 x 16 x 16 (us, both gradients; in brackets the two separate
+// A group's outputs are taken in equal blocks of up to 64, one after the other over the same units, where the device has
+// workgroups for the room this makes: the two tiles of 128 outputs leave room for one per CU.  grad_input has one owner all
+// along, who writes it for the first block and adds to it for the others.  128 images of 64 x 16 x 16 (us, both gradients; in brackets the two separate
 // kernels): 128 outputs, p = 8, 1109 -> 556 (811); 192 outputs 834 (1398), at p = 37.3 1301 (2222), which the separate kernels
 // took before; 128 channels to 128 outputs, p = 37.3, 2874 -> 1533 (2810), to 256, p = 8, 2003 (3388).
 inline int outputs_in_block(int NG) {
@@ -71,33 +71,41 @@ inline int outputs_in_block(int NG) {
     return (NG + blocks - 1) / blocks;
 }
 
-// A tile's g and 1/out are staged for up to 32 outputs at a time, in equal shares of a group's outputs: staged whole, the
-// panels of 64 outputs let a CU hold two workgroups, in halves three.
+// A tile's g and 1/out are staged for up to 32 outputs at a time, in equal shares of a block's outputs, for the same reason:
+// staged whole, the panels of 64 outputs let a CU hold two workgroups, in halves three.
 inline int outputs_staged(int block) {
     const int shares = (block + 31) / 32;
     return (block + shares - 1) / shares;
 }
 
-inline size_t lds_bytes(int NG, size_t plane_floats) {
+struct Pieces { int block, chunk; };   // outputs whose tiles are in LDS, and of which g and 1/out are staged, at a time
+inline Pieces least_pieces(int NG) {
     const int block = outputs_in_block(NG);
-    return ((size_t)2 * block * WLD + (size_t)2 * outputs_staged(block) * TR + plane_floats) * sizeof(float);
+    return {block, outputs_staged(block)};
 }
 
 // IMG: a tile's grad_input sums are parked as [64 columns][64 positions] over the g and 1/out panels; what that
 // takes beyond the panels' 128 floats per staged output
-inline int park_extra(int NG) { return std::max(0, TCP * TR - 2 * outputs_staged(outputs_in_block(NG)) * TR); }
+inline int park_extra(int chunk) { return std::max(0, TCP * TR - 2 * chunk * TR); }
 
 // IMG: the floats behind the panels: the parked tile's overhang, the ring of image rows, a word that stays zero,
 // and the two tables (image row, tap row) -> output row and (image column, tap column) -> output column
-inline size_t image_floats(int NG, int ring_rows, int H, int W) {
-    return (size_t)park_extra(NG) + (size_t)kPlanes * ring_rows * W + 4 + 3 * (size_t)(H + W);
+inline size_t image_floats(int chunk, int ring_rows, int H, int W) {
+    return (size_t)park_extra(chunk) + (size_t)kPlanes * ring_rows * W + 4 + 3 * (size_t)(H + W);
 }
+
+inline size_t lds_bytes(const Pieces& p, size_t plane_floats) {
+    return ((size_t)2 * p.block * WLD + (size_t)2 * p.chunk * TR + plane_floats) * sizeof(float);
+}
+
+// Workgroups that one CU's LDS admits: 160 KB, dealt out in pieces of 1280 bytes; 256 bytes are the kernel's own static words.
+inline long on_a_cu(size_t lds) { return (long)(160 * 1024 / ((lds + 256 + 1279) / 1280 * 1280)); }
 
 }  // namespace
 
 // BLOCKS: more outputs per group than one block holds (its own instantiation: the loop around everything costs registers,
 // 3 % on 32 and 64 outputs).
-// WAVES: what LDS allows per SIMD, four workgroups per CU (128 registers) up to 32 outputs per group, three (168) above
+// WAVES: what LDS allows per SIMD, four workgroups per CU (128 registers) up to 39 outputs per group, three (168) above
 // (64 -> 64 channels on 128 images of 16 x 16, p = 8: 326 -> 299 us; to 128 outputs 604 -> 556).  With four, nothing that
 // only larger groups need may cost a register: outputs are staged whole (ONE_CHUNK: the loop over chunks around it had the
 // instance for columns spill 108 bytes and the one for images 172, against 0 and 60 without it; 64 images of 71 inputs x
@@ -111,7 +119,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                           float* __restrict__ grad_input, float* __restrict__ grad_weight, float e, ConvBwd d,
                           ImgWin win) {
     constexpr int TC = IMG ? 9 * kPlanes : TCP;   // columns per tile
-    constexpr bool ONE_CHUNK = WAVES == 4;        // up to 32 outputs are staged whole
+    constexpr bool ONE_CHUNK = WAVES == 4;        // the whole group is staged at once
     extern __shared__ __align__(16) float lds[];
     const int K = d.K;
     float* Ws = lds;                     // [block][WLD]  w[n][k0 + c]
@@ -571,17 +579,16 @@ int ring_rows_for(const ImgWin& win, int HW) {
 template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
 hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
-                                hipStream_t stream) {
-    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, outputs_in_block(pr.NG),
-              outputs_staged(outputs_in_block(pr.NG))};
+                                const Pieces& pieces, hipStream_t stream) {
+    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, pieces.block, pieces.chunk};
     d.tiles_k = IMG ? (win.CG + kPlanes - 1) / kPlanes : (d.K + TCP - 1) / TCP;
     d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
     const long pairs = (long)d.tiles_k * d.G;
     if constexpr (IMG) {
         d.ring_rows = ring_rows_for(win, pr.HW);
-        d.park_extra = park_extra(d.NG);
+        d.park_extra = park_extra(d.chunk);
     }
-    const size_t lds = lds_bytes(d.NG, IMG ? image_floats(d.NG, d.ring_rows, win.H, win.W) : 0);
+    const size_t lds = lds_bytes(pieces, IMG ? image_floats(d.chunk, d.ring_rows, win.H, win.W) : 0);
     // Units per workgroup.  A CU issues at the same rate whether two, three or four workgroups share it, so what a
     // launch takes is what the busiest CU has to work through: workgroups per CU (dealt round robin) times units per
     // workgroup.  With few long workgroups that is uneven -- 860 workgroups of three images on 256 CUs leave twelve
@@ -619,10 +626,22 @@ template <bool IMG, int IE>
 hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
+    // The fewest pieces with which a CU still holds as many workgroups as the launch has for it (three at most).  Pieces buy
+    // room for more of them and cost a barrier per chunk and a walk over the rows per block; where the launch cannot use the
+    // room they only cost: 44 images of 28 x 25 x 32 to 67 outputs, p = 20.5 (176 workgroups), 568 us in two blocks, 472 whole;
+    // 41 of 9 x 30 x 31 to 78, p = 1.5, 768 and 607; 79 of 12 x 7 x 31 to 33, p = 20.5, 88 and 84.
+    const long units = IMG ? pr.B : ((long)pr.B * pr.HW + TR - 1) / TR;
+    const long wgs = units * (IMG ? (win.CG + kPlanes - 1) / kPlanes : (pr.K + TCP - 1) / TCP) * pr.G;
+    const long wanted = std::min(3L, (wgs + pr.num_cu - 1) / pr.num_cu);
+    const int ring_rows = IMG ? ring_rows_for(win, pr.HW) : 0;
+    Pieces pieces = least_pieces(pr.NG);
+    auto lds_of = [&](const Pieces& c) { return lds_bytes(c, IMG ? image_floats(c.chunk, ring_rows, win.H, win.W) : 0); };
+    for (const Pieces& c : {Pieces{pr.NG, pr.NG}, Pieces{pr.NG, outputs_staged(pr.NG)}})
+        if (lds_of(c) <= kMaxLds && on_a_cu(lds_of(c)) >= wanted) { pieces = c; break; }
 #define LDIST_LAUNCH(BLOCKS, WAVES, HALF) \
-    launch_conv_backward_blocks<IMG, IE, BLOCKS, WAVES, HALF>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, stream)
-    if (outputs_in_block(pr.NG) < pr.NG) return LDIST_LAUNCH(true, 3, IMG);
-    if (pr.NG > 32) return LDIST_LAUNCH(false, 3, IMG);
+    launch_conv_backward_blocks<IMG, IE, BLOCKS, WAVES, HALF>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, pieces, stream)
+    if (pieces.block < pr.NG) return LDIST_LAUNCH(true, 3, IMG);
+    if (pieces.chunk < pr.NG || on_a_cu(lds_of(pieces)) < 4) return LDIST_LAUNCH(false, 3, IMG);
     // Halving shortens the launch where every column tile is halved; beside whole tiles, which take as long as before, it only
     // costs its registers (6 % of four-output layers, nothing gained by any with 2 to 17 column tiles).
     if (IMG && win.CG * 9 <= TCP / 2) return LDIST_LAUNCH(false, 4, IMG);
@@ -658,7 +677,8 @@ bool norm_conv_backward_fused_applicable(const Problem& pr) {
 bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO, int num_cu) {
     if (g_tile_override >= 2 || (long)q.HO * q.WO <= 1) return false;
     const ImgWin win{q.C, q.C / G, q.H, q.W, q.HO, q.WO, q.S, q.P, q.D};
-    if (lds_bytes(CO / G, image_floats(CO / G, ring_rows_for(win, q.HO * q.WO), q.H, q.W)) > kMaxLds) return false;
+    const Pieces least = least_pieces(CO / G);
+    if (lds_bytes(least, image_floats(least.chunk, ring_rows_for(win, q.HO * q.WO), q.H, q.W)) > kMaxLds) return false;
     // the kernel's 32-bit byte offsets: a tile's planes of one image, one image's outputs of a group
     if (4L * kPlanes * q.H * q.W >= (1L << 31) || 4L * (CO / G) * q.HO * q.WO >= (1L << 31)) return false;
     return forced_on() || (long)q.B * q.HO * q.WO >= 64L * num_cu;

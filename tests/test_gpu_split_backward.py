@@ -51,6 +51,17 @@ def test_forward_tiles_of_eight_groups(shape, p):
     torch.testing.assert_close(got, oracle.norm_dist_forward(x, w, G, p), rtol=1e-5, atol=1e-6)
 
 
+# Groups that a workgroup takes whole, in chunks and in blocks: with workgroups for several per CU, 96 and 200 outputs go in
+# blocks, 40 and 64 in chunks; with one or two per CU they stay whole as far as LDS reaches (270 and 300 do not fit whole).
+@pytest.mark.parametrize("p", [8.0, 37.3])
+@pytest.mark.parametrize("case", [(600, 2, 3, 4, 40), (800, 1, 3, 3, 64), (600, 2, 3, 4, 96), (520, 1, 4, 4, 200), (300, 1, 4, 5, 33),
+                                  (280, 3, 4, 4, 67), (9, 8, 5, 7, 130), (5, 2, 6, 6, 270), (3, 10, 5, 5, 300)])
+def test_conv_backward_in_pieces(case, p):
+    from test_gpu_parity import test_norm_conv_backward_both_gradients_in_one_pass_from_the_image as from_the_image
+    B, C, H, W, outputs = case
+    from_the_image((B, C, H, W, outputs, 1, 1, 1, 1), p)
+
+
 # More outputs per group than one block of 64 holds: just over it, equal blocks, a short last one.
 @pytest.mark.parametrize("p", [8.0, 5.5, 37.3])
 @pytest.mark.parametrize("outputs", [65, 96, 257])
