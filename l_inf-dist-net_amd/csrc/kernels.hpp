@@ -160,8 +160,8 @@ hipError_t norm_backward_fused(const float* grad_output, const float* input, con
                                float* grad_input, float* grad_weight, float p, const Problem& pr, hipStream_t stream);
 // Both p-norm gradients of a convolution-shaped layer in one pass (norm_conv_backward.hip), from the unfolded
 // input or from the image.
-bool norm_conv_backward_fused_applicable(const Problem& pr);
-bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO, int num_cu);
+bool norm_conv_backward_fused_applicable(const Problem& pr, float p);
+bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO, float p, int num_cu);
 hipError_t norm_conv_backward_fused_columns(const float* grad_output, const float* input, const float* weight,
                                             const float* output, float* grad_input, float* grad_weight, float p,
                                             const Problem& pr, hipStream_t stream);

@@ -234,7 +234,7 @@ int ldist_norm_dist_backward(const float* grad_output, const float* input, const
     if (ldist::norm_backward_fused_applicable(pr, p, grad_output, input, weight, output, grad_input, grad_weight))
         return finish(ldist::norm_backward_fused(grad_output, input, weight, output, grad_input, grad_weight, p, pr,
                                                  (hipStream_t)stream));
-    if (ldist::norm_conv_backward_fused_applicable(pr))
+    if (ldist::norm_conv_backward_fused_applicable(pr, p))
         return finish(ldist::norm_conv_backward_fused_columns(grad_output, input, weight, output, grad_input, grad_weight,
                                                               p, pr, (hipStream_t)stream));
     if (hipError_t e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, true, (hipStream_t)stream);
@@ -430,7 +430,7 @@ int ldist_norm_dist_conv_backward(const float* grad_output, const float* img, co
     ldist::Problem pr{};
     if (!grad_output || !img || !weight || !output || !grad_img || !grad_weight) return LDIST_EINVAL;
     if (int rc = norm_conv_prepare(B, C, H, W, CO, G, KH, KW, stride, padding, dilation, p, q, pr)) return rc;
-    if (ldist::norm_conv_backward_fused_image_applicable(q, G, CO, pr.num_cu))
+    if (ldist::norm_conv_backward_fused_image_applicable(q, G, CO, p, pr.num_cu))
         return finish(ldist::norm_conv_backward_fused_image(grad_output, img, weight, output, grad_img, grad_weight, p, q,
                                                             G, CO, pr.num_cu, pr.device, (hipStream_t)stream));
     if (hipError_t e = ldist::norm_conv_backward_input(grad_output, img, weight, output, grad_img, p, q, G, CO, pr.num_cu,

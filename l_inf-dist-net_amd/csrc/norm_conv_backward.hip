@@ -664,24 +664,56 @@ hipError_t dispatch_conv_backward(const float* grad_output, const float* input, 
 
 bool forced_on() { return g_tile_override == 0 || g_tile_override == 1; }   // tests and tuning
 
+// Groups of up to this many outputs take the one-pass kernel whenever the layer has the rows: two tiles and two panels of
+// theirs fit one workgroup's LDS beside the ring of any image.
+constexpr int kWholeGroup = 140;
+
+// Whether a larger group is better off in blocks here than on the two separate kernels.  Those cut grad_input and
+// grad_weight into tiles of their own and fill the device whatever the shape; here a launch has `units` (images, or tiles of
+// 64 rows) x column tiles x groups workgroups that each walk all outputs, and a CU with a single one of them runs at about
+// 0.6 of its rate.  `fill` is the share of the device that this keeps busy, `columns` the columns the separate kernels pad to
+// against those padded to here.  A shared term saves half the work and more where it is a logarithm and an exponential, less
+// where it is a few multiplications.  Separate kernels and this one, us, measured on 400 layers (the lines lie where the
+// ratio passes 1):
+//   61 images of 7 x 32 x 26 to 215 outputs, p = 8, fill 0.14                 309 and 1332
+//   24 images of 4 x 29 x 29 to 383 outputs, p = 20.5, fill 0.06              340 and 2964
+//   51 images of 12 columns x 580 to 441 outputs, p = 3, fill 0.90            153 and 237
+//   252 images of 14 x 31 x 18 to 366 outputs, two groups, p = 70, fill 0.98  2012 and 1240
+//   140 images of 41 x 17 x 34 to 199 outputs, p = 8, fill 0.82               2541 and 1964
+bool blocks_pay(long units, int tiles_k, int G, double columns, float p, int num_cu) {
+    const long wgs = units * tiles_k * G, on_busiest = (wgs + num_cu - 1) / num_cu;
+    const double fill = (double)wgs / num_cu / (on_busiest == 1 ? 1.0 / 0.6 : (double)on_busiest);
+    const int ie = small_int_power(p - 1.0f);
+    if (!(ie == 1 || ie == 2 || ie == 3 || ie == 7)) return fill * columns >= 0.66;   // the exponents of dispatch_conv_backward
+    return wgs >= 4L * num_cu || (tiles_k > 1 ? fill >= 0.82 : fill * columns >= 1.2);
+}
+
 }  // namespace
 
 // Whether the one-pass kernel takes a layer given as unfolded columns: the conv layout with enough rows to give
 // every CU work.
-bool norm_conv_backward_fused_applicable(const Problem& pr) {
+bool norm_conv_backward_fused_applicable(const Problem& pr, float p) {
     if (pr.HW == 1 || g_tile_override >= 2) return false;
-    return forced_on() || (long)pr.B * pr.HW >= 64L * pr.num_cu;
+    if (forced_on()) return true;
+    const long rows = (long)pr.B * pr.HW;
+    return rows >= 64L * pr.num_cu && (pr.NG <= kWholeGroup ||
+                                       blocks_pay((rows + TR - 1) / TR, (pr.K + TCP - 1) / TCP, pr.G, 1.0, p, pr.num_cu));
 }
 
 // The same for a layer given as an image: also the ring of image rows of seven channel planes must fit LDS.
-bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO, int num_cu) {
+bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO, float p, int num_cu) {
     if (g_tile_override >= 2 || (long)q.HO * q.WO <= 1) return false;
     const ImgWin win{q.C, q.C / G, q.H, q.W, q.HO, q.WO, q.S, q.P, q.D};
     const Pieces least = least_pieces(CO / G);
     if (lds_bytes(least, image_floats(least.chunk, ring_rows_for(win, q.HO * q.WO), q.H, q.W)) > kMaxLds) return false;
     // the kernel's 32-bit byte offsets: a tile's planes of one image, one image's outputs of a group
     if (4L * kPlanes * q.H * q.W >= (1L << 31) || 4L * (CO / G) * q.HO * q.WO >= (1L << 31)) return false;
-    return forced_on() || (long)q.B * q.HO * q.WO >= 64L * num_cu;
+    if (forced_on()) return true;
+    if ((long)q.B * q.HO * q.WO < 64L * num_cu) return false;
+    if (CO / G <= kWholeGroup) return true;
+    const int tiles_k = (win.CG + kPlanes - 1) / kPlanes, last = win.CG - kPlanes * (tiles_k - 1), L = q.HO * q.WO;
+    const double here = (tiles_k - 1) * TCP + (last * 9 <= TCP / 2 ? TCP / 2 : TCP), there = (win.CG * 9 + 63) / 64 * 64;
+    return blocks_pay(q.B, tiles_k, G, there / here * L / ((L + TR - 1) / TR * TR), p, num_cu);
 }
 
 // From the unfolded input (B, CI, HW): every element of grad_input is written, grad_weight is added to.

@@ -62,6 +62,34 @@ def test_conv_backward_in_pieces(case, p):
     from_the_image((B, C, H, W, outputs, 1, 1, 1, 1), p)
 
 
+# Large groups left to the library: the two separate kernels where the layer has few images or column tiles, blocks in one pass
+# where it fills the device.
+@pytest.mark.parametrize("p", [3.0, 20.5])
+@pytest.mark.parametrize("case", [(17, 4, 31, 33, 171), (260, 7, 8, 8, 170), (520, 9, 6, 7, 150)])
+def test_conv_backward_of_large_groups(case, p):
+    import torch.nn.functional as F
+    from gpu_common import DEV, cpp, say
+    B, C, H, W, outputs = case
+    say("large group", case, "p", p)
+    g = gen(sum(case))
+    img, w = torch.rand(B, C, H, W, generator=g), torch.randn(outputs, C * 9, generator=g) / (C * 9) ** 0.5
+    cols = F.unfold(img, 3, 1, 1, 1).contiguous()
+    go = torch.randn(B, outputs, H * W, generator=g)
+    out = oracle.norm_dist_forward(cols, w, 1, p)
+    ex, mx = oracle.norm_dist_backward_input(go, cols, w, out, 1, p, with_abs_terms=True)
+    ew, mw = oracle.norm_dist_backward_weight(go, cols, w, out, 1, p, with_abs_terms=True)
+    fold = lambda t: F.fold(t.double(), (H, W), 3, 1, 1, 1)
+    gi, gw = torch.full((B, C, H, W), float("nan"), device=DEV), torch.zeros((outputs, C * 9), device=DEV)
+    cpp.norm_dist_conv_backward(*(t.to(DEV) for t in (go, img, w, out)), gi, gw, 1, p, 3, 1, 1, 1)
+    gx, gc = torch.full(cols.shape, float("nan"), device=DEV), torch.zeros_like(gw)
+    cpp.norm_dist_backward(*(t.to(DEV) for t in (go, cols, w, out)), gx, gc, 1, p)
+    torch.cuda.synchronize()
+    assert_sum_close(gi.cpu(), fold(ex), fold(mx), p, 1e-5, 1e-6)
+    assert_sum_close(gx.cpu(), ex, mx, p, 1e-5, 1e-6)
+    for got in (gw, gc):
+        assert_sum_close(got.cpu(), ew, mw, p, 1e-5, 1e-6)
+
+
 # More outputs per group than one block of 64 holds: just over it, equal blocks, a short last one.
 @pytest.mark.parametrize("p", [8.0, 5.5, 37.3])
 @pytest.mark.parametrize("outputs", [65, 96, 257])
