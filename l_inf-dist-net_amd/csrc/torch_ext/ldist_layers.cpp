@@ -531,6 +531,9 @@ std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Ten
 struct Margins : public Function<Margins> {
     static Tensor forward(AutogradContext* ctx, const Tensor& lower, const Tensor& upper, const Tensor& targets) {
         const On on(upper);
+        // torch's own look-up of the label's lower bound, for what it does with a target that is no class: the kernel below
+        // would leave NaN in such a row and go on
+        lower.gather(1, targets.view({-1, 1}));
         Tensor m = torch::empty_like(upper);
         done("certified_margins", ldist_certified_margins(in(lower), in(upper), targets.const_data_ptr<int64_t>(),
                                                           (int)upper.size(0), (int)upper.size(1), out(m), on.stream));

@@ -129,6 +129,27 @@ def test_margins_and_their_gradients(both_routes):
     torch.testing.assert_close(ga, gb, rtol=1e-6, atol=1e-6)
 
 
+def test_margins_look_the_label_up_as_torch_does(both_routes):
+    """What torch's gather does with a target that is no class, both routes do: it sees the targets on either."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    up, t = torch.randn(5, 10, generator=gen(8)).to(DEV), torch.arange(5, device=DEV)
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func is torch.ops.aten.gather.default:
+                self.indices.append(args[2].flatten().clone())
+            return func(*args, **(kwargs or {}))
+
+    def run():
+        mode = Seen()
+        mode.indices = []
+        with mode:
+            pkg.BoundFinalIdentity()(up, up - 1, up + 1, t)
+        return mode.indices
+    for indices in both_routes(run):
+        assert len(indices) == 1 and torch.equal(indices[0], t)
+
+
 def test_attack_and_optimizer_agree(both_routes):
     def run():
         torch.manual_seed(0)
