@@ -597,12 +597,14 @@ void adamw_step(const std::vector<Tensor>& params, const std::vector<Tensor>& gr
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "Native host path of the L_p / L_inf distance layers on MI355X (gfx950)";
-    m.def("norm_dist", &norm_dist);
-    m.def("inf_dist_bound", &inf_dist_bound);
-    m.def("layer", &layer);
-    m.def("layer_bounds", &layer_bounds);
-    m.def("layer_value_bounds", &layer_value_bounds);
-    m.def("margins", &margins);
-    m.def("pgd_step", &pgd_step);
-    m.def("adamw_step", &adamw_step);
+    // Without the interpreter lock, which nothing in here needs: threads that each drive a stream run side by side.
+    using no_lock = py::call_guard<py::gil_scoped_release>;
+    m.def("norm_dist", &norm_dist, no_lock());
+    m.def("inf_dist_bound", &inf_dist_bound, no_lock());
+    m.def("layer", &layer, no_lock());
+    m.def("layer_bounds", &layer_bounds, no_lock());
+    m.def("layer_value_bounds", &layer_value_bounds, no_lock());
+    m.def("margins", &margins, no_lock());
+    m.def("pgd_step", &pgd_step, no_lock());
+    m.def("adamw_step", &adamw_step, no_lock());
 }

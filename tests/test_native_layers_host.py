@@ -1,0 +1,56 @@
+"""The native host path of the layers (csrc/torch_ext/ldist_layers.cpp) where no GPU is needed: what it does before it looks at
+the device of its tensors."""
+import threading
+import time
+
+import pytest
+import torch
+
+import __graft_entry__ as entry
+
+pkg = entry.load_package()
+
+
+@pytest.fixture(scope="module")
+def ops():
+    module = pkg.norm_dist_cpp._compiled("ldist_layers")
+    if module is None:
+        pytest.skip("torch_ext has not been built")
+    return module
+
+
+def _longest_pause_of_another_thread(call):
+    """Seconds of `call`, and the longest time another thread found no turn meanwhile."""
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0.001)
+    other = threading.Thread(target=tick)
+    other.start()
+    time.sleep(0.02)
+    begin = time.perf_counter()
+    with pytest.raises(RuntimeError, match="CUDA"):
+        call()
+    end = time.perf_counter()
+    stop.set()
+    other.join()
+    inside = [begin] + [t for t in ticks if begin < t < end] + [end]
+    return end - begin, max(b - a for a, b in zip(inside, inside[1:]))
+
+
+def test_other_threads_run_during_a_call(ops):
+    """The functions make strided tensors contiguous before they refuse what is not on a GPU: time to spend without the
+    interpreter lock.  Held, no other thread would have a turn before the call returns."""
+    wide = torch.zeros(6000, 6000).t()
+    targets = torch.zeros(6000, dtype=torch.int64)
+    threads = torch.get_num_threads()
+    torch.set_num_threads(1)
+    try:
+        for call in (lambda: ops.pgd_step(wide, wide, wide, 0.1, 0.1, 0.0, 1.0), lambda: ops.margins(wide, wide, targets),
+                     lambda: ops.layer(wide, wide.view(6000, 6000, 1, 1), None, None, 0.0, False, 1, 8.0, 1, 1, 0, 1, True, 0)):
+            took, pause = _longest_pause_of_another_thread(call)
+            assert pause < 0.5 * took, (took, pause)
+    finally:
+        torch.set_num_threads(threads)
