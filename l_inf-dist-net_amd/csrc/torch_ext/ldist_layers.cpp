@@ -404,6 +404,12 @@ Tensor as_output(const Tensor& y, const Tensor& x, const Window& win) {
     return y.view({y.size(0), y.size(1), ho, wo});
 }
 
+// What the library would refuse, before `positions` divides by the stride.
+void check_window(const Window& win) {
+    TORCH_CHECK(win.trivial() || (win.k > 0 && win.stride > 0 && win.pad >= 0 && win.dil > 0),
+                "the window needs a positive size, stride and dilation, and no negative padding");
+}
+
 // The weight of a layer on x (B, CI, H, W) or (B, CI) is (CO, CI/G, k, k): the kernels that read the image take its
 // channels from the image and the reduction's length from the window, so both have to agree with what the weight holds.
 void check_weight(const Tensor& w, const Tensor& x, int64_t G, const Window& win) {
@@ -424,6 +430,7 @@ std::tuple<Tensor, bool> layer(const Tensor& x, const Tensor& weight, const OptT
                                double momentum, bool training, int64_t G, double p, int64_t k, int64_t stride, int64_t pad,
                                int64_t dil, bool finite_p_from_image, int64_t folded_max_row) {
     const Window win{k, stride, pad, dil};
+    check_window(win);
     const Tensor w = weight.contiguous();
     check_weight(w, x, G, win);
     check_per_channel(bias, "bias", w);
@@ -471,6 +478,7 @@ std::tuple<Tensor, Tensor, bool> layer_bounds(const Tensor& lower, const Tensor&
                                               int64_t dil) {
     at::NoGradGuard no_grad;
     const Window win{k, stride, pad, dil};
+    check_window(win);
     const Tensor w = weight.contiguous();
     check_weight(w, lower, G, win);
     check_per_channel(bias, "bias", w);

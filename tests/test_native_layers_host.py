@@ -54,3 +54,13 @@ def test_other_threads_run_during_a_call(ops):
             assert pause < 0.5 * took, (took, pause)
     finally:
         torch.set_num_threads(threads)
+
+
+@pytest.mark.parametrize("stride,padding,dilation", [(0, 1, 1), (-1, 1, 1), (1, -1, 1), (1, 1, 0)])
+def test_a_window_that_is_none_is_refused_with_an_exception(ops, stride, padding, dilation):
+    """A stride of zero would divide the process away, on whatever device the tensors are."""
+    x, w = torch.zeros(2, 3, 8, 8), torch.zeros(4, 3, 3, 3)
+    for call in (lambda: ops.layer(x, w, None, None, 0.0, False, 1, 8.0, 3, stride, padding, dilation, True, 0),
+                 lambda: ops.layer_bounds(x, x, w, None, None, 1, 3, stride, padding, dilation)):
+        with pytest.raises(RuntimeError, match="window"):
+            call()
