@@ -237,7 +237,8 @@ int ldist_norm_dist_backward(const float* grad_output, const float* input, const
     if (ldist::norm_conv_backward_fused_applicable(pr, p))
         return finish(ldist::norm_conv_backward_fused_columns(grad_output, input, weight, output, grad_input, grad_weight,
                                                               p, pr, (hipStream_t)stream));
-    if (hipError_t e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, true, (hipStream_t)stream);
+    const bool shared = ldist::g_tile_override < 0;   // forced onto the separate kernels, grad_input keeps a fixed order
+    if (hipError_t e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, shared, (hipStream_t)stream);
         e != hipSuccess)
         return finish(e);
     return finish(ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr,

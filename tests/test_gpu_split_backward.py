@@ -147,3 +147,43 @@ def test_conv_backward_below_two(outputs, p):
     assert_sum_close(gx.cpu(), ex, mx, p, 1e-5, 1e-6)
     for got in (gw, gc):
         assert_sum_close(got.cpu(), ew, mw, p, 1e-5, 1e-6)
+
+
+# ldist_set_tile_override(2): the separate kernels, whose grad_input is added up in the order that its own entry point keeps.
+@pytest.mark.parametrize("shape", [(40, 1040, 130, 1, 1), (64, 2048, 96, 2, 1), (3, 520, 24, 1, 20)])
+def test_forced_separate_kernels_keep_the_order_of_grad_input(shape):
+    from gpu_common import DEV, cpp, gpu_norm_forward, say, set_tile
+    B, CO, CI, G, HW = shape
+    say("fixed order", shape)
+    x, w = make_inputs(B, CO, CI, G, HW, seed=sum(shape))
+    go = torch.randn(B, CO, HW, generator=gen(7)).to(DEV)
+    out = gpu_norm_forward(x, w, G, 37.3).to(DEV)
+    x, w = x.to(DEV), w.to(DEV)
+    own, both, gw = torch.empty_like(x), torch.empty_like(x), torch.zeros_like(w)
+    try:
+        set_tile(2)
+        cpp.norm_dist_backward_input(go, x, w, out, own, G, 37.3)
+        cpp.norm_dist_backward(go, x, w, out, both, gw, G, 37.3)
+        torch.cuda.synchronize()
+    finally:
+        set_tile(-1)
+    assert torch.equal(own, both)
+
+
+# The same split in the unfolded layout: few tiles, many outputs.
+@pytest.mark.parametrize("p", [3.0, 37.3])
+@pytest.mark.parametrize("shape", [(3, 520, 24, 1, 20), (2, 1030, 70, 2, 33), (1, 300, 9, 1, 2)])
+def test_shared_grad_input_of_columns(shape, p):
+    from gpu_common import DEV, cpp, say
+    B, CO, CI, G, HW = shape
+    say("split grad_input, columns", shape, "p", p)
+    x, w = make_inputs(B, CO, CI, G, HW, seed=sum(shape))
+    go = torch.randn(B, CO, HW, generator=gen(7))
+    out = oracle.norm_dist_forward(x, w, G, p)
+    ex, mx = oracle.norm_dist_backward_input(go, x, w, out, G, p, with_abs_terms=True)
+    ew, mw = oracle.norm_dist_backward_weight(go, x, w, out, G, p, with_abs_terms=True)
+    gx, gw = torch.full((B, CI, HW), float("nan"), device=DEV), torch.zeros((CO, CI // G), device=DEV)
+    cpp.norm_dist_backward(*(t.to(DEV) for t in (go, x, w, out)), gx, gw, G, p)
+    torch.cuda.synchronize()
+    assert_sum_close(gx.cpu(), ex, mx, p, 1e-5, 1e-6)
+    assert_sum_close(gw.cpu(), ew, mw, p, 1e-5, 1e-6)
