@@ -171,6 +171,14 @@ LDIST_API int ldist_norm_dist_backward(const float* grad_output, const float* in
                                        const float* output, int B, int CO, int CI, int G, int HW, float* grad_input,
                                        float* grad_weight, float p, ldist_stream_t stream);
 
+/* Either p-norm gradient or both (a NULL gradient is left out), every sum added up in one order: the same bits in every run.
+ * What torch.use_deterministic_algorithms(True) asks of the layers.  The separate kernels, never shared out over workgroups,
+ * so small layers take several times as long as in ldist_norm_dist_backward.  No counterpart in the reference, whose atomics
+ * keep no order.  grad_input and grad_weight as there. */
+LDIST_API int ldist_norm_dist_backward_ordered(const float* grad_output, const float* input, const float* weight,
+                                               const float* output, int B, int CO, int CI, int G, int HW, float* grad_input,
+                                               float* grad_weight, float p, ldist_stream_t stream);
+
 /* The two scatter backward passes again, but writing EVERY element of the
  * gradient (zeros where nothing lands) so the caller can pass uninitialised
  * memory and skip its own zero fill.  No counterpart in the reference, which

@@ -31,6 +31,7 @@ SIGNATURES = {
     "ldist_norm_dist_forward_values": [_F, _F, _i, _i, _i, _i, _i, _F, _f, _S],
     "ldist_norm_dist_backward_input": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _f, _S],
     "ldist_norm_dist_backward_weight": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _f, _S],
+    "ldist_norm_dist_backward_ordered": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _S],
     "ldist_norm_dist_backward": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _S],
     "ldist_mean_shift": [_F, _i, _i, _i, _F, _F, _F, _f, _S],
     "ldist_unfold": [_F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _S],

@@ -108,7 +108,8 @@ hipError_t inf_backward_weight(const float* grad_output, const int32_t* pos, flo
                                bool overwrite, hipStream_t stream);
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
                         bool values_only, hipStream_t stream);
-// `shared`: a small problem's outputs may be shared out over workgroups whose sums meet by float atomics, in no fixed order.
+// `shared`, here and for grad_weight: a small problem's outputs (rows) may be shared out over workgroups whose sums meet by
+// float atomics, in no fixed order.
 hipError_t norm_backward_input(const float* grad_output, const float* input, const float* weight,
                                const float* output, float* grad_input, float p, const Problem& pr, bool shared,
                                hipStream_t stream);
@@ -123,7 +124,7 @@ hipError_t norm_backward_weight_tiled(const float* grad_output, const float* inp
                                       const float* output, float* grad_weight, float p, const Problem& pr,
                                       hipStream_t stream);
 hipError_t norm_backward_weight(const float* grad_output, const float* input, const float* weight,
-                                const float* output, float* grad_weight, float p, const Problem& pr,
+                                const float* output, float* grad_weight, float p, const Problem& pr, bool shared,
                                 hipStream_t stream);
 
 hipError_t mean_shift(const float* x, float* y, float* mean_out, float* running_mean, float momentum, int B, int C,

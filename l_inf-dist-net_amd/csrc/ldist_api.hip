@@ -221,7 +221,7 @@ int ldist_norm_dist_backward_weight(const float* grad_output, const float* input
     if (!grad_output || !input || !weight || !output || !grad_weight || !valid_p(p)) return LDIST_EINVAL;
     ldist::Problem pr{};
     if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
-    return finish(ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr,
+    return finish(ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr, true,
                                               (hipStream_t)stream));
 }
 
@@ -241,8 +241,22 @@ int ldist_norm_dist_backward(const float* grad_output, const float* input, const
     if (hipError_t e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, shared, (hipStream_t)stream);
         e != hipSuccess)
         return finish(e);
-    return finish(ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr,
+    return finish(ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr, true,
                                               (hipStream_t)stream));
+}
+
+int ldist_norm_dist_backward_ordered(const float* grad_output, const float* input, const float* weight, const float* output,
+                                     int B, int CO, int CI, int G, int HW, float* grad_input, float* grad_weight, float p,
+                                     ldist_stream_t stream) {
+    if (!grad_output || !input || !weight || !output || (!grad_input && !grad_weight) || !valid_p(p)) return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
+    hipError_t e = hipSuccess;
+    if (grad_input)
+        e = ldist::norm_backward_input(grad_output, input, weight, output, grad_input, p, pr, false, (hipStream_t)stream);
+    if (e == hipSuccess && grad_weight)
+        e = ldist::norm_backward_weight(grad_output, input, weight, output, grad_weight, p, pr, false, (hipStream_t)stream);
+    return finish(e);
 }
 
 int ldist_mean_shift(const float* x, int B, int C, int L, float* y, float* mean_out, float* running_mean,

@@ -22,11 +22,11 @@ hipError_t norm_backward_input(const float* grad_output, const float* input, con
 }
 
 hipError_t norm_backward_weight(const float* grad_output, const float* input, const float* weight,
-                                const float* output, float* grad_weight, float p, const Problem& pr,
+                                const float* output, float* grad_weight, float p, const Problem& pr, bool shared,
                                 hipStream_t stream) {
     if (norm_backward_weight_tiled_applicable(pr, p, grad_output, input, weight, output, grad_weight))
         return norm_backward_weight_tiled(grad_output, input, weight, output, grad_weight, p, pr, stream);
-    return launch_norm_backward<true, false>(grad_output, input, weight, output, grad_weight, p, pr, true, stream, ImgWin{});
+    return launch_norm_backward<true, false>(grad_output, input, weight, output, grad_weight, p, pr, shared, stream, ImgWin{});
 }
 
 }  // namespace ldist

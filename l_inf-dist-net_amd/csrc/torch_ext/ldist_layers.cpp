@@ -191,7 +191,13 @@ struct ColumnLayer : public Function<ColumnLayer> {
         } else {
             const Tensor &x = saved[0], &w = saved[1], &aux = saved[2];
             if (want_w) gw = torch::zeros_like(w);   // the kernels add onto this buffer
-            if (want_x && want_w)
+            if (at::globalContext().deterministicAlgorithms()) {
+                if (want_x || want_w)
+                    done("norm_dist_backward_ordered",
+                         ldist_norm_dist_backward_ordered(in(g), in(x), in(w), in(aux), s.B, s.CO, s.CI, (int)G, s.HW,
+                                                          want_x ? out(gx) : nullptr, want_w ? out(gw) : nullptr, (float)p,
+                                                          on.stream));
+            } else if (want_x && want_w)
                 done("norm_dist_backward", ldist_norm_dist_backward(in(g), in(x), in(w), in(aux), s.B, s.CO, s.CI, (int)G, s.HW,
                                                                     out(gx), out(gw), (float)p, on.stream));
             else if (want_x)

@@ -122,6 +122,22 @@ def norm_dist_backward(grad_output, input, weight, output, grad_input, grad_weig
           _p(grad_input), _p(grad_weight), float(p))
 
 
+def norm_dist_backward_ordered(grad_output, input, weight, output, grad_input, grad_weight, G, p):
+    """Either gradient or both (None: not wanted), the same bits in every run; buffers as for norm_dist_backward."""
+    grads = [(t, n) for t, n in ((grad_input, "grad_input"), (grad_weight, "grad_weight")) if t is not None]
+    for t, n in [(grad_output, "grad_output"), (input, "input"), (weight, "weight"), (output, "output")] + grads:
+        _check_input(t, n)
+    dev = _same_device(grad_output, input, weight, output, *(t for t, _ in grads))
+    B, CO, CI, HW = grad_output.size(0), output.size(1), input.size(1), input.size(2)
+    _expect(weight.size(0) == CO and weight.size(1) * G == CI, "weight must be (CO, CI/G)")
+    _expect(tuple(output.shape) == (B, CO, HW) and tuple(grad_output.shape) == (B, CO, HW),
+            "output and grad_output must be (B, CO, HW)")
+    _expect(input.size(0) == B and (grad_input is None or grad_input.shape == input.shape), "grad_input must match input")
+    _expect(grad_weight is None or grad_weight.shape == weight.shape, "grad_weight must match weight")
+    _call("ldist_norm_dist_backward_ordered", dev, _p(grad_output), _p(input), _p(weight), _p(output), B, CO, CI, G, HW,
+          *(None if t is None else _p(t) for t in (grad_input, grad_weight)), float(p))
+
+
 def inf_dist_forward(input, weight, output, pos, G):
     """model/norm_dist.cpp:54-62."""
     for t, n in ((input, "input"), (weight, "weight"), (output, "output")):

@@ -224,3 +224,31 @@ def test_empty_batches_and_other_dimensions():
         pkg.norm_dist(x, w, 1, INF)
     with pytest.raises((RuntimeError, IndexError)):
         pkg.norm_dist(x.view(4, 12, 1), w.view(8, 12, 1, 1), 1, INF)
+
+
+# Small layers whose sums are shared out over workgroups unless asked not to: outputs, rows (300 x 40 -> 24), a window.
+@pytest.mark.parametrize("p", [3.0, 8.0, 37.3])
+@pytest.mark.parametrize("case", [(64, 512, 1024, 0), (300, 40, 24, 0), (33, 130, 260, 0), (6, 5, 300, 11)])
+def test_deterministic_p_norm_gradients(both_routes, case, p):
+    B, cin, cout, hw = case
+    x = torch.rand(*((B, cin, hw, hw) if hw else (B, cin)), generator=gen(21)).to(DEV)
+    layer = pkg.NormDistConv(cin, cout, 3, padding=1, p=p) if hw else pkg.NormDist(cin, cout, p=p)
+    layer = layer.to(DEV)
+
+    def run():
+        layer.zero_grad()
+        xi = x.clone().requires_grad_()
+        y = layer(xi)[0]
+        y.backward(torch.sin(torch.arange(y.numel(), device=DEV, dtype=torch.float32)).view_as(y))
+        return [xi.grad, layer.weight.grad.clone()]
+    torch.use_deterministic_algorithms(True)
+    try:
+        native, python = both_routes(lambda: [run() for _ in range(6)])
+    finally:
+        torch.use_deterministic_algorithms(False)
+    for got in native[1:] + python:
+        _same(native[0], got)
+    # The shared form: the same sums in another order, of terms that are powers of numbers rounded a few times (p * 2^-23 and a
+    # few times that); the terms' signs alternate, which a factor of eight covers.
+    for a, b in zip(native[0], run()):
+        assert (a - b).norm() <= 8 * 2.0 ** -23 * (p + 2) * b.norm()
