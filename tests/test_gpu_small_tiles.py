@@ -67,3 +67,23 @@ def test_long_reductions_at_large_exponents_pass_over_small_terms(shape, tile):
     for p in (128.0, 1000.0):
         got, want = gpu_norm_forward(x, w, G, p), oracle.norm_dist_forward(x, w, G, p)
         torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-6)
+
+
+# The forward pass without gradients at the kernel that the library chooses by itself: a few rows, small tiles, the large
+# tiles, a handful of outputs, k that is odd or shorter than a vector, a window's positions.
+@pytest.mark.parametrize("p", [2.0, 3.0, 8.0, 37.3, 300.0])
+@pytest.mark.parametrize("shape", [(1, 1000, 1030, 1, 1), (5, 40, 3, 1, 1), (33, 130, 257, 2, 1), (100, 513, 2051, 1, 1),
+                                   (1030, 700, 64, 1, 1), (40, 10, 400, 1, 1), (6, 48, 54, 2, 35)])
+def test_values_without_gradients(shape, p):
+    from gpu_common import DEV, cpp, say
+    import __graft_entry__ as entry
+    B, CO, CI, G, HW = shape
+    say("values", shape, "p", p)
+    x, w = make_inputs(B, CO, CI, G, HW, seed=sum(shape))
+    want = oracle.norm_dist_forward(x, w, G, p)
+    x, w = x.to(DEV), w.to(DEV)
+    got = torch.full((B, CO, HW), float("nan"), device=DEV)
+    cpp.norm_dist_forward_values(x, w, got, G, p)
+    torch.testing.assert_close(got.cpu(), want, rtol=1e-5, atol=1e-6)
+    with torch.no_grad():
+        assert torch.equal(got, entry.load_package().norm_dist(x, w, G, p))
