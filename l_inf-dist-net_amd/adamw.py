@@ -95,7 +95,8 @@ class AdamW(Optimizer):
                 if ops is not None and _fused_ok(prm, grad, m, v):
                     for tensors, t in zip(fused, (prm, grad, m, v)):
                         tensors.append(t)
-                    hyper.append((-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd, state["step"]))
+                    hyper.append((*(float(v) for v in (-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd)),
+                                  int(state["step"])))
                 elif _fused_ok(prm, grad, m, v):
                     norm_dist_cpp.adamw_lp_step(prm, grad, m, v, p_norm, lr, beta1, beta2, eps, wd, state["step"])
                 else:

@@ -78,3 +78,19 @@ def test_the_python_route_takes_the_same_entry_points(monkeypatch):
     pkg.norm_dist(x, w, 2, 8.0)
     assert called == [("norm_dist_forward_values", (5, 8, 1), 2, 8.0), ("norm_dist_forward_values", (5, 8, 1), 2, 3.5),
                       ("norm_dist_forward", (5, 8, 1), 2, 8.0)]
+
+
+def test_adamw_takes_any_number_as_a_step_or_rate(ops, monkeypatch):
+    """A restored state may hold the step count as a float or a tensor; a rate may be a tensor."""
+    layer = pkg.NormDist(6, 4, p=8.0)
+    opt = pkg.AdamW(layer, lr=torch.tensor(1e-2))
+    for prm in layer.parameters():
+        prm.grad = torch.ones_like(prm)
+    opt.step()
+    monkeypatch.setattr("%s._fused_ok" % type(opt).__module__, lambda *tensors: True)
+    monkeypatch.setattr(pkg.norm_dist_cpp, "layer_ops", ops)
+    for step in (3.0, torch.tensor(3.0), 3):
+        for state in opt.state.values():
+            state["step"] = step
+        with pytest.raises(RuntimeError, match="CUDA"):   # as far as the look at the device, with every argument taken
+            opt.step()
