@@ -41,7 +41,7 @@ class BoundFinalIdentity(nn.Module):
         if lower is None or upper is None or targets is None:
             return x
         ops = norm_dist_cpp.native_ops()
-        if (ops is not None and upper.is_cuda and upper.dim() == 2 and upper.numel() > 0 and
+        if (ops is not None and upper.is_cuda and upper.dim() == 2 and 0 < upper.numel() < 2 ** 31 and
                 lower.dtype == upper.dtype == torch.float32 and targets.dtype == torch.int64 and
                 lower.shape == upper.shape and targets.numel() == upper.size(0)):
             return x, ops.margins(lower, upper, targets)   # two kernels instead of four

@@ -2,6 +2,7 @@
 the device of its tensors."""
 import threading
 import time
+from unittest import mock
 
 import pytest
 import torch
@@ -94,3 +95,24 @@ def test_adamw_takes_any_number_as_a_step_or_rate(ops, monkeypatch):
             state["step"] = step
         with pytest.raises(RuntimeError, match="CUDA"):   # as far as the look at the device, with every argument taken
             opt.step()
+
+
+def test_tensors_past_the_native_range_are_left_to_torch(monkeypatch):
+    """The native margins and attack step address 2^31 - 1 values; torch, which ran both before, takes more."""
+    ops = mock.Mock()
+    monkeypatch.setattr(pkg.norm_dist_cpp, "native_ops", lambda: ops)
+    monkeypatch.setattr(pkg.AttackPGD, "_project", lambda self, x, centre=None: x)
+
+    def tensor(rows, columns, dtype=torch.float32):
+        t = mock.MagicMock(is_cuda=True, dtype=dtype, shape=(rows, columns))
+        t.dim.return_value, t.numel.return_value, t.size.return_value = 2, rows * columns, rows
+        for operation in ("__add__", "__sub__", "__rmul__"):
+            getattr(t, operation).return_value = t
+        return t
+
+    for columns, native in ((1, True), (8, False)):
+        t = tensor(2 ** 28, columns)
+        pkg.BoundFinalIdentity()(t, t, t, tensor(2 ** 28, 1, torch.int64))
+        pkg.AttackPGD(None, 0.1, 0.03, 3, 1.0, 0.0)._ascend(t, t, t)
+        assert ops.margins.called == ops.pgd_step.called == native
+        ops.reset_mock()
