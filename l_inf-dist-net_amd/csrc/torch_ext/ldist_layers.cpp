@@ -1,9 +1,10 @@
 // PyTorch-ROCm C++ extension `ldist_layers`: the layers' host path in native code, over the C ABI of libldist_hip.so.
 // What norm_dist.py, mlp.py, harness.py and adamw.py do in Python for tensors they keep the Python route for (CPU
 // tensors, other types, hooked sub-modules), done here for float32 GPU tensors: the same entry points in the same order
-// with the same results.  A layer's forward is one call and one autograd node, and its backward runs without the
-// interpreter; a Python autograd function costs 15 to 30 us per call and direction, more than the kernels of a layer of
-// a thousand neurons take.
+// with the same results, except that a forward pass at finite p that no gradient follows takes
+// ldist_norm_dist_forward_values here and ldist_norm_dist_forward there: the last bits may differ.  A layer's forward is
+// one call and one autograd node, and its backward runs without the interpreter; a Python autograd function costs 15 to
+// 30 us per call and direction, more than the kernels of a layer of a thousand neurons take.
 #include <torch/extension.h>
 
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>

@@ -64,7 +64,8 @@ def norm_dist_forward(input, weight, output, G, p):
 
 def norm_dist_forward_values(input, weight, output, G, p):
     """norm_dist_forward for a forward pass that no gradient follows: free to sum in the order of whichever kernel is
-    fastest for the size (no counterpart in the reference)."""
+    fastest for the size (no counterpart in the reference).  The layers' native host path makes this call; their Python
+    route keeps norm_dist_forward."""
     for t, n in ((input, "input"), (weight, "weight"), (output, "output")):
         _check_input(t, n)
     dev = _same_device(input, weight, output)
@@ -556,8 +557,8 @@ def use_torch_extension(on=True):
 
 
 # The layers' host path in native code (csrc/torch_ext/ldist_layers.cpp: routes, autograd nodes, optimizer loop), over
-# the same library with the same results; None: the Python route of norm_dist.py, which also serves CPU tensors, other
-# types and modules with hooks inside.
+# the same library with the same results (without a gradient and at finite p to the last bits: norm_dist_forward_values);
+# None: the Python route of norm_dist.py, which also serves CPU tensors, other types and modules with hooks inside.
 layer_ops = None
 
 

@@ -80,7 +80,7 @@ def test_layer_routes_agree(both_routes, case, shift, bias, p):
 
     for train, grad in ((True, True), (False, True), (False, False)):
         (a, ra), (b, rb) = both_routes(lambda: step(train, grad))
-        _same(a, b, exact=math.isinf(p) or not grad)
+        _same(a, b, exact=math.isinf(p))   # finite p without gradients may sum in another order
         assert ra == rb
     if math.isinf(p):
         with torch.no_grad():

@@ -67,20 +67,6 @@ def test_a_window_that_is_none_is_refused_with_an_exception(ops, stride, padding
             call()
 
 
-def test_the_python_route_takes_the_same_entry_points(monkeypatch):
-    """Without a gradient to follow, finite p runs norm_dist_forward_values on either route: the same bits."""
-    called = []
-    for name in ("norm_dist_forward", "norm_dist_forward_values"):
-        monkeypatch.setattr(pkg.norm_dist_cpp, name, lambda *args, name=name: called.append((name, tuple(args[2].shape), *args[3:])))
-    x, w = torch.rand(5, 6, 1), torch.rand(8, 3, requires_grad=True)
-    pkg.norm_dist(x, w.detach(), 2, 8.0)
-    with torch.no_grad():
-        pkg.norm_dist(x, w, 2, 3.5)
-    pkg.norm_dist(x, w, 2, 8.0)
-    assert called == [("norm_dist_forward_values", (5, 8, 1), 2, 8.0), ("norm_dist_forward_values", (5, 8, 1), 2, 3.5),
-                      ("norm_dist_forward", (5, 8, 1), 2, 8.0)]
-
-
 def test_adamw_takes_any_number_as_a_step_or_rate(ops, monkeypatch):
     """A restored state may hold the step count as a float or a tensor; a rate may be a tensor."""
     layer = pkg.NormDist(6, 4, p=8.0)
