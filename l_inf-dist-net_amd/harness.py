@@ -7,6 +7,7 @@ Same public names, signatures and results as the reference's model/model.py:3-29
 attack.py:4-36 (AttackPGD), main.py:60-105 (train) and main.py:166-194 (certified_test).
 """
 import contextlib
+import numbers
 
 import torch
 import torch.nn as nn
@@ -105,7 +106,7 @@ class AttackPGD:
         ops = norm_dist_cpp.native_ops()
         if (ops is not None and type(self)._project is AttackPGD._project and adv.is_cuda and adv.numel() < 2 ** 31 and
                 adv.dtype == grad.dtype == inputs.dtype == torch.float32 and adv.shape == inputs.shape and
-                not any(isinstance(v, torch.Tensor) for v in (self.eps, self.step_size, self.up, self.down))):
+                all(isinstance(v, numbers.Real) for v in (self.eps, self.step_size, self.up, self.down))):
             return ops.pgd_step(adv, grad, inputs, self.step_size, self.eps, self.down, self.up)   # one kernel
         return self._project(adv + self.step_size * grad.sign(), centre=inputs)
 

@@ -4,6 +4,7 @@ import threading
 import time
 from unittest import mock
 
+import numpy as np
 import pytest
 import torch
 
@@ -102,3 +103,18 @@ def test_tensors_past_the_native_range_are_left_to_torch(monkeypatch):
         pkg.AttackPGD(None, 0.1, 0.03, 3, 1.0, 0.0)._ascend(t, t, t)
         assert ops.margins.called == ops.pgd_step.called == native
         ops.reset_mock()
+
+
+def test_attack_ranges_per_channel_are_left_to_torch(monkeypatch):
+    """`down` and `up` may be anything that torch.as_tensor takes and that broadcasts; the native step takes numbers."""
+    ops = mock.Mock()
+    monkeypatch.setattr(pkg.norm_dist_cpp, "native_ops", lambda: ops)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+    x, grad = torch.rand(2, 3, 4, 4), torch.randn(2, 3, 4, 4)
+    low = np.array([0.1, 0.2, 0.3], dtype=np.float32).reshape(3, 1, 1)
+    for down, up in ((low, 1.0), (0.0, low + 0.5), (low.tolist(), (low + 0.5).tolist())):
+        got = pkg.AttackPGD(None, 0.1, 0.03, 1, up, down)._ascend(x, grad, x)
+        want = torch.minimum(torch.maximum(x + 0.03 * grad.sign(), torch.as_tensor(down)), torch.as_tensor(up))
+        assert not ops.pgd_step.called and torch.equal(got, want.float())
+    pkg.AttackPGD(None, np.float32(0.1), 0.03, 1, 1, 0)._ascend(x, grad, x)
+    assert ops.pgd_step.called
