@@ -74,34 +74,36 @@ class AdamW(Optimizer):
                 loss = closure()
         fused, hyper = ([], [], [], []), []   # tensors and hyper-parameters of the native call
         ops = norm_dist_cpp.layer_ops
-        for group in self.param_groups:
-            module = group["module"]
-            p_norm = module.p if isinstance(module, NormDistConv) else get_p_norm(module)
-            beta1, beta2 = group["betas"]
-            lr, eps, wd = group["lr"], group["eps"], group["weight_decay"]
-            for prm in group["params"]:
-                grad = prm.grad
-                if grad is None:
-                    continue
-                if grad.is_sparse:
-                    raise RuntimeError("AdamW does not support sparse gradients")
-                state = self.state[prm]
-                if not state:
-                    state["step"] = 0
-                    state["exp_avg"] = torch.zeros_like(prm, memory_format=torch.preserve_format)
-                    state["exp_avg_sq"] = torch.zeros_like(prm, memory_format=torch.preserve_format)
-                state["step"] += 1
-                m, v = state["exp_avg"], state["exp_avg_sq"]
-                if ops is not None and _fused_ok(prm, grad, m, v):
-                    for tensors, t in zip(fused, (prm, grad, m, v)):
-                        tensors.append(t)
-                    hyper.append((*(float(v) for v in (-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd)),
-                                  int(state["step"])))
-                elif _fused_ok(prm, grad, m, v):
-                    norm_dist_cpp.adamw_lp_step(prm, grad, m, v, p_norm, lr, beta1, beta2, eps, wd, state["step"])
-                else:
-                    lp_weight_decay_(prm, p_norm, lr, wd, eps)
-                    _adam_(prm, grad, m, v, lr, beta1, beta2, eps, state["step"])
-        if hyper:
-            ops.adamw_step(*fused, hyper)
+        try:
+            for group in self.param_groups:
+                module = group["module"]
+                p_norm = module.p if isinstance(module, NormDistConv) else get_p_norm(module)
+                beta1, beta2 = group["betas"]
+                lr, eps, wd = group["lr"], group["eps"], group["weight_decay"]
+                for prm in group["params"]:
+                    grad = prm.grad
+                    if grad is None:
+                        continue
+                    if grad.is_sparse:
+                        raise RuntimeError("AdamW does not support sparse gradients")
+                    state = self.state[prm]
+                    if not state:
+                        state["step"] = 0
+                        state["exp_avg"] = torch.zeros_like(prm, memory_format=torch.preserve_format)
+                        state["exp_avg_sq"] = torch.zeros_like(prm, memory_format=torch.preserve_format)
+                    state["step"] += 1
+                    m, v = state["exp_avg"], state["exp_avg_sq"]
+                    if ops is not None and _fused_ok(prm, grad, m, v):
+                        hyper.append((*(float(v) for v in (-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd)),
+                                      int(state["step"])))
+                        for tensors, t in zip(fused, (prm, grad, m, v)):
+                            tensors.append(t)
+                    elif _fused_ok(prm, grad, m, v):
+                        norm_dist_cpp.adamw_lp_step(prm, grad, m, v, p_norm, lr, beta1, beta2, eps, wd, state["step"])
+                    else:
+                        lp_weight_decay_(prm, p_norm, lr, wd, eps)
+                        _adam_(prm, grad, m, v, lr, beta1, beta2, eps, state["step"])
+        finally:   # a parameter that raises leaves those before it with their step taken
+            if hyper:
+                ops.adamw_step(*fused, hyper)
         return loss

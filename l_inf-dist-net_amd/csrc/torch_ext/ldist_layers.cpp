@@ -593,6 +593,8 @@ Tensor pgd_step(const Tensor& adv, const Tensor& grad, const Tensor& centre, dou
 // weight decay and the step count after this one.
 void adamw_step(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& exp_avgs,
                 const std::vector<Tensor>& exp_avg_sqs, const std::vector<std::tuple<double, double, double, double, double, double, int64_t>>& hyper) {
+    TORCH_CHECK(grads.size() == params.size() && exp_avgs.size() == params.size() && exp_avg_sqs.size() == params.size() &&
+                hyper.size() == params.size(), "every parameter needs its gradient, moments and hyper-parameters");
     for (size_t i = 0; i < params.size(); i++) {
         const Tensor &w = params[i], &g = grads[i], &m = exp_avgs[i], &v = exp_avg_sqs[i];
         for (const Tensor* t : {&w, &g, &m, &v}) {

@@ -118,3 +118,25 @@ def test_attack_ranges_per_channel_are_left_to_torch(monkeypatch):
         assert not ops.pgd_step.called and torch.equal(got, want.float())
     pkg.AttackPGD(None, np.float32(0.1), 0.03, 1, 1, 0)._ascend(x, grad, x)
     assert ops.pgd_step.called
+
+
+def test_adamw_steps_what_comes_before_a_parameter_that_raises(monkeypatch):
+    """The native loop takes its parameters together; those before a refused gradient have had their step all the same."""
+    ops, net = mock.Mock(), torch.nn.Sequential(pkg.NormDist(6, 4, p=8.0), pkg.NormDist(4, 3, p=8.0))
+    opt, params = pkg.AdamW(net), list(net.parameters())
+    monkeypatch.setattr("%s._fused_ok" % type(opt).__module__, lambda *tensors: True)
+    monkeypatch.setattr(pkg.norm_dist_cpp, "layer_ops", ops)
+    for prm in params:
+        prm.grad = torch.ones_like(prm)
+    params[2].grad = params[2].grad.to_sparse()
+    with pytest.raises(RuntimeError, match="sparse"):
+        opt.step()
+    (taken, _, _, _, hyper), _ = ops.adamw_step.call_args
+    assert [id(t) for t in taken] == [id(t) for t in params[:2]]
+    assert [h[-1] for h in hyper] == [opt.state[t]["step"] for t in params[:2]] == [1, 1]
+    opt.param_groups[3]["lr"] = "none"             # the next one raises behind its count
+    params[2].grad = torch.ones_like(params[2])
+    with pytest.raises(ValueError):
+        opt.step()
+    (taken, *others, hyper), _ = ops.adamw_step.call_args
+    assert len(taken) == len(hyper) == 3 and all(len(tensors) == 3 for tensors in others)
