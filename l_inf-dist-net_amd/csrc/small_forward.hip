@@ -603,10 +603,7 @@ constexpr ForwardModel kModels[] = {
 // at the rate it reaches with that many workgroups (a single one leaves the vector unit idle nearly half the time,
 // since a wave issues every 4.3 clocks at best).  A handful of rows: the reading of the weights plus the arithmetic.
 int small_forward_tile(const Problem& pr, ForwardKind kind, float p) {
-    if (pr.HW != 1 || pr.K < 4) return -1;
-    // Past the 31-bit byte offsets that a lane addresses its tile's panels by: values alone have no larger tiles, but the
-    // few-rows kernel, whose rows are 64-bit pointers, takes any number of rows.
-    if (4LL * 80 * pr.G * pr.K >= (1LL << 31)) return kind == ForwardKind::kValues ? kFewRows : -1;
+    if (pr.HW != 1 || pr.K < 4 || 4LL * 80 * pr.G * pr.K >= (1LL << 31)) return -1;
     if (g_tile_override >= 10) return g_tile_override - 10;
     if (g_tile_override >= 0) return kind == ForwardKind::kValues ? kQuadTileCount - 1 : -1;   // values: there are no larger tiles
     const ForwardModel& model = kModels[kind != ForwardKind::kNorm ? (int)kind : small_int_power(p) >= 2 ? 3 : 4];
