@@ -64,7 +64,8 @@ LDIST_API int ldist_last_hip_error(void);
  * one width) included, 2 / 3 / 4 keep them off; 5 forces that one-pass kernel on and is
  * like 2 for every other kernel.  10..16 force the seven small tiles (32x80, 32x40, 16x40, 32x64, 32x32, 16x32, 64x80) and 30 the
  * few-rows kernel of the fully connected forward passes with more than 16 outputs per group and at least 4 inputs, which
- * otherwise are chosen by an estimate of their time.  Process-wide; not thread safe. */
+ * otherwise are chosen by an estimate of their time; for the p-norm backward they are like 2.  Under any override
+ * grad_input of the separate p-norm backward kernels is added up in one order.  Process-wide; not thread safe. */
 LDIST_API int ldist_set_tile_override(int choice);
 /* Tuning knob, no counterpart in the reference: 1 (default) orders the tiles of
  * the forward kernels so that each of the 8 XCDs works on one contiguous run of
@@ -161,12 +162,18 @@ LDIST_API int ldist_norm_dist_backward_weight(const float* grad_output, const fl
  * norm_dist_backward_weight_cuda, model/norm_dist.cpp:9-12, which its autograd function calls one after the other,
  * model/norm_dist.py:41-46).  No single counterpart in the reference.  Every term
  *   g[m,n] * (|x-w| / output[m,n])^(p-1) * sign(x-w)
- * belongs to both sums.  One kernel evaluates it once and adds it to both for fully connected layers large enough to
- * fill the device at every exponent p > 2 (p = 2 is cheaper as two kernels, p = 3 too unless the tiles fill nine
- * tenths of the device; grad_weight then
- * collects one addend per tile of 128 rows with float atomics, in no fixed order), and for the unfolded-conv layout (HW > 1) with up to
- * about 140 outputs per group (one addend per workgroup); other shapes run the two separate kernels.  grad_input is written whole and may be uninitialised;
- * grad_weight is added to and must hold zeros (or the values to accumulate onto) on entry. */
+ * belongs to both sums.  One kernel evaluates it once and adds it to both for
+ *   fully connected layers at p > 2 with at least 128 outputs per group, inputs and outputs per group multiples of four and
+ *     16-byte aligned tensors, at any batch (beyond p = 3, 4 and 8, layers of 2^23 weights and more need over 32 rows);
+ *   the unfolded-conv layout (HW > 1) from 64 rows (B * HW) per CU on, with up to 140 outputs per group, and with more
+ *     where an estimate of both ways' time says so.
+ * Other shapes run the two separate kernels.
+ * grad_input is written whole and may be uninitialised.  In fully connected layers of few tiles, and in the separate kernels
+ * likewise (either layout), several workgroups share a tile's outputs: grad_input is then zero-filled first and their sums
+ * meet in it by float atomics, in no fixed order.
+ * grad_weight is added to and must hold zeros (or the values to accumulate onto) on entry; it collects one addend per tile of
+ * 64 rows (fully connected), per workgroup (conv layout) or per share of the rows (separate kernel) with float atomics, in no
+ * fixed order.  ldist_norm_dist_backward_ordered below keeps one. */
 LDIST_API int ldist_norm_dist_backward(const float* grad_output, const float* input, const float* weight,
                                        const float* output, int B, int CO, int CI, int G, int HW, float* grad_input,
                                        float* grad_weight, float p, ldist_stream_t stream);

@@ -8,8 +8,8 @@ namespace ldist {
 
 // y[b,c,l] = (x[b,c,l] - mean[c]) + bias[c], in this order and each step rounded as the two torch operations round it;
 // either vector may be absent.  y may be x.  One lane per VEC neighbouring values: VEC = 4 needs 16-byte aligned
-// tensors and, for L == 1, C % 4 == 0 (mean and bias are then read with 128-bit loads too), for L > 1, L % 4 == 0 (the
-// four values share a channel).
+// tensors and, for L == 1, C % 4 == 0 (four values of one row), for L > 1, L % 4 == 0 (the four values share a channel).
+// mean and bias are read a value at a time, from cache: they need no alignment.
 template <int VEC, bool ROWS>
 __global__ void __launch_bounds__(256)
 channel_shift_kernel(const float* __restrict__ mean, const float* __restrict__ bias, const float* x, float* y, int C, int L,

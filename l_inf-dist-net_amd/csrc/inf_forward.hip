@@ -416,8 +416,10 @@ struct InfForward {
 // it the kernels of small_forward.hip and few_rows_forward.hip are one v_sub_f32 and half a v_max3_f32 per (row, output,
 // input) and nothing else, and their registers leave room for four waves per SIMD.  fc layout, K a multiple of four.
 // ---------------------------------------------------------------------------
-// The shapes the values-only kernel takes: the fc layout with 128-bit loads and more than a handful of outputs per
-// group (the skinny kernels serve those, and pos costs them nothing).  Everything else computes pos as well.
+// The shapes that have a values-only form: the fc layout with more than a handful of outputs per group (the skinny kernels
+// serve those) and 4 | K, aligned tensors and rows that 32-bit byte offsets reach, as fwd_engine.hpp's loads ask for.  The
+// kernels behind it (small_forward.hip, few_rows_forward.hip) read rows of any alignment from K = 4 on; passes of other
+// shapes compute pos as well, which nobody reads then.
 bool inf_forward_values_applicable(const Problem& pr, const void* input, const void* weight) {
     return pr.HW == 1 && pr.NG > kSkinnyMaxNG && can_vec4(pr, input, weight);
 }

@@ -180,8 +180,7 @@ __device__ __forceinline__ void read_frag(Frag<GEO, NX, KP>& f, const LaneAddr<G
     for (int e = 0; e < KP; e++) {
         const unsigned at = lp.w + (r + e) * (GEO::SN * 4u);
         const vec4f a = *(lds_vec4f*)(uintptr_t)at;
-        f.w[e][0] = a.x; f.w[e][1] = a.y; f.w[e][2] = a.z;
-        if constexpr (GEO::TN > 3) f.w[e][3] = a.w;
+        f.w[e][0] = a.x; f.w[e][1] = a.y; f.w[e][2] = a.z; f.w[e][3] = a.w;
         if constexpr (GEO::TN == 8) {
             const vec4f b = *(lds_vec4f*)(uintptr_t)(at + GEO::BN / 2 * 4u);
             f.w[e][4] = b.x; f.w[e][5] = b.y; f.w[e][6] = b.z; f.w[e][7] = b.w;
