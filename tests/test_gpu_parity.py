@@ -1442,10 +1442,11 @@ FUSED_BACKWARD_SHAPES = [sh for sh in TILED_BACKWARD_SHAPES if sh[4] == 1] + [(5
 @pytest.mark.parametrize("shape", FUSED_BACKWARD_SHAPES + [(1030, 24, 44, 1, 1), (512, 64, 20, 1, 1)])
 def test_norm_backward_both_gradients_in_one_pass(shape, p, tile):
     """norm_dist_backward against the oracle: the kernel that evaluates every term once for both gradients, forced
-    with the tile override (by itself it only takes large layers, and p = 2 and 3 never), in its general form
-    (logarithm and exponential) and its multiply-only forms for p = 2, 3, 4, 8; then override 2, which switches it
-    off, so that the same call runs the two separate kernels (515 and 1030 rows, 20 and 44 columns: partial tiles of
-    those).  grad_weight is added onto the buffer (0.125 here) like the separate call's."""
+    with the tile override (by itself it takes layers of at least 128 outputs, and p = 2 never; 0, 1 and 5 force the
+    same 64 x 64 tiles), in its general form (logarithm and exponential) and its multiply-only forms for p = 2, 3, 4,
+    8; then override 2, which switches it off, so that the same call runs the two separate kernels (515 and 1030 rows,
+    20 and 44 columns: partial tiles of those).  grad_weight is added onto the buffer (0.125 here) like the separate
+    call's."""
     from gpu_common import DEV, cpp, say, set_tile
     B, CO, CI, G, HW = shape
     say("norm_backward fused", shape, "p", p, "tile", tile)
@@ -1467,9 +1468,9 @@ def test_norm_backward_both_gradients_in_one_pass(shape, p, tile):
 
 @pytest.mark.parametrize("p", [8.0, 4.0, 20.5, 100.0])
 def test_norm_backward_one_pass_on_48_column_tiles(p):
-    """A layer of about 3072 inputs at batch 500: 128 x 80 and 128 x 64 tiles would leave CUs idle, so the one-call
-    backward takes its 128 x 48 geometry (three columns per lane, the weight panel at a pitch of four) of its own
-    accord; ragged in rows (500), outputs (260 = 4 stages of 64 + 4) and columns (3068 = 63 tiles of 48 + 44)."""
+    """A layer of about 3072 inputs at batch 500, which the one-call backward takes of its own accord, on 64 x 64 tiles
+    as every layer (the name is from the 48-column tiles it had); ragged in rows (500 = 7 tiles of 64 + 52), outputs
+    (260 = 4 stages of 64 + 4) and columns (3068 = 47 tiles of 64 + 60)."""
     from gpu_common import DEV, cpp, say, set_tile
     B, CO, CI, G, HW = 500, 260, 3068, 1, 1
     say("norm_backward one pass, 48-column tiles", "p", p)

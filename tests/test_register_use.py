@@ -24,7 +24,7 @@ def scratch_of(source, tmp_path):
 
 
 def test_one_pass_conv_backward_at_four_waves(tmp_path):
-    """norm_conv_backward_kernel<IMG, IE, BLOCKS, 4, ...>: layers of up to 32 outputs per group."""
+    """norm_conv_backward_kernel<IMG, IE, BLOCKS, 4, ...>: groups staged whole, of up to 39 outputs."""
     four = {name: size for name, size in scratch_of("norm_conv_backward.hip", tmp_path).items()
             if re.search(r"norm_conv_backward_kernelILb[01]ELi\dELb[01]ELi4E", name)}
     columns = [size for name, size in four.items() if "kernelILb0E" in name]
