@@ -37,6 +37,14 @@ void check(const Tensor& t, const char* name, const torch::Device& dev) {
     TORCH_CHECK(t.device() == dev, "all tensors must be on the same device");
 }
 
+// A saved tensor is what an unpack hook made of it (torch.autograd.graph.saved_tensors_hooks): the kernels read it as it was
+// saved, so it has to be that still.  `like`: a tensor of the backward pass that autograd has checked.
+void check_saved(const Tensor& t, const char* name, at::ScalarType type, at::IntArrayRef shape, const Tensor& like) {
+    TORCH_CHECK(t.is_cuda() && t.device() == like.device(), "saved ", name, " must be a CUDA tensor on the gradient's device");
+    TORCH_CHECK(t.is_contiguous(), "saved ", name, " must be contiguous");
+    TORCH_CHECK(t.scalar_type() == type && t.sizes() == shape, "saved ", name, " must have the type and shape that it was saved with");
+}
+
 // Pins the device of `t` for a scope and knows its current stream.
 struct On {
     explicit On(const Tensor& t) : guard(t.device()) {}
@@ -170,16 +178,24 @@ struct ColumnLayer : public Function<ColumnLayer> {
         const double p = ctx->saved_data["p"].toDouble();
         const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1);
         const bool want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
-        const On on(saved[0]);
+        const auto w_shape = ctx->saved_data["w"].toIntVector();
         Tensor gx, gw, gb;
         Tensor g = grads[0].contiguous();
+        const On on(g);
+        if (std::isinf(p)) {
+            check_saved(saved[0], "argmax", torch::kInt32, s.output(), g);
+        } else {
+            check_saved(saved[0], "input", torch::kFloat32, s.input(), g);
+            check_saved(saved[1], "weight", torch::kFloat32, w_shape, g);
+            check_saved(saved[2], "output", torch::kFloat32, s.output(), g);
+        }
         if (want_b) gb = sum_per_channel(g);
         if (ctx->saved_data["mean"].toBool()) g = mean_shifted(on, g, Tensor(), 0.0);
         if (want_x) gx = torch::empty(s.input(), g.options());
         if (std::isinf(p)) {
             // the scatter kernels write every element, zeros included: no fill needed here
             const int32_t* pos = saved[0].const_data_ptr<int32_t>();
-            if (want_w) gw = torch::empty(ctx->saved_data["w"].toIntVector(), g.options());
+            if (want_w) gw = torch::empty(w_shape, g.options());
             if (want_x && want_w)
                 done("inf_dist_backward", ldist_inf_dist_backward_overwrite(in(g), pos, s.B, s.CO, s.CI, (int)G, s.HW, out(gx),
                                                                             out(gw), on.stream));
@@ -286,8 +302,9 @@ struct InfImageLayer : public Function<InfImageLayer> {
         const Window win{v[0], v[1], v[2], v[3]};
         const int G = (int)ctx->saved_data["G"].toInt();
         const bool want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
-        const On on(pos);
         Tensor g = grads[0].contiguous();
+        const On on(g);
+        check_saved(pos, "argmax", torch::kInt32, g.sizes(), g);
         Tensor gi, gw, gb;
         if (want_b) gb = sum_per_channel(g);
         if (ctx->saved_data["mean"].toBool()) g = mean_shifted(on, g, Tensor(), 0.0);
@@ -325,6 +342,8 @@ struct NormImageLayer : public Function<NormImageLayer> {
         Tensor raw = norm_image_forward(on, img, w, G, p, win);
         Tensor y = shifted(on, raw, bias, shift, true);
         ctx->save_for_backward({img, w, raw});
+        ctx->saved_data["img"] = img.sizes().vec();
+        ctx->saved_data["w"] = w.sizes().vec();
         ctx->saved_data["G"] = G;
         ctx->saved_data["p"] = p;
         ctx->saved_data["window"] = std::vector<int64_t>{win.k, win.stride, win.pad, win.dil};
@@ -337,12 +356,15 @@ struct NormImageLayer : public Function<NormImageLayer> {
         const Tensor &img = saved[0], &w = saved[1], &raw = saved[2];
         const auto v = ctx->saved_data["window"].toIntVector();
         const Window win{v[0], v[1], v[2], v[3]};
-        const int G = (int)ctx->saved_data["G"].toInt(), CO = (int)w.size(0);
+        const int G = (int)ctx->saved_data["G"].toInt(), CO = (int)ctx->saved_data["w"].toIntVector()[0];
         const float p = (float)ctx->saved_data["p"].toDouble();
         const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1);
         const bool want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
-        const On on(img);
         Tensor g = grads[0].contiguous();
+        const On on(g);
+        check_saved(img, "input", torch::kFloat32, ctx->saved_data["img"].toIntVector(), g);
+        check_saved(w, "weight", torch::kFloat32, ctx->saved_data["w"].toIntVector(), g);
+        check_saved(raw, "output", torch::kFloat32, g.sizes(), g);
         Tensor gi, gw, gb;
         if (want_b) gb = sum_per_channel(g);
         if (ctx->saved_data["mean"].toBool()) g = mean_shifted(on, g, Tensor(), 0.0);

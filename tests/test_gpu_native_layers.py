@@ -252,3 +252,25 @@ def test_deterministic_p_norm_gradients(both_routes, case, p):
     # few times that); the terms' signs alternate, which a factor of eight covers.
     for a, b in zip(native[0], run()):
         assert (a - b).norm() <= 8 * 2.0 ** -23 * (p + 2) * b.norm()
+
+
+@pytest.mark.parametrize("changed", ["host", "strided", "wider type", "shorter"])
+@pytest.mark.parametrize("p", [INF, 8.0])
+@pytest.mark.parametrize("case", ["fc", "image"])
+def test_saved_tensors_that_a_hook_has_changed_are_refused(case, p, changed):
+    """What an unpack hook returns is not what was saved: the native nodes say so before a kernel reads it."""
+    from gpu_common import say
+    say("saved tensors", case, p, changed)
+    back = {"host": lambda t: t.cpu(), "wider type": lambda t: t.double(), "shorter": lambda t: t[:-1].contiguous(),
+            "strided": lambda t: torch.stack([t, t], -1)[..., 0]}[changed]
+    layer = (pkg.NormDist(12, 20, p=p, bias=False) if case == "fc" else
+             pkg.NormDistConv(4, 20, 3, padding=1, p=p, bias=False)).to(DEV)
+    x = torch.rand(*((6, 12) if case == "fc" else (6, 4, 7, 8)), device=DEV, requires_grad=True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, back):
+        y = layer(x)[0]
+    with pytest.raises(RuntimeError, match="saved"):
+        y.sum().backward()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(DEV)):   # as it was saved: taken
+        y = layer(x)[0]
+    got = torch.autograd.grad(y.sum(), x)[0]
+    _same([got], [torch.autograd.grad(layer(x)[0].sum(), x)[0]], exact=p == INF)
