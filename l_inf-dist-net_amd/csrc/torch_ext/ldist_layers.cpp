@@ -396,18 +396,23 @@ Tensor norm_dist(const Tensor& x, const Tensor& w, int64_t G, double p) {
     return distances(On(x), x, w, G, p);
 }
 
-std::tuple<Tensor, Tensor> inf_dist_bound(const Tensor& lower, const Tensor& upper, const Tensor& w, int64_t G) {
+// `w`: a layer's weight with its window, (CO, CI/G, k, k), or the matrix that it is.
+std::tuple<Tensor, Tensor> bounds_of_columns(const Tensor& lower, const Tensor& upper, const Tensor& w, int64_t G) {
     check(lower, "input_lower", lower.device());
     check(upper, "input_upper", lower.device());
     check(w, "weight", lower.device());
     TORCH_CHECK(lower.sizes() == upper.sizes(), "input_upper must match input_lower");
-    TORCH_CHECK(w.dim() == 2 || w.dim() == 4, "weight must be (CO, CI/G)");
     const On on(lower);
     const Sizes s = sizes_of(lower, w, G);
     Tensor lo = torch::empty(s.output(), lower.options()), hi = torch::empty_like(lo);
     done("inf_dist_bound_forward", ldist_inf_dist_bound_forward(in(lower), in(upper), in(w), s.B, s.CO, s.CI, (int)G, s.HW,
                                                                 out(lo), out(hi), on.stream));
     return {lo, hi};
+}
+
+std::tuple<Tensor, Tensor> inf_dist_bound(const Tensor& lower, const Tensor& upper, const Tensor& w, int64_t G) {
+    TORCH_CHECK(lower.dim() == 3 && w.dim() == 2, "input_lower must be 3-D, weight 2-D");
+    return bounds_of_columns(lower, upper, w, G);
 }
 
 Shift make_shift(const OptTensor& running, double momentum, bool training, const torch::Device& dev) {
@@ -529,12 +534,12 @@ std::tuple<Tensor, Tensor, bool> layer_bounds(const Tensor& lower, const Tensor&
                                                                               (int)G, WINDOW_ARGS(win), out(lo), out(hi),
                                                                               on.stream));
     } else if (win.trivial()) {
-        std::tie(lo, hi) = inf_dist_bound(as_columns(lower), as_columns(upper), w, G);
+        std::tie(lo, hi) = bounds_of_columns(as_columns(lower), as_columns(upper), w, G);
     } else {
         const Tensor l = lower.contiguous(), u = upper.contiguous();
         check(l, "lower_img", w.device());
         check(u, "upper_img", w.device());
-        std::tie(lo, hi) = inf_dist_bound(unfolded(on, l, win), unfolded(on, u, win), w, G);
+        std::tie(lo, hi) = bounds_of_columns(unfolded(on, l, win), unfolded(on, u, win), w, G);
     }
     lo = shifted(on, lo, bias, shift, false);
     hi = shifted(on, hi, bias, shift, false);

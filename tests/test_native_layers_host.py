@@ -68,6 +68,15 @@ def test_a_window_that_is_none_is_refused_with_an_exception(ops, stride, padding
             call()
 
 
+@pytest.mark.parametrize("weight", [(8, 12, 1, 1), (8, 3, 2, 2), (8, 12, 1), (96,)])
+def test_weights_that_are_no_matrix_are_refused(ops, weight):
+    """As the entry points of the library's torch extension do, whatever the weight's values would make of it."""
+    x, w = torch.zeros(4, 12, 5), torch.zeros(weight)
+    for call in (lambda: ops.norm_dist(x, w, 1, 8.0), lambda: ops.inf_dist_bound(x, x, w, 1)):
+        with pytest.raises(RuntimeError, match="weight 2-D"):
+            call()
+
+
 def test_adamw_takes_any_number_as_a_step_or_rate(ops, monkeypatch):
     """A restored state may hold the step count as a float or a tensor; a rate may be a tensor."""
     layer = pkg.NormDist(6, 4, p=8.0)
