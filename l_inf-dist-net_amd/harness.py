@@ -104,7 +104,8 @@ class AttackPGD:
     def _ascend(self, adv, grad, inputs):
         """One signed-gradient step and its projections."""
         ops = norm_dist_cpp.native_ops()
-        if (ops is not None and type(self)._project is AttackPGD._project and adv.is_cuda and adv.numel() < 2 ** 31 and
+        own = getattr(self._project, "__func__", None) is AttackPGD._project   # not a subclass's or an object's of its own
+        if (ops is not None and own and adv.is_cuda and adv.numel() < 2 ** 31 and
                 adv.dtype == grad.dtype == inputs.dtype == torch.float32 and adv.shape == inputs.shape and
                 all(isinstance(v, numbers.Real) for v in (self.eps, self.step_size, self.up, self.down))):
             return ops.pgd_step(adv, grad, inputs, self.step_size, self.eps, self.down, self.up)   # one kernel

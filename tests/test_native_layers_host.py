@@ -129,6 +129,23 @@ def test_attack_ranges_per_channel_are_left_to_torch(monkeypatch):
     assert ops.pgd_step.called
 
 
+def test_an_attack_with_a_projection_of_its_own_uses_it(monkeypatch):
+    """Replaced in a subclass or on the object: the native step knows the plain projection only."""
+    ops = mock.Mock()
+    monkeypatch.setattr(pkg.norm_dist_cpp, "native_ops", lambda: ops)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+
+    class Halved(pkg.AttackPGD):
+        def _project(self, x, centre=None):
+            return x / 2
+    replaced = pkg.AttackPGD(None, 0.1, 0.03, 1, 1.0, 0.0)
+    replaced._project = lambda x, centre=None: x / 2
+    x, grad = torch.rand(2, 3, 4, 4), torch.randn(2, 3, 4, 4)
+    for attack in (Halved(None, 0.1, 0.03, 1, 1.0, 0.0), replaced):
+        assert torch.equal(attack._ascend(x, grad, x), (x + 0.03 * grad.sign()) / 2)
+    assert not ops.pgd_step.called
+
+
 def test_adamw_steps_what_comes_before_a_parameter_that_raises(monkeypatch):
     """The native loop takes its parameters together; those before a refused gradient have had their step all the same."""
     ops, net = mock.Mock(), torch.nn.Sequential(pkg.NormDist(6, 4, p=8.0), pkg.NormDist(4, 3, p=8.0))
