@@ -94,7 +94,7 @@ class AdamW(Optimizer):
                     state["step"] += 1
                     m, v = state["exp_avg"], state["exp_avg_sq"]
                     if ops is not None and _fused_ok(prm, grad, m, v):
-                        hyper.append((*(float(v) for v in (-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd)),
+                        hyper.append((*map(float, (-1.0 if p_norm is None else p_norm, lr, beta1, beta2, eps, wd)),
                                       int(state["step"])))
                         for tensors, t in zip(fused, (prm, grad, m, v)):
                             tensors.append(t)
