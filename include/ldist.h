@@ -91,6 +91,24 @@ LDIST_API int ldist_inf_dist_forward(const float* input, const float* weight, in
 LDIST_API int ldist_inf_dist_forward_values(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
                                   float* output, ldist_stream_t stream);
 
+/* L_inf forward passes of large fully connected layers that evaluate only the differences which can be the maximum
+ * (lists of every row's outermost values; same results, bit for bit).  No counterpart in the reference.  They need
+ * device scratch memory from the caller, free again for other work on the stream when the call returns:
+ * ldist_inf_dist_workspace says how much, 0 where a layer has no such form (call the plain entry point); `what` is one
+ * of LDIST_WITH_POS, LDIST_VALUES_ONLY (pos == NULL), LDIST_BOUNDS.  workspace: 16-byte aligned, contents of no matter.
+ * LDIST_EUNSUPPORTED where the size is 0, and without pos also where ldist_inf_dist_forward_values has no form for the
+ * tensors: nothing is enqueued then. */
+enum { LDIST_WITH_POS = 0, LDIST_VALUES_ONLY = 1, LDIST_BOUNDS = 2 };
+LDIST_API int ldist_inf_dist_workspace(int B, int CO, int CI, int G, int HW, int what, int64_t* bytes);
+LDIST_API int ldist_inf_dist_forward_ws(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
+                                        float* output, int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream);
+LDIST_API int ldist_inf_dist_bound_forward_ws(const float* input_lower, const float* input_upper, const float* weight, int B,
+                                              int CO, int CI, int G, int HW, float* output_lower, float* output_upper,
+                                              void* workspace, int64_t bytes, ldist_stream_t stream);
+/* Testing knob: -1 (default) by size; 0 the workspace forms cover nothing; 1 they cover every fully connected layer of
+ * one group with more than 16 outputs and up to 40960 inputs, and rely on their lists alone.  Process-wide. */
+LDIST_API int ldist_set_extremes(int choice);
+
 /* Interval-bound forward.  Replaces inf_dist_bound_forward_cuda
  * (model/norm_dist.cpp:15-16, model/inf_dist_cuda.cu:181-188).
  *   output_upper = max_k max(|l-w|, |u-w|)

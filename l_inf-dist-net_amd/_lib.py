@@ -20,6 +20,9 @@ _d = ctypes.c_double
 SIGNATURES = {
     "ldist_inf_dist_forward": [_F, _F, _i, _i, _i, _i, _i, _F, _I, _S],
     "ldist_inf_dist_forward_values": [_F, _F, _i, _i, _i, _i, _i, _F, _S],
+    "ldist_inf_dist_workspace": [_i, _i, _i, _i, _i, _i, ctypes.c_void_p],
+    "ldist_inf_dist_forward_ws": [_F, _F, _i, _i, _i, _i, _i, _F, _I, ctypes.c_void_p, ctypes.c_int64, _S],
+    "ldist_inf_dist_bound_forward_ws": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, ctypes.c_void_p, ctypes.c_int64, _S],
     "ldist_inf_dist_bound_forward": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _S],
     "ldist_inf_dist_value_bound_forward": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _F, _F, _F, _S],
     "ldist_inf_dist_backward_input": [_F, _I, _i, _i, _i, _i, _i, _F, _S],

@@ -27,6 +27,7 @@ bound_forward_kernel(const float* __restrict__ lower, const float* __restrict__ 
     static_assert(2 * (KS - 1) * TM * TN * NGRP <= NBUF * STAGE, "merge area fits in the panels");
     extern __shared__ __align__(16) float lds[];
 
+    if (gated_off(d)) return;
     int tm, tn, g;
     tile_of_block(d, tm, tn, g);
     const int m0 = tm * BM, n0 = tn * BN;

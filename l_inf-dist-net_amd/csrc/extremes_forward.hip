@@ -1,0 +1,1005 @@
+// L_inf forward passes of large fully connected layers that evaluate only the differences that can be a maximum.
+//
+// max_k |x[m,k] - w[n,k]| is attained where x[m,k] or w[n,k] lies far out: if a short list of row m holds its q_x
+// outermost inputs, and one of row n its q_w outermost weights, then every k in neither list has
+//     |x - w| <= max(max x - min w, max w - min x)   over what the two lists left out,
+// two numbers per row.  The maximum over the k in either list is therefore the maximum over all k wherever it exceeds
+// that bound, which can be read off afterwards: rounding is monotone, so the statement holds for the rounded differences
+// too, and the results (argmax with its sign included) are the same bits as those of the full walk.  Outputs that do not
+// pass are walked in full by the wave that finds them.  With K = 5120 inputs, lists of 1 to 4 % suffice for all but one
+// output in a thousand, for inputs and weights of comparable spread as for very different ones.
+//
+// Launches, all on the caller's stream:
+//   sample   64 x 64 outputs in full, and for their rows what lists of eight lengths would leave out;
+//   select   the list lengths that cost least by that sample (or none: `dense`, and the kernels of the full walk, which
+//            are launched last and otherwise leave at once, do the work), and every row's list;
+//   scan     first every row's list against all outputs, then every weight row's list against all rows.
+//
+// The reduction is cut into C chunks of at most 2560 k with lists and bounds of their own, so that a chunk of eight rows
+// of the other operand fits half a CU's LDS.  Rows with NaN or infinities (bounds: boxes that are not l <= u) get an infinite
+// bound: their outputs are walked in full with the comparisons of the other kernels.
+//
+// 5120 x 5120 with positions, batch 272 / 512: 300 / 470 -> 165 / 205 us; values at 1024 780 -> 155; bounds at 1024 2170 -> 225.
+// Data that the lists cannot help cost 12 to 60 us beside the full walk of 480 to 2170.
+#include "kernels.hpp"
+#include "quad_engine.hpp"
+#include "wave_reduce.hpp"
+
+namespace ldist {
+namespace {
+
+typedef float F4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxChunk = 2560;              // eight rows of it: 80 KB of LDS, two workgroups per CU
+constexpr int kLengths[8] = {0, 8, 16, 32, 48, 64, 96, 128};   // of a chunk's list
+constexpr int kMaxList = 128;
+constexpr int kBins = 512;                   // of the histogram of |v - center|: 256 to the octave, the top two octaves
+constexpr int kBinShift = 15;
+constexpr int kSampled = 64;                 // rows of either operand that the sample looks at
+constexpr int kSampleRows = 4;               // of them in one workgroup
+constexpr int kSampleGroups = kSampled / kSampleRows;
+constexpr float kNever = 3.402823466e38f;    // bound of an empty remainder; finite, so that infinite bounds stay infinite beside it
+
+// How many entries of a list are meant to be taken, so that those of rows with a few more still fit.
+__device__ __forceinline__ constexpr int typical(int length) { return length - length / 8 - length / 16; }
+
+struct Header {
+    float center;
+    int qx, qw;
+    int dense;         // the lists are not worth it
+    int full;          // the full walk has to do the work: dense, or the lists left too many outputs unsettled
+    int failed;        // how many
+    int taken[2][8];   // tiles of a scan that the workgroups of an XCD have taken beyond their first
+};
+
+// One operand: its rows, their lists in blocks of 16 rows (entry-major, so that 16 neighbouring lanes read 128 bytes)
+// and per chunk and row what the lists left out.
+struct Side {
+    const float *v, *v2;   // v2: the upper ends where v are the lower ends of boxes
+    int rows, blocks;
+    char* lists;           // [chunk][block][entry][16] of {value, 32 k} or {lower, upper, 32 k, 0}
+    float* rest;           // [chunk][2 or 4][rows]: max, min; boxes: max of the upper ends, min of the lower, max of the lower, min of the upper
+};
+
+struct Search {
+    Side x, w;
+    float *out, *out2;     // distances, or the lower and upper bounds
+    int32_t* pos;
+    Header* head;
+    unsigned char* counts; // [workgroup of the sample][combination of lengths]: outputs that would not pass
+    float* reach;          // [x, w][length][sampled row]: how far from the center a list of that length begins
+    float* partial;        // [row of x][pitch] of the first scan's {value, position}, {upper, lower bound}, or values
+    int pitch;
+    int* walk;             // [failed]: their indices
+    int walk_most;
+    int K, C, KC;
+    int lanes_first, lanes_second;   // rows per workgroup of the two scans
+    float price_x, price_w, price_fail, price_dense;   // of a list entry, of an output that does not pass, of the full walk
+};
+
+__device__ __forceinline__ float wave_max_f(float x) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) x = __builtin_fmaxf(x, __shfl_xor(x, o));
+    return x;
+}
+__device__ __forceinline__ float wave_min_f(float x) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) x = __builtin_fminf(x, __shfl_xor(x, o));
+    return x;
+}
+__device__ __forceinline__ int sum_from_lane(int x, int lane) {   // over this lane and those above it
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_down(x, o);
+        if (lane + o < 64) x += y;
+    }
+    return x;
+}
+__device__ __forceinline__ bool not_finite(float v) { return !(__builtin_fabsf(v) < __builtin_inff()); }
+
+// A chunk of a row in a wave's registers: lane l holds k = 64 j + l.
+template <int NV>
+struct RowChunk {
+    float v[NV];
+    __device__ __forceinline__ void load(const float* row, int kc, int lane) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)row, 0, kc * 4, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < NV; j++)
+            v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane * 4, j * 256, 0));
+    }
+    // k past the chunk as `center`, which no list takes.
+    __device__ __forceinline__ void center_past(int kc, int lane, float center) {
+        if (kc >= NV * 64) return;
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            v[j] = lane < kc - j * 64 ? v[j] : center;
+            if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // no more lane masks at a time than there are registers for
+        }
+    }
+    // Keeps the compiler from carrying what one pass over the values derives from them into the next (registers).
+    __device__ __forceinline__ void opaque() {
+#pragma unroll
+        for (int j = 0; j < NV; j++) asm volatile("" : "+v"(v[j]));
+    }
+};
+
+// ---- sample ----------------------------------------------------------------------------------------------------------
+// Distance from the center as a bin of a histogram: 256 to the octave, two octaves below the largest; negative: below.
+struct Bins {
+    unsigned base;
+    __device__ __forceinline__ explicit Bins(float most) : base(__float_as_uint(most) - ((unsigned)(kBins - 1) << kBinShift)) {}
+    __device__ __forceinline__ int of(float u) const { return min((int)(__float_as_uint(u) - base) >> kBinShift, kBins - 1); }
+    __device__ __forceinline__ float edge(int bin) const {   // lower edge
+        return __uint_as_float((unsigned)max((int)(base + ((unsigned)bin << kBinShift)), 0));
+    }
+};
+
+// found(i, distance from the center at which a list of the i-th length begins), for one row chunk.
+template <int NV, class F>
+__device__ __forceinline__ void lengths_of(RowChunk<NV>& a, float center, int* hist, int lane, F&& found) {
+    float most = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) most = __builtin_fmaxf(most, __builtin_fabsf(a.v[j] - center));
+    const Bins bins(wave_max_f(most));
+    a.opaque();
+#pragma unroll
+    for (int j = 0; j < kBins / 256; j++) *reinterpret_cast<int4*>(hist + (j * 64 + lane) * 4) = make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < NV; j++) {   // a quarter of normally distributed values get here
+        const int bin = bins.of(__builtin_fabsf(a.v[j] - center));
+        if (bin >= 0) atomicAdd(hist + bin, 1);
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    constexpr int OWN = kBins / 64;
+    int upward[OWN], sum = 0;   // values in this lane's bins, from each bin up; then in all bins from there up
+#pragma unroll
+    for (int j = OWN / 4 - 1; j >= 0; j--) {
+        const int4 h = *reinterpret_cast<const int4*>(hist + lane * OWN + j * 4);
+        upward[4 * j + 3] = sum += h.w;
+        upward[4 * j + 2] = sum += h.z;
+        upward[4 * j + 1] = sum += h.y;
+        upward[4 * j] = sum += h.x;
+    }
+    const int above = sum_from_lane(sum, lane) - sum;
+#pragma unroll
+    for (int j = 0; j < OWN; j++) upward[j] += above;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        int taken = 0;   // of this lane's bins
+#pragma unroll
+        for (int j = 0; j < OWN; j++) taken += upward[j] <= typical(kLengths[i]);
+        const unsigned long long over = __ballot(upward[0] > typical(kLengths[i]));
+        int cut = 0;
+        if (over) {
+            const int at = 63 - __builtin_clzll(over);
+            cut = (at + 1) * OWN - __builtin_amdgcn_readlane(taken, at);
+        }
+        found(i, bins.edge(cut));
+    }
+}
+
+// A workgroup looks at 4 x 4 outputs: wave i at row i % 8 (four of x, four of w) in every other chunk, then all at the outputs.
+template <int NV, bool PAIR>
+__global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
+    constexpr int NO = kSampleRows * kSampleRows, NB = PAIR ? 2 : 1, WAVES = 16;
+    __shared__ __align__(16) int hist[WAVES][kBins];
+    __shared__ float rest[NB][2 * kSampleRows][8][16];   // [bound][row][length][chunk]: the most that the list leaves out
+    __shared__ float reach[2 * kSampleRows][8][16];
+    __shared__ float outs[WAVES][NB * NO];
+    __shared__ float part[WAVES];
+    __shared__ int fails[64];
+    static_assert(NO == WAVES, "a wave for every output");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bx = blockIdx.x / kSampleGroups, bw = blockIdx.x % kSampleGroups;
+    auto sampled = [](int i, int rows) { return (int)((long long)i * rows / kSampled); };
+    if (tid < 64) fails[tid] = 0;
+    const int r = wave & 7;
+    const bool of_x = r < kSampleRows;
+    const Side& side = of_x ? s.x : s.w;
+    const int row = sampled((of_x ? bx : bw) * kSampleRows + (r & (kSampleRows - 1)), side.rows);
+    RowChunk<NV> a, b;   // boxes: both ends, then a alone, the middles
+    auto load = [&](int ch) {
+        const int k0 = ch * s.KC, kc = min(s.KC, s.K - k0);
+        a.load(side.v + (size_t)row * s.K + k0, kc, lane);
+        if constexpr (PAIR) { if (of_x) b.load(side.v2 + (size_t)row * s.K + k0, kc, lane); }
+    };
+    const int first = wave >> 3;
+    if (first < s.C) load(first);
+    // a center common to both operands: the mean of 1024 weights; any number is correct
+    float c = s.w.v[(size_t)((long long)tid * s.w.rows / 1024) * s.K + (size_t)((long long)tid * 61 % s.K)];
+#pragma unroll
+    for (int o = 32; o; o >>= 1) c += __shfl_xor(c, o);
+    if (lane == 0) part[wave] = c;
+    __syncthreads();
+    c = 0.f;
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) c += part[i];
+    const float center = not_finite(c) ? 0.f : c / 1024.f;
+    if (blockIdx.x == 0) {
+        if (tid == 0) s.head->center = center;
+        if (tid < 16) s.head->taken[tid >> 3][tid & 7] = 0;
+        if (tid == 16) s.head->failed = 0;
+    }
+#pragma unroll 1
+    for (int ch = first; ch < s.C; ch += WAVES / 8) {
+        if (ch != first) load(ch);
+        const int kc = min(s.KC, s.K - ch * s.KC);
+        float widest = 0.f, width = 0.f;   // of the boxes, and the mean; half of each
+        if constexpr (PAIR) {
+            if (of_x) {
+#pragma unroll
+                for (int j = 0; j < NV; j++) {
+                    const float half = 0.5f * (b.v[j] - a.v[j]);
+                    widest = __builtin_fmaxf(widest, half);
+                    width += half;
+                    a.v[j] = 0.5f * (a.v[j] + b.v[j]);
+                }
+                widest = wave_max_f(widest);
+#pragma unroll
+                for (int o = 32; o; o >>= 1) width += __shfl_xor(width, o);
+                width /= kc;
+            }
+        }
+        a.center_past(kc, lane, center);
+        lengths_of<NV>(a, center, hist[wave], lane, [&](int i, float edge) {
+            if (lane == 0) {
+                reach[r][i][ch] = edge;
+                rest[0][r][i][ch] = edge + widest;                    // upper bounds reach further than the middles,
+                if constexpr (PAIR) rest[1][r][i][ch] = edge - width;   // lower bounds less far
+            }
+        });
+    }
+
+    float up[NO], lo[NO];
+#pragma unroll
+    for (int i = 0; i < NO; i++) up[i] = lo[i] = 0.f;
+    const float *xr[kSampleRows], *ur[kSampleRows], *wr[kSampleRows];
+#pragma unroll
+    for (int i = 0; i < kSampleRows; i++) {
+        xr[i] = s.x.v + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
+        if constexpr (PAIR) ur[i] = s.x.v2 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
+        wr[i] = s.w.v + (size_t)sampled(bw * kSampleRows + i, s.w.rows) * s.K;
+    }
+    constexpr int AHEAD = PAIR ? 3 : 5;
+    for (int kb = 0; kb < s.K; kb += 1024 * AHEAD) {
+        float x[AHEAD][kSampleRows], u[AHEAD][kSampleRows], w[AHEAD][kSampleRows];
+#pragma unroll
+        for (int e = 0; e < AHEAD; e++) {
+            const int k = min(kb + e * 1024 + tid, s.K - 1);   // past the end: the last k again
+#pragma unroll
+            for (int i = 0; i < kSampleRows; i++) { x[e][i] = xr[i][k]; w[e][i] = wr[i][k]; if constexpr (PAIR) u[e][i] = ur[i][k]; }
+        }
+#pragma unroll
+        for (int e = 0; e < AHEAD; e++)
+#pragma unroll
+            for (int i = 0; i < kSampleRows; i++)
+#pragma unroll
+                for (int j = 0; j < kSampleRows; j++) {
+                    const float dl = x[e][i] - w[e][j];
+                    float& U = up[i * kSampleRows + j];
+                    U = __builtin_fmaxf(U, __builtin_fabsf(dl));
+                    if constexpr (PAIR) {
+                        const float du = u[e][i] - w[e][j];
+                        float& L = lo[i * kSampleRows + j];
+                        U = __builtin_fmaxf(U, __builtin_fabsf(du));
+                        L = __builtin_fmaxf(__builtin_fmaxf(L, dl), -du);
+                    }
+                }
+    }
+#pragma unroll
+    for (int i = 0; i < NO; i++) {
+        const float u = wave_max(up[i]);   // in lane 63
+        if (lane == 63) outs[wave][i] = u;
+        if constexpr (PAIR) {
+            const float l = wave_max(lo[i]);
+            if (lane == 63) outs[wave][NO + i] = l;
+        }
+    }
+    __syncthreads();
+    if (tid < NB * NO) {
+        float best = outs[0][tid];
+#pragma unroll
+        for (int i = 1; i < WAVES; i++) best = __builtin_fmaxf(best, outs[i][tid]);
+        outs[0][tid] = best;
+    }
+    __syncthreads();
+    {   // wave: output, lane: combination of lengths
+        const int ix = lane >> 3, iw = lane & 7;
+        bool ok = true;
+#pragma unroll
+        for (int q = 0; q < NB; q++) {
+            float bound = 0.f;
+            for (int ch = 0; ch < s.C; ch++)
+                bound = __builtin_fmaxf(bound, rest[q][wave / kSampleRows][ix][ch] + rest[0][kSampleRows + wave % kSampleRows][iw][ch]);
+            ok &= PAIR ? outs[0][q * NO + wave] >= bound : outs[0][wave] > bound;
+        }
+        if (!ok) atomicAdd(&fails[lane], 1);
+    }
+    __syncthreads();
+    if (tid < 64) {
+        s.counts[blockIdx.x * 64 + tid] = (unsigned char)fails[tid];
+    } else if (tid < 128) {   // 8 rows x 8 lengths; of x from the workgroups with bw == 0, of w from those with bx == 0
+        const int rr = (tid >> 3) & 7, i = tid & 7;
+        if (rr < kSampleRows ? bw == 0 : bx == 0) {
+            float sum = 0.f;
+            for (int ch = 0; ch < s.C; ch++) sum += reach[rr][i][ch];
+            s.reach[((rr < kSampleRows ? 0 : 1) * 8 + i) * kSampled + (rr < kSampleRows ? bx : bw) * kSampleRows + (rr & (kSampleRows - 1))] = sum / s.C;
+        }
+    }
+}
+
+// ---- select ----------------------------------------------------------------------------------------------------------
+// The cheapest lengths by the sample; every workgroup works this out for itself.
+__device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][64], int wave, int lane, int& ix, int& iw, int& dense) {
+    constexpr int SHARE = kSampleGroups * kSampleGroups / 8;
+    int part = 0;
+#pragma unroll
+    for (int b = 0; b < SHARE; b++) part += s.counts[(wave * SHARE + b) * 64 + lane];
+    sums[wave][lane] = part;
+    __syncthreads();
+    int fails = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) fails += sums[i][lane];
+    float cost = s.C * (s.price_x * kLengths[lane >> 3] + s.price_w * kLengths[lane & 7]) +
+                 s.price_fail * ((float)fails / (kSampled * kSampled));
+    int pick = lane;
+#pragma unroll
+    for (int o = 32; o; o >>= 1) {
+        const float c = __shfl_xor(cost, o);
+        const int p = __shfl_xor(pick, o);
+        if (c < cost || (c == cost && p < pick)) { cost = c; pick = p; }
+    }
+    pick = __builtin_amdgcn_readfirstlane(pick);
+    ix = pick >> 3;
+    iw = pick & 7;
+    dense = __builtin_amdgcn_readfirstlane(cost > s.price_dense ? 1 : 0);
+}
+
+// A workgroup makes the lists of 16 rows in one chunk, a wave those of two rows: all values beyond `t` from the center,
+// where t starts as what the sampled rows needed on the average and is moved where the list would overflow or stay half empty
+// (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly.
+// Bound by reading the operands once.
+template <int NV, bool PAIR>
+__global__ void __launch_bounds__(512, PAIR ? 3 : 5) extremes_select_kernel(Search s) {
+    extern __shared__ __align__(16) char stage[];   // [entry][16] as in Side::lists
+    __shared__ int sums[8][64];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per = s.x.blocks + s.w.blocks, ch = blockIdx.x / per;
+    int block = blockIdx.x % per;
+    const bool of_x = block < s.x.blocks;
+    const Side& side = of_x ? s.x : s.w;
+    if (!of_x) block -= s.x.blocks;
+    const int k0 = ch * s.KC;
+    auto row_at = [&](int i) { return __builtin_amdgcn_readfirstlane(min(block * 16 + wave * 2 + i, side.rows - 1)); };
+
+    auto lists = [&](auto pair) {
+        constexpr bool P = decltype(pair)::value;
+        RowChunk<NV> a, b;
+        int kc = min(s.KC, s.K - k0);
+        auto load = [&](int i, int lane) {
+            const size_t at = (size_t)row_at(i) * s.K + k0;
+            a.load(side.v + at, kc, lane);
+            if constexpr (P) b.load(side.v2 + at, kc, lane);
+        };
+        load(0, tid & 63);
+        int ix, iw, dense;
+        choose_lengths(s, sums, wave, tid & 63, ix, iw, dense);
+        const int q = kLengths[of_x ? ix : iw];
+        if (blockIdx.x == 0 && tid == 0) { s.head->qx = kLengths[ix]; s.head->qw = kLengths[iw]; s.head->dense = s.head->full = dense; }
+        if (dense) return;
+        const float center = s.head->center;
+        float guess = s.reach[((of_x ? 0 : 1) * 8 + (of_x ? ix : iw)) * kSampled + (tid & 63)];
+#pragma unroll
+        for (int o = 32; o; o >>= 1) guess += __shfl_xor(guess, o);
+        guess = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(guess * (1.f / kSampled))));
+#pragma unroll 1
+        for (int i = 0; i < 2; i++) {
+            // what is derived from these is made where it is used, not kept in registers over the loop
+            asm volatile("" : "+s"(kc));
+            int lane = tid & 63;
+            asm volatile("" : "+v"(lane));
+            if (i) load(i, lane);
+            const int row = row_at(i), r = wave * 2 + i;
+            a.center_past(kc, lane, center);
+            if constexpr (P) b.center_past(kc, lane, center);
+            float odd = 0.f;   // NaN if there is a NaN or an infinity
+            bool crossed = false;
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+                odd = __builtin_fmaf(a.v[j], 0.f, odd);
+                if constexpr (P) { odd = __builtin_fmaf(b.v[j], 0.f, odd); crossed |= a.v[j] > b.v[j]; }
+            }
+            const bool bad = __any(odd != 0.f || crossed);
+            // twice the middle of a box, where values are compared by themselves
+            constexpr float F = P ? 2.f : 1.f;
+            auto key = [&](int j) {
+                if constexpr (P) return a.v[j] + b.v[j];
+                else return a.v[j];
+            };
+            auto count = [&](float t) {
+                const float hi = F * (center + t), lo = F * (center - t);
+                int n = 0;
+#pragma unroll
+                for (int j = 0; j < NV; j++) n += __builtin_popcountll(__ballot(key(j) > hi) | __ballot(key(j) < lo));
+                return n;
+            };
+            float hi, lo;
+            if (q == 0) {   // no list: everything is left out
+                hi = -kNever;
+                lo = kNever;
+#pragma unroll
+                for (int j = 0; j < NV; j++) { hi = __builtin_fmaxf(hi, key(j)); lo = __builtin_fminf(lo, key(j)); }
+                hi = wave_max_f(hi);
+                lo = wave_min_f(lo);
+            } else {
+                float t = guess;
+                int n = count(t);
+                if (n > q || n < q / 2) {
+                    float most = 0.f;
+#pragma unroll
+                    for (int j = 0; j < NV; j++) most = __builtin_fmaxf(most, __builtin_fabsf(key(j) - F * center));
+                    float in = 0.f, out = wave_max_f(most) * (1.f / F);   // too long a list, and none at all
+                    if (n > q) in = t; else out = __builtin_fminf(out, t);
+#pragma unroll 1
+                    for (int step = 0; step < 10; step++) {
+                        t = 0.5f * (in + out);
+                        n = count(t);
+                        if (n > q) { in = t; continue; }
+                        out = t;
+                        if (n >= q - q / 4) break;
+                    }
+                    t = out;
+                }
+                hi = F * (center + t);
+                lo = F * (center - t);
+            }
+            int base = 0;
+            float most = -kNever, least = kNever, most_lower = -kNever, least_upper = kNever;
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+                const bool in = key(j) > hi || key(j) < lo;
+                const unsigned long long m = __ballot(in);
+                if (m) {
+                    const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                    if (in && at < q) {
+                        const unsigned k32 = (unsigned)(lane + j * 64) * 32u;
+                        if constexpr (P) reinterpret_cast<uint4*>(stage)[at * 16 + r] = make_uint4(__float_as_uint(a.v[j]), __float_as_uint(b.v[j]), k32, 0u);
+                        else reinterpret_cast<uint2*>(stage)[at * 16 + r] = make_uint2(__float_as_uint(a.v[j]), k32);
+                    }
+                    base += __builtin_popcountll(m);
+                }
+                if constexpr (P) {
+                    most = __builtin_fmaxf(most, in ? -kNever : b.v[j]);
+                    least = __builtin_fminf(least, in ? kNever : a.v[j]);
+                    most_lower = __builtin_fmaxf(most_lower, in ? -kNever : a.v[j]);
+                    least_upper = __builtin_fminf(least_upper, in ? kNever : b.v[j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // a list that is not full repeats the chunk's first value
+            const unsigned v0 = __builtin_amdgcn_readfirstlane(__float_as_uint(a.v[0]));
+            const unsigned v1 = P ? __builtin_amdgcn_readfirstlane(__float_as_uint(b.v[0])) : 0u;
+            for (int e = base + lane; e < q; e += 64) {
+                if constexpr (P) reinterpret_cast<uint4*>(stage)[e * 16 + r] = make_uint4(v0, v1, 0u, 0u);
+                else reinterpret_cast<uint2*>(stage)[e * 16 + r] = make_uint2(v0, 0u);
+            }
+            if constexpr (P) {
+                most = wave_max_f(most);
+                least = wave_min_f(least);
+                most_lower = wave_max_f(most_lower);
+                least_upper = wave_min_f(least_upper);
+            } else {
+                most = hi;
+                least = lo;
+            }
+            if (lane == 0 && block * 16 + r < side.rows) {
+                const float inf = __builtin_inff();
+                float* rest = side.rest + (size_t)ch * (P ? 4 : 2) * side.rows + row;
+                rest[0] = bad ? inf : most;
+                rest[side.rows] = bad ? -inf : least;
+                if constexpr (P) {
+                    rest[2 * side.rows] = bad ? inf : most_lower;
+                    rest[3 * side.rows] = bad ? -inf : least_upper;
+                }
+            }
+        }
+        __syncthreads();
+        constexpr int E = P ? 16 : 8;   // bytes of an entry
+        uint4* dst = reinterpret_cast<uint4*>(side.lists + ((size_t)ch * side.blocks + block) * q * 16 * E);
+        for (int i = tid; i < q * E; i += 512) dst[i] = reinterpret_cast<const uint4*>(stage)[i];
+    };
+    if constexpr (PAIR) {
+        if (of_x) { lists(std::true_type{}); return; }
+    }
+    lists(std::false_type{});
+}
+
+// ---- scan ------------------------------------------------------------------------------------------------------------
+enum { kWithPos, kOnlyValues, kBoxes };
+__device__ __host__ constexpr int strip_rows(bool pairs) { return pairs ? 4 : 8; }   // 32 bytes per k
+
+// Lanes own rows of one operand (`ln`) and walk their lists; a strip of rows of the other (`sd`) lies in LDS, 32 bytes per
+// k, so that an entry costs two 128-bit reads at a place of its own for eight differences (boxes in the strip: four rows,
+// lower and upper end).  Odd lanes read the second half first: two lanes at the same k mod 8 then miss each other's banks.
+//
+// Bound by the vector unit (3.5 instructions per difference with the position) beside those reads, 60 % of whose cycles are
+// bank conflicts of random places: 5120 x 5120 at batch 512, 96 + 128 entries per row: 59 + 70 us, of which 25 are w from
+// memory.  Four rows per strip with four workgroups per CU read the lists twice as often: 92 + 105 us before, and 73 + 91 with
+// eight rows, both with the first pass's results stored one by one to 64 rows at a time (35 us of that pass); a strip's next chunk fetched between the
+// entries made their loads wait for it (they return in order): 82 us.
+//
+// First pass: lanes are rows of x, results into s.partial.  Second: lanes are rows of w; takes what the first left, checks the
+// bound and notes the outputs that fail it.
+template <int MODE, bool SECOND>
+__global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
+    constexpr bool BOX = MODE == kBoxes, PAIR_ENTRY = BOX && !SECOND, PAIR_STRIP = BOX && SECOND;
+    constexpr int RS = strip_rows(PAIR_STRIP), U = kMaxChunk / 512, NT = 512;
+    extern __shared__ __align__(16) char lds[];
+    if (s.head->dense) return;
+    const Side& ln = SECOND ? s.w : s.x;
+    const Side& sd = SECOND ? s.x : s.w;
+    const int q = SECOND ? s.head->qw : s.head->qx;
+    const bool both = s.head->qx != 0;   // second pass: the first has left something
+    if (!SECOND && !both) return;
+    const int K = s.K, KC = s.KC, C = s.C, N = s.w.rows;
+    const int LG = SECOND ? s.lanes_second : s.lanes_first, EG = NT / LG;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int eg = __builtin_amdgcn_readfirstlane(tid / LG), at = tid % LG;
+    const unsigned odd = (lane & 1) * 16u;   // which half a lane reads first
+
+    // Every XCD takes a contiguous run of tiles.  First pass: the lane blocks of one strip beside each other, so that w
+    // streams from memory once.  Second: an eighth of the strips, which then stay in the XCD's L2, under every lane block in
+    // turn, whose lists are read once.
+    const int strips = (sd.rows + RS - 1) / RS, blocks = (ln.rows + LG - 1) / LG, tiles = strips * blocks;
+    const int together = SECOND ? (strips + 7) / 8 : 1;
+    auto place = [&](int t, int& strip, int& block) {
+        const int group = t / (together * blocks), i = t - group * together * blocks, n = min(together, strips - group * together);
+        block = i / n;
+        strip = group * together + i - block * n;
+    };
+    const int xcd = blockIdx.x % 8;
+    const int t_begin = (int)((long long)tiles * xcd / 8), t_end = (int)((long long)tiles * (xcd + 1) / 8);
+    int tile = t_begin + (int)(blockIdx.x / 8);
+    if (tile >= t_end) return;
+    // The first tile is fixed, the others are taken as workgroups get there; lane 0 has the next one in hand a tile ahead.
+    auto take = [&] { return t_begin + (int)(gridDim.x / 8) + atomicAdd(&s.head->taken[SECOND][xcd], 1); };
+    int in_hand = tid == 0 ? take() : 0;
+
+    while (true) {
+        int strip, block;
+        place(tile, strip, block);
+        const int s0 = strip * RS, row0 = block * LG;
+        const int l = min(row0 + at, ln.rows - 1);
+        const bool live = row0 + at < ln.rows;
+        const bool wave_live = __builtin_amdgcn_readfirstlane(row0 + (at & ~63)) < ln.rows;
+        // values: the difference of the largest magnitude, with its sign, and 32 k; boxes: upper and lower bound
+        float best[RS], low[RS];
+        unsigned key[RS];
+#pragma unroll
+        for (int j = 0; j < RS; j++) { best[j] = low[j] = 0.f; key[j] = 0u; }
+        int next_tile = t_end;
+#pragma unroll 1
+        for (int ch = 0; ch < C; ch++) {
+            const int k0 = ch * KC, kc = min(KC, K - k0);
+            __syncthreads();   // everyone is done with the strip before
+            if (ch + 1 == C) {   // hand out the next tile
+                if (tid == 0) *reinterpret_cast<int*>(lds) = in_hand;
+                __syncthreads();
+                next_tile = __builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile int*>(lds));
+                __syncthreads();
+                if (tid == 0 && next_tile < t_end) in_hand = take();
+            }
+            {
+                const auto rl = __builtin_amdgcn_make_buffer_rsrc((void*)(sd.v + (size_t)s0 * K + k0), 0, 0x7fffffff, 0x00020000);
+                const auto ru = __builtin_amdgcn_make_buffer_rsrc((void*)((PAIR_STRIP ? sd.v2 : sd.v) + (size_t)s0 * K + k0), 0, 0x7fffffff, 0x00020000);
+                float t[U][8];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (u * NT >= kc || q == 0) continue;
+                    const unsigned k4 = (unsigned)min(u * NT + tid, kc - 1) * 4u;   // lanes past the chunk store nothing
+#pragma unroll
+                    for (int j = 0; j < RS; j++) {
+                        const int row = min(j, sd.rows - 1 - s0) * K * 4;
+                        t[u][PAIR_STRIP ? 2 * j : j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rl, k4, row, 0));
+                        if constexpr (PAIR_STRIP) t[u][2 * j + 1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ru, k4, row, 0));
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int k = u * NT + tid;
+                    if (k < kc && q != 0) {
+                        *reinterpret_cast<F4*>(lds + k * 32) = F4{t[u][0], t[u][1], t[u][2], t[u][3]};
+                        *reinterpret_cast<F4*>(lds + k * 32 + 16) = F4{t[u][4], t[u][5], t[u][6], t[u][7]};
+                    }
+                }
+            }
+            using Entry = typename std::conditional<PAIR_ENTRY, uint4, uint2>::type;
+            const Entry* list = reinterpret_cast<const Entry*>(ln.lists) + (((size_t)ch * ln.blocks + l / 16) * q) * 16 + (l & 15);
+            const unsigned kb = (unsigned)k0 * 32u;
+            auto entry = [&](const Entry& en) {
+                unsigned k32;
+                if constexpr (PAIR_ENTRY) k32 = en.z;
+                else k32 = en.y;
+                const float v = __uint_as_float(en.x);
+                const unsigned from = k32 ^ odd;
+                const F4 half[2] = {*reinterpret_cast<const F4*>(lds + from), *reinterpret_cast<const F4*>(lds + (from ^ 16u))};
+#pragma unroll
+                for (int j = 0; j < RS; j++) {
+                    if constexpr (PAIR_STRIP) {
+                        const float dl = half[j / 2][2 * (j & 1)] - v, du = half[j / 2][2 * (j & 1) + 1] - v;
+                        best[j] = __builtin_fmaxf(__builtin_fmaxf(best[j], __builtin_fabsf(dl)), __builtin_fabsf(du));
+                        low[j] = __builtin_fmaxf(__builtin_fmaxf(low[j], dl), -du);
+                    } else {
+                        const float other = half[j / 4][j & 3];
+                        if constexpr (BOX) {
+                            const float dl = v - other, du = __uint_as_float(en.y) - other;
+                            best[j] = __builtin_fmaxf(__builtin_fmaxf(best[j], __builtin_fabsf(dl)), __builtin_fabsf(du));
+                            low[j] = __builtin_fmaxf(__builtin_fmaxf(low[j], dl), -du);
+                        } else {
+                            const float df = SECOND ? other - v : v - other;
+                            if constexpr (MODE == kWithPos) {
+                                const bool wins = __builtin_fabsf(df) > __builtin_fabsf(best[j]);
+                                best[j] = wins ? df : best[j];
+                                key[j] = wins ? kb + k32 : key[j];
+                            } else {
+                                best[j] = __builtin_fmaxf(best[j], __builtin_fabsf(df));
+                            }
+                        }
+                    }
+                }
+            };
+            // entries eg, eg + EG, ... four at a time; a place past the end repeats the last
+            const int quads = ((q - eg + EG - 1) / EG + 3) / 4;
+            Entry en[4], en_next[4];
+            auto read = [&](Entry (&e)[4], int i) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) e[c] = list[min(eg + (4 * i + c) * EG, q - 1) * 16];
+            };
+            if (wave_live && q != 0) read(en, 0);
+            __syncthreads();
+            if (wave_live && q != 0) {
+#pragma unroll 1
+                for (int i = 0; i < quads; i++) {
+                    read(en_next, i + 1);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) entry(en[c]);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) en[c] = en_next[c];
+                }
+            }
+        }
+
+        // odd lanes hold the halves the other way round
+        auto swap = [&](auto& p, auto& r) { const auto c = p; p = lane & 1 ? r : p; r = lane & 1 ? c : r; };
+#pragma unroll
+        for (int j = 0; j < RS / 2; j++) {
+            swap(best[j], best[j + RS / 2]);
+            if constexpr (BOX) swap(low[j], low[j + RS / 2]);
+            if constexpr (MODE == kWithPos) swap(key[j], key[j + RS / 2]);
+        }
+        if (EG > 1) {   // the groups of lanes that shared a row's list
+            float* pa = reinterpret_cast<float*>(lds);
+            unsigned* pb = reinterpret_cast<unsigned*>(lds + NT / 2 * RS * 4);
+            for (int half = EG / 2; half > 0; half /= 2) {
+                __syncthreads();
+                if (eg >= half && eg < 2 * half) {
+#pragma unroll
+                    for (int j = 0; j < RS; j++) {
+                        pa[j * (NT / 2) + tid - half * LG] = best[j];
+                        if constexpr (MODE != kOnlyValues) pb[j * (NT / 2) + tid - half * LG] = BOX ? __float_as_uint(low[j]) : key[j];
+                    }
+                }
+                __syncthreads();
+                if (eg < half) {
+#pragma unroll
+                    for (int j = 0; j < RS; j++) {
+                        const float o = pa[j * (NT / 2) + tid];
+                        if constexpr (MODE == kWithPos) {
+                            const unsigned ok = pb[j * (NT / 2) + tid];
+                            const float ao = __builtin_fabsf(o), ab = __builtin_fabsf(best[j]);
+                            if (ao > ab || (ao == ab && ok < key[j])) { best[j] = o; key[j] = ok; }
+                        } else {
+                            best[j] = __builtin_fmaxf(best[j], o);
+                            if constexpr (BOX) low[j] = __builtin_fmaxf(low[j], __uint_as_float(pb[j * (NT / 2) + tid]));
+                        }
+                    }
+                }
+            }
+        }
+        auto pos_of = [&](int j) { return best[j] == 0.f ? 0 : (int)((key[j] >> 5) | (__float_as_uint(best[j]) & 0x80000000u)); };
+        if (eg == 0 && wave_live) {
+            if constexpr (!SECOND) {
+                if (live) {   // 16 * RS bytes of a row (8 * RS without positions): whole sectors, and all of a lane's in few stores
+                    if constexpr (MODE == kOnlyValues) {
+                        float* to = s.partial + (size_t)l * s.pitch + s0;
+#pragma unroll
+                        for (int j = 0; j < RS; j += 4) *reinterpret_cast<F4*>(to + j) = F4{best[j], best[j + 1], best[j + 2], best[j + 3]};
+                    } else {
+                        float* to = s.partial + 2 * ((size_t)l * s.pitch + s0);
+                        auto second = [&](int j) { return BOX ? low[j] : __int_as_float(pos_of(j)); };
+#pragma unroll
+                        for (int j = 0; j < RS; j += 2)
+                            *reinterpret_cast<F4*>(to + 2 * j) = F4{__builtin_fabsf(best[j]), second(j), __builtin_fabsf(best[j + 1]), second(j + 1)};
+                    }
+                }
+            } else {
+                float limit[RS], limit_low[RS];   // what neither list holds
+#pragma unroll
+                for (int j = 0; j < RS; j++) limit[j] = limit_low[j] = -kNever;
+                for (int ch = 0; ch < C; ch++) {
+                    const float* lr = ln.rest + (size_t)ch * 2 * ln.rows + l;
+                    const float lh = lr[0], ll = lr[ln.rows];
+#pragma unroll
+                    for (int j = 0; j < RS; j++) {
+                        const float* sr = sd.rest + (size_t)ch * (BOX ? 4 : 2) * sd.rows + min(s0 + j, sd.rows - 1);
+                        limit[j] = __builtin_fmaxf(limit[j], __builtin_fmaxf(sr[0] - ll, lh - sr[sd.rows]));
+                        if constexpr (BOX) limit_low[j] = __builtin_fmaxf(limit_low[j], __builtin_fmaxf(sr[2 * sd.rows] - ll, lh - sr[3 * sd.rows]));
+                    }
+                }
+                unsigned failed = 0;
+#pragma unroll
+                for (int j = 0; j < RS; j++)
+                    if (live && s0 + j < sd.rows) {
+                        const size_t o = (size_t)(s0 + j) * N + l;
+                        const size_t from = (size_t)(s0 + j) * s.pitch + l;   // what the first pass left
+                        float have = 0.f, with = 0.f;
+                        if constexpr (MODE == kOnlyValues) {
+                            if (both) have = s.partial[from];
+                        } else if (both) {
+                            const float2 both = reinterpret_cast<const float2*>(s.partial)[from];
+                            have = both.x;
+                            with = both.y;
+                        }
+                        // an infinite limit is a row that the lists cannot speak for, whatever they found
+                        if constexpr (BOX) {
+                            const float lo = __builtin_fmaxf(low[j], with), up = __builtin_fmaxf(best[j], have);
+                            if (up >= limit[j] && lo >= limit_low[j] && limit[j] < __builtin_inff()) {
+                                s.out[o] = lo;
+                                s.out2[o] = up;
+                            } else {
+                                failed |= 1u << j;
+                            }
+                        } else if constexpr (MODE == kOnlyValues) {
+                            const float v = __builtin_fmaxf(best[j], have);
+                            if (v >= limit[j] && limit[j] < __builtin_inff()) s.out[o] = v;
+                            else failed |= 1u << j;
+                        } else {
+                            float v = __builtin_fabsf(best[j]);
+                            int p = pos_of(j);
+                            const int hp = __float_as_int(with);
+                            if (have > v || (have == v && (hp & 0x7fffffff) < (p & 0x7fffffff))) { v = have; p = hp; }
+                            if (v > limit[j]) {   // at the limit a lower k might hold the same value
+                                s.out[o] = v;
+                                s.pos[o] = p;
+                            } else {
+                                failed |= 1u << j;
+                            }
+                        }
+                    }
+                if (__ballot(failed != 0)) {
+                    int n = 0;
+#pragma unroll
+                    for (int j = 0; j < RS; j++) n += __builtin_popcountll(__ballot(failed >> j & 1));
+                    int first = lane == 0 ? atomicAdd(&s.head->failed, n) : 0;
+                    first = __builtin_amdgcn_readfirstlane(first);
+#pragma unroll
+                    for (int j = 0; j < RS; j++) {
+                        const unsigned long long m = __ballot(failed >> j & 1);
+                        if (failed >> j & 1)
+                            s.walk[first + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0))] =
+                                (s0 + j) * N + l;
+                        first += __builtin_popcountll(m);
+                    }
+                }
+            }
+        }
+        tile = next_tile;
+        if (tile >= t_end) return;
+    }
+}
+
+// ---- walk ------------------------------------------------------------------------------------------------------------
+// The outputs that the lists could not settle, a wave for each, all k and the comparisons of the other kernels.  More than
+// `s.walk_most` of them: the full walk of the layer is cheaper, and follows.
+template <int MODE>
+__global__ void __launch_bounds__(256) extremes_walk_kernel(Search s) {
+    if (s.head->dense) return;
+    const int failed = s.head->failed;
+    if (failed > s.walk_most) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) s.head->full = 1;
+        return;
+    }
+    const int lane = threadIdx.x & 63, K = s.K, N = s.w.rows;
+    for (int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); i < failed; i += gridDim.x * 4) {
+        const int o = __builtin_amdgcn_readfirstlane(s.walk[i]);
+        const float* xr = s.x.v + (size_t)(o / N) * K;
+        const float* wr = s.w.v + (size_t)(o % N) * K;
+        if constexpr (MODE == kBoxes) {
+            const float* ur = s.x.v2 + (size_t)(o / N) * K;
+            float up = 0.f, lo = 0.f;
+            auto one = [&](float x, float u, float w) {
+                const float tl = x - w, tu = u - w, al = __builtin_fabsf(tl), au = __builtin_fabsf(tu);
+                up = __builtin_fmaxf(up, __builtin_fmaxf(al, au));
+                if (!(tl < 0.f && tu > 0.f)) lo = __builtin_fmaxf(lo, __builtin_fminf(al, au));
+            };
+            for (int kb = 0; kb < K; kb += 256 * 4) {
+                float4_any x[4], u[4], w[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int k = min(kb + c * 256 + lane * 4, K - 4);   // the last vector is moved back, those past the end repeat it
+                    x[c] = *reinterpret_cast<const float4_any*>(xr + k);
+                    u[c] = *reinterpret_cast<const float4_any*>(ur + k);
+                    w[c] = *reinterpret_cast<const float4_any*>(wr + k);
+                }
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) one(x[c].v[e], u[c].v[e], w[c].v[e]);
+            }
+            up = wave_max(up);
+            lo = wave_max(lo);
+            if (lane == 63) { s.out[o] = lo; s.out2[o] = up; }
+        } else {
+            float v = 0.f;
+            int p = 0;   // k with the sign of the difference
+            auto one = [&](float x, float w, int k) {
+                const float df = x - w, a = __builtin_fabsf(df);
+                const bool wins = a > v;
+                v = wins ? a : v;
+                p = wins ? (int)((unsigned)k | (__float_as_uint(df) & 0x80000000u)) : p;
+            };
+            for (int kb = 0; kb < K; kb += 256 * 5) {
+                float4_any x[5], w[5];
+#pragma unroll
+                for (int c = 0; c < 5; c++) {
+                    const int k = min(kb + c * 256 + lane * 4, K - 4);   // the last vector is moved back, those past the end repeat it
+                    x[c] = *reinterpret_cast<const float4_any*>(xr + k);
+                    w[c] = *reinterpret_cast<const float4_any*>(wr + k);
+                }
+#pragma unroll
+                for (int c = 0; c < 5; c++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) one(x[c].v[e], w[c].v[e], min(kb + c * 256 + lane * 4, K - 4) + e);
+            }
+            wave_best(v, p);
+            if (lane == 63) {
+                s.out[o] = v;
+                if constexpr (MODE == kWithPos) s.pos[o] = v > 0.f ? p : 0;
+            }
+        }
+    }
+}
+
+}  // namespace
+
+// ---- host ------------------------------------------------------------------------------------------------------------
+namespace {
+
+struct Layout {
+    int C, KC, mb, nb, pitch;
+    size_t counts, reach, partial, walk, x_lists, w_lists, x_rest, w_rest, total;   // byte offsets in the workspace
+};
+
+Layout layout_of(const Problem& pr, ForwardKind kind) {
+    const bool boxes = kind == ForwardKind::kBounds;
+    Layout l{};
+    l.C = (pr.K + kMaxChunk - 1) / kMaxChunk;
+    l.KC = ((pr.K + l.C - 1) / l.C + 63) / 64 * 64;
+    l.mb = (pr.B + 15) / 16;
+    l.nb = (pr.NG + 15) / 16;
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const size_t here = at; at += (bytes + 255) / 256 * 256; return here; };
+    take(sizeof(Header));
+    l.counts = take((size_t)kSampleGroups * kSampleGroups * 64);
+    l.pitch = (pr.NG + 7) / 8 * 8;
+    l.partial = take((size_t)pr.B * l.pitch * (kind == ForwardKind::kValues ? 1 : 2) * sizeof(float));
+    l.walk = take((size_t)pr.B * pr.NG * sizeof(int));
+    l.reach = take(2 * 8 * kSampled * sizeof(float));
+    l.x_lists = take((size_t)l.C * l.mb * kMaxList * 16 * (boxes ? 16 : 8));
+    l.w_lists = take((size_t)l.C * l.nb * kMaxList * 16 * 8);
+    l.x_rest = take((size_t)l.C * (boxes ? 4 : 2) * pr.B * sizeof(float));
+    l.w_rest = take((size_t)l.C * 2 * pr.NG * sizeof(float));
+    l.total = at;
+    return l;
+}
+
+template <int MODE, bool SECOND>
+hipError_t launch_scan(const Search& s, const Problem& pr, hipStream_t stream) {
+    auto kern = extremes_scan_kernel<MODE, SECOND>;
+    static LdsRecord allowed = {};
+    const size_t strip = (size_t)s.KC * 32, lds = strip > 16384 ? strip : 16384;   // the strip, or what the groups of lanes hand over
+    if (hipError_t e = allow_lds(kern, (size_t)kMaxChunk * 32, pr.device, allowed); e != hipSuccess) return e;
+    const Side &ln = SECOND ? s.w : s.x, &sd = SECOND ? s.x : s.w;
+    const int rows = strip_rows(MODE == kBoxes && SECOND), lanes = SECOND ? s.lanes_second : s.lanes_first;
+    const long tiles = (long)((sd.rows + rows - 1) / rows) * ((ln.rows + lanes - 1) / lanes);
+    const long most = 2L * pr.num_cu / 8 * 8;   // two strips fit a CU
+    const unsigned grid = (unsigned)(tiles < most ? (tiles + 7) / 8 * 8 : most);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, stream, s);
+    return hipGetLastError();
+}
+
+template <bool PAIR>
+hipError_t launch_lists(const Search& s, hipStream_t stream) {
+    const unsigned grid = (unsigned)(s.C * (s.x.blocks + s.w.blocks));
+    const size_t stage = (size_t)kMaxList * 16 * (PAIR ? 16 : 8);
+#define LISTS(NV)                                                                                                                 \
+    do {                                                                                                                          \
+        hipLaunchKernelGGL((extremes_sample_kernel<NV, PAIR>), dim3(kSampleGroups * kSampleGroups), dim3(1024), 0, stream, s);     \
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;                                                          \
+        hipLaunchKernelGGL((extremes_select_kernel<NV, PAIR>), dim3(grid), dim3(512), stage, stream, s);                          \
+    } while (0)
+    if (s.KC <= 1024) LISTS(16);
+    else if (s.KC <= 1536) LISTS(24);
+    else if (s.KC <= 2048) LISTS(32);
+    else LISTS(40);
+#undef LISTS
+    return hipGetLastError();
+}
+
+// Lanes of a workgroup that own different rows (the others share their lists): as many as leave two tiles per workgroup.
+int lanes_for(int rows, int strips, int num_cu) {
+    int lanes = 512;
+    while (lanes > 128 && (long)strips * ((rows + lanes - 1) / lanes) < 4L * num_cu) lanes /= 2;
+    while (lanes > 64 && rows <= lanes / 2) lanes /= 2;
+    return lanes;
+}
+
+}  // namespace
+
+// The layers for which the lists are expected to be faster, by an estimate of their time on normally distributed values
+// (lists of about 50 and 100 entries per chunk), fitted to eight sizes of weights from 1024 x 784 to 5120 x 5120 at
+// batches of 32 to 1024, against that of the full walk: e.g. 1024 x 3072 at batch 512 (positions) 92 us in full and
+// 80 with lists, at 272 56 and 78; 5120 x 5120 at 64, 128 and 1024 93, 165, 909 and 120, 138, 282 us.
+// The size alone decides, for the caller asks for the workspace before there is a device to ask.
+size_t extremes_workspace(const Problem& pr, ForwardKind kind) {
+    if (g_extremes == 0 || pr.HW != 1 || pr.G != 1 || pr.NG <= 16 || pr.K < 4 || pr.K > 16 * kMaxChunk) return 0;
+    if (g_extremes < 0) {
+        if (g_tile_override >= 0 || pr.K < 512) return 0;
+        const double outputs = (double)pr.B * pr.NG, weights = (double)pr.NG * pr.K;
+        const bool boxes = kind == ForwardKind::kBounds;
+        const double us = (boxes ? 65 : 55) + 2.1e-6 * weights + (boxes ? 5.3e-5 : 3.5e-5) * outputs;
+        if (1.1 * us + 5 > full_walk_us(pr, kind, 256)) return 0;
+    }
+    return layout_of(pr, kind).total;
+}
+
+hipError_t extremes_forward(const float* x, const float* x2, const float* w, float* out, float* out2, int32_t* pos, void* workspace,
+                            const Problem& pr, hipStream_t stream, const int** gate) {
+    const bool boxes = x2 != nullptr;
+    const Layout l = layout_of(pr, boxes ? ForwardKind::kBounds : pos ? ForwardKind::kInf : ForwardKind::kValues);
+    char* ws = static_cast<char*>(workspace);
+    Search s{};
+    s.head = reinterpret_cast<Header*>(ws);
+    s.counts = reinterpret_cast<unsigned char*>(ws + l.counts);
+    s.reach = reinterpret_cast<float*>(ws + l.reach);
+    s.partial = reinterpret_cast<float*>(ws + l.partial);
+    s.pitch = l.pitch;
+    s.walk = reinterpret_cast<int*>(ws + l.walk);
+    s.walk_most = g_extremes > 0 ? pr.B * pr.NG : pr.B * pr.NG / 16;
+    s.x = Side{x, x2, pr.B, l.mb, ws + l.x_lists, reinterpret_cast<float*>(ws + l.x_rest)};
+    s.w = Side{w, nullptr, pr.NG, l.nb, ws + l.w_lists, reinterpret_cast<float*>(ws + l.w_rest)};
+    s.out = out; s.out2 = out2; s.pos = pos;
+    s.K = pr.K; s.C = l.C; s.KC = l.KC;
+    s.lanes_first = lanes_for(pr.B, (pr.NG + 7) / 8, pr.num_cu);
+    const int second_rows = strip_rows(boxes);
+    s.lanes_second = lanes_for(pr.NG, (pr.B + second_rows - 1) / second_rows, pr.num_cu);
+    s.price_x = 1.f;
+    s.price_w = boxes ? 2.f : 1.f;
+    s.price_fail = 6.f * pr.K;   // in list entries of one row: a walked output reads two rows, 3 ns with all waves at it, an entry 0.1 ps per output
+    s.price_dense = g_extremes > 0 ? 3e38f : (boxes ? 0.5f : 0.2f) * pr.K;
+    *gate = &s.head->full;
+    if (hipError_t e = boxes ? launch_lists<true>(s, stream) : launch_lists<false>(s, stream); e != hipSuccess) return e;
+#define SCANS(MODE)                                                                                                       \
+    do {                                                                                                                  \
+        if (hipError_t e = launch_scan<MODE, false>(s, pr, stream); e != hipSuccess) return e;                   \
+        if (hipError_t e = launch_scan<MODE, true>(s, pr, stream); e != hipSuccess) return e;                    \
+        hipLaunchKernelGGL(extremes_walk_kernel<MODE>, dim3(4 * pr.num_cu), dim3(256), 0, stream, s);                     \
+        return hipGetLastError();                                                                                         \
+    } while (0)
+    if (boxes) SCANS(kBoxes);
+    if (pos) SCANS(kWithPos);
+    SCANS(kOnlyValues);
+#undef SCANS
+}
+
+}  // namespace ldist

@@ -253,7 +253,7 @@ inline bool can_vec4_out(const Problem& pr, const void* a, const void* b = nullp
     return aligned16(a) && aligned16(b) && (pr.HW == 1 ? pr.NG % 4 == 0 : pr.HW % 4 == 0);
 }
 
-inline Dims make_dims(const Problem& pr) { return Dims{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, g_xcd_remap, 0}; }
+inline Dims make_dims(const Problem& pr) { return Dims{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, g_xcd_remap, 0, pr.gate}; }
 
 // Dims::m_block for a kernel whose workgroup reads x_rows rows of the input panels (BM times the number of panels)
 // and w_rows rows of weights per stage: `resident` workgroups share an L2 at a time (workgroups per CU times the CUs

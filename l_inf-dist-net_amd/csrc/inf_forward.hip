@@ -32,6 +32,7 @@ inf_forward_kernel(const float* __restrict__ input, const float* __restrict__ we
     constexpr int STAGE = Stage::STAGE, NBUF = Stage::NBUF;
     extern __shared__ __align__(16) float lds[];
 
+    if (gated_off(d)) return;
     int tm, tn, g;
     tile_of_block(d, tm, tn, g);
     const int m0 = tm * BM, n0 = tn * BN;

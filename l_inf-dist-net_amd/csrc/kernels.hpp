@@ -11,6 +11,7 @@ struct Problem {
     int B, G, K, NG, HW;  // K = CI/G, NG = CO/G
     int num_cu;           // compute units of the current device
     int device;
+    const int* gate = nullptr;   // of a launch that may find nothing to do on the device: it leaves at once where *gate is 0
 };
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -30,6 +31,8 @@ enum class TileChoice { M128N80K2, M128N64K1, M256N32K1, M32N32K8 };
 // (inf_forward.hip; by itself it takes them where M128N80K2 would be chosen) and leaves every other kernel's choice alone.
 extern int g_tile_override;
 extern int g_xcd_remap;  // 1 (default): XCD-aware tile order; 0: plain order (tuning)
+
+extern int g_extremes;   // -1 (default): extremes_forward.hip where its rule says so; 0: never; 1: wherever it can run, without a full walk after it (tests)
 
 inline TileChoice choose_tile(int M, int NG, int G, int num_cu) {
     if (g_tile_override >= 0 && g_tile_override <= 3) return static_cast<TileChoice>(g_tile_override);
@@ -66,6 +69,13 @@ inline hipError_t allow_lds(Kern kern, size_t bytes, int device, LdsRecord& done
     return e;
 }
 
+enum class ForwardKind { kInf, kValues, kBounds, kNorm };
+// Large fully connected layers: only the differences that can be the maximum (extremes_forward.hip).  The size of its
+// workspace, 0 where the layer is not one of them; the launches, which leave *gate != 0 on the device where the full walk has
+// to follow.  `x2`: the upper ends of boxes, nullptr for distances; pos == nullptr: values only.
+size_t extremes_workspace(const Problem& pr, ForwardKind kind);
+hipError_t extremes_forward(const float* x, const float* x2, const float* w, float* out, float* out2, int32_t* pos, void* workspace,
+                            const Problem& pr, hipStream_t stream, const int** gate);
 hipError_t inf_forward(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr,
                        hipStream_t stream);
 // Values without pos, for forward passes that no gradient follows (inf_forward.hip); the fc layout with 128-bit loads.
@@ -75,8 +85,8 @@ hipError_t inf_forward_values(const float* input, const float* weight, float* ou
 // Small tiles with the reduction split over many k-groups, for fully connected layers whose outputs are too few to fill
 // the device with the tiles above, and the kernel for a handful of rows (small_forward.hip, which also estimates which of
 // them is fastest; -1: the larger tiles).
-enum class ForwardKind { kInf, kValues, kBounds, kNorm };
 int small_forward_tile(const Problem& pr, ForwardKind kind, float p);
+double full_walk_us(const Problem& pr, ForwardKind kind, int num_cu);   // its estimate for a layer that walks all k
 // pos == nullptr: values only
 hipError_t inf_forward_small(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr, int tile,
                              hipStream_t stream);

@@ -12,6 +12,7 @@
 namespace ldist {
 int g_tile_override = -1;
 int g_xcd_remap = 1;
+int g_extremes = -1;
 }
 
 namespace {
@@ -40,13 +41,18 @@ int current_device(ldist::Problem& pr) {
     return LDIST_OK;
 }
 
-int check_dims(int B, int CO, int CI, int G, int HW, ldist::Problem& pr) {
+int check_sizes(int B, int CO, int CI, int G, int HW, ldist::Problem& pr) {
     if (B <= 0 || CO <= 0 || CI <= 0 || G <= 0 || HW <= 0) return LDIST_EINVAL;
     if (CI % G != 0 || CO % G != 0) return LDIST_EINVAL;
     const long long lim = 1LL << 31;
     const long long rows = (long long)B * HW;
     if (rows >= lim || rows * CI >= lim || rows * CO >= lim || (long long)CO * (CI / G) >= lim) return LDIST_ERANGE;
     pr.B = B; pr.G = G; pr.K = CI / G; pr.NG = CO / G; pr.HW = HW;
+    return LDIST_OK;
+}
+
+int check_dims(int B, int CO, int CI, int G, int HW, ldist::Problem& pr) {
+    if (int rc = check_sizes(B, CO, CI, G, HW, pr)) return rc;
     return current_device(pr);
 }
 
@@ -102,6 +108,59 @@ int ldist_set_tile_override(int choice) {
     if (choice < -1 || (choice > 5 && choice < 10) || (choice > 16 && choice != 30)) return LDIST_EINVAL;
     ldist::g_tile_override = choice;
     return LDIST_OK;
+}
+
+int ldist_set_extremes(int choice) {
+    if (choice < -1 || choice > 1) return LDIST_EINVAL;
+    ldist::g_extremes = choice;
+    return LDIST_OK;
+}
+
+int ldist_inf_dist_workspace(int B, int CO, int CI, int G, int HW, int what, int64_t* bytes) {
+    if (!bytes || what < LDIST_WITH_POS || what > LDIST_BOUNDS) return LDIST_EINVAL;
+    *bytes = 0;
+    ldist::Problem pr{};
+    if (int rc = check_sizes(B, CO, CI, G, HW, pr)) return rc;
+    *bytes = (int64_t)ldist::extremes_workspace(pr, static_cast<ldist::ForwardKind>(what));
+    return LDIST_OK;
+}
+
+// The workspace forms of the forward passes: the lists, then the full walk where the lists were not worth it.
+static int extremes_entry(const float* x, const float* x2, const float* w, ldist::Problem& pr, ldist::ForwardKind kind, float* out,
+                          float* out2, int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream) {
+    const size_t need = ldist::extremes_workspace(pr, kind);
+    if (need == 0) return LDIST_EUNSUPPORTED;
+    if (bytes < 0 || (size_t)bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return LDIST_EINVAL;
+    const hipError_t e = ldist::extremes_forward(x, x2, w, out, out2, pos, workspace, pr, (hipStream_t)stream, &pr.gate);
+    return finish(e);
+}
+
+int ldist_inf_dist_forward_ws(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output,
+                              int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream) {
+    if (!input || !weight || !output || !workspace) return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
+    // without pos the full walk is that of ldist_inf_dist_forward_values
+    if (!pos && !ldist::inf_forward_values_applicable(pr, input, weight)) return LDIST_EUNSUPPORTED;
+    if (int rc = extremes_entry(input, nullptr, weight, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues, output,
+                                nullptr, pos, workspace, bytes, stream))
+        return rc;
+    if (ldist::g_extremes > 0) return LDIST_OK;
+    return finish(pos ? ldist::inf_forward(input, weight, output, pos, pr, (hipStream_t)stream)
+                      : ldist::inf_forward_values(input, weight, output, pr, (hipStream_t)stream));
+}
+
+int ldist_inf_dist_bound_forward_ws(const float* input_lower, const float* input_upper, const float* weight, int B, int CO,
+                                    int CI, int G, int HW, float* output_lower, float* output_upper, void* workspace,
+                                    int64_t bytes, ldist_stream_t stream) {
+    if (!input_lower || !input_upper || !weight || !output_lower || !output_upper || !workspace) return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
+    if (int rc = extremes_entry(input_lower, input_upper, weight, pr, ldist::ForwardKind::kBounds, output_lower, output_upper,
+                                nullptr, workspace, bytes, stream))
+        return rc;
+    if (ldist::g_extremes > 0) return LDIST_OK;
+    return finish(ldist::bound_forward(input_lower, input_upper, weight, output_lower, output_upper, pr, (hipStream_t)stream));
 }
 
 int ldist_inf_dist_forward(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,

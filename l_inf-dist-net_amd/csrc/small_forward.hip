@@ -42,6 +42,7 @@ inf_forward_quad_kernel(const float* __restrict__ input, const float* __restrict
     constexpr int ANY = 63;                                 // in a tag: several groups hold the maximum
     using Stage = QStager<GEO, 1>;
     extern __shared__ __align__(16) float lds[];
+    if (gated_off(d)) return;
     int tm, tn, g;
     tile_of_block(d, tm, tn, g);
     const int m0 = tm * GEO::BM, n0 = tn * GEO::BN;
@@ -197,6 +198,7 @@ bound_forward_quad_kernel(const float* __restrict__ lower, const float* __restri
     constexpr int TM = GEO::TM, TN = GEO::TN, KK = GEO::KK, NGRP = GEO::NGRP;
     using Stage = QStager<GEO, 2>;
     extern __shared__ __align__(16) float lds[];
+    if (gated_off(d)) return;
     int tm, tn, g;
     tile_of_block(d, tm, tn, g);
     const int m0 = tm * GEO::BM, n0 = tn * GEO::BN;
@@ -601,21 +603,18 @@ constexpr ForwardModel kModels[] = {
     /* other p */ {{4.55, 4.75, 4.42, 4.70, 4.81, 4.80, 4.33}, 4.3, 5.2, 0.82, 0, 200, 120, 25.4, 16.1, 4.7},
 };
 
-// Which kernel a fully connected layer takes: the one with the shortest estimate.  Tiles: the busiest CU's share of them
+// The kernel with the shortest estimate, and the estimate.  Tiles: the busiest CU's share of them
 // at the rate it reaches with that many workgroups (a single one leaves the vector unit idle nearly half the time,
 // since a wave issues every 4.3 clocks at best).  A handful of rows: the reading of the weights plus the arithmetic.
-int small_forward_tile(const Problem& pr, ForwardKind kind, float p) {
-    if (pr.HW != 1 || pr.K < 4 || 4LL * 80 * pr.G * pr.K >= (1LL << 31)) return -1;
-    if (g_tile_override >= 10) return g_tile_override - 10;
-    if (g_tile_override >= 0) return kind == ForwardKind::kValues ? kQuadTileCount - 1 : -1;   // values: there are no larger tiles
+static int fastest_forward(const Problem& pr, ForwardKind kind, float p, double cus, double& best) {
     const ForwardModel& model = kModels[kind != ForwardKind::kNorm ? (int)kind : small_int_power(p) >= 2 ? 3 : 4];
-    const double M = pr.B, K = pr.K, cus = pr.num_cu;
+    const double M = pr.B, K = pr.K;
     // the busiest CU's time for its tiles of bm x bn (k of them the parts of a tile that do not grow with K)
     auto tiles_us = [&](int bm, int bn, int resident, double k, double rate) {
         const double per_cu = std::ceil(std::ceil(M / bm) * std::ceil((double)pr.NG / bn) * pr.G / cus);
         return per_cu * bm * bn * (K + k) * cus * 1e-6 / (rate * (per_cu < 2 && resident > 1 ? model.one_fill : 1.0));
     };
-    double best = model.few_us + 4e-6 * pr.G * pr.NG * K / 4.4 + 1e-6 * M * pr.G * pr.NG * (K + model.few_k) / model.few;
+    best = model.few_us + 4e-6 * pr.G * pr.NG * K / 4.4 + 1e-6 * M * pr.G * pr.NG * (K + model.few_k) / model.few;
     int pick = kFewRows;
     for (int i = 0; i < kQuadTileCount; i++) {
         const QuadTile& t = kQuadTiles[i];
@@ -627,9 +626,24 @@ int small_forward_tile(const Problem& pr, ForwardKind kind, float p) {
     if (pr.K % 4 == 0 && kind != ForwardKind::kValues) {
         const bool halves = M > 64 && kind == ForwardKind::kInf;
         const double us = model.big_us + tiles_us(halves ? 64 : 128, 80, halves ? 2 : 1, model.big_k, model.big);
-        if (us < best) pick = -1;
+        if (us < best) { best = us; pick = -1; }
     }
     return pick;
+}
+
+// Which kernel a fully connected layer takes.
+int small_forward_tile(const Problem& pr, ForwardKind kind, float p) {
+    if (pr.HW != 1 || pr.K < 4 || 4LL * 80 * pr.G * pr.K >= (1LL << 31)) return -1;
+    if (g_tile_override >= 10) return g_tile_override - 10;
+    if (g_tile_override >= 0) return kind == ForwardKind::kValues ? kQuadTileCount - 1 : -1;   // values: there are no larger tiles
+    double us;
+    return fastest_forward(pr, kind, p, pr.num_cu, us);
+}
+
+double full_walk_us(const Problem& pr, ForwardKind kind, int num_cu) {
+    double us;
+    fastest_forward(pr, kind, 0.f, num_cu, us);
+    return us;
 }
 
 hipError_t inf_forward_small(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr, int tile,

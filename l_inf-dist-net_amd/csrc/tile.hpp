@@ -34,7 +34,9 @@ struct Dims {
     int ovec;             // outputs may be written with 128-bit stores
     int xcd_remap;        // 1: hand each XCD a contiguous run of tiles
     int m_block;          // > 0: row tiles are walked in blocks of this many (tile_of_block); 0: all of them
+    const int* gate;      // not nullptr: nothing to do where *gate is 0 (Problem::gate)
 };
+__device__ __forceinline__ bool gated_off(const Dims& d) { return d.gate && *d.gate == 0; }
 
 // XOR applied to the m (or n) coordinate of LDS row kk.  It permutes aligned
 // groups of four floats inside aligned blocks of 32, so 128-bit accesses stay

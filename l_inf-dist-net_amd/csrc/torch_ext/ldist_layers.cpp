@@ -15,6 +15,7 @@
 #include <tuple>
 #include <vector>
 
+#include "inf_forward.hpp"
 #include "ldist.h"
 
 namespace {
@@ -128,13 +129,13 @@ Tensor distances(const On& on, const Tensor& x, const Tensor& w, int64_t G, doub
     const Sizes s = sizes_of(x, w, G);
     Tensor y = torch::empty(s.output(), x.options());
     if (std::isinf(p)) {
-        const int rc = ldist_inf_dist_forward_values(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y), on.stream);
+        const int rc = ldist_torch::inf_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y), nullptr, y, on.stream);
         if (rc != LDIST_EUNSUPPORTED) {
             done("inf_dist_forward_values", rc);
         } else {
             Tensor pos = torch::empty(s.output(), x.options().dtype(torch::kInt32));
-            done("inf_dist_forward", ldist_inf_dist_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y),
-                                                            pos.data_ptr<int32_t>(), on.stream));
+            done("inf_dist_forward", ldist_torch::inf_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y),
+                                                              pos.data_ptr<int32_t>(), y, on.stream));
         }
     } else {
         done("norm_dist_forward_values", ldist_norm_dist_forward_values(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y),
@@ -153,8 +154,8 @@ struct ColumnLayer : public Function<ColumnLayer> {
         Tensor raw = torch::empty(s.output(), x.options());
         if (inf) {
             Tensor pos = torch::empty(s.output(), x.options().dtype(torch::kInt32));
-            done("inf_dist_forward", ldist_inf_dist_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(raw),
-                                                            pos.data_ptr<int32_t>(), on.stream));
+            done("inf_dist_forward", ldist_torch::inf_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(raw),
+                                                              pos.data_ptr<int32_t>(), raw, on.stream));
             ctx->save_for_backward({pos});
         } else {
             done("norm_dist_forward", ldist_norm_dist_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(raw), (float)p,
@@ -405,8 +406,8 @@ std::tuple<Tensor, Tensor> bounds_of_columns(const Tensor& lower, const Tensor& 
     const On on(lower);
     const Sizes s = sizes_of(lower, w, G);
     Tensor lo = torch::empty(s.output(), lower.options()), hi = torch::empty_like(lo);
-    done("inf_dist_bound_forward", ldist_inf_dist_bound_forward(in(lower), in(upper), in(w), s.B, s.CO, s.CI, (int)G, s.HW,
-                                                                out(lo), out(hi), on.stream));
+    done("inf_dist_bound_forward", ldist_torch::inf_bound_forward(in(lower), in(upper), in(w), s.B, s.CO, s.CI, (int)G, s.HW,
+                                                                  out(lo), out(hi), lo, on.stream));
     return {lo, hi};
 }
 

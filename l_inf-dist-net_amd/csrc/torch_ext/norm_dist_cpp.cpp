@@ -12,6 +12,7 @@
 #include <initializer_list>
 #include <string>
 
+#include "inf_forward.hpp"
 #include "ldist.h"
 
 namespace {
@@ -100,8 +101,8 @@ void inf_dist_forward(torch::Tensor& input, torch::Tensor& weight, torch::Tensor
     Call c("inf_dist_forward", {{"input", input}, {"weight", weight}, {"output", output}}, {{"pos", pos}});
     const Shape s = forward_shape("inf_dist_forward", input, weight, output, G);
     same_shape("inf_dist_forward", pos, output, "pos and output");
-    c.done(ldist_inf_dist_forward(in(input), in(weight), s.B, s.CO, s.CI, G, s.HW, out(output), pos.data_ptr<int32_t>(),
-                                  c.stream()));
+    c.done(ldist_torch::inf_forward(in(input), in(weight), s.B, s.CO, s.CI, G, s.HW, out(output), pos.data_ptr<int32_t>(),
+                                    output, c.stream()));
 }
 
 void inf_dist_bound_forward(torch::Tensor& input_lower, torch::Tensor& input_upper, torch::Tensor& weight,
@@ -111,8 +112,8 @@ void inf_dist_bound_forward(torch::Tensor& input_lower, torch::Tensor& input_upp
     const Shape s = forward_shape("inf_dist_bound_forward", input_lower, weight, output_lower, G);
     same_shape("inf_dist_bound_forward", input_upper, input_lower, "input_upper and input_lower");
     same_shape("inf_dist_bound_forward", output_upper, output_lower, "output_upper and output_lower");
-    c.done(ldist_inf_dist_bound_forward(in(input_lower), in(input_upper), in(weight), s.B, s.CO, s.CI, G, s.HW,
-                                        out(output_lower), out(output_upper), c.stream()));
+    c.done(ldist_torch::inf_bound_forward(in(input_lower), in(input_upper), in(weight), s.B, s.CO, s.CI, G, s.HW,
+                                          out(output_lower), out(output_upper), output_lower, c.stream()));
 }
 
 // The scatter gradients: sizes come from grad_output and the gradient buffer (model/norm_dist.cpp:79-80,87-88); the

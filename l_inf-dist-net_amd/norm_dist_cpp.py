@@ -8,6 +8,8 @@ RuntimeError) plus the shape relations the reference leaves unchecked, then
 calls the matching C-ABI entry point of libldist_hip.so on the current HIP
 stream of the tensors' device.
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -139,6 +141,22 @@ def norm_dist_backward_ordered(grad_output, input, weight, output, grad_input, g
           *(None if t is None else _p(t) for t in (grad_input, grad_weight)), float(p))
 
 
+def _with_workspace(name, what, sizes, dev, args):
+    """Calls the form `name` of a forward pass that takes scratch memory, where the library has one for the layer; False
+    elsewhere: the plain entry point is the way.  `args`: pointers before and after the sizes."""
+    need = ctypes.c_int64()
+    with torch.cuda.device(dev):
+        if _lib.lib().ldist_inf_dist_workspace(*sizes, what, ctypes.byref(need)) != 0 or need.value == 0:
+            return False
+        scratch = torch.empty(need.value, dtype=torch.uint8, device=dev)   # free for later work on the stream on return
+        rc = getattr(_lib.lib(), name)(*args[0], *sizes, *args[1], _p(scratch), need.value,
+                                       torch.cuda.current_stream(dev).cuda_stream)
+    if rc == _lib.EUNSUPPORTED:
+        return False
+    _lib.check(rc, name)
+    return True
+
+
 def inf_dist_forward(input, weight, output, pos, G):
     """model/norm_dist.cpp:54-62."""
     for t, n in ((input, "input"), (weight, "weight"), (output, "output")):
@@ -149,7 +167,9 @@ def inf_dist_forward(input, weight, output, pos, G):
     _expect(input.dim() == 3 and weight.dim() == 2, "input must be 3-D, weight 2-D")
     _expect(weight.size(0) == CO and weight.size(1) * G == CI, "weight must be (CO, CI/G)")
     _expect(tuple(output.shape) == (B, CO, HW) and tuple(pos.shape) == (B, CO, HW), "output and pos must be (B, CO, HW)")
-    _call("ldist_inf_dist_forward", dev, _p(input), _p(weight), B, CO, CI, G, HW, _p(output), _p(pos))
+    if not _with_workspace("ldist_inf_dist_forward_ws", 0, (B, CO, CI, G, HW), dev,
+                           ((_p(input), _p(weight)), (_p(output), _p(pos)))):
+        _call("ldist_inf_dist_forward", dev, _p(input), _p(weight), B, CO, CI, G, HW, _p(output), _p(pos))
 
 
 def inf_dist_forward_values(input, weight, output, G):
@@ -164,6 +184,8 @@ def inf_dist_forward_values(input, weight, output, G):
     _expect(input.dim() == 3 and weight.dim() == 2, "input must be 3-D, weight 2-D")
     _expect(weight.size(0) == CO and weight.size(1) * G == CI, "weight must be (CO, CI/G)")
     _expect(tuple(output.shape) == (B, CO, HW), "output must be (B, CO, HW)")
+    if _with_workspace("ldist_inf_dist_forward_ws", 1, (B, CO, CI, G, HW), dev, ((_p(input), _p(weight)), (_p(output), None))):
+        return True
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream(dev).cuda_stream
         rc = _lib.lib().ldist_inf_dist_forward_values(_p(input), _p(weight), B, CO, CI, G, HW, _p(output), stream)
@@ -184,8 +206,10 @@ def inf_dist_bound_forward(input_lower, input_upper, weight, output_lower, outpu
     _expect(weight.size(0) == CO and weight.size(1) * G == CI, "weight must be (CO, CI/G)")
     _expect(tuple(output_lower.shape) == (B, CO, HW) and tuple(output_upper.shape) == (B, CO, HW),
             "outputs must be (B, CO, HW)")
-    _call("ldist_inf_dist_bound_forward", dev, _p(input_lower), _p(input_upper), _p(weight), B, CO, CI, G, HW,
-          _p(output_lower), _p(output_upper))
+    if not _with_workspace("ldist_inf_dist_bound_forward_ws", 2, (B, CO, CI, G, HW), dev,
+                           ((_p(input_lower), _p(input_upper), _p(weight)), (_p(output_lower), _p(output_upper)))):
+        _call("ldist_inf_dist_bound_forward", dev, _p(input_lower), _p(input_upper), _p(weight), B, CO, CI, G, HW,
+              _p(output_lower), _p(output_upper))
 
 
 def inf_dist_value_bound_forward(input, input_lower, input_upper, weight, output, output_lower, output_upper, G,
