@@ -350,6 +350,9 @@ LDIST_API int ldist_norm_dist_conv_backward(const float* grad_output, const floa
  * geometry allows and also switches off the rule that leaves small or channel-heavy layers, which
  * would keep too few waves on a CU, to the general path.  Process-wide; not thread safe. */
 LDIST_API int ldist_set_conv_rows_override(int rows);
+/* The same for the groups of lanes that share the channels of a tile in ldist_inf_dist_conv_forward and
+ * ldist_inf_dist_bound_conv_forward: 0 (default) = chosen by shape; 1 to 8 where the shape allows that many. */
+LDIST_API int ldist_set_conv_groups_override(int groups);
 /* Testing and tuning knob, no counterpart in the reference: how ldist_inf_dist_conv_forward keeps the
  * image rows in LDS.  0 (default) = by shape; 1 = only the variant that holds all channels of a group;
  * 2 = only the variant that stages four channels at a time (needs C/G % 4 == 0); 3 = neither, so that

@@ -80,6 +80,8 @@ def lib():
         handle.ldist_set_tile_override.restype = ctypes.c_int
         handle.ldist_set_conv_rows_override.argtypes = [ctypes.c_int]
         handle.ldist_set_conv_rows_override.restype = ctypes.c_int
+        handle.ldist_set_conv_groups_override.argtypes = [ctypes.c_int]
+        handle.ldist_set_conv_groups_override.restype = ctypes.c_int
         handle.ldist_set_conv_staging_override.argtypes = [ctypes.c_int]
         handle.ldist_set_conv_staging_override.restype = ctypes.c_int
         handle.ldist_version.restype = ctypes.c_int

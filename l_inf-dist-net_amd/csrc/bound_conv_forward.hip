@@ -23,8 +23,9 @@ namespace {
 
 using namespace convimg;
 
-template <int S>
-__global__ void __launch_bounds__(kMaxThreads, 2)
+// GROUPED: several groups of lanes share the channels (share_channels).
+template <int S, bool GROUPED>
+__global__ void __launch_bounds__(GROUPED ? 2 * kMaxThreads : kMaxThreads, 2)
 bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restrict__ upper,
                           const float* __restrict__ weight, float* __restrict__ out_lower,
                           float* __restrict__ out_upper, ConvFwd a) {
@@ -33,11 +34,12 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
     constexpr int BNP = kBNP;
     constexpr float INF = __builtin_inff();
     extern __shared__ __align__(16) float lds[];
-    float* xl = lds;                                    // 2 x [xhalf]: lower rows of the stage's channels
-    float* xu = lds + a.xwords;                         // 2 x [xhalf]: upper rows
-    float* wst = lds + 2 * a.xwords;                    // 2 x [kKC][kBNP]
+    const int NT = GROUPED ? a.GT : blockDim.x, kg = GROUPED ? threadIdx.x / NT : 0;
+    const int tid = threadIdx.x - kg * NT;              // inside the group, which has stages of its own
+    float* xl = lds + kg * (2 * a.xwords + 2 * kKC * kBNP);   // 2 x [xhalf]: lower rows of the stage's channels
+    float* xu = xl + a.xwords;                          // 2 x [xhalf]: upper rows
+    float* wst = xu + a.xwords;                         // 2 x [kKC][kBNP]
     const int xhalf = a.xwords / 2;
-    const int tid = threadIdx.x, NT = blockDim.x;
 
     int id = blockIdx.x;
     const int tn = id % a.tiles_n; id /= a.tiles_n;
@@ -89,7 +91,7 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
     }
     auto xload = [&](int ch) {
         const size_t base = (size_t)ch * kCC * a.H * a.W;
-        const unsigned left = (unsigned)min(a.CG - ch * kCC, kCC);   // channels this stage really has (1..4)
+        const unsigned left = (unsigned)max(min(a.CG - ch * kCC, kCC), 0);   // channels this stage really has (a k-group's last stages may have none)
 #pragma unroll
         for (int r = 0; r < XR; r++) {
             const bool real = ((unsigned)goff[r] >> 28) < left;   // -1 reads as channel 15: never real
@@ -144,12 +146,13 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
         return bad;
     };
 
-    wload(0);
-    xload(0);
+    const int nstage = GROUPED ? (a.CGP / kCC + a.KG - 1) / a.KG : a.CGP / kCC, ch0 = kg * nstage;   // this group's stages: ch0 .. ch0 + nstage - 1
+    wload(ch0);
+    xload(ch0);
     bool bad0 = loaded_irregular();
     xstore(xl, xu);
     wstore(wst);
-    bad0 |= rest(0, xl, xu, wst);
+    bad0 |= rest(ch0, xl, xu, wst);
     int irregular = __syncthreads_or(bad0);
 
     // ---- lane geometry ----
@@ -164,11 +167,10 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
         for (int t = 0; t < kTN; t++) { lo[e][t] = 0.f; up[e][t] = 0.f; }
 
     struct Row { float l[NXR * 4], u[NXR * 4], w[3][kTN]; };
-    const int nstage = a.CGP / kCC;
     for (int ch = 0; ch < nstage; ch++) {
         if (ch + 1 < nstage) {
-            wload(ch + 1);
-            xload(ch + 1);
+            wload(ch0 + ch + 1);
+            xload(ch0 + ch + 1);
         }
         const float* wrow = wst + (ch & 1) * kKC * BNP + kTN * nl;   // walks down the 9*kCC rows of the stage
         const float* lrow = xl + (ch & 1) * xhalf + xlane_off;       // walk down the window rows of its channels
@@ -248,11 +250,18 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
             float* sw = wst + ((ch + 1) & 1) * kKC * BNP;
             xstore(xl + ((ch + 1) & 1) * xhalf, xu + ((ch + 1) & 1) * xhalf);
             wstore(sw);
-            bad |= rest(ch + 1, xl + ((ch + 1) & 1) * xhalf, xu + ((ch + 1) & 1) * xhalf, sw);
+            bad |= rest(ch0 + ch + 1, xl + ((ch + 1) & 1) * xhalf, xu + ((ch + 1) & 1) * xhalf, sw);
         }
         irregular = __syncthreads_or(bad);
     }
 
+    if constexpr (GROUPED) {   // output t of a lane is finished by group t mod KG
+        meet_groups(lds, a, kg, tid, [&](int e, int t) { return make_float2(up[e][t], lo[e][t]); },
+                    [&](int e, int t, float2 other) {
+                        up[e][t] = __builtin_fmaxf(up[e][t], other.x);
+                        lo[e][t] = __builtin_fmaxf(lo[e][t], other.y);
+                    });
+    }
     const int h = h0 + hr;
     if (h >= a.HO) return;
     const int L = a.HO * a.WO;
@@ -260,6 +269,7 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
     for (int t = 0; t < kTN; t++) {
         const int n = n0 + kTN * nl + t;
         if (n >= a.NG) break;
+        if (GROUPED && owner_of(t, a.KG) != kg) continue;
         const size_t at = (((size_t)b * a.G + g) * a.NG + n) * L + (size_t)h * a.WO + w0;
         if (a.vec_out) {
             *reinterpret_cast<float4*>(out_lower + at) = make_float4(lo[0][t], lo[1][t], lo[2][t], lo[3][t]);
@@ -282,17 +292,20 @@ bool bound_conv_forward_supported(const ConvGeom& q, int G, int CO) {
 }
 
 hipError_t bound_conv_forward(const float* lower, const float* upper, const float* weight, float* out_lower,
-                              float* out_upper, const ConvGeom& q, int G, int CO, int device, hipStream_t stream) {
+                              float* out_upper, const ConvGeom& q, int G, int CO, int device, int num_cu, hipStream_t stream) {
     ConvFwd a{};
     if (!plan(q, G, CO, a, 2)) return hipErrorInvalidValue;   // the API layer asks bound_conv_forward_supported first
+    share_channels(q, a, 2, num_cu, {27e3, 36e3, 24e3, 0.0, 1});
     a.vec_in = 0;
     a.vec_out = q.WO % kTM == 0 && aligned16(out_lower) && aligned16(out_upper);   // every run of 8 positions whole and aligned
-    const size_t lds = (2 * (size_t)a.xwords + 2 * (size_t)kKC * kBNP) * sizeof(float);
+    const size_t lds = lds_bytes(a, 2);
     // The dynamic-LDS limit is raised to what the largest launch so far needed, not to the whole 160 KB: the
     // workgroup-wide vote keeps a little static LDS of its own, and the two must fit together.
-    static std::atomic<size_t> raised[64][2] = {};   // callers may come from several threads
-    const int ki = q.S - 1;
-    auto kern = q.S == 1 ? bound_conv_forward_kernel<1> : bound_conv_forward_kernel<2>;
+    static std::atomic<size_t> raised[64][4] = {};   // callers may come from several threads
+    const bool grouped = a.KG > 1;
+    const int ki = (q.S - 1) * 2 + grouped;
+    auto kern = q.S == 1 ? (grouped ? bound_conv_forward_kernel<1, true> : bound_conv_forward_kernel<1, false>)
+                         : (grouped ? bound_conv_forward_kernel<2, true> : bound_conv_forward_kernel<2, false>);
     const int di = device >= 0 && device < 64 ? device : 0;
     if (lds > raised[di][ki].load(std::memory_order_acquire) || di != device) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -304,7 +317,7 @@ hipError_t bound_conv_forward(const float* lower, const float* upper, const floa
         }
     }
     const unsigned grid = (unsigned)((long long)q.B * G * a.tiles_h * a.tiles_n);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(a.ML * a.NL), lds, stream, lower, upper, weight, out_lower, out_upper, a);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(a.KG * a.GT), lds, stream, lower, upper, weight, out_lower, out_upper, a);
     return hipGetLastError();
 }
 

@@ -13,6 +13,7 @@ constexpr int kKC = kCC * 9;      // k values per weight stage
 constexpr int kMaxThreads = 256;
 constexpr int kBNP = 68;          // row length of the weight stage: 64 outputs + 4, a constant so that reads take immediate offsets
 constexpr int kWRegs = 9;         // weight words a lane carries from global to LDS per stage (64 outputs x 36 / 256)
+constexpr int kRest = 6;          // weight words a lane has in flight beyond those, where a workgroup has fewer lanes
 // image words a lane carries per stage when the channels are staged (4 channels x rows held x padded width / lanes)
 __host__ __device__ constexpr int x_regs(int S) { return S == 1 ? 7 : 10; }
 
@@ -27,6 +28,7 @@ struct ConvFwd {
     int resident;                // 1: all channels of the image rows stay in LDS; 0: staged kCC channels at a time
     int xwords;                  // floats of the image area in LDS
     int cstride;                 // resident: floats between channels (NR*WP padded to 4 mod 8); staged: unused
+    int KG, GT;                  // groups of lanes that share a tile's channels, lanes of one
 };
 
 constexpr size_t kLdsLimit = 160 * 1024;
@@ -127,10 +129,112 @@ inline bool plan(const ConvGeom& q, int G, int CO, ConvFwd& a, int nx = 1) {
         }
         if (have) {
             a = pick;
+            a.KG = 1;
+            a.GT = a.ML * a.NL;
             return (long long)q.B * G * a.tiles_h * a.tiles_n < (1LL << 31);
         }
     }
     return false;
+}
+
+inline size_t lds_bytes(const ConvFwd& a, int nx) {
+    const size_t weights = 2 * (size_t)kKC * kBNP;
+    return sizeof(float) * (a.resident ? a.xwords + a.KG * weights : a.KG * (nx * (size_t)a.xwords + weights));
+}
+
+// Clocks of a launch: what the busiest CU's workgroups take, one set of as many as fit after the other.  `one` and `two`: a stage's
+// clocks with one wave per SIMD and with two; `fixed`, `search`: what a workgroup's start and end take, and what the groups
+// divide at the end (the search for the position).
+struct StageClocks { double one, two, fixed, search; int rest; };   // rest: weight words in flight beyond the parked ones
+inline double launch_clocks(const ConvFwd& a, int nx, int num_cu, const StageClocks& c) {
+    const int waves = (a.KG * a.GT + 63) / 64, stages = (a.CGP / kCC + a.KG - 1) / a.KG;
+    long at_once = (long)(kLdsLimit / (lds_bytes(a, nx) + (nx > 1 ? 256 : 0)));
+    if (at_once * waves > 8) at_once = 8 / waves;
+    if (at_once < 1) at_once = 1;
+    const long per_cu = ((long)a.B * a.G * a.tiles_h * a.tiles_n + num_cu - 1) / num_cu;
+    const int unparked = kKC * a.BN - kWRegs * a.GT;   // weights of a stage that lanes fetch without having them in flight
+    const double extra = unparked > 0 ? (c.rest > 1 ? 4e3 : 2e3) * ((unparked + c.rest * a.GT - 1) / (c.rest * a.GT)) : 0.0;
+    auto set = [&](long workgroups) {
+        return stages * ((workgroups * waves > 4 ? c.two : c.one) + extra) + c.fixed + c.search / (a.KG < kTN ? a.KG : kTN);
+    };
+    return per_cu / at_once * set(at_once) + (per_cu % at_once ? set(per_cu % at_once) : 0.0);
+}
+
+// The launch shape of layers that would leave CUs idle: plan() fills a CU, not the device.  77 images of 14 x 14 and 64
+// outputs are 154 workgroups of four waves then, three tenths of what the device can issue.  Here the tile may be smaller
+// and its channels are shared by up to eight groups of lanes (eight waves in all, two per SIMD), which have stages of their
+// own and meet in LDS at the end.  That layer with 64 channels: bounds 190 -> 117 us, values 85 -> 46; the same images at
+// 28 x 28, 32 channels, 32 outputs: 141 -> 119 and 47 -> 47.  The clocks were fitted to these.  A shape is changed where that gains 7 %,
+// and only below four rounds of workgroups: beyond, the last round's share is small.
+inline void share_channels(const ConvGeom& q, ConvFwd& a, int nx, int num_cu, const StageClocks& clocks_of) {
+    if (g_conv_rows_override > 0 && g_conv_groups_override <= 0) return;
+    const int forced = g_conv_groups_override;
+    const double before = launch_clocks(a, nx, num_cu, clocks_of);
+    double best = forced > 0 ? 1e300 : 0.93 * before;
+    if (forced <= 0 && (double)a.B * a.G * a.tiles_h * a.tiles_n > 4.0 * 2 * num_cu) return;   // at least four rounds
+    const int S = q.S, quads = (a.NG + kTN - 1) / kTN, first_tiles = (quads + 15) / 16, nstage = a.CGP / kCC;
+    ConvFwd pick = a;
+    int last_nl = 0;
+    for (int tiles_n = first_tiles; tiles_n <= quads && tiles_n <= 8 * first_tiles; tiles_n++) {
+        ConvFwd c = a;
+        c.NL = (quads + tiles_n - 1) / tiles_n;
+        if (c.NL == last_nl || a.SEG * c.NL > kMaxThreads) continue;
+        last_nl = c.NL;
+        c.BN = c.NL * kTN;
+        c.tiles_n = (quads + c.NL - 1) / c.NL;
+        for (int R = 1; R <= q.HO && R * a.SEG * c.NL <= kMaxThreads; R++) {
+            if (g_conv_rows_override > 0 && R != g_conv_rows_override) continue;
+            c.R = R; c.NR = (R - 1) * S + 3; c.ML = R * a.SEG;
+            c.tiles_h = (q.HO + R - 1) / R;
+            c.GT = c.ML * c.NL;
+            c.cstride = channel_stride(c.NR * a.WP);
+            const int words = kCC * c.NR * a.WP, carried = x_regs(S) * c.GT;
+            if (!a.resident && words > carried) continue;
+            c.xwords = a.resident ? a.CGP * c.cstride : 2 * ((carried + 3) / 4 * 4);
+            int last_per = nstage + 1;
+            for (c.KG = 1; c.KG * c.GT <= 2 * kMaxThreads && c.KG <= nstage; c.KG++) {
+                const int per = (nstage + c.KG - 1) / c.KG;
+                if (per == last_per || (forced > 0 && c.KG != forced)) continue;   // a group more than the stages are worth
+                last_per = per;
+                if (lds_bytes(c, nx) > kLdsLimit - (nx > 1 ? 1024 : 0)) break;
+                const double clocks = launch_clocks(c, nx, num_cu, clocks_of);
+                if (clocks < best) { best = clocks; pick = c; }
+            }
+        }
+    }
+    if (pick.KG != a.KG || pick.R != a.R || pick.NL != a.NL) {
+        const long long grid = (long long)pick.B * pick.G * pick.tiles_h * pick.tiles_n;
+        if (grid < (1LL << 31)) a = pick;
+    }
+}
+
+// Which group of lanes finishes output t of a lane.
+__device__ __forceinline__ int owner_of(int t, int groups) { return t % groups; }
+
+// The groups' results of a lane's outputs meet with the owner of each: mine(e, t) gives an output's
+// two numbers, take(e, t, numbers) sees those of every other group.  Lies over the weight stages (64 bytes per lane of at
+// most 256, where a group has 19 KB), which nothing reads any more when the caller has passed a barrier.
+template <class MINE, class TAKE>
+__device__ __forceinline__ void meet_groups(float* park, const ConvFwd& a, int kg, int tid, MINE&& mine, TAKE&& take) {
+    float2* const p = reinterpret_cast<float2*>(park);
+    const int all = a.KG * a.GT;
+#pragma unroll
+    for (int t = 0; t < kTN; t++) {
+        const int owner = owner_of(t, a.KG);
+        if (t > 0) __syncthreads();
+        if (kg != owner) {
+#pragma unroll
+            for (int e = 0; e < kTM; e++) p[e * all + kg * a.GT + tid] = mine(e, t);
+        }
+        __syncthreads();
+        if (kg == owner) {
+            for (int g = 0; g < a.KG; g++) {
+                if (g == kg) continue;
+#pragma unroll
+                for (int e = 0; e < kTM; e++) take(e, t, p[e * all + g * a.GT + tid]);
+            }
+        }
+    }
 }
 
 }  // namespace convimg

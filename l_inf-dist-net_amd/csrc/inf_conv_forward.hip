@@ -22,6 +22,7 @@
 namespace ldist {
 
 int g_conv_rows_override = 0;      // > 0: output rows per workgroup forced (tests and tuning)
+int g_conv_groups_override = 0;    // > 0: groups of lanes that share the channels forced, where the shape allows it (tests)
 int g_conv_staging_override = 0;   // 1: image rows resident in LDS only; 2: staged only; 3: neither; 0: by shape
 
 namespace {
@@ -31,15 +32,18 @@ using namespace convimg;
 // POS = false: values only, for a forward pass that no gradient follows (pos has no reader then): the maximum is kept
 // across channels without the per-channel record, and the search after the loop is left out.  Same subtractions and
 // maxima: the values are those of POS = true bit for bit.
-template <int S, bool RESIDENT, bool POS>
-__global__ void __launch_bounds__(kMaxThreads, 2)
+// GROUPED: several groups of lanes share the channels (share_channels).
+template <int S, bool RESIDENT, bool POS, bool GROUPED>
+__global__ void __launch_bounds__(GROUPED ? 2 * kMaxThreads : kMaxThreads, 2)
 inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__ weight, float* __restrict__ out,
                         int32_t* __restrict__ pos, ConvFwd a) {
     constexpr int NXR = (7 * S + 2) / 4 + 1;          // 128-bit reads per window row: pixels 0 .. 7*S + 2
     extern __shared__ __align__(16) float lds[];
-    float* tile = lds;                                  // RESIDENT: [CGP][NR][WP]; staged: 2 x [xwords / 2]
-    float* wst = lds + a.xwords;                        // 2 x [kKC][kBNP]
-    const int tid = threadIdx.x, NT = blockDim.x;
+    const int NT = GROUPED ? a.GT : blockDim.x, kg = GROUPED ? threadIdx.x / NT : 0;
+    const int tid = threadIdx.x - kg * NT;              // inside the group, which has stages of its own
+    // RESIDENT: [CGP][NR][WP], all groups'; staged: 2 x [xwords / 2] per group
+    float* tile = lds + (RESIDENT ? 0 : kg * (a.xwords + 2 * kKC * kBNP));
+    float* wst = tile + a.xwords + (RESIDENT ? kg * 2 * kKC * kBNP : 0);   // 2 x [kKC][kBNP]
 
     int id = blockIdx.x;
     const int tn = id % a.tiles_n; id /= a.tiles_n;
@@ -81,13 +85,25 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
     // directly; with 256 lanes this loop is empty.
     auto wrest = [&](int ch, float* stage) {
         const int kb = ch * kKC;
-        for (int idx = tid + kWRegs * NT; idx < kKC * a.BN; idx += NT) {
-            const int n = idx / kKC, kk = idx - n * kKC;
-            const bool real = n < nvalid && kb + kk < K;
-            stage[kk * BNP + n] = real ? wgrp[(unsigned)(n * K + kb + kk)] : 0.f;
+        constexpr int REST = POS ? 1 : kRest;   // with pos there are no registers for more
+        for (int first = tid + kWRegs * NT; first < kKC * a.BN; first += REST * NT) {
+            float v[REST];
+#pragma unroll
+            for (int r = 0; r < REST; r++) {
+                const int idx = first + r * NT, n = idx / kKC, kk = idx - n * kKC;
+                const bool real = n < nvalid && kb + kk < K;
+                v[r] = wgrp[real ? (unsigned)(n * K + kb + kk) : 0u];
+                v[r] = real ? v[r] : 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < REST; r++) {
+                const int idx = first + r * NT, n = idx / kKC, kk = idx - n * kKC;
+                if (idx < kKC * a.BN) stage[kk * BNP + n] = v[r];
+            }
         }
     };
-    wload(0);
+    const int nstage = GROUPED ? (a.CGP / kCC + a.KG - 1) / a.KG : a.CGP / kCC, ch0 = kg * nstage;   // this group's stages: ch0 .. ch0 + nstage - 1
+    wload(ch0);
 
     const float* src = img + ((size_t)b * a.G + g) * a.CG * a.H * a.W;   // the group's channels of this image
     // ---- staged: what each lane moves per stage is the same every time, only the channel base advances ----
@@ -108,11 +124,12 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
         }
     }
     auto xload = [&](int ch) {
-        const float* base = src + (size_t)ch * kCC * a.H * a.W;
+        const bool real = !GROUPED || ch * kCC < a.CG;    // a group's last stages may have no channels (CG % kCC == 0 here)
+        const float* base = src + (real ? (size_t)ch * kCC * a.H * a.W : 0);
 #pragma unroll
         for (int r = 0; r < kXRegs; r++) {
             const float v = base[goff[r] < 0 ? 0 : goff[r]];   // branch-free: padding reads a valid word, replaced by 0
-            xreg[r] = goff[r] < 0 ? 0.f : v;
+            xreg[r] = goff[r] < 0 || !real ? 0.f : v;
         }
     };
     auto xstore = [&](float* stage) {
@@ -122,13 +139,14 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
     // A workgroup too small to carry a whole stage in kXRegs words per lane (tiny images) moves the rest
     // directly; with 256 lanes this loop is empty.
     auto xrest = [&](int ch, float* stage) {
-        const float* base = src + (size_t)ch * kCC * a.H * a.W;
+        const bool there = !GROUPED || ch * kCC < a.CG;
+        const float* base = src + (there ? (size_t)ch * kCC * a.H * a.W : 0);
         const int plane = NR * WP;
         for (int idx = tid + kXRegs * NT; idx < kCC * plane; idx += NT) {
             const int c = idx / plane, rem = idx - c * plane;
             const int row = rem / WP, col = rem - row * WP;
             const int y = y0 + row, x = col - a.P;
-            const bool real = (unsigned)y < (unsigned)a.H && (unsigned)x < (unsigned)a.W;
+            const bool real = there && (unsigned)y < (unsigned)a.H && (unsigned)x < (unsigned)a.W;
             stage[idx] = real ? base[(c * a.H + y) * a.W + x] : 0.f;
         }
     };
@@ -136,6 +154,7 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
     // ---- RESIDENT: image rows -> LDS once, padding as zeros ----
     if constexpr (RESIDENT) {
         const int words = a.CGP * CST;
+        const int tid = threadIdx.x, NT = blockDim.x;   // all groups together
         for (int i = tid * 4; i < words; i += NT * 4) *reinterpret_cast<float4*>(tile + i) = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
         const int rows = a.CG * NR;
@@ -165,20 +184,34 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
                     }
             }
         } else {
-            for (int i = tid; i < rows * a.W; i += NT) {
-                const int row = i / a.W, x = i - row * a.W;
-                const int c = row / NR, r = row - c * NR;
-                const int y = y0 + r;
-                if ((unsigned)y < (unsigned)a.H) tile[c * CST + r * WP + a.P + x] = src[((size_t)c * a.H + y) * a.W + x];
+            // eight words in flight per lane (one: 30 of 85 us of a 64-channel layer of 77 images of 14 x 14 were this copy)
+            constexpr int UN = 8;
+            const int total = rows * a.W;
+            for (int i0 = tid; i0 < total; i0 += UN * NT) {
+                float v[UN];
+                int at[UN];
+#pragma unroll
+                for (int u = 0; u < UN; u++) {
+                    const int i = i0 + u * NT;
+                    const int row = i / a.W, x = i - row * a.W;
+                    const int c = row / NR, r = row - c * NR;
+                    const int y = y0 + r;
+                    const bool real = i < total && (unsigned)y < (unsigned)a.H;
+                    at[u] = real ? c * CST + r * WP + a.P + x : -1;
+                    v[u] = src[real ? ((size_t)c * a.H + y) * a.W + x : 0];
+                }
+#pragma unroll
+                for (int u = 0; u < UN; u++)
+                    if (at[u] >= 0) tile[at[u]] = v[u];
             }
         }
     } else {
-        xload(0);
+        xload(ch0);
         xstore(tile);
-        xrest(0, tile);
+        xrest(ch0, tile);
     }
     wstore(wst);
-    wrest(0, wst);
+    wrest(ch0, wst);
     __syncthreads();
 
     // ---- lane geometry ----
@@ -194,18 +227,20 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
 #pragma unroll
         for (int t = 0; t < kTN; t++) { acc[e][t] = 0.f; cm[e][t] = 0.f; unit[e][t] = 0; }
 
-    const int nstage = a.CGP / kCC;
-    const float* xch = xlane;
+    const float* xch = xlane + (RESIDENT ? ch0 * kCC * CST : 0);
     for (int ch = 0; ch < nstage; ch++) {
         if (ch + 1 < nstage) {
-            wload(ch + 1);
-            if constexpr (!RESIDENT) xload(ch + 1);
+            wload(ch0 + ch + 1);
+            if constexpr (!RESIDENT) xload(ch0 + ch + 1);
         }
         const float* wrow = wst + (ch & 1) * kKC * BNP + kTN * nl;   // walks down the 9*kCC rows of the stage
         // walks down the window rows of the stage's channels
         const float* xrow = RESIDENT ? xch : tile + (ch & 1) * xhalf + xlane_off;
         static_assert(kTrack == 1 && kCC % 2 == 0, "a unit is a channel; units in pairs");
-        if constexpr (RESIDENT) {
+        // a group's last stages may lie past the channels; staged images read as zeros there
+        const bool past = GROUPED && RESIDENT && (ch0 + ch) * kCC >= a.CG;
+        if (past) {
+        } else if constexpr (RESIDENT) {
             // A unit (one channel: nine differences per position and output) continues the running maximum: cur
             // starts from prev, which is left alone, so the unit raised the maximum iff cur > prev afterwards, and the
             // two arrays swap roles from unit to unit (no copy, one compare and one select per unit and output).
@@ -273,7 +308,7 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
             };
 #pragma unroll 1
             for (int u = 0; u < kCC; u += 2) {
-                const int un = ch * kCC + u;
+                const int un = (ch0 + ch) * kCC + u;
                 unit_pass(acc, cm, un);
                 unit_pass(cm, acc, un + 1);
             }
@@ -321,7 +356,7 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
                 }
                 xrow += kTrack * CST;
                 wrow += 9 * kTrack * BNP;
-                const int un = ch * (kCC / kTrack) + u;
+                const int un = (ch0 + ch) * (kCC / kTrack) + u;
 #pragma unroll
                 for (int e = 0; e < kTM; e++)
 #pragma unroll
@@ -336,15 +371,25 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
         xch += kCC * CST;
         if (ch + 1 < nstage) {
             wstore(wst + ((ch + 1) & 1) * kKC * BNP);
-            wrest(ch + 1, wst + ((ch + 1) & 1) * kKC * BNP);
+            wrest(ch0 + ch + 1, wst + ((ch + 1) & 1) * kKC * BNP);
             if constexpr (!RESIDENT) {
                 xstore(tile + ((ch + 1) & 1) * xhalf);
-                xrest(ch + 1, tile + ((ch + 1) & 1) * xhalf);
+                xrest(ch0 + ch + 1, tile + ((ch + 1) & 1) * xhalf);
             }
         }
         __syncthreads();
     }
 
+    if constexpr (GROUPED) {   // output t of a lane is finished by group t mod KG; of equal maxima the lower channel's counts
+        // RESIDENT: the image rows stay for the search
+        meet_groups(RESIDENT ? lds + a.xwords : lds, a, kg, tid,
+                    [&](int e, int t) { return make_float2(acc[e][t], __int_as_float(unit[e][t])); },
+                    [&](int e, int t, float2 other) {
+                        const int u = __float_as_int(other.y);
+                        if (POS && (other.x > acc[e][t] || (other.x == acc[e][t] && u < unit[e][t]))) unit[e][t] = u;
+                        acc[e][t] = __builtin_fmaxf(acc[e][t], other.x);
+                    });
+    }
     const int h = h0 + hr;
     if (h >= a.HO) return;
     const int L = a.HO * a.WO;
@@ -353,6 +398,7 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
         for (int t = 0; t < kTN; t++) {
             const int n = n0 + kTN * nl + t;
             if (n >= a.NG) break;
+            if (GROUPED && owner_of(t, a.KG) != kg) continue;
             const size_t at = (((size_t)b * a.G + g) * a.NG + n) * L + (size_t)h * a.WO + w0;
             if (a.vec_out) {
                 *reinterpret_cast<float4*>(out + at) = make_float4(acc[0][t], acc[1][t], acc[2][t], acc[3][t]);
@@ -394,6 +440,7 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
     for (int step = 0; step < STEPS; step++) {
         const int t = step / (kTM / EB), e0 = (step % (kTM / EB)) * EB;
         if (step + 1 < STEPS) issue(step + 1, wq[(step + 1) & 1]);
+        if (GROUPED && owner_of(t, a.KG) != kg) continue;   // another group has this output
         float xq[EB][9];
 #pragma unroll
         for (int eb = 0; eb < EB; eb++) {
@@ -455,20 +502,21 @@ bool inf_conv_forward_supported(const ConvGeom& q, int G, int CO) {
 
 // pos == nullptr: values only (the kernel without the argmax).
 hipError_t inf_conv_forward(const float* img, const float* weight, float* out, int32_t* pos, const ConvGeom& q, int G,
-                            int CO, int device, hipStream_t stream) {
+                            int CO, int device, int num_cu, hipStream_t stream) {
     ConvFwd a{};
     if (!plan(q, G, CO, a)) return hipErrorInvalidValue;   // the API layer asks inf_conv_forward_supported first
     const bool with_pos = pos != nullptr;
+    share_channels(q, a, 1, num_cu, with_pos ? StageClocks{10e3, 13e3, 14e3, 20e3, 1} : StageClocks{9e3, 11.5e3, 14e3, 0.0, kRest});
     a.vec_in = q.W % 4 == 0 && aligned16(img);
     a.vec_out = q.WO % kTM == 0 && aligned16(out) && aligned16(pos);   // every run of 8 positions whole and aligned
-    const size_t lds = ((size_t)a.xwords + 2 * (size_t)kKC * kBNP) * sizeof(float);
-    static std::atomic<bool> raised[64][8] = {};   // callers may come from several threads
-    const int ki = ((q.S - 1) * 2 + a.resident) * 2 + (with_pos ? 1 : 0);
+    const size_t lds = lds_bytes(a, 1);
+    static std::atomic<bool> raised[64][16] = {};   // callers may come from several threads
+    const int ki = (((q.S - 1) * 2 + a.resident) * 2 + (with_pos ? 1 : 0)) * 2 + (a.KG > 1 ? 1 : 0);
     using Kern = void (*)(const float*, const float*, float*, int32_t*, ConvFwd);
-    const Kern table[8] = {inf_conv_forward_kernel<1, false, false>, inf_conv_forward_kernel<1, false, true>,
-                           inf_conv_forward_kernel<1, true, false>,  inf_conv_forward_kernel<1, true, true>,
-                           inf_conv_forward_kernel<2, false, false>, inf_conv_forward_kernel<2, false, true>,
-                           inf_conv_forward_kernel<2, true, false>,  inf_conv_forward_kernel<2, true, true>};
+#define BOTH(S, RESIDENT, POS) inf_conv_forward_kernel<S, RESIDENT, POS, false>, inf_conv_forward_kernel<S, RESIDENT, POS, true>
+    const Kern table[16] = {BOTH(1, false, false), BOTH(1, false, true), BOTH(1, true, false), BOTH(1, true, true),
+                            BOTH(2, false, false), BOTH(2, false, true), BOTH(2, true, false), BOTH(2, true, true)};
+#undef BOTH
     const Kern kern = table[ki];
     if (!(device >= 0 && device < 64 && raised[device][ki].load(std::memory_order_acquire))) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -477,7 +525,7 @@ hipError_t inf_conv_forward(const float* img, const float* weight, float* out, i
         if (device >= 0 && device < 64) raised[device][ki].store(true, std::memory_order_release);
     }
     const unsigned grid = (unsigned)((long long)q.B * G * a.tiles_h * a.tiles_n);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(a.ML * a.NL), lds, stream, img, weight, out, pos, a);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(a.KG * a.GT), lds, stream, img, weight, out, pos, a);
     return hipGetLastError();
 }
 

@@ -400,7 +400,8 @@ static int inf_conv_forward_entry(const float* img, const float* weight, int B, 
     if (!ldist::inf_conv_forward_supported(q, G, CO)) return LDIST_EUNSUPPORTED;
     ldist::Problem pr{};
     if (int rc = current_device(pr)) return rc;
-    return finish(ldist::inf_conv_forward(img, weight, output, pos, q, G, CO, pr.device, (hipStream_t)stream));
+    return finish(ldist::inf_conv_forward(img, weight, output, pos, q, G, CO, pr.device, pr.num_cu,
+                                          (hipStream_t)stream));
 }
 
 int ldist_inf_dist_conv_forward(const float* img, const float* weight, int B, int C, int H, int W, int CO, int G,
@@ -438,7 +439,7 @@ int ldist_inf_dist_bound_conv_forward(const float* lower_img, const float* upper
     ldist::Problem pr{};
     if (int rc = current_device(pr)) return rc;
     return finish(ldist::bound_conv_forward(lower_img, upper_img, weight, output_lower, output_upper, q, G, CO,
-                                            pr.device, (hipStream_t)stream));
+                                            pr.device, pr.num_cu, (hipStream_t)stream));
 }
 
 int ldist_norm_dist_conv_supported(int C, int H, int W, int CO, int G, int KH, int KW, int stride, int padding,
@@ -524,6 +525,12 @@ int ldist_set_conv_staging_override(int mode) {
 int ldist_set_conv_rows_override(int rows) {
     if (rows < 0) return LDIST_EINVAL;
     ldist::g_conv_rows_override = rows;
+    return LDIST_OK;
+}
+
+int ldist_set_conv_groups_override(int groups) {
+    if (groups < 0 || groups > 8) return LDIST_EINVAL;
+    ldist::g_conv_groups_override = groups;
     return LDIST_OK;
 }
 
