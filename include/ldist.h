@@ -345,6 +345,30 @@ LDIST_API int ldist_norm_dist_conv_backward(const float* grad_output, const floa
                                             const float* output, int B, int C, int H, int W, int CO, int G, int KH, int KW,
                                             int stride, int padding, int dilation, float* grad_img, float* grad_weight,
                                             float p, ldist_stream_t stream);
+/* The forward passes with the evaluation-mode shift and bias of the layer in the same launch: what is stored for channel c
+ * is (v - mean[c]) + bias[c], either of which may be null; otherwise as the entry point without `_shifted`.  Fully
+ * connected layers (HW = 1) and 3x3 image layers.  pos may be null: values only (LDIST_EUNSUPPORTED where there is no
+ * such form).  workspace may be null, else it is that of ldist_inf_dist_workspace.  The p-norm form, for passes that no
+ * gradient follows, returns LDIST_EUNSUPPORTED for large layers: apply ldist_channel_shift there. */
+LDIST_API int ldist_inf_dist_forward_shifted(const float* input, const float* weight, int B, int CO, int CI, int G,
+                                             const float* mean, const float* bias, float* output, int32_t* pos,
+                                             void* workspace, int64_t bytes, ldist_stream_t stream);
+LDIST_API int ldist_inf_dist_bound_forward_shifted(const float* input_lower, const float* input_upper, const float* weight,
+                                                   int B, int CO, int CI, int G, const float* mean, const float* bias,
+                                                   float* output_lower, float* output_upper, void* workspace,
+                                                   int64_t bytes, ldist_stream_t stream);
+LDIST_API int ldist_norm_dist_forward_values_shifted(const float* input, const float* weight, int B, int CO, int CI, int G,
+                                                     const float* mean, const float* bias, float* output, float p,
+                                                     ldist_stream_t stream);
+LDIST_API int ldist_inf_dist_conv_forward_shifted(const float* img, const float* weight, int B, int C, int H, int W, int CO,
+                                                  int G, int KH, int KW, int stride, int padding, int dilation,
+                                                  const float* mean, const float* bias, float* output, int32_t* pos,
+                                                  ldist_stream_t stream);
+LDIST_API int ldist_inf_dist_bound_conv_forward_shifted(const float* lower_img, const float* upper_img, const float* weight,
+                                                        int B, int C, int H, int W, int CO, int G, int KH, int KW,
+                                                        int stride, int padding, int dilation, const float* mean,
+                                                        const float* bias, float* output_lower, float* output_upper,
+                                                        ldist_stream_t stream);
 /* Testing and tuning knob, no counterpart in the reference: output rows per workgroup of
  * ldist_inf_dist_conv_forward; 0 (default) = chosen by shape.  A positive value is clamped to what the
  * geometry allows and also switches off the rule that leaves small or channel-heavy layers, which

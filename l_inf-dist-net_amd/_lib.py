@@ -50,6 +50,11 @@ SIGNATURES = {
     "ldist_norm_dist_conv_backward": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _F, _f, _S],
     "ldist_fold": [_F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _S],
     "ldist_inf_dist_backward_input_folded": [_F, _I, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _S],
+    "ldist_inf_dist_forward_shifted": [_F, _F, _i, _i, _i, _i, _F, _F, _F, _I, ctypes.c_void_p, ctypes.c_int64, _S],
+    "ldist_inf_dist_bound_forward_shifted": [_F, _F, _F, _i, _i, _i, _i, _F, _F, _F, _F, ctypes.c_void_p, ctypes.c_int64, _S],
+    "ldist_norm_dist_forward_values_shifted": [_F, _F, _i, _i, _i, _i, _F, _F, _F, _f, _S],
+    "ldist_inf_dist_conv_forward_shifted": [_F, _F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _F, _F, _I, _S],
+    "ldist_inf_dist_bound_conv_forward_shifted": [_F, _F, _F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _F, _F, _F, _S],
     "ldist_adamw_lp_step": [_F, _F, _F, _F, _i, _i, _d, _d, _d, _d, _d, _d, _i, _S],
 }
 

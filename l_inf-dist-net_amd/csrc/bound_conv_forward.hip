@@ -271,6 +271,12 @@ bound_conv_forward_kernel(const float* __restrict__ lower, const float* __restri
         if (n >= a.NG) break;
         if (GROUPED && owner_of(t, a.KG) != kg) continue;
         const size_t at = (((size_t)b * a.G + g) * a.NG + n) * L + (size_t)h * a.WO + w0;
+        if (a.mean || a.bias)
+#pragma unroll
+            for (int e = 0; e < kTM; e++) {
+                lo[e][t] = shifted_value(a.mean, a.bias, g * a.NG + n, lo[e][t]);
+                up[e][t] = shifted_value(a.mean, a.bias, g * a.NG + n, up[e][t]);
+            }
         if (a.vec_out) {
             *reinterpret_cast<float4*>(out_lower + at) = make_float4(lo[0][t], lo[1][t], lo[2][t], lo[3][t]);
             *reinterpret_cast<float4*>(out_lower + at + 4) = make_float4(lo[4][t], lo[5][t], lo[6][t], lo[7][t]);
@@ -292,11 +298,14 @@ bool bound_conv_forward_supported(const ConvGeom& q, int G, int CO) {
 }
 
 hipError_t bound_conv_forward(const float* lower, const float* upper, const float* weight, float* out_lower,
-                              float* out_upper, const ConvGeom& q, int G, int CO, int device, int num_cu, hipStream_t stream) {
+                              float* out_upper, const ConvGeom& q, int G, int CO, int device, int num_cu, const float* mean,
+                              const float* bias, hipStream_t stream) {
     ConvFwd a{};
     if (!plan(q, G, CO, a, 2)) return hipErrorInvalidValue;   // the API layer asks bound_conv_forward_supported first
     share_channels(q, a, 2, num_cu, {27e3, 36e3, 24e3, 0.0, 1});
     a.vec_in = 0;
+    a.mean = mean;
+    a.bias = bias;
     a.vec_out = q.WO % kTM == 0 && aligned16(out_lower) && aligned16(out_upper);   // every run of 8 positions whole and aligned
     const size_t lds = lds_bytes(a, 2);
     // The dynamic-LDS limit is raised to what the largest launch so far needed, not to the whole 160 KB: the

@@ -122,6 +122,12 @@ bound_forward_kernel(const float* __restrict__ lower, const float* __restrict__ 
                 }
     }
 
+    if constexpr (!CONV) {
+        if (d.mean || d.bias) {
+            shift_patch<GEO>(lo, d.mean, d.bias, d, n0, g, tx);
+            shift_patch<GEO>(up, d.mean, d.bias, d, n0, g, tx);
+        }
+    }
     store_patch<GEO, CONV>(out_lower, lo, d, m0, n0, g, tx, ty, d.ovec != 0);
     store_patch<GEO, CONV>(out_upper, up, d, m0, n0, g, tx, ty, d.ovec != 0);
 }
@@ -168,8 +174,9 @@ bound_forward_skinny_kernel(const float* __restrict__ lower, const float* __rest
             for (int q = 1; q < 4; q++) { l = __builtin_fmaxf(l, sl[q][tid]); u = __builtin_fmaxf(u, su[q][tid]); }
             const int r = tid / NB, j = tid % NB;
             if (rows.m0 + r < d.M && nb + j < d.NG) {
-                out_lower[rows.ooff[r] + (size_t)(nb + j) * d.HW] = l;
-                out_upper[rows.ooff[r] + (size_t)(nb + j) * d.HW] = u;
+                const int c = rows.g * d.NG + nb + j;
+                out_lower[rows.ooff[r] + (size_t)(nb + j) * d.HW] = shifted_value(d.mean, d.bias, c, l);
+                out_upper[rows.ooff[r] + (size_t)(nb + j) * d.HW] = shifted_value(d.mean, d.bias, c, u);
             }
         }
         __syncthreads();

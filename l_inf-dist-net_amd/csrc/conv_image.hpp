@@ -2,6 +2,7 @@
 // (inf_conv_forward.hip: values and argmax; bound_conv_forward.hip: interval bounds).
 #pragma once
 #include "kernels.hpp"
+#include "tile.hpp"
 
 namespace ldist {
 namespace convimg {
@@ -28,6 +29,7 @@ struct ConvFwd {
     int resident;                // 1: all channels of the image rows stay in LDS; 0: staged kCC channels at a time
     int xwords;                  // floats of the image area in LDS
     int cstride;                 // resident: floats between channels (NR*WP padded to 4 mod 8); staged: unused
+    const float *mean, *bias;    // per channel: (v - mean) + bias is stored; either may be null
     int KG, GT;                  // groups of lanes that share a tile's channels, lanes of one
 };
 

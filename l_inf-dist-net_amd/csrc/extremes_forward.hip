@@ -64,6 +64,7 @@ struct Side {
 struct Search {
     Side x, w;
     float *out, *out2;     // distances, or the lower and upper bounds
+    const float *mean, *bias;   // of Problem
     int32_t* pos;
     Header* head;
     unsigned char* counts; // [workgroup of the sample][combination of lengths]: outputs that would not pass
@@ -754,14 +755,14 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                         if constexpr (BOX) {
                             const float lo = __builtin_fmaxf(low[j], with), up = __builtin_fmaxf(best[j], have);
                             if (up >= limit[j] && lo >= limit_low[j] && limit[j] < __builtin_inff()) {
-                                s.out[o] = lo;
-                                s.out2[o] = up;
+                                s.out[o] = shifted_value(s.mean, s.bias, l, lo);
+                                s.out2[o] = shifted_value(s.mean, s.bias, l, up);
                             } else {
                                 failed |= 1u << j;
                             }
                         } else if constexpr (MODE == kOnlyValues) {
                             const float v = __builtin_fmaxf(best[j], have);
-                            if (v >= limit[j] && limit[j] < __builtin_inff()) s.out[o] = v;
+                            if (v >= limit[j] && limit[j] < __builtin_inff()) s.out[o] = shifted_value(s.mean, s.bias, l, v);
                             else failed |= 1u << j;
                         } else {
                             float v = __builtin_fabsf(best[j]);
@@ -769,7 +770,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                             const int hp = __float_as_int(with);
                             if (have > v || (have == v && (hp & 0x7fffffff) < (p & 0x7fffffff))) { v = have; p = hp; }
                             if (v > limit[j]) {   // at the limit a lower k might hold the same value
-                                s.out[o] = v;
+                                s.out[o] = shifted_value(s.mean, s.bias, l, v);
                                 s.pos[o] = p;
                             } else {
                                 failed |= 1u << j;
@@ -838,7 +839,10 @@ __global__ void __launch_bounds__(256) extremes_walk_kernel(Search s) {
             }
             up = wave_max(up);
             lo = wave_max(lo);
-            if (lane == 63) { s.out[o] = lo; s.out2[o] = up; }
+            if (lane == 63) {
+                s.out[o] = shifted_value(s.mean, s.bias, o % N, lo);
+                s.out2[o] = shifted_value(s.mean, s.bias, o % N, up);
+            }
         } else {
             float v = 0.f;
             int p = 0;   // k with the sign of the difference
@@ -863,7 +867,7 @@ __global__ void __launch_bounds__(256) extremes_walk_kernel(Search s) {
             }
             wave_best(v, p);
             if (lane == 63) {
-                s.out[o] = v;
+                s.out[o] = shifted_value(s.mean, s.bias, o % N, v);
                 if constexpr (MODE == kWithPos) s.pos[o] = v > 0.f ? p : 0;
             }
         }
@@ -979,6 +983,7 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* w, flo
     s.x = Side{x, x2, pr.B, l.mb, ws + l.x_lists, reinterpret_cast<float*>(ws + l.x_rest)};
     s.w = Side{w, nullptr, pr.NG, l.nb, ws + l.w_lists, reinterpret_cast<float*>(ws + l.w_rest)};
     s.out = out; s.out2 = out2; s.pos = pos;
+    s.mean = pr.mean; s.bias = pr.bias;
     s.K = pr.K; s.C = l.C; s.KC = l.KC;
     s.lanes_first = lanes_for(pr.B, (pr.NG + 7) / 8, pr.num_cu);
     const int second_rows = strip_rows(boxes);

@@ -156,7 +156,7 @@ inf_forward_few_rows_kernel(const float* __restrict__ input, const float* __rest
     const int m = rows.m0 + o / kFewCols, n = rows.n0 + o % kFewCols;
     if (half == 0 && o < NO && m < d.M && n < d.NG) {
         const size_t at = ((size_t)m * d.G + rows.g) * d.NG + n;
-        output[at] = best;
+        output[at] = shifted_value(d.mean, d.bias, rows.g * d.NG + n, best);
         if constexpr (POS) {
             int found = 0;
             if (best > 0.f) {
@@ -257,8 +257,8 @@ bound_forward_few_rows_kernel(const float* __restrict__ lower, const float* __re
     const int o = lane >> 1, m = rows.m0 + o / kFewCols, n = rows.n0 + o % kFewCols;
     if ((lane & 1) == 0 && o < NO && m < d.M && n < d.NG) {
         const size_t at = ((size_t)m * d.G + rows.g) * d.NG + n;
-        out_lower[at] = l;
-        out_upper[at] = u;
+        out_lower[at] = shifted_value(d.mean, d.bias, rows.g * d.NG + n, l);
+        out_upper[at] = shifted_value(d.mean, d.bias, rows.g * d.NG + n, u);
     }
 }
 
@@ -348,7 +348,8 @@ norm_forward_few_rows_kernel(const float* __restrict__ input, const float* __res
         result = pow_pos(sum, 1.0f / p) * mx;
     }
     const int o = lane >> 1, m = rows.m0 + o / kFewCols, n = rows.n0 + o % kFewCols;
-    if ((lane & 1) == 0 && o < NO && m < d.M && n < d.NG) output[((size_t)m * d.G + rows.g) * d.NG + n] = result;
+    if ((lane & 1) == 0 && o < NO && m < d.M && n < d.NG)
+        output[((size_t)m * d.G + rows.g) * d.NG + n] = shifted_value(d.mean, d.bias, rows.g * d.NG + n, result);
 }
 
 static Dims few_dims(const Problem& pr, int rm) {

@@ -249,11 +249,31 @@ __device__ __forceinline__ void store_patch(T* __restrict__ dst, const T (&val)[
     }
 }
 
+// (v - mean[c]) + bias[c] for the lane's patch; either pointer may be null.
+template <class GEO>
+__device__ __forceinline__ void shift_patch(float (&val)[GEO::TM][GEO::TN], const float* __restrict__ mean,
+                                            const float* __restrict__ bias, const Dims& d, int n0, int g, int tx) {
+#pragma unroll
+    for (int j = 0; j < GEO::TN; j++) {
+        const int n = n0 + GEO::col(tx, j);
+        if (n >= d.NG) continue;
+        const int c = g * d.NG + n;
+        const float mu = mean ? mean[c] : 0.f, b = bias ? bias[c] : 0.f;
+#pragma unroll
+        for (int i = 0; i < GEO::TM; i++) {
+            float v = val[i][j];
+            if (mean) v -= mu;
+            if (bias) v += b;
+            val[i][j] = v;
+        }
+    }
+}
+
 inline bool can_vec4_out(const Problem& pr, const void* a, const void* b = nullptr) {
     return aligned16(a) && aligned16(b) && (pr.HW == 1 ? pr.NG % 4 == 0 : pr.HW % 4 == 0);
 }
 
-inline Dims make_dims(const Problem& pr) { return Dims{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, g_xcd_remap, 0, pr.gate}; }
+inline Dims make_dims(const Problem& pr) { return Dims{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, g_xcd_remap, 0, pr.mean, pr.bias, pr.gate}; }
 
 // Dims::m_block for a kernel whose workgroup reads x_rows rows of the input panels (BM times the number of panels)
 // and w_rows rows of weights per stage: `resident` workgroups share an L2 at a time (workgroups per CU times the CUs

@@ -400,6 +400,9 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
             if (n >= a.NG) break;
             if (GROUPED && owner_of(t, a.KG) != kg) continue;
             const size_t at = (((size_t)b * a.G + g) * a.NG + n) * L + (size_t)h * a.WO + w0;
+            if (a.mean || a.bias)
+#pragma unroll
+                for (int e = 0; e < kTM; e++) acc[e][t] = shifted_value(a.mean, a.bias, g * a.NG + n, acc[e][t]);
             if (a.vec_out) {
                 *reinterpret_cast<float4*>(out + at) = make_float4(acc[0][t], acc[1][t], acc[2][t], acc[3][t]);
                 *reinterpret_cast<float4*>(out + at + 4) = make_float4(acc[4][t], acc[5][t], acc[6][t], acc[7][t]);
@@ -480,6 +483,9 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
         const int n = n0 + kTN * nl + t;
         if (n >= a.NG) continue;
         const size_t at = (((size_t)b * a.G + g) * a.NG + n) * L + (size_t)h * a.WO + w0;
+        if (a.mean || a.bias)
+#pragma unroll
+            for (int e = 0; e < kTM; e++) acc[e][t] = shifted_value(a.mean, a.bias, g * a.NG + n, acc[e][t]);
         if (a.vec_out) {
             *reinterpret_cast<float4*>(out + at) = make_float4(acc[0][t], acc[1][t], acc[2][t], acc[3][t]);
             *reinterpret_cast<float4*>(out + at + 4) = make_float4(acc[4][t], acc[5][t], acc[6][t], acc[7][t]);
@@ -502,11 +508,14 @@ bool inf_conv_forward_supported(const ConvGeom& q, int G, int CO) {
 
 // pos == nullptr: values only (the kernel without the argmax).
 hipError_t inf_conv_forward(const float* img, const float* weight, float* out, int32_t* pos, const ConvGeom& q, int G,
-                            int CO, int device, int num_cu, hipStream_t stream) {
+                            int CO, int device, int num_cu, const float* mean, const float* bias,
+                            hipStream_t stream) {
     ConvFwd a{};
     if (!plan(q, G, CO, a)) return hipErrorInvalidValue;   // the API layer asks inf_conv_forward_supported first
     const bool with_pos = pos != nullptr;
     share_channels(q, a, 1, num_cu, with_pos ? StageClocks{10e3, 13e3, 14e3, 20e3, 1} : StageClocks{9e3, 11.5e3, 14e3, 0.0, kRest});
+    a.mean = mean;
+    a.bias = bias;
     a.vec_in = q.W % 4 == 0 && aligned16(img);
     a.vec_out = q.WO % kTM == 0 && aligned16(out) && aligned16(pos);   // every run of 8 positions whole and aligned
     const size_t lds = lds_bytes(a, 1);

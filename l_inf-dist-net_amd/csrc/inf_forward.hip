@@ -343,7 +343,13 @@ inf_forward_kernel(const float* __restrict__ input, const float* __restrict__ we
         const int ml = CONV ? inner : outer, nl = CONV ? outer : inner;
         const int m = m0 + ml, n = n0 + nl;
         if (m >= d.M || n >= d.NG) continue;
-        const float4 v4 = *reinterpret_cast<const float4*>(cand_v + 4 * q);
+        float4 v4 = *reinterpret_cast<const float4*>(cand_v + 4 * q);
+        if constexpr (!CONV) {
+            if (d.mean || d.bias) {
+                auto shifted = [&](int e, float v) { return shifted_value(d.mean, d.bias, g * d.NG + min(n + e, d.NG - 1), v); };
+                v4 = make_float4(shifted(0, v4.x), shifted(1, v4.y), shifted(2, v4.z), shifted(3, v4.w));
+            }
+        }
         const int4 p4 = *reinterpret_cast<const int4*>(cand_c + 4 * q);
         const float vs[4] = {v4.x, v4.y, v4.z, v4.w};
         const int ps[4] = {p4.x, p4.y, p4.z, p4.w};
@@ -517,7 +523,7 @@ inf_forward_skinny_kernel(const float* __restrict__ input, const float* __restri
             for (int q = 1; q < 4; q++) take_better(v, p, sv[q][tid], sp[q][tid]);
             const int r = tid / NB, j = tid % NB;
             if (rows.m0 + r < d.M && nb + j < d.NG) {
-                output[rows.ooff[r] + (size_t)(nb + j) * d.HW] = v;
+                output[rows.ooff[r] + (size_t)(nb + j) * d.HW] = shifted_value(d.mean, d.bias, rows.g * d.NG + nb + j, v);
                 pos[rows.ooff[r] + (size_t)(nb + j) * d.HW] = v > 0.f ? p : 0;
             }
         }

@@ -11,6 +11,7 @@ struct Problem {
     int B, G, K, NG, HW;  // K = CI/G, NG = CO/G
     int num_cu;           // compute units of the current device
     int device;
+    const float *mean = nullptr, *bias = nullptr;   // per output channel: what a forward pass stores is (v - mean) + bias (fc layout; the kernels say which)
     const int* gate = nullptr;   // of a launch that may find nothing to do on the device: it leaves at once where *gate is 0
 };
 
@@ -193,13 +194,16 @@ hipError_t norm_conv_backward_weight(const float* grad_output, const float* img,
 extern int g_conv_rows_override;
 extern int g_conv_groups_override;
 extern int g_conv_staging_override;
+// Whether norm_forward without gradients applies Problem::mean and bias.
+bool norm_forward_shifts(const Problem& pr, float p);
 bool inf_conv_forward_supported(const ConvGeom& q, int G, int CO);
 hipError_t inf_conv_forward(const float* img, const float* weight, float* out, int32_t* pos, const ConvGeom& q, int G,
-                            int CO, int device, int num_cu, hipStream_t stream);
+                            int CO, int device, int num_cu, const float* mean, const float* bias, hipStream_t stream);
 // Interval-bound forward straight from the lower and upper images (same geometries; channels always staged).
 bool bound_conv_forward_supported(const ConvGeom& q, int G, int CO);
 hipError_t bound_conv_forward(const float* lower, const float* upper, const float* weight, float* out_lower,
-                              float* out_upper, const ConvGeom& q, int G, int CO, int device, int num_cu, hipStream_t stream);
+                              float* out_upper, const ConvGeom& q, int G, int CO, int device, int num_cu, const float* mean, const float* bias,
+                              hipStream_t stream);
 hipError_t inf_backward_input_folded(const float* grad_output, const int32_t* pos, float* grad_img, const ConvGeom& q,
                                      int G, int CO, hipStream_t stream);
 

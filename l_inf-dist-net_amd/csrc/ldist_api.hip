@@ -163,6 +163,56 @@ int ldist_inf_dist_bound_forward_ws(const float* input_lower, const float* input
     return finish(ldist::bound_forward(input_lower, input_upper, weight, output_lower, output_upper, pr, (hipStream_t)stream));
 }
 
+// Forward passes whose results leave with the evaluation-mode shift and bias applied, (v - mean) + bias: fully connected layers,
+// every kernel of which does so on its way out.  `workspace` may be null.
+int ldist_inf_dist_forward_shifted(const float* input, const float* weight, int B, int CO, int CI, int G, const float* mean,
+                                   const float* bias, float* output, int32_t* pos, void* workspace, int64_t bytes,
+                                   ldist_stream_t stream) {
+    if (!input || !weight || !output) return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, 1, pr)) return rc;
+    if (!pos && !ldist::inf_forward_values_applicable(pr, input, weight)) return LDIST_EUNSUPPORTED;
+    pr.mean = mean;
+    pr.bias = bias;
+    if (workspace) {
+        const int rc = extremes_entry(input, nullptr, weight, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues,
+                                      output, nullptr, pos, workspace, bytes, stream);
+        if (rc != LDIST_OK && rc != LDIST_EUNSUPPORTED) return rc;
+        if (rc == LDIST_OK && ldist::g_extremes > 0) return LDIST_OK;
+    }
+    return finish(pos ? ldist::inf_forward(input, weight, output, pos, pr, (hipStream_t)stream)
+                      : ldist::inf_forward_values(input, weight, output, pr, (hipStream_t)stream));
+}
+
+int ldist_inf_dist_bound_forward_shifted(const float* input_lower, const float* input_upper, const float* weight, int B, int CO,
+                                         int CI, int G, const float* mean, const float* bias, float* output_lower,
+                                         float* output_upper, void* workspace, int64_t bytes, ldist_stream_t stream) {
+    if (!input_lower || !input_upper || !weight || !output_lower || !output_upper) return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, 1, pr)) return rc;
+    pr.mean = mean;
+    pr.bias = bias;
+    if (workspace) {
+        const int rc = extremes_entry(input_lower, input_upper, weight, pr, ldist::ForwardKind::kBounds, output_lower, output_upper,
+                                      nullptr, workspace, bytes, stream);
+        if (rc != LDIST_OK && rc != LDIST_EUNSUPPORTED) return rc;
+        if (rc == LDIST_OK && ldist::g_extremes > 0) return LDIST_OK;
+    }
+    return finish(ldist::bound_forward(input_lower, input_upper, weight, output_lower, output_upper, pr, (hipStream_t)stream));
+}
+
+int ldist_norm_dist_forward_values_shifted(const float* input, const float* weight, int B, int CO, int CI, int G,
+                                           const float* mean, const float* bias, float* output, float p,
+                                           ldist_stream_t stream) {
+    if (!input || !weight || !output || !valid_p(p)) return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, 1, pr)) return rc;
+    if (!ldist::norm_forward_shifts(pr, p)) return LDIST_EUNSUPPORTED;
+    pr.mean = mean;
+    pr.bias = bias;
+    return finish(ldist::norm_forward(input, weight, output, p, pr, true, (hipStream_t)stream));
+}
+
 int ldist_inf_dist_forward(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
                            float* output, int32_t* pos, ldist_stream_t stream) {
     if (!input || !weight || !output || !pos) return LDIST_EINVAL;
@@ -390,7 +440,7 @@ int ldist_inf_dist_conv_forward_supported(int C, int H, int W, int CO, int G, in
 // pos == nullptr: values only
 static int inf_conv_forward_entry(const float* img, const float* weight, int B, int C, int H, int W, int CO, int G,
                                   int KH, int KW, int stride, int padding, int dilation, float* output, int32_t* pos,
-                                  ldist_stream_t stream) {
+                                  ldist_stream_t stream, const float* mean = nullptr, const float* bias = nullptr) {
     ldist::ConvGeom q{};
     if (!img || !weight || !output || CO <= 0 || G <= 0) return LDIST_EINVAL;
     if (int rc = conv_geometry(B, C, H, W, KH, KW, stride, padding, dilation, q)) return rc;
@@ -400,7 +450,7 @@ static int inf_conv_forward_entry(const float* img, const float* weight, int B, 
     if (!ldist::inf_conv_forward_supported(q, G, CO)) return LDIST_EUNSUPPORTED;
     ldist::Problem pr{};
     if (int rc = current_device(pr)) return rc;
-    return finish(ldist::inf_conv_forward(img, weight, output, pos, q, G, CO, pr.device, pr.num_cu,
+    return finish(ldist::inf_conv_forward(img, weight, output, pos, q, G, CO, pr.device, pr.num_cu, mean, bias,
                                           (hipStream_t)stream));
 }
 
@@ -418,6 +468,13 @@ int ldist_inf_dist_conv_forward_values(const float* img, const float* weight, in
                                   stream);
 }
 
+int ldist_inf_dist_conv_forward_shifted(const float* img, const float* weight, int B, int C, int H, int W, int CO, int G,
+                                        int KH, int KW, int stride, int padding, int dilation, const float* mean,
+                                        const float* bias, float* output, int32_t* pos, ldist_stream_t stream) {
+    return inf_conv_forward_entry(img, weight, B, C, H, W, CO, G, KH, KW, stride, padding, dilation, output, pos, stream, mean,
+                                  bias);
+}
+
 int ldist_inf_dist_bound_conv_forward_supported(int C, int H, int W, int CO, int G, int KH, int KW, int stride,
                                                 int padding, int dilation) {
     ldist::ConvGeom q{};
@@ -429,6 +486,14 @@ int ldist_inf_dist_bound_conv_forward_supported(int C, int H, int W, int CO, int
 int ldist_inf_dist_bound_conv_forward(const float* lower_img, const float* upper_img, const float* weight, int B, int C,
                                       int H, int W, int CO, int G, int KH, int KW, int stride, int padding,
                                       int dilation, float* output_lower, float* output_upper, ldist_stream_t stream) {
+    return ldist_inf_dist_bound_conv_forward_shifted(lower_img, upper_img, weight, B, C, H, W, CO, G, KH, KW, stride, padding,
+                                                     dilation, nullptr, nullptr, output_lower, output_upper, stream);
+}
+
+int ldist_inf_dist_bound_conv_forward_shifted(const float* lower_img, const float* upper_img, const float* weight, int B, int C,
+                                              int H, int W, int CO, int G, int KH, int KW, int stride, int padding,
+                                              int dilation, const float* mean, const float* bias, float* output_lower,
+                                              float* output_upper, ldist_stream_t stream) {
     ldist::ConvGeom q{};
     if (!lower_img || !upper_img || !weight || !output_lower || !output_upper || CO <= 0 || G <= 0) return LDIST_EINVAL;
     if (int rc = conv_geometry(B, C, H, W, KH, KW, stride, padding, dilation, q)) return rc;
@@ -439,7 +504,7 @@ int ldist_inf_dist_bound_conv_forward(const float* lower_img, const float* upper
     ldist::Problem pr{};
     if (int rc = current_device(pr)) return rc;
     return finish(ldist::bound_conv_forward(lower_img, upper_img, weight, output_lower, output_upper, q, G, CO,
-                                            pr.device, pr.num_cu, (hipStream_t)stream));
+                                            pr.device, pr.num_cu, mean, bias, (hipStream_t)stream));
 }
 
 int ldist_norm_dist_conv_supported(int C, int H, int W, int CO, int G, int KH, int KW, int stride, int padding,

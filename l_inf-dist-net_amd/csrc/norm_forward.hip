@@ -64,7 +64,7 @@ norm_forward_skinny_kernel(const float* __restrict__ input, const float* __restr
                     const float sum = v + 1e-10f * pow_pos(1e-10f * __builtin_amdgcn_rcpf(mx), p);  // seeded sum
                     const int r = tid / NB, j = tid % NB;
                     if (rows.m0 + r < d.M && nb + j < d.NG)
-                        output[rows.ooff[r] + (size_t)(nb + j) * d.HW] = pow_pos(sum, 1.0f / p) * mx;
+                        output[rows.ooff[r] + (size_t)(nb + j) * d.HW] = shifted_value(d.mean, d.bias, rows.g * d.NG + nb + j, pow_pos(sum, 1.0f / p) * mx);
                 }
             }
             __syncthreads();
@@ -120,6 +120,10 @@ static hipError_t norm_forward_eight_groups(const float* input, const float* wei
     if (wide < square && wide <= flat) return launch_eight_groups<Geo<32, 40, 4, 5, 8>>(pr, stream, input, weight, output, p);
     if (flat < square) return launch_eight_groups<Geo<16, 32, 2, 4, 8>>(pr, stream, input, weight, output, p);
     return launch_eight_groups<Geo<32, 32, 4, 4, 8>>(pr, stream, input, weight, output, p);
+}
+
+bool norm_forward_shifts(const Problem& pr, float p) {
+    return pr.HW == 1 && (pr.NG <= kSkinnyMaxNG || small_forward_tile(pr, ForwardKind::kNorm, p) >= 0);
 }
 
 // `values_only`: no gradient follows.  Such a pass may sum in any order and takes whichever kernel is fastest for the

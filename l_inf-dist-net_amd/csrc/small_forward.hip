@@ -19,6 +19,21 @@ __device__ __forceinline__ void q_store_tile(T* __restrict__ dst, const T* cand,
         if (m >= d.M || n >= d.NG) continue;
         T* at = dst + ((size_t)m * d.G + g) * d.NG + n;
         const T* from = cand + ml * GEO::BN + nl;
+        if constexpr (std::is_same<T, float>::value) {
+            if (d.mean || d.bias) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = shifted_value(d.mean, d.bias, g * d.NG + min(n + e, d.NG - 1), from[e]);
+                if (d.ovec && n + 3 < d.NG) {
+                    *reinterpret_cast<float4*>(at) = make_float4(v[0], v[1], v[2], v[3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < d.NG) at[e] = v[e];
+                }
+                continue;
+            }
+        }
         if (d.ovec && n + 3 < d.NG) {
             *reinterpret_cast<V4*>(at) = *reinterpret_cast<const V4*>(from);
         } else {

@@ -15,6 +15,22 @@ inline torch::Tensor workspace(int B, int CO, int CI, int G, int HW, int what, c
     return torch::empty({bytes}, like.options().dtype(torch::kUInt8).requires_grad(false));
 }
 
+// The same with the evaluation-mode shift and bias (either may be null) applied by the forward kernel; fully connected layers.
+inline int inf_forward_shifted(const float* x, const float* w, int B, int CO, int CI, int G, const float* mean, const float* bias,
+                               float* y, int32_t* pos, const torch::Tensor& like, ldist_stream_t stream) {
+    const torch::Tensor ws = workspace(B, CO, CI, G, 1, pos ? LDIST_WITH_POS : LDIST_VALUES_ONLY, like);
+    return ldist_inf_dist_forward_shifted(x, w, B, CO, CI, G, mean, bias, y, pos, ws.defined() ? ws.data_ptr() : nullptr,
+                                          ws.defined() ? ws.numel() : 0, stream);
+}
+
+inline int inf_bound_forward_shifted(const float* lower, const float* upper, const float* w, int B, int CO, int CI, int G,
+                                     const float* mean, const float* bias, float* out_lower, float* out_upper,
+                                     const torch::Tensor& like, ldist_stream_t stream) {
+    const torch::Tensor ws = workspace(B, CO, CI, G, 1, LDIST_BOUNDS, like);
+    return ldist_inf_dist_bound_forward_shifted(lower, upper, w, B, CO, CI, G, mean, bias, out_lower, out_upper,
+                                                ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, stream);
+}
+
 // pos == nullptr: values only; LDIST_EUNSUPPORTED where only the form with pos exists.  `like`: a tensor of the call.
 inline int inf_forward(const float* x, const float* w, int B, int CO, int CI, int G, int HW, float* y, int32_t* pos,
                        const torch::Tensor& like, ldist_stream_t stream) {

@@ -79,6 +79,9 @@ struct Shift {
     double momentum = 0;
     bool training = false;
     bool batch_mean() const { return training && running.defined(); }
+    const float* running_mean() const { return running.defined() ? running.const_data_ptr<float>() : nullptr; }
+    // nothing but per-channel constants follow the distances: the forward kernels can apply them on their way out
+    bool constant(const OptTensor& bias) const { return !batch_mean() && (running.defined() || (bias.has_value() && bias->defined())); }
 };
 
 Tensor mean_shifted(const On& on, const Tensor& x, const Tensor& running, double momentum) {
@@ -125,9 +128,28 @@ Tensor sum_per_channel(const Tensor& g) { return g.dim() == 2 ? g.sum(0) : g.sum
 
 // No gradient follows: the argmax that the forward with gradients records has no reader, and p-norm sums may be taken in
 // any order.
-Tensor distances(const On& on, const Tensor& x, const Tensor& w, int64_t G, double p) {
+// The layer's shift and bias included.
+Tensor distances(const On& on, const Tensor& x, const Tensor& w, int64_t G, double p, const OptTensor& bias, const Shift& shift) {
     const Sizes s = sizes_of(x, w, G);
     Tensor y = torch::empty(s.output(), x.options());
+    if (s.HW == 1 && shift.constant(bias)) {
+        const float *mean = shift.running_mean(), *b = in(bias);
+        int rc;
+        if (std::isinf(p)) {
+            rc = ldist_torch::inf_forward_shifted(in(x), in(w), s.B, s.CO, s.CI, (int)G, mean, b, out(y), nullptr, y, on.stream);
+            if (rc == LDIST_EUNSUPPORTED) {
+                Tensor pos = torch::empty(s.output(), x.options().dtype(torch::kInt32));
+                rc = ldist_torch::inf_forward_shifted(in(x), in(w), s.B, s.CO, s.CI, (int)G, mean, b, out(y),
+                                                      pos.data_ptr<int32_t>(), y, on.stream);
+            }
+        } else {
+            rc = ldist_norm_dist_forward_values_shifted(in(x), in(w), s.B, s.CO, s.CI, (int)G, mean, b, out(y), (float)p, on.stream);
+        }
+        if (rc != LDIST_EUNSUPPORTED) {
+            done("dist_forward_shifted", rc);
+            return y;
+        }
+    }
     if (std::isinf(p)) {
         const int rc = ldist_torch::inf_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y), nullptr, y, on.stream);
         if (rc != LDIST_EUNSUPPORTED) {
@@ -141,7 +163,7 @@ Tensor distances(const On& on, const Tensor& x, const Tensor& w, int64_t G, doub
         done("norm_dist_forward_values", ldist_norm_dist_forward_values(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(y),
                                                                         (float)p, on.stream));
     }
-    return y;
+    return shifted(on, y, bias, shift, false);
 }
 
 // Distances of columns (B, CI, L) with gradients, then the shift: one node.
@@ -151,17 +173,21 @@ struct ColumnLayer : public Function<ColumnLayer> {
         const On on(x);
         const Sizes s = sizes_of(x, w, G);
         const bool inf = std::isinf(p);
+        const bool fused = inf && s.HW == 1 && shift.constant(bias);
         Tensor raw = torch::empty(s.output(), x.options());
         if (inf) {
             Tensor pos = torch::empty(s.output(), x.options().dtype(torch::kInt32));
-            done("inf_dist_forward", ldist_torch::inf_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(raw),
-                                                              pos.data_ptr<int32_t>(), raw, on.stream));
+            int32_t* const at = pos.data_ptr<int32_t>();
+            done("inf_dist_forward",
+                 fused ? ldist_torch::inf_forward_shifted(in(x), in(w), s.B, s.CO, s.CI, (int)G, shift.running_mean(), in(bias),
+                                                          out(raw), at, raw, on.stream)
+                       : ldist_torch::inf_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(raw), at, raw, on.stream));
             ctx->save_for_backward({pos});
         } else {
             done("norm_dist_forward", ldist_norm_dist_forward(in(x), in(w), s.B, s.CO, s.CI, (int)G, s.HW, out(raw), (float)p,
                                                               on.stream));
         }
-        Tensor y = shifted(on, raw, bias, shift, !inf);
+        Tensor y = fused ? raw : shifted(on, raw, bias, shift, !inf);
         if (!inf) ctx->save_for_backward({x, w, raw});
         ctx->saved_data["w"] = w.sizes().vec();
         ctx->saved_data["sizes"] = std::vector<int64_t>{s.B, s.CO, s.CI, s.HW, s.flat};
@@ -258,11 +284,19 @@ struct Unfold : public Function<Unfold> {
 // ---- layers straight from the image -------------------------------------------------------------------------------
 // p = infinity.  Forward: the kernel that reads the image where it covers the geometry, else unfold + distances;
 // backward: the image gradient directly (scatter and fold fused).
+// The layer's shift and bias included.
 Tensor inf_image_forward(const On& on, const Tensor& img, const Tensor& w, int64_t G, const Window& win, bool from_image,
-                         Tensor* pos) {
+                         Tensor* pos, const OptTensor& bias, const Shift& shift) {
     const auto [ho, wo] = win.positions(img);
     const int CO = (int)w.size(0);
     Tensor y = torch::empty({img.size(0), CO, ho * wo}, img.options());
+    if (from_image && shift.constant(bias)) {
+        if (pos) *pos = torch::empty({img.size(0), CO, ho * wo}, img.options().dtype(torch::kInt32));
+        done("inf_dist_conv_forward", ldist_inf_dist_conv_forward_shifted(in(img), in(w), IMAGE_ARGS(img), CO, (int)G,
+                                                                          WINDOW_ARGS(win), shift.running_mean(), in(bias), out(y),
+                                                                          pos ? pos->data_ptr<int32_t>() : nullptr, on.stream));
+        return y;
+    }
     if (pos || !from_image) {
         Tensor own = torch::empty({img.size(0), CO, ho * wo}, img.options().dtype(torch::kInt32));
         if (from_image) {
@@ -279,7 +313,7 @@ Tensor inf_image_forward(const On& on, const Tensor& img, const Tensor& w, int64
         done("inf_dist_conv_forward_values", ldist_inf_dist_conv_forward_values(in(img), in(w), IMAGE_ARGS(img), CO, (int)G,
                                                                                 WINDOW_ARGS(win), out(y), on.stream));
     }
-    return y;
+    return shifted(on, y, bias, shift, false);
 }
 
 struct InfImageLayer : public Function<InfImageLayer> {
@@ -287,7 +321,7 @@ struct InfImageLayer : public Function<InfImageLayer> {
                           bool from_image, Shift shift) {
         const On on(img);
         Tensor pos;
-        Tensor raw = inf_image_forward(on, img, w, G, win, from_image, &pos);
+        Tensor y = inf_image_forward(on, img, w, G, win, from_image, &pos, bias, shift);
         ctx->save_for_backward({pos});
         ctx->saved_data["G"] = G;
         ctx->saved_data["img"] = img.sizes().vec();
@@ -295,7 +329,7 @@ struct InfImageLayer : public Function<InfImageLayer> {
         ctx->saved_data["window"] = std::vector<int64_t>{win.k, win.stride, win.pad, win.dil};
         ctx->saved_data["bias"] = bias.has_value() && bias->defined();
         ctx->saved_data["mean"] = shift.batch_mean();
-        return shifted(on, raw, bias, shift, false);
+        return y;
     }
     static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
         const Tensor pos = ctx->get_saved_variables()[0];
@@ -394,11 +428,13 @@ Tensor norm_dist(const Tensor& x, const Tensor& w, int64_t G, double p) {
     check(w, "weight", x.device());
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(w)))
         return ColumnLayer::apply(x, w, OptTensor(), G, p, Shift());
-    return distances(On(x), x, w, G, p);
+    return distances(On(x), x, w, G, p, OptTensor(), Shift());
 }
 
 // `w`: a layer's weight with its window, (CO, CI/G, k, k), or the matrix that it is.
-std::tuple<Tensor, Tensor> bounds_of_columns(const Tensor& lower, const Tensor& upper, const Tensor& w, int64_t G) {
+// The layer's shift and bias included.
+std::tuple<Tensor, Tensor> bounds_of_columns(const Tensor& lower, const Tensor& upper, const Tensor& w, int64_t G,
+                                             const OptTensor& bias, const Shift& shift) {
     check(lower, "input_lower", lower.device());
     check(upper, "input_upper", lower.device());
     check(w, "weight", lower.device());
@@ -406,14 +442,20 @@ std::tuple<Tensor, Tensor> bounds_of_columns(const Tensor& lower, const Tensor& 
     const On on(lower);
     const Sizes s = sizes_of(lower, w, G);
     Tensor lo = torch::empty(s.output(), lower.options()), hi = torch::empty_like(lo);
+    if (s.HW == 1 && shift.constant(bias)) {
+        done("inf_dist_bound_forward",
+             ldist_torch::inf_bound_forward_shifted(in(lower), in(upper), in(w), s.B, s.CO, s.CI, (int)G, shift.running_mean(),
+                                                    in(bias), out(lo), out(hi), lo, on.stream));
+        return {lo, hi};
+    }
     done("inf_dist_bound_forward", ldist_torch::inf_bound_forward(in(lower), in(upper), in(w), s.B, s.CO, s.CI, (int)G, s.HW,
                                                                   out(lo), out(hi), lo, on.stream));
-    return {lo, hi};
+    return {shifted(on, lo, bias, shift, false), shifted(on, hi, bias, shift, false)};
 }
 
 std::tuple<Tensor, Tensor> inf_dist_bound(const Tensor& lower, const Tensor& upper, const Tensor& w, int64_t G) {
     TORCH_CHECK(lower.dim() == 3 && w.dim() == 2, "input_lower must be 3-D, weight 2-D");
-    return bounds_of_columns(lower, upper, w, G);
+    return bounds_of_columns(lower, upper, w, G, OptTensor(), Shift());
 }
 
 Shift make_shift(const OptTensor& running, double momentum, bool training, const torch::Device& dev) {
@@ -489,20 +531,19 @@ std::tuple<Tensor, bool> layer(const Tensor& x, const Tensor& weight, const OptT
                         : NormImageLayer::apply(img, w, bias, G, p, win, shift);
             } else {
                 const On on(img);
-                Tensor raw = inf ? inf_image_forward(on, img, w, G, win, from_image, nullptr)
-                                 : norm_image_forward(on, img, w, G, p, win);
-                y = shifted(on, raw, bias, shift, false);
+                y = inf ? inf_image_forward(on, img, w, G, win, from_image, nullptr, bias, shift)
+                        : shifted(on, norm_image_forward(on, img, w, G, p, win), bias, shift, false);
             }
         } else {
             const Tensor cols = grad && wants_grad(img) ? Unfold::apply(img, win) : unfolded(On(img), img, win);
             if (grad) y = ColumnLayer::apply(cols, w, bias, G, p, shift);
-            else { const On on(cols); y = shifted(on, distances(on, cols, w, G, p), bias, shift, false); }
+            else { const On on(cols); y = distances(on, cols, w, G, p, bias, shift); }
         }
     } else {
         const Tensor cols = as_columns(x);
         check(cols, "input", w.device());
         if (grad) y = ColumnLayer::apply(cols, w, bias, G, p, shift);
-        else { const On on(cols); y = shifted(on, distances(on, cols, w, G, p), bias, shift, false); }
+        else { const On on(cols); y = distances(on, cols, w, G, p, bias, shift); }
     }
     return {as_output(y, x, win), from_image};
 }
@@ -531,19 +572,17 @@ std::tuple<Tensor, Tensor, bool> layer_bounds(const Tensor& lower, const Tensor&
         const auto [ho, wo] = win.positions(l);
         lo = torch::empty({l.size(0), w.size(0), ho * wo}, l.options());
         hi = torch::empty_like(lo);
-        done("inf_dist_bound_conv_forward", ldist_inf_dist_bound_conv_forward(in(l), in(u), in(w), IMAGE_ARGS(l), (int)w.size(0),
-                                                                              (int)G, WINDOW_ARGS(win), out(lo), out(hi),
-                                                                              on.stream));
+        done("inf_dist_bound_conv_forward",
+             ldist_inf_dist_bound_conv_forward_shifted(in(l), in(u), in(w), IMAGE_ARGS(l), (int)w.size(0), (int)G, WINDOW_ARGS(win),
+                                                       shift.running_mean(), in(bias), out(lo), out(hi), on.stream));
     } else if (win.trivial()) {
-        std::tie(lo, hi) = bounds_of_columns(as_columns(lower), as_columns(upper), w, G);
+        std::tie(lo, hi) = bounds_of_columns(as_columns(lower), as_columns(upper), w, G, bias, shift);
     } else {
         const Tensor l = lower.contiguous(), u = upper.contiguous();
         check(l, "lower_img", w.device());
         check(u, "upper_img", w.device());
-        std::tie(lo, hi) = bounds_of_columns(unfolded(on, l, win), unfolded(on, u, win), w, G);
+        std::tie(lo, hi) = bounds_of_columns(unfolded(on, l, win), unfolded(on, u, win), w, G, bias, shift);
     }
-    lo = shifted(on, lo, bias, shift, false);
-    hi = shifted(on, hi, bias, shift, false);
     return {as_output(lo, lower, win), as_output(hi, lower, win), from_image};
 }
 

@@ -17,26 +17,6 @@
 
 namespace ldist {
 
-// (v - mean[c]) + bias[c] for the lane's patch; either pointer may be null.
-template <class GEO>
-__device__ __forceinline__ void shift_patch(float (&val)[GEO::TM][GEO::TN], const float* __restrict__ mean,
-                                            const float* __restrict__ bias, const Dims& d, int n0, int g, int tx) {
-#pragma unroll
-    for (int j = 0; j < GEO::TN; j++) {
-        const int n = n0 + GEO::col(tx, j);
-        if (n >= d.NG) continue;
-        const int c = g * d.NG + n;
-        const float mu = mean ? mean[c] : 0.f, b = bias ? bias[c] : 0.f;
-#pragma unroll
-        for (int i = 0; i < GEO::TM; i++) {
-            float v = val[i][j];
-            if (mean) v -= mu;
-            if (bias) v += b;
-            val[i][j] = v;
-        }
-    }
-}
-
 template <class GEO, bool CONV, int VEC>
 __global__ void __launch_bounds__(GEO::NT, 2)
 value_bound_forward_kernel(const float* __restrict__ input, const float* __restrict__ lower,
