@@ -1,9 +1,9 @@
 // Forward kernels for fully connected layers with a handful of rows (serving one or a few inputs): bound by reading the
 // weights once, so they go from memory into registers, never through LDS.
 //
-// A wave owns RM rows x 4 outputs and its 64 lanes split k, four consecutive k each per trip (a trip is 256 k): a lane
-// loads four weight vectors and RM input vectors with 128-bit loads, the next trip's before the arithmetic of this one.
-// The four waves of a workgroup take 16 neighbouring outputs and read the same rows, which they find in the vector
+// A wave owns RM rows x four outputs (one or two rows: as many outputs) and its 64 lanes split k, four consecutive k each per trip (a trip is 256 k): a lane
+// loads the weight vectors and RM input vectors with 128-bit loads, the next trip's before the arithmetic of this one.
+// The four waves of a workgroup take neighbouring outputs and read the same rows, which they find in the vector
 // cache.  At the end the lanes' results meet through LDS: every wave writes its 4 * RM results of 64 lanes and two lanes
 // take one output.  k past the end: the last vector of a row is moved back to end with the row, vectors beyond it
 // repeat that one, which changes no maximum (sums blank the repeated values).
@@ -17,14 +17,17 @@
 
 namespace ldist {
 
-constexpr int kFewCols = 4;      // outputs per wave
+// Outputs per wave.  A row by itself: one, so that 5120 outputs are five workgroups on every CU with five trips' loads in flight
+// per wave: 1 x 5120 -> 5120, values, 21.6 -> 19.3 us (four outputs: 1.25 workgroups per CU); more rows find work enough in four.
+constexpr int few_cols(int rows) { return rows <= 2 ? rows : 4; }
 
 typedef float FewF4 __attribute__((ext_vector_type(4)));
 
 template <int RM, int NX>
 struct FewRows {
+    static constexpr int COLS = few_cols(RM);
     const float* xr[NX][RM];
-    const float* wr[kFewCols];
+    const float* wr[COLS];
     int K, lane, m0, n0, g;
 
     __device__ __forceinline__ FewRows(const float* const (&input)[NX], const float* weight, const Dims& d) {
@@ -34,21 +37,21 @@ struct FewRows {
         int tm, tn;
         tile_of_block(d, tm, tn, g);
         m0 = tm * RM;
-        n0 = (tn * 4 + wave) * kFewCols;
+        n0 = (tn * 4 + wave) * COLS;
 #pragma unroll
         for (int q = 0; q < NX; q++)
 #pragma unroll
             for (int i = 0; i < RM; i++) xr[q][i] = input[q] + ((size_t)min(m0 + i, d.M - 1) * d.G + g) * K;
 #pragma unroll
-        for (int j = 0; j < kFewCols; j++) wr[j] = weight + ((size_t)g * d.NG + min(n0 + j, d.NG - 1)) * K;
+        for (int j = 0; j < COLS; j++) wr[j] = weight + ((size_t)g * d.NG + min(n0 + j, d.NG - 1)) * K;
     }
     __device__ __forceinline__ int trips() const { return (K + 255) / 256; }
     __device__ __forceinline__ int k_of(int trip) const { return trip * 256 + lane * 4; }
-    struct Vecs { FewF4 x[NX][RM], w[kFewCols]; };
+    struct Vecs { FewF4 x[NX][RM], w[COLS]; };
     __device__ __forceinline__ void load(Vecs& v, int trip) const {
         const int k = min(k_of(trip), K - 4);
 #pragma unroll
-        for (int j = 0; j < kFewCols; j++) v.w[j] = vec(wr[j] + k);
+        for (int j = 0; j < COLS; j++) v.w[j] = vec(wr[j] + k);
 #pragma unroll
         for (int q = 0; q < NX; q++)
 #pragma unroll
@@ -68,6 +71,19 @@ struct FewRows {
                 Vecs v;
                 load(v, t);
                 f(v, t);
+            }
+            return;
+        }
+        if constexpr (RM <= 2) {
+            constexpr int AHEAD = RM == 1 ? 5 : 3;
+#pragma unroll 1
+            for (int t = 0; t < n; t += AHEAD) {
+                Vecs v[AHEAD];
+#pragma unroll
+                for (int c = 0; c < AHEAD; c++) load(v[c], min(t + c, n - 1));
+#pragma unroll
+                for (int c = 0; c < AHEAD; c++)
+                    if (t + c < n) f(v[c], t + c);
             }
             return;
         }
@@ -93,7 +109,7 @@ template <int RM, bool POS>
 __global__ void __launch_bounds__(256, 3)
 inf_forward_few_rows_kernel(const float* __restrict__ input, const float* __restrict__ weight, float* __restrict__ output,
                             int32_t* __restrict__ pos, Dims d) {
-    constexpr int NO = RM * kFewCols;
+    constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
     __shared__ float park[4][NO][kFewPitch];   // first the values, then the tags: both at once would cost a workgroup per CU
     const float* const ins[1] = {input};
     const FewRows<RM, 1> rows(ins, weight, d);
@@ -197,7 +213,7 @@ template <int RM>
 __global__ void __launch_bounds__(256, 3)
 bound_forward_few_rows_kernel(const float* __restrict__ lower, const float* __restrict__ upper, const float* __restrict__ weight,
                               float* __restrict__ out_lower, float* __restrict__ out_upper, Dims d) {
-    constexpr int NO = RM * kFewCols;
+    constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
     __shared__ float park[4][NO][kFewPitch];
     const float* const ins[2] = {lower, upper};
     const FewRows<RM, 2> rows(ins, weight, d);
@@ -268,7 +284,7 @@ template <int RM, int IP>
 __global__ void __launch_bounds__(256, 3)
 norm_forward_few_rows_kernel(const float* __restrict__ input, const float* __restrict__ weight, float* __restrict__ output,
                              float p, Dims d) {
-    constexpr int NO = RM * kFewCols;
+    constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
     __shared__ float park[4][NO][kFewPitch];
     const float* const ins[1] = {input};
     const FewRows<RM, 1> rows(ins, weight, d);
@@ -355,7 +371,7 @@ norm_forward_few_rows_kernel(const float* __restrict__ input, const float* __res
 static Dims few_dims(const Problem& pr, int rm) {
     Dims d = make_dims(pr);
     d.tiles_m = (d.M + rm - 1) / rm;
-    d.tiles_n = (d.NG + 4 * kFewCols - 1) / (4 * kFewCols);
+    d.tiles_n = (d.NG + 4 * few_cols(rm) - 1) / (4 * few_cols(rm));
     return d;
 }
 
