@@ -737,6 +737,12 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                         if constexpr (BOX) limit_low[j] = __builtin_fmaxf(limit_low[j], __builtin_fmaxf(sr[2 * sd.rows] - ll, lh - sr[3 * sd.rows]));
                     }
                 }
+                const float mu = s.mean ? s.mean[l] : 0.f, add = s.bias ? s.bias[l] : 0.f;   // before the stores, which they might alias
+                auto stored = [&](float v) {
+                    if (s.mean) v = v - mu;
+                    if (s.bias) v = v + add;
+                    return v;
+                };
                 unsigned failed = 0;
 #pragma unroll
                 for (int j = 0; j < RS; j++)
@@ -755,14 +761,14 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                         if constexpr (BOX) {
                             const float lo = __builtin_fmaxf(low[j], with), up = __builtin_fmaxf(best[j], have);
                             if (up >= limit[j] && lo >= limit_low[j] && limit[j] < __builtin_inff()) {
-                                s.out[o] = shifted_value(s.mean, s.bias, l, lo);
-                                s.out2[o] = shifted_value(s.mean, s.bias, l, up);
+                                s.out[o] = stored(lo);
+                                s.out2[o] = stored(up);
                             } else {
                                 failed |= 1u << j;
                             }
                         } else if constexpr (MODE == kOnlyValues) {
                             const float v = __builtin_fmaxf(best[j], have);
-                            if (v >= limit[j] && limit[j] < __builtin_inff()) s.out[o] = shifted_value(s.mean, s.bias, l, v);
+                            if (v >= limit[j] && limit[j] < __builtin_inff()) s.out[o] = stored(v);
                             else failed |= 1u << j;
                         } else {
                             float v = __builtin_fabsf(best[j]);
@@ -770,7 +776,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                             const int hp = __float_as_int(with);
                             if (have > v || (have == v && (hp & 0x7fffffff) < (p & 0x7fffffff))) { v = have; p = hp; }
                             if (v > limit[j]) {   // at the limit a lower k might hold the same value
-                                s.out[o] = shifted_value(s.mean, s.bias, l, v);
+                                s.out[o] = stored(v);
                                 s.pos[o] = p;
                             } else {
                                 failed |= 1u << j;
