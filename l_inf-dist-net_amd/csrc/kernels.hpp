@@ -164,6 +164,9 @@ hipError_t unfold(const float* img, float* cols, const ConvGeom& q, hipStream_t 
 hipError_t fold(const float* gcols, float* gimg, const ConvGeom& q, hipStream_t stream);
 // L_inf forward straight from the image (3x3 window, dilation 1, stride 1 or 2; a group's channels
 // either few enough to stay in LDS or a multiple of four); inf_conv_forward_supported tells whether a geometry is covered.
+bool norm_backward_few_applicable(const Problem& pr);   // layers of few outputs (norm_backward_few.hip)
+hipError_t norm_backward_few(const float* grad_output, const float* input, const float* weight, const float* output,
+                             float* grad_input, float* grad_weight, float p, const Problem& pr, hipStream_t stream);
 // Both p-norm gradients in one pass over the terms (norm_backward_fused.hip; the fc layout).
 bool norm_backward_fused_applicable(const Problem& pr, float p, const void* grad_output, const void* input,
                                     const void* weight, const void* output, const void* grad_input,

@@ -343,6 +343,9 @@ int ldist_norm_dist_backward(const float* grad_output, const float* input, const
     if (ldist::norm_backward_fused_applicable(pr, p, grad_output, input, weight, output, grad_input, grad_weight))
         return finish(ldist::norm_backward_fused(grad_output, input, weight, output, grad_input, grad_weight, p, pr,
                                                  (hipStream_t)stream));
+    if (ldist::norm_backward_few_applicable(pr))
+        return finish(ldist::norm_backward_few(grad_output, input, weight, output, grad_input, grad_weight, p, pr,
+                                               (hipStream_t)stream));
     if (ldist::norm_conv_backward_fused_applicable(pr, p))
         return finish(ldist::norm_conv_backward_fused_columns(grad_output, input, weight, output, grad_input, grad_weight,
                                                               p, pr, (hipStream_t)stream));
