@@ -133,6 +133,8 @@ bool norm_forward_shifts(const Problem& pr, float p) {
 // gradients of a five-layer net.
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
                         bool values_only, hipStream_t stream) {
+    if (pr.NG <= kSkinnyMaxNG && values_only && few_rows_of_few_outputs(pr))
+        return norm_forward_few_rows(input, weight, output, p, pr, stream);
     if (pr.NG <= kSkinnyMaxNG) {
         const Dims d = make_dims(pr);
         const bool vec = pr.HW == 1 && pr.K % 4 == 0 && aligned16(input) && aligned16(weight);

@@ -3,6 +3,7 @@
 // (row, output) partial results are reduced inside each wave with DPP moves and then across
 // the four waves through LDS.  These kernels are bound by reading x once and w from L2.
 #pragma once
+#include "kernels.hpp"
 #include "tile.hpp"
 #include "wave_reduce.hpp"
 
@@ -87,6 +88,11 @@ __device__ __forceinline__ void skinny_sweep(const float* const (&input)[NX], co
         else if ((ng) <= 12) { if (vec) LAUNCH(12, true); else LAUNCH(12, false); } \
         else { if (vec) LAUNCH(16, true); else LAUNCH(16, false); }                \
     } while (0)
+
+// One or two rows: a workgroup for each leaves the weights to one or two CUs, which have too few loads in flight to bring them
+// from memory at any rate; the few-rows kernel (a wave per output) spreads them.  1 x 5120 -> 10: 18 -> 6 us; 1024 lanes per row
+// instead of 256: 16, and 272 and 1024 rows 18 -> 28 and 29 -> 50.
+inline bool few_rows_of_few_outputs(const Problem& pr) { return pr.HW == 1 && pr.B <= 2 && pr.K >= 1024 && g_tile_override < 0; }
 
 inline unsigned skinny_grid(const Dims& d, int rw) { return (unsigned)((d.M + rw - 1) / rw) * d.G; }
 
