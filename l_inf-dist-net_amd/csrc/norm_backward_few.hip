@@ -128,9 +128,9 @@ hipError_t launch_few(const float* grad_output, const float* input, const float*
 
 }  // namespace
 
-// Every fully connected layer of up to 16 outputs per group, where the order of the sums is free.
+// Every fully connected layer of up to 16 outputs per group, where the order of the sums is free; a launch has fewer than 2^32 lanes.
 bool norm_backward_few_applicable(const Problem& pr) {
-    return pr.HW == 1 && pr.NG <= kSkinnyMaxNG && g_tile_override < 0 && (long long)((pr.K + kCols - 1) / kCols) * pr.G < (1LL << 31);
+    return pr.HW == 1 && pr.NG <= kSkinnyMaxNG && g_tile_override < 0 && (long long)((pr.K + kCols - 1) / kCols) * pr.G < (1LL << 23);
 }
 
 hipError_t norm_backward_few(const float* grad_output, const float* input, const float* weight, const float* output,
