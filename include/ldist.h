@@ -222,7 +222,7 @@ LDIST_API int ldist_inf_dist_backward_weight_overwrite(const float* grad_output,
 LDIST_API int ldist_inf_dist_backward_overwrite(const float* grad_output, const int32_t* pos, int B, int CO, int CI, int G,
                                       int HW, float* grad_input, float* grad_weight, ldist_stream_t stream);
 
-/* Per-channel mean shift of a contiguous (B, C, L) tensor in one kernel:
+/* Per-channel mean shift of a contiguous (B, C, L) tensor:
  *   mean[c] = mean over b and l of x[b,c,l];   y[b,c,l] = x[b,c,l] - mean[c]
  *   running_mean[c] = (1 - momentum) * running_mean[c] + momentum * mean[c]   (when running_mean != NULL)
  * No native counterpart in the reference: this is the training-mode arithmetic of its MeanNorm

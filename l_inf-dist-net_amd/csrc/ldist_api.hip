@@ -377,7 +377,7 @@ int ldist_mean_shift(const float* x, int B, int C, int L, float* y, float* mean_
     if ((long long)B * C * L >= (1LL << 31)) return LDIST_ERANGE;
     ldist::Problem pr{};
     if (int rc = current_device(pr)) return rc;
-    return finish(ldist::mean_shift(x, y, mean_out, running_mean, momentum, B, C, L, (hipStream_t)stream));
+    return finish(ldist::mean_shift(x, y, mean_out, running_mean, momentum, B, C, L, pr.num_cu, (hipStream_t)stream));
 }
 
 int ldist_adamw_lp_step(float* param, const float* grad, float* exp_avg, float* exp_avg_sq, int rows, int cols,

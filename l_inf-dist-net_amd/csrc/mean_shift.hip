@@ -1,9 +1,11 @@
 // Per-channel mean shift of a (B, C, L) tensor: y[b,c,l] = x[b,c,l] - mean_c, mean_c the mean of
-// x over b and l, in one kernel; optionally moves a running mean.  This is the training-mode
+// x over b and l; optionally moves a running mean.  This is the training-mode
 // arithmetic of the reference's MeanNorm (model/norm_dist.py:85-96), which runs it as five
 // small torch kernels per layer and direction; the same kernel serves the backward pass
 // (gx = gy - mean(gy)).  HBM-bound: a workgroup owns a slab small enough that its second read
 // comes from cache, so the tensor is fetched once and written once.
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "wave_reduce.hpp"
 
@@ -99,9 +101,8 @@ mean_shift_rows_kernel(const float* __restrict__ x, float* __restrict__ y, float
 }
 
 // L > 1: for a fixed (b, c) the L values are contiguous.  Workgroup = one channel; lanes run along l
-// (128-bit accesses when VEC == 4: L % 4 == 0 and 16-byte aligned bases).  A channel is one workgroup's work and
-// there are often fewer channels than CUs, so the workgroup is as large as it can be: what limits this kernel is
-// how many loads one CU keeps in flight.
+// (128-bit accesses when VEC == 4: L % 4 == 0 and 16-byte aligned bases).  A channel is one workgroup's work, and
+// the workgroup is as large as it can be: what limits this kernel is how many loads one CU keeps in flight.
 template <int VEC>
 __global__ void __launch_bounds__(kMsChanThreads)
 mean_shift_channel_kernel(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ mean_out,
@@ -177,8 +178,112 @@ mean_shift_channel_kernel(const float* __restrict__ x, float* __restrict__ y, fl
     }
 }
 
+// The same for channels that are fewer than the CUs and long, in two launches that share a channel out.  The sums are the ones of
+// the kernel above, in the same order and so the same bits: a workgroup of the first launch is one of its sixteen waves.  They go
+// from one launch to the other through y: every workgroup of the second finds all sixteen in the first places of its own part,
+// which it overwrites after reading them, so neither the order of workgroups nor scratch memory matters.  Bound by memory.
+constexpr int kMsWaves = kMsChanThreads / 64;
+constexpr int kMsPartThreads = 256, kMsPartUnroll = 4;
+
+template <int VEC>
+struct ChannelWalk {
+    int c, C, L, per_b;
+    __device__ __forceinline__ size_t at(int i) const {
+        const int b = i / per_b, q = i - b * per_b;
+        return ((size_t)b * C + c) * L + (size_t)q * VEC;
+    }
+};
+
+template <int VEC>
+__global__ void __launch_bounds__(64)
+mean_shift_sums_kernel(const float* __restrict__ x, float* __restrict__ y, int B, int C, int L, int parts, int len) {
+    typedef float V __attribute__((ext_vector_type(VEC)));
+    constexpr int UN = 32;   // loads in flight: a lane's work of 32 x 1024 x 1024 values is one such trip
+    const int c = blockIdx.x / kMsWaves, wave = blockIdx.x % kMsWaves, lane = threadIdx.x;
+    const ChannelWalk<VEC> walk{c, C, L, L / VEC};
+    const int total = B * walk.per_b;
+    float s = 0.f;
+    for (int i0 = wave * 64 + lane; i0 < total; i0 += UN * kMsChanThreads) {
+        V v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            const int i = i0 + u * kMsChanThreads;
+            v[u] = i < total ? *reinterpret_cast<const V*>(x + walk.at(i)) : V(0.f);
+        }
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            if constexpr (VEC == 4) s += (v[u][0] + v[u][1]) + (v[u][2] + v[u][3]);
+            else s += v[u][0];
+        }
+    }
+    s = __shfl(wave_sum(s), 63);
+    if (lane < parts) y[walk.at(lane * len + wave)] = s;
+}
+
+template <int VEC>
+__global__ void __launch_bounds__(kMsPartThreads)
+mean_shift_part_kernel(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ mean_out,
+                       float* __restrict__ running_mean, float momentum, int B, int C, int L, int parts, int len) {
+    typedef float V __attribute__((ext_vector_type(VEC)));
+    __shared__ float sums[kMsWaves];
+    constexpr int UN = kMsPartUnroll;
+    const int c = blockIdx.x / parts, part = blockIdx.x - c * parts;
+    const ChannelWalk<VEC> walk{c, C, L, L / VEC};
+    const int begin = part * len, end = min(B * walk.per_b, begin + len);
+    if (threadIdx.x < kMsWaves) sums[threadIdx.x] = y[walk.at(begin + threadIdx.x)];
+    __syncthreads();   // read by all before any of it is overwritten
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < kMsWaves; q++) t += sums[q];
+    const float mean = t / ((float)B * (float)L);
+    if (part == 0 && threadIdx.x == 0) {
+        if (mean_out) mean_out[c] = mean;
+        if (running_mean) move_running_mean(running_mean, c, mean, momentum);
+    }
+    for (int i0 = begin + threadIdx.x; i0 < end; i0 += UN * kMsPartThreads) {
+        size_t at[UN];
+        V v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            at[u] = walk.at(min(i0 + u * kMsPartThreads, end - 1));
+            v[u] = *reinterpret_cast<const V*>(x + at[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (i0 + u * kMsPartThreads < end) *reinterpret_cast<V*>(y + at[u]) = v[u] - mean;
+    }
+}
+
+// Parts of a channel: four workgroups per CU, each with a full trip of loads (1024 vectors); 1: one workgroup does it all.
+// The lines, us, one workgroup per channel -> shared, images x channels x L with four values to a vector:
+//   128 x 32 x 1024 21.5 -> 12.2, 128 x 64 x 1024 24.3 -> 20.3, 128 x 96 x 1024 26.6 -> 26.6, 128 x 128 x 1024 36.4 -> 38.0;
+//   77 x 32 x 784 11.9 -> 9.2, 32 x 32 x 1024 7.2 -> 6.7, 128 x 64 x 256 8.0 -> 8.4, 77 x 64 x 196 4.9 -> 7.6
+// and with one: 128 x 32 x 841 60.8 -> 21.1, 128 x 128 x 841 66.8 -> 40.9, 128 x 256 x 841 78.8 -> 84.8; 128 x 32 x 101 8.9 -> 7.1,
+// 128 x 32 x 49 6.0 -> 6.4.
+static int channel_parts(int C, int total, int vec, int num_cu) {
+    if (C > num_cu / (vec == 4 ? 4 : 2) || total < 12 * kMsChanThreads) return 1;
+    if (total >= (1 << 30)) return 1;   // 31-bit indices, a trip past the end included
+    return std::min(std::min(4 * num_cu / C, total / (kMsPartUnroll * kMsPartThreads)), 64);
+}
+
+template <int VEC>
+static void launch_channels(const float* x, float* y, float* mean_out, float* running_mean, float momentum, int B, int C, int L,
+                            int num_cu, hipStream_t stream) {
+    const int total = B * (L / VEC), parts = channel_parts(C, total, VEC, num_cu);
+    if (parts == 1) {
+        hipLaunchKernelGGL(mean_shift_channel_kernel<VEC>, dim3((unsigned)C), dim3(kMsChanThreads), 0, stream, x, y, mean_out,
+                           running_mean, momentum, B, C, L);
+        return;
+    }
+    // the last part has at least len - parts + 1 vectors, of 1024 - 63: room for the sixteen sums
+    const int len = (total + parts - 1) / parts;
+    hipLaunchKernelGGL(mean_shift_sums_kernel<VEC>, dim3((unsigned)(C * kMsWaves)), dim3(64), 0, stream, x, y, B, C, L, parts, len);
+    hipLaunchKernelGGL(mean_shift_part_kernel<VEC>, dim3((unsigned)(C * parts)), dim3(kMsPartThreads), 0, stream, x, y, mean_out,
+                       running_mean, momentum, B, C, L, parts, len);
+}
+
 hipError_t mean_shift(const float* x, float* y, float* mean_out, float* running_mean, float momentum, int B, int C,
-                      int L, hipStream_t stream) {
+                      int L, int num_cu, hipStream_t stream) {
     if (L == 1) {
         const unsigned grid = (unsigned)((C + kMsCols - 1) / kMsCols);
         if (C % 4 == 0 && aligned16(x) && aligned16(y))
@@ -188,11 +293,9 @@ hipError_t mean_shift(const float* x, float* y, float* mean_out, float* running_
             hipLaunchKernelGGL(mean_shift_rows_kernel<false>, dim3(grid), dim3(kMsThreads), 0, stream, x, y,
                                mean_out, running_mean, momentum, B, C);
     } else if (L % 4 == 0 && aligned16(x) && aligned16(y)) {
-        hipLaunchKernelGGL(mean_shift_channel_kernel<4>, dim3((unsigned)C), dim3(kMsChanThreads), 0, stream, x, y,
-                           mean_out, running_mean, momentum, B, C, L);
+        launch_channels<4>(x, y, mean_out, running_mean, momentum, B, C, L, num_cu, stream);
     } else {
-        hipLaunchKernelGGL(mean_shift_channel_kernel<1>, dim3((unsigned)C), dim3(kMsChanThreads), 0, stream, x, y,
-                           mean_out, running_mean, momentum, B, C, L);
+        launch_channels<1>(x, y, mean_out, running_mean, momentum, B, C, L, num_cu, stream);
     }
     return hipGetLastError();
 }
