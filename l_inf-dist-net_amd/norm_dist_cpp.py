@@ -297,7 +297,7 @@ def inf_dist_backward_overwrite(grad_output, pos, grad_input, grad_weight, G):
 
 
 def mean_shift(x, y, mean_out=None, running_mean=None, momentum=0.0):
-    """y = x minus its per-channel mean over dims 0 and 2 of a (B, C, L) tensor, in one kernel.
+    """y = x minus its per-channel mean over dims 0 and 2 of a (B, C, L) tensor.
 
     Not in the reference's binding: there the same arithmetic is MeanNorm's torch code
     (model/norm_dist.py:85-96).  ``mean_out`` (C) receives the mean, ``running_mean`` (C) is moved
