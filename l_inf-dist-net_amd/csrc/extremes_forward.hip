@@ -358,7 +358,8 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
 
 // A workgroup makes the lists of 16 rows in one chunk, a wave those of two rows: all values beyond `t` from the center,
 // where t starts as what the sampled rows needed on the average and is moved where the list would overflow or stay half empty
-// (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly.
+// (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly,
+// unless more values tie at the outer end than the list has places: such a row's bounds are those of all its values.
 // Bound by reading the operands once.
 template <int NV, bool PAIR>
 __global__ void __launch_bounds__(512, PAIR ? 3 : 5) extremes_select_kernel(Search s) {
@@ -439,7 +440,8 @@ __global__ void __launch_bounds__(512, PAIR ? 3 : 5) extremes_select_kernel(Sear
                     float most = 0.f;
 #pragma unroll
                     for (int j = 0; j < NV; j++) most = __builtin_fmaxf(most, __builtin_fabsf(key(j) - F * center));
-                    float in = 0.f, out = wave_max_f(most) * (1.f / F);   // too long a list, and none at all
+                    // too long a list, and one of no more than what ties at the outer end: center + t, rounded, may lie inside it
+                    float in = 0.f, out = wave_max_f(most) * (1.f / F);
                     if (n > q) in = t; else out = __builtin_fminf(out, t);
 #pragma unroll 1
                     for (int step = 0; step < 10; step++) {
@@ -476,6 +478,21 @@ __global__ void __launch_bounds__(512, PAIR ? 3 : 5) extremes_select_kernel(Sear
                     least_upper = __builtin_fminf(least_upper, in ? kNever : b.v[j]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+            }
+            if (__builtin_expect(base > q, 0)) {   // the list has lost values that no bound above speaks for
+#pragma unroll
+                for (int j = 0; j < NV; j++) {
+                    most = __builtin_fmaxf(most, P ? b.v[j] : a.v[j]);
+                    least = __builtin_fminf(least, a.v[j]);
+                    if constexpr (P) {
+                        most_lower = __builtin_fmaxf(most_lower, a.v[j]);
+                        least_upper = __builtin_fminf(least_upper, b.v[j]);
+                    }
+                }
+                if constexpr (!P) {
+                    hi = wave_max_f(most);
+                    lo = wave_min_f(least);
+                }
             }
             // a list that is not full repeats the chunk's first value
             const unsigned v0 = __builtin_amdgcn_readfirstlane(__float_as_uint(a.v[0]));
