@@ -110,6 +110,7 @@ __global__ void __launch_bounds__(256, 3)
 inf_forward_few_rows_kernel(const float* __restrict__ input, const float* __restrict__ weight, float* __restrict__ output,
                             int32_t* __restrict__ pos, Dims d) {
     constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
+    if (gated_off(d)) return;
     __shared__ float park[4][NO][kFewPitch];   // first the values, then the tags: both at once would cost a workgroup per CU
     const float* const ins[1] = {input};
     const FewRows<RM, 1> rows(ins, weight, d);
@@ -214,6 +215,7 @@ __global__ void __launch_bounds__(256, 3)
 bound_forward_few_rows_kernel(const float* __restrict__ lower, const float* __restrict__ upper, const float* __restrict__ weight,
                               float* __restrict__ out_lower, float* __restrict__ out_upper, Dims d) {
     constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
+    if (gated_off(d)) return;
     __shared__ float park[4][NO][kFewPitch];
     const float* const ins[2] = {lower, upper};
     const FewRows<RM, 2> rows(ins, weight, d);
