@@ -94,8 +94,9 @@ LDIST_API int ldist_inf_dist_forward_values(const float* input, const float* wei
 /* L_inf forward passes of large fully connected layers that evaluate only the differences which can be the maximum
  * (lists of every row's outermost values; same results, bit for bit).  No counterpart in the reference.  They need
  * device scratch memory from the caller, free again for other work on the stream when the call returns:
- * ldist_inf_dist_workspace says how much, 0 where a layer has no such form (call the plain entry point); `what` is one
- * of LDIST_WITH_POS, LDIST_VALUES_ONLY (pos == NULL), LDIST_BOUNDS.  workspace: 16-byte aligned, contents of no matter.
+ * ldist_inf_dist_workspace says how much, 0 where a layer has no such form (call the plain entry point), and 256 MiB at
+ * most: batches that would need more are taken in parts; `what` is one of LDIST_WITH_POS, LDIST_VALUES_ONLY
+ * (pos == NULL), LDIST_BOUNDS.  workspace: 16-byte aligned, contents of no matter.
  * LDIST_EUNSUPPORTED where the size is 0, and without pos also where ldist_inf_dist_forward_values has no form for the
  * tensors: nothing is enqueued then. */
 enum { LDIST_WITH_POS = 0, LDIST_VALUES_ONLY = 1, LDIST_BOUNDS = 2 };

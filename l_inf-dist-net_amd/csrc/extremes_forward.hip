@@ -71,7 +71,7 @@ struct Search {
     float* reach;          // [x, w][length][sampled row]: how far from the center a list of that length begins
     float* partial;        // [row of x][pitch] of the first scan's {value, position}, {upper, lower bound}, or values
     int pitch;
-    int* walk;             // [failed]: their indices
+    int* walk;             // [walk_most]: indices of outputs that fail
     int walk_most;
     int K, C, KC;
     int lanes_first, lanes_second;   // rows per workgroup of the two scans
@@ -809,9 +809,8 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
 #pragma unroll
                     for (int j = 0; j < RS; j++) {
                         const unsigned long long m = __ballot(failed >> j & 1);
-                        if (failed >> j & 1)
-                            s.walk[first + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0))] =
-                                (s0 + j) * N + l;
+                        const int at = first + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                        if ((failed >> j & 1) && at < s.walk_most) s.walk[at] = (s0 + j) * N + l;   // more: the full walk follows
                         first += __builtin_popcountll(m);
                     }
                 }
@@ -907,6 +906,9 @@ struct Layout {
     size_t counts, reach, partial, walk, x_lists, w_lists, x_rest, w_rest, total;   // byte offsets in the workspace
 };
 
+// More outputs than these go to the full walk; forced lists have none after them.
+int walk_most(const Problem& pr) { return g_extremes > 0 ? pr.B * pr.NG : pr.B * pr.NG / 16; }
+
 Layout layout_of(const Problem& pr, ForwardKind kind) {
     const bool boxes = kind == ForwardKind::kBounds;
     Layout l{};
@@ -920,7 +922,7 @@ Layout layout_of(const Problem& pr, ForwardKind kind) {
     l.counts = take((size_t)kSampleGroups * kSampleGroups * 64);
     l.pitch = (pr.NG + 7) / 8 * 8;
     l.partial = take((size_t)pr.B * l.pitch * (kind == ForwardKind::kValues ? 1 : 2) * sizeof(float));
-    l.walk = take((size_t)pr.B * pr.NG * sizeof(int));
+    l.walk = take((size_t)walk_most(pr) * sizeof(int));
     l.reach = take(2 * 8 * kSampled * sizeof(float));
     l.x_lists = take((size_t)l.C * l.mb * kMaxList * 16 * (boxes ? 16 : 8));
     l.w_lists = take((size_t)l.C * l.nb * kMaxList * 16 * 8);
@@ -978,16 +980,36 @@ int lanes_for(int rows, int strips, int num_cu) {
 // batches of 32 to 1024, against that of the full walk: e.g. 1024 x 3072 at batch 512 (positions) 92 us in full and
 // 80 with lists, at 272 56 and 78; 5120 x 5120 at 64, 128 and 1024 93, 165, 909 and 120, 138, 282 us.
 // The size alone decides, for the caller asks for the workspace before there is a device to ask.
-size_t extremes_workspace(const Problem& pr, ForwardKind kind) {
+static bool lists_pay(const Problem& pr, ForwardKind kind) {
+    if (g_tile_override >= 0 || pr.K < 512) return false;
+    const double outputs = (double)pr.B * pr.NG, weights = (double)pr.NG * pr.K;
+    const bool boxes = kind == ForwardKind::kBounds;
+    const double us = (boxes ? 65 : 55) + 2.1e-6 * weights + (boxes ? 5.3e-5 : 3.5e-5) * outputs;
+    return 1.1 * us + 5 <= full_walk_us(pr, kind, 256);
+}
+
+// Rows of one sequence of launches: all of them where its scratch memory stays below kScratchMost, else equal shares of whole
+// blocks (each lists the weights again, 17 + 32 us of some 900 at 4096 x 5120 x 5120).  0: the lists of the weights alone leave
+// room for less than kFewestRows, or the layer has none.
+constexpr size_t kScratchMost = (size_t)256 << 20;
+constexpr int kFewestRows = 256;
+static int rows_at_once(const Problem& pr, ForwardKind kind) {
     if (g_extremes == 0 || pr.HW != 1 || pr.G != 1 || pr.NG <= 16 || pr.K < 4 || pr.K > 16 * kMaxChunk) return 0;
-    if (g_extremes < 0) {
-        if (g_tile_override >= 0 || pr.K < 512) return 0;
-        const double outputs = (double)pr.B * pr.NG, weights = (double)pr.NG * pr.K;
-        const bool boxes = kind == ForwardKind::kBounds;
-        const double us = (boxes ? 65 : 55) + 2.1e-6 * weights + (boxes ? 5.3e-5 : 3.5e-5) * outputs;
-        if (1.1 * us + 5 > full_walk_us(pr, kind, 256)) return 0;
+    Problem part = pr;
+    for (int shares = 1;; shares++) {
+        part.B = shares == 1 ? pr.B : ((pr.B + shares - 1) / shares + 15) / 16 * 16;
+        if (shares > 1 && part.B < kFewestRows) return 0;
+        if (layout_of(part, kind).total <= kScratchMost) break;
     }
-    return layout_of(pr, kind).total;
+    return g_extremes > 0 || lists_pay(part, kind) ? part.B : 0;
+}
+
+size_t extremes_workspace(const Problem& pr, ForwardKind kind, int& rows) {
+    rows = rows_at_once(pr, kind);
+    if (rows == 0) return 0;
+    Problem part = pr;
+    part.B = rows;
+    return layout_of(part, kind).total;
 }
 
 hipError_t extremes_forward(const float* x, const float* x2, const float* w, float* out, float* out2, int32_t* pos, void* workspace,
@@ -1002,7 +1024,7 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* w, flo
     s.partial = reinterpret_cast<float*>(ws + l.partial);
     s.pitch = l.pitch;
     s.walk = reinterpret_cast<int*>(ws + l.walk);
-    s.walk_most = g_extremes > 0 ? pr.B * pr.NG : pr.B * pr.NG / 16;
+    s.walk_most = walk_most(pr);
     s.x = Side{x, x2, pr.B, l.mb, ws + l.x_lists, reinterpret_cast<float*>(ws + l.x_rest)};
     s.w = Side{w, nullptr, pr.NG, l.nb, ws + l.w_lists, reinterpret_cast<float*>(ws + l.w_rest)};
     s.out = out; s.out2 = out2; s.pos = pos;

@@ -79,6 +79,46 @@ int conv_geometry(int B, int C, int H, int W, int KH, int KW, int stride, int pa
     return LDIST_OK;
 }
 
+// The workspace forms of the forward passes: the lists, then the full walk where the lists were not worth it, for as many rows
+// at a time as the workspace is for.  full(part, in, at): the full walk of such a part, whose inputs and outputs begin there.
+template <class FULL>
+int extremes_entry(const float* x, const float* x2, const float* w, const ldist::Problem& pr, ldist::ForwardKind kind,
+                          float* out, float* out2, int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream, FULL&& full) {
+    int rows;
+    const size_t need = ldist::extremes_workspace(pr, kind, rows);
+    if (need == 0) return LDIST_EUNSUPPORTED;
+    if (bytes < 0 || (size_t)bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return LDIST_EINVAL;
+    for (long long first = 0; first < pr.B; first += rows) {
+        ldist::Problem part = pr;
+        part.B = first + rows < pr.B ? rows : (int)(pr.B - first);
+        const size_t in = (size_t)first * pr.K, at = (size_t)first * pr.NG;
+        hipError_t e = ldist::extremes_forward(x + in, x2 ? x2 + in : nullptr, w, out + at, out2 ? out2 + at : nullptr,
+                                               pos ? pos + at : nullptr, workspace, part, (hipStream_t)stream, &part.gate);
+        if (e == hipSuccess && ldist::g_extremes <= 0) e = full(part, in, at);
+        if (int rc = finish(e)) return rc;
+    }
+    return LDIST_OK;
+}
+
+// Distances, without pos: values only.
+int distances_entry(const float* x, const float* w, const ldist::Problem& pr, float* out, int32_t* pos, void* workspace,
+                           int64_t bytes, ldist_stream_t stream) {
+    return extremes_entry(x, nullptr, w, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues, out, nullptr, pos,
+                          workspace, bytes, stream, [&](const ldist::Problem& part, size_t in, size_t at) {
+                              return pos ? ldist::inf_forward(x + in, w, out + at, pos + at, part, (hipStream_t)stream)
+                                         : ldist::inf_forward_values(x + in, w, out + at, part, (hipStream_t)stream);
+                          });
+}
+
+int bounds_entry(const float* lower, const float* upper, const float* w, const ldist::Problem& pr, float* out_lower,
+                        float* out_upper, void* workspace, int64_t bytes, ldist_stream_t stream) {
+    return extremes_entry(lower, upper, w, pr, ldist::ForwardKind::kBounds, out_lower, out_upper, nullptr, workspace, bytes, stream,
+                          [&](const ldist::Problem& part, size_t in, size_t at) {
+                              return ldist::bound_forward(lower + in, upper + in, w, out_lower + at, out_upper + at, part,
+                                                          (hipStream_t)stream);
+                          });
+}
+
 }  // namespace
 
 extern "C" {
@@ -121,18 +161,9 @@ int ldist_inf_dist_workspace(int B, int CO, int CI, int G, int HW, int what, int
     *bytes = 0;
     ldist::Problem pr{};
     if (int rc = check_sizes(B, CO, CI, G, HW, pr)) return rc;
-    *bytes = (int64_t)ldist::extremes_workspace(pr, static_cast<ldist::ForwardKind>(what));
+    int rows;
+    *bytes = (int64_t)ldist::extremes_workspace(pr, static_cast<ldist::ForwardKind>(what), rows);
     return LDIST_OK;
-}
-
-// The workspace forms of the forward passes: the lists, then the full walk where the lists were not worth it.
-static int extremes_entry(const float* x, const float* x2, const float* w, ldist::Problem& pr, ldist::ForwardKind kind, float* out,
-                          float* out2, int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream) {
-    const size_t need = ldist::extremes_workspace(pr, kind);
-    if (need == 0) return LDIST_EUNSUPPORTED;
-    if (bytes < 0 || (size_t)bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return LDIST_EINVAL;
-    const hipError_t e = ldist::extremes_forward(x, x2, w, out, out2, pos, workspace, pr, (hipStream_t)stream, &pr.gate);
-    return finish(e);
 }
 
 int ldist_inf_dist_forward_ws(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output,
@@ -142,12 +173,7 @@ int ldist_inf_dist_forward_ws(const float* input, const float* weight, int B, in
     if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
     // without pos the full walk is that of ldist_inf_dist_forward_values
     if (!pos && !ldist::inf_forward_values_applicable(pr, input, weight)) return LDIST_EUNSUPPORTED;
-    if (int rc = extremes_entry(input, nullptr, weight, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues, output,
-                                nullptr, pos, workspace, bytes, stream))
-        return rc;
-    if (ldist::g_extremes > 0) return LDIST_OK;
-    return finish(pos ? ldist::inf_forward(input, weight, output, pos, pr, (hipStream_t)stream)
-                      : ldist::inf_forward_values(input, weight, output, pr, (hipStream_t)stream));
+    return distances_entry(input, weight, pr, output, pos, workspace, bytes, stream);
 }
 
 int ldist_inf_dist_bound_forward_ws(const float* input_lower, const float* input_upper, const float* weight, int B, int CO,
@@ -156,11 +182,7 @@ int ldist_inf_dist_bound_forward_ws(const float* input_lower, const float* input
     if (!input_lower || !input_upper || !weight || !output_lower || !output_upper || !workspace) return LDIST_EINVAL;
     ldist::Problem pr{};
     if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
-    if (int rc = extremes_entry(input_lower, input_upper, weight, pr, ldist::ForwardKind::kBounds, output_lower, output_upper,
-                                nullptr, workspace, bytes, stream))
-        return rc;
-    if (ldist::g_extremes > 0) return LDIST_OK;
-    return finish(ldist::bound_forward(input_lower, input_upper, weight, output_lower, output_upper, pr, (hipStream_t)stream));
+    return bounds_entry(input_lower, input_upper, weight, pr, output_lower, output_upper, workspace, bytes, stream);
 }
 
 // Forward passes whose results leave with the evaluation-mode shift and bias applied, (v - mean) + bias: fully connected layers,
@@ -175,10 +197,8 @@ int ldist_inf_dist_forward_shifted(const float* input, const float* weight, int 
     pr.mean = mean;
     pr.bias = bias;
     if (workspace) {
-        const int rc = extremes_entry(input, nullptr, weight, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues,
-                                      output, nullptr, pos, workspace, bytes, stream);
-        if (rc != LDIST_OK && rc != LDIST_EUNSUPPORTED) return rc;
-        if (rc == LDIST_OK && ldist::g_extremes > 0) return LDIST_OK;
+        const int rc = distances_entry(input, weight, pr, output, pos, workspace, bytes, stream);
+        if (rc != LDIST_EUNSUPPORTED) return rc;
     }
     return finish(pos ? ldist::inf_forward(input, weight, output, pos, pr, (hipStream_t)stream)
                       : ldist::inf_forward_values(input, weight, output, pr, (hipStream_t)stream));
@@ -193,10 +213,8 @@ int ldist_inf_dist_bound_forward_shifted(const float* input_lower, const float* 
     pr.mean = mean;
     pr.bias = bias;
     if (workspace) {
-        const int rc = extremes_entry(input_lower, input_upper, weight, pr, ldist::ForwardKind::kBounds, output_lower, output_upper,
-                                      nullptr, workspace, bytes, stream);
-        if (rc != LDIST_OK && rc != LDIST_EUNSUPPORTED) return rc;
-        if (rc == LDIST_OK && ldist::g_extremes > 0) return LDIST_OK;
+        const int rc = bounds_entry(input_lower, input_upper, weight, pr, output_lower, output_upper, workspace, bytes, stream);
+        if (rc != LDIST_EUNSUPPORTED) return rc;
     }
     return finish(ldist::bound_forward(input_lower, input_upper, weight, output_lower, output_upper, pr, (hipStream_t)stream));
 }
