@@ -142,13 +142,16 @@ def norm_dist_backward_ordered(grad_output, input, weight, output, grad_input, g
 
 
 def _with_workspace(name, what, sizes, dev, args):
-    """Calls the form `name` of a forward pass that takes scratch memory, where the library has one for the layer; False
-    elsewhere: the plain entry point is the way.  `args`: pointers before and after the sizes."""
+    """Calls the form `name` of a forward pass that takes scratch memory, where the library has one for the layer and there is
+    memory for it; False elsewhere: the plain entry point is the way.  `args`: pointers before and after the sizes."""
     need = ctypes.c_int64()
     with torch.cuda.device(dev):
         if _lib.lib().ldist_inf_dist_workspace(*sizes, what, ctypes.byref(need)) != 0 or need.value == 0:
             return False
-        scratch = torch.empty(need.value, dtype=torch.uint8, device=dev)   # free for later work on the stream on return
+        try:
+            scratch = torch.empty(need.value, dtype=torch.uint8, device=dev)   # free for later work on the stream on return
+        except torch.OutOfMemoryError:
+            return False
         rc = getattr(_lib.lib(), name)(*args[0], *sizes, *args[1], _p(scratch), need.value,
                                        torch.cuda.current_stream(dev).cuda_stream)
     if rc == _lib.EUNSUPPORTED:

@@ -1,4 +1,5 @@
-"""Scratch memory of the lists of outermost values (csrc/extremes_forward.hip): bounded, by taking large batches in parts."""
+"""Scratch memory of the lists of outermost values (csrc/extremes_forward.hip): bounded, by taking large batches in parts, and not
+needed where there is none."""
 import ctypes
 
 import pytest
@@ -70,3 +71,41 @@ def test_a_batch_in_parts_against_the_full_walk(extension):
         pkg._lib.lib().ldist_set_extremes(-1)
         cpp.use_torch_extension(True)
     assert differing(got, want) == dict.fromkeys(WHAT, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("extension", [True, False])
+def test_no_memory_for_the_scratch(extension):
+    """An allocator that has room for the results but not for the lists: the full walk, not an error."""
+    from gpu_common import DEV, cpp, say
+    B, CO, K = 1024, 5120, 5120
+    say("extremes without memory", extension)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x, w = torch.randn(B, K, 1, device=DEV, generator=g), torch.randn(CO, K, device=DEV, generator=g) / K ** 0.5
+    up = x + 0.1
+    assert min(workspace(B, CO, K, what) for what in WHAT) > 30 << 20
+    want = run(WHAT, x, up, w)
+    a, b = torch.empty(B, CO, 1, device=DEV), torch.empty(B, CO, 1, device=DEV)
+    pos = torch.empty(B, CO, 1, device=DEV, dtype=torch.int32)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    cpp.use_torch_extension(extension)
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / total)
+    try:
+        held = []                      # what the allocator has free inside its segments
+        with pytest.raises(torch.OutOfMemoryError):
+            while len(held) < 1000:
+                held.append(torch.empty(30 << 20, dtype=torch.uint8, device=DEV))
+        cpp.inf_dist_forward(x, w, a, pos, 1)
+        first = (a.cpu(), pos.cpu())
+        assert cpp.inf_dist_forward_values(x, w, a, 1)
+        second = a.cpu()
+        cpp.inf_dist_bound_forward(x, up, w, a, b, 1)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        cpp.use_torch_extension(True)
+    want = {form: [t.cpu() for t in tensors] for form, tensors in want.items()}
+    assert [torch.equal(i, j) for i, j in zip(first, want["positions"])] == [True, True]
+    assert torch.equal(second, want["values"][0])
+    assert torch.equal(a.cpu(), want["bounds"][0]) and torch.equal(b.cpu(), want["bounds"][1])
