@@ -31,7 +31,8 @@ norm_backward_few_kernel(const float* __restrict__ grad_output, const float* __r
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kb = blockIdx.x % col_blocks, rest = blockIdx.x / col_blocks, chunk = rest % chunks, g = rest / chunks;
     const int K = d.K, NG = d.NG, k = kb * kCols + lane, kc = min(k, K - 1);
-    const int m_begin = chunk * rows_per_wg, m_end = min(d.M, m_begin + rows_per_wg);
+    // rows are counted unsigned: a stage past the last of nearly 2^31 of them still has a number
+    const unsigned rows_all = d.M, m_begin = (unsigned)chunk * rows_per_wg, m_end = min(rows_all, m_begin + rows_per_wg);
     const float ev = in_vgpr(e);
     auto spower = [&](float u) {
         if constexpr (IE == 0) return __builtin_copysignf(pow_pos(__builtin_fabsf(u), ev), u);
@@ -44,11 +45,11 @@ norm_backward_few_kernel(const float* __restrict__ grad_output, const float* __r
         w[j] = weight[((size_t)g * NG + min(j, NG - 1)) * K + kc];
         gw[j] = 0.f;
     }
-    for (int m0 = m_begin; m0 < m_end; m0 += kRows) {
-        const int rows = min(kRows, m_end - m0), mine = wave * (kRows / 4);
+    for (unsigned m0 = m_begin; m0 < m_end; m0 += kRows) {
+        const int rows = min((unsigned)kRows, m_end - m0), mine = wave * (kRows / 4);
         float x[kRows / 4];
 #pragma unroll
-        for (int r = 0; r < kRows / 4; r++) x[r] = input[((size_t)min(m0 + mine + r, d.M - 1) * d.G + g) * K + kc];
+        for (int r = 0; r < kRows / 4; r++) x[r] = input[((size_t)min(m0 + mine + r, rows_all - 1) * d.G + g) * K + kc];
         __syncthreads();   // the stage before is done with
         bool unsafe = false;
         for (int i = tid; i < kRows * NB; i += 256) {
@@ -107,10 +108,10 @@ hipError_t launch_few(const float* grad_output, const float* input, const float*
     const Dims d = make_dims(pr);
     const int col_blocks = (pr.K + kCols - 1) / kCols;
     // rows are shared out until there are four workgroups per CU; every share costs an atomic addition per weight
-    const long want = 4L * pr.num_cu / ((long)col_blocks * pr.G), most = (d.M + kRows - 1) / kRows;
+    const long all = d.M, want = 4L * pr.num_cu / ((long)col_blocks * pr.G), most = (all + kRows - 1) / kRows;
     long chunks = want < 1 ? 1 : want < most ? want : most;
-    const int rows_per_wg = (int)((d.M + chunks * kRows - 1) / (chunks * kRows)) * kRows;
-    chunks = (d.M + rows_per_wg - 1) / rows_per_wg;
+    const int rows_per_wg = (int)((all + chunks * kRows - 1) / (chunks * kRows)) * kRows;   // below 2^31: chunks is 1 for few rows only
+    chunks = (all + rows_per_wg - 1) / rows_per_wg;
     const unsigned grid = (unsigned)(col_blocks * chunks * pr.G);
 #define LAUNCH(IE)                                                                                                            \
     hipLaunchKernelGGL((norm_backward_few_kernel<NB, IE>), dim3(grid), dim3(256), 0, stream, grad_output, input, weight, output,  \

@@ -72,3 +72,25 @@ def test_values_of_one_and_two_rows(case, p):
     exact = df.amax(-1) * (df / df.amax(-1, keepdim=True)).pow(p).sum(-1).pow(1 / p)
     # a term is off by p + 45 units at the most, which the root divides by p; root and scale add a few
     torch.testing.assert_close(out.cpu().double().view(B, N), exact, rtol=((p + 45) / p + 20) * 2.0 ** -23, atol=0.0)
+
+
+@pytest.mark.parametrize("p", [2.0, 37.3])
+def test_both_gradients_of_as_many_rows_as_an_index_counts(p):
+    """One input, one output, 2^31 - 100 rows: counting rows past the last of them in 32 bits with a sign would start over."""
+    from gpu_common import DEV, cpp, say
+    B = 2 ** 31 - 100
+    say("few outputs backward, rows", B, p)
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("48 GiB of device memory")
+    x, out = torch.full((B, 1, 1), 0.5, device=DEV), torch.full((B, 1, 1), 0.5, device=DEV)
+    go, gi = torch.zeros(B, 1, 1, device=DEV), torch.full((B, 1, 1), float("nan"), device=DEV)
+    rows = torch.tensor([0, 63, 64, B // 2, 2 ** 31 - 2 ** 21 - 1, 2 ** 31 - 2 ** 21, B - 2 ** 20, B - 65, B - 2, B - 1], device=DEV)
+    signs = torch.tensor([1.0, -1.0], device=DEV).repeat(5)
+    x[rows, 0, 0] = 0.5 * signs
+    go[rows, 0, 0] = 2.0 ** torch.arange(10, device=DEV)
+    gw = torch.zeros(1, 1, device=DEV)
+    cpp.norm_dist_backward(go, x, torch.zeros(1, 1, device=DEV), out, gi, gw, 1, p)   # |x - w| = out: the powers are one
+    assert gw.item() == -(go[rows, 0, 0] * signs).sum().item()
+    assert torch.equal(gi[rows, 0, 0], go[rows, 0, 0] * signs)
+    gi[rows, 0, 0] = 0.0
+    assert not any(part.any().item() for part in gi.view(-1).split(2 ** 28))      # NaN counts as true
