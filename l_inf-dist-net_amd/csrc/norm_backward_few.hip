@@ -31,8 +31,8 @@ norm_backward_few_kernel(const float* __restrict__ grad_output, const float* __r
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kb = blockIdx.x % col_blocks, rest = blockIdx.x / col_blocks, chunk = rest % chunks, g = rest / chunks;
     const int K = d.K, NG = d.NG, k = kb * kCols + lane, kc = min(k, K - 1);
-    // rows are counted unsigned: a stage past the last of nearly 2^31 of them still has a number
-    const unsigned rows_all = d.M, m_begin = (unsigned)chunk * rows_per_wg, m_end = min(rows_all, m_begin + rows_per_wg);
+    const int m_begin = chunk * rows_per_wg;
+    int left = min(d.M - m_begin, rows_per_wg);   // rows to come: what is past them may have no number below 2^31
     const float ev = in_vgpr(e);
     auto spower = [&](float u) {
         if constexpr (IE == 0) return __builtin_copysignf(pow_pos(__builtin_fabsf(u), ev), u);
@@ -45,11 +45,11 @@ norm_backward_few_kernel(const float* __restrict__ grad_output, const float* __r
         w[j] = weight[((size_t)g * NG + min(j, NG - 1)) * K + kc];
         gw[j] = 0.f;
     }
-    for (unsigned m0 = m_begin; m0 < m_end; m0 += kRows) {
-        const int rows = min((unsigned)kRows, m_end - m0), mine = wave * (kRows / 4);
+    for (int m0 = m_begin;; m0 += kRows) {
+        const int rows = min(kRows, left), mine = wave * (kRows / 4);
         float x[kRows / 4];
 #pragma unroll
-        for (int r = 0; r < kRows / 4; r++) x[r] = input[((size_t)min(m0 + mine + r, rows_all - 1) * d.G + g) * K + kc];
+        for (int r = 0; r < kRows / 4; r++) x[r] = input[((size_t)(m0 + min(mine + r, rows - 1)) * d.G + g) * K + kc];
         __syncthreads();   // the stage before is done with
         bool unsafe = false;
         for (int i = tid; i < kRows * NB; i += 256) {
@@ -89,6 +89,7 @@ norm_backward_few_kernel(const float* __restrict__ grad_output, const float* __r
         };
         if (factored) walk([&](float df, int r, int j) { return cs[r][j] * spower(df); });
         else walk([&](float df, int r, int j) { return cs[r][j] * spower(df * rs[r][j]); });
+        if ((left -= kRows) <= 0) break;
     }
 #pragma unroll
     for (int j = 0; j < NB; j++) sums[wave][j][lane] = gw[j];
