@@ -533,7 +533,7 @@ inf_forward_skinny_kernel(const float* __restrict__ input, const float* __restri
 
 hipError_t inf_forward(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr,
                        hipStream_t stream) {
-    if (pr.NG <= kSkinnyMaxNG && few_rows_of_few_outputs(pr)) return inf_forward_few_rows(input, weight, output, pos, pr, stream);
+    if (pr.NG <= kSkinnyMaxNG && few_rows_of_few_outputs(pr, false, false)) return inf_forward_few_rows(input, weight, output, pos, pr, stream);
     if (pr.NG <= kSkinnyMaxNG) {
         const Dims d = make_dims(pr);
         const bool vec = pr.HW == 1 && pr.K % 4 == 0 && aligned16(input) && aligned16(weight);

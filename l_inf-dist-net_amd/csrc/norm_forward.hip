@@ -133,7 +133,7 @@ bool norm_forward_shifts(const Problem& pr, float p) {
 // gradients of a five-layer net.
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
                         bool values_only, hipStream_t stream) {
-    if (pr.NG <= kSkinnyMaxNG && values_only && few_rows_of_few_outputs(pr))
+    if (pr.NG <= kSkinnyMaxNG && values_only && few_rows_of_few_outputs(pr, true, small_int_power(p) < 2 || small_int_power(p) == 7))
         return norm_forward_few_rows(input, weight, output, p, pr, stream);
     if (pr.NG <= kSkinnyMaxNG) {
         const Dims d = make_dims(pr);

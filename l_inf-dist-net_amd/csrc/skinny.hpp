@@ -92,7 +92,15 @@ __device__ __forceinline__ void skinny_sweep(const float* const (&input)[NX], co
 // One or two rows: a workgroup for each leaves the weights to one or two CUs, which have too few loads in flight to bring them
 // from memory at any rate; the few-rows kernel (a wave per output) spreads them.  1 x 5120 -> 10: 18 -> 6 us; 1024 lanes per row
 // instead of 256: 16, and 272 and 1024 rows 18 -> 28 and 29 -> 50.
-inline bool few_rows_of_few_outputs(const Problem& pr) { return pr.HW == 1 && pr.B <= 2 && pr.K >= 1024 && g_tile_override < 0; }
+// Few of the few outputs are few waves there, each with all of a long row, where the workgroup of a row has four: up to four
+// outputs (us, that workgroup / few-rows) p = 37.3, 2 x 1024 3.3 / 5.3, 2 x 12000 9.5 / 29, 1 x 12000 9.4 / 13; p = 8, 2 x 5120
+// 5.7 / 7.9, but 1 x 5000 5.6 / 4.9; L_inf, 2 x 5120 5.7 / 6.8, but 2 x 2000 4.6 / 4.5 and 1 x 5000 5.4 / 4.4; 5 to 8 outputs,
+// L_inf 2 x 12000 11.4 / 12.0, 2 x 40000 25 / 32, all others the other way.  `terms_cost`: powers by logarithm and exponential.
+inline bool few_rows_of_few_outputs(const Problem& pr, bool norm, bool terms_cost) {
+    if (pr.HW != 1 || pr.B > 2 || pr.K < 1024 || g_tile_override >= 0) return false;
+    if (pr.B == 1 && !terms_cost) return true;
+    return norm ? pr.NG > 4 : pr.NG > 8 || pr.K < (pr.NG > 4 ? 8192 : 2048);
+}
 
 inline unsigned skinny_grid(const Dims& d, int rw) { return (unsigned)((d.M + rw - 1) / rw) * d.G; }
 
