@@ -1,8 +1,8 @@
 // Forward kernels for fully connected layers with a handful of rows (serving one or a few inputs): bound by reading the
 // weights once, so they go from memory into registers, never through LDS.
 //
-// A wave owns RM rows x four outputs (one or two rows: as many outputs) and its 64 lanes split k, four consecutive k each per trip (a trip is 256 k): a lane
-// loads the weight vectors and RM input vectors with 128-bit loads, the next trip's before the arithmetic of this one.
+// A wave owns RM rows x four outputs (one or two rows: also one or two) and its 64 lanes split k, four consecutive k each per trip
+// (a trip is 256 k): a lane loads the weight vectors and RM input vectors with 128-bit loads, the next trip's before the arithmetic of this one.
 // The four waves of a workgroup take neighbouring outputs and read the same rows, which they find in the vector
 // cache.  At the end the lanes' results meet through LDS: every wave writes its 4 * RM results of 64 lanes and two lanes
 // take one output.  k past the end: the last vector of a row is moved back to end with the row, vectors beyond it
@@ -10,6 +10,8 @@
 //
 // Against tiles of rows x outputs (32 x 32 is the smallest of fwd_engine.hpp) nothing is computed for absent rows:
 // 1 x 5120 -> 5120, values: 60 -> 27 us, of which 21 us are the 105 MB of weights at the rate of a large copy.
+#include <cmath>
+
 #include "quad_engine.hpp"
 #include "fwd_engine.hpp"
 #include "pow.hpp"
@@ -17,15 +19,30 @@
 
 namespace ldist {
 
-// Outputs per wave.  A row by itself: one, so that 5120 outputs are five workgroups on every CU with five trips' loads in flight
-// per wave: 1 x 5120 -> 5120, values, 21.6 -> 19.3 us (four outputs: 1.25 workgroups per CU); more rows find work enough in four.
+// Outputs per wave of one and two rows: as many as rows, or four.  Few of them make more waves, with five or three trips' loads
+// in flight each: 1 x 5120 -> 5120, values, 17.4 -> 16.7 us; with four its 320 workgroups are 1.25 to a CU.  Four read the rows
+// less often, and are better where they fill the CUs and where the rows are short.  Us, as many as rows / four:
+//   1 x 5120 -> 1024 4.1 / 6.2, 1 x 3072 -> 4096 9.6 / 9.2, 1 x 800 -> 4096 3.5 / 3.2, -> 5120 3.9 / 3.7; with positions 5.0 / 6.1,
+//   10.5 / 10.1, 4.5 / 3.8, 4.8 / 4.3; p = 37.3 7.9 / 12.0, 16.4 / 16.1, 5.8 / 5.0, 6.2 / 6.5
+//   2 x 5120 -> 1024 6.3 / 7.3, 2 x 5120 -> 4096 16.2 / 14.1, 2 x 800 -> 5120 4.6 / 4.0; p = 37.3 15.6 / 18.1, 30.6 / 26.6, 9.0 / 8.8;
+//   with positions 7.4 / 10.6, 14.9 / 18.8, 5.7 / 5.0
+//   bounds, which read two inputs: 1 x 5120 -> 1024 7.0 / 7.9, -> 3000 12.3 / 11.6, 1 x 3072 -> 5120 12.5 / 12.0;
+//   2 x 5120 -> 1024 11.8 / 11.1, 2 x 1000 -> 20000 18.5 / 14.8
 constexpr int few_cols(int rows) { return rows <= 2 ? rows : 4; }
+enum class FewKind { kValues, kPos, kNorm, kBounds };
+static int cols_of(const Problem& pr, FewKind kind) {
+    if (pr.B > 2) return 4;
+    const double per_cu = (double)pr.NG * pr.G / (16.0 * pr.num_cu);   // workgroups, with four
+    const bool enough = per_cu >= 0.7, full = per_cu >= 0.7 * std::ceil(per_cu), brief = pr.K < 2048;
+    if (kind == FewKind::kBounds) return pr.B == 2 || enough ? 4 : 1;
+    if (kind == FewKind::kPos && pr.B == 2) return per_cu > 1 && brief ? 4 : 2;
+    return enough && (full || brief) ? 4 : pr.B;
+}
 
 typedef float FewF4 __attribute__((ext_vector_type(4)));
 
-template <int RM, int NX>
+template <int RM, int NX, int COLS = few_cols(RM)>
 struct FewRows {
-    static constexpr int COLS = few_cols(RM);
     const float* xr[NX][RM];
     const float* wr[COLS];
     int K, lane, m0, n0, g;
@@ -74,7 +91,7 @@ struct FewRows {
             }
             return;
         }
-        if constexpr (RM <= 2) {
+        if constexpr (COLS <= 2) {
             constexpr int AHEAD = RM == 1 ? 5 : 3;
 #pragma unroll 1
             for (int t = 0; t < n; t += AHEAD) {
@@ -105,15 +122,17 @@ struct FewRows {
 constexpr int kFewPitch = 68;
 
 // L_inf.  A lane keeps the trip in which its maximum was raised; (trip, lane) is the order of k.
-template <int RM, bool POS>
+template <int RM, bool POS, int COLS = few_cols(RM)>
 __global__ void __launch_bounds__(256, 3)
 inf_forward_few_rows_kernel(const float* __restrict__ input, const float* __restrict__ weight, float* __restrict__ output,
                             int32_t* __restrict__ pos, Dims d) {
-    constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
-    if (gated_off(d)) return;
+    constexpr int kFewCols = COLS, NO = RM * kFewCols;
+    if constexpr (RM == 8) {   // lists, which may leave this launch nothing to do, are for larger batches than the other forms; 0.2 us
+        if (gated_off(d)) return;
+    }
     __shared__ float park[4][NO][kFewPitch];   // first the values, then the tags: both at once would cost a workgroup per CU
     const float* const ins[1] = {input};
-    const FewRows<RM, 1> rows(ins, weight, d);
+    const FewRows<RM, 1, COLS> rows(ins, weight, d);
     const int wave = threadIdx.x >> 6, lane = rows.lane;
     float acc[RM][kFewCols];
     int trip[RM][kFewCols];
@@ -121,7 +140,7 @@ inf_forward_few_rows_kernel(const float* __restrict__ input, const float* __rest
     for (int i = 0; i < RM; i++)
 #pragma unroll
         for (int j = 0; j < kFewCols; j++) { acc[i][j] = 0.f; trip[i][j] = 0; }
-    rows.walk([&](const typename FewRows<RM, 1>::Vecs& v, int t) {
+    rows.walk([&](const typename FewRows<RM, 1, COLS>::Vecs& v, int t) {
 #pragma unroll
         for (int i = 0; i < RM; i++)
 #pragma unroll
@@ -178,8 +197,8 @@ inf_forward_few_rows_kernel(const float* __restrict__ input, const float* __rest
             int found = 0;
             if (best > 0.f) {
                 const int kc = min((tag >> 6) * 256 + (tag & 63) * 4, d.K - 4);
-                const FewF4 df = FewRows<RM, 1>::vec(input + ((size_t)m * d.G + rows.g) * d.K + kc) -
-                                 FewRows<RM, 1>::vec(weight + ((size_t)rows.g * d.NG + n) * d.K + kc);
+                const FewF4 df = FewRows<RM, 1, COLS>::vec(input + ((size_t)m * d.G + rows.g) * d.K + kc) -
+                                 FewRows<RM, 1, COLS>::vec(weight + ((size_t)rows.g * d.NG + n) * d.K + kc);
 #pragma unroll
                 for (int e = 3; e >= 0; e--)
                     if (__builtin_fabsf(df[e]) == best) found = (kc + e) | (__float_as_int(df[e]) & 0x80000000);
@@ -210,20 +229,22 @@ __device__ __forceinline__ float few_reduce(float (*park)[kFewPitch], const floa
 }
 
 // Interval bounds: a trip whose vectors hold l > u, a NaN or an infinity takes the reference's literal predicate.
-template <int RM>
+template <int RM, int COLS>
 __global__ void __launch_bounds__(256, 3)
 bound_forward_few_rows_kernel(const float* __restrict__ lower, const float* __restrict__ upper, const float* __restrict__ weight,
                               float* __restrict__ out_lower, float* __restrict__ out_upper, Dims d) {
-    constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
-    if (gated_off(d)) return;
+    constexpr int kFewCols = COLS, NO = RM * kFewCols;
+    if constexpr (RM == 4) {   // lists, which may leave this launch nothing to do, are for larger batches than the other forms; 0.2 us
+        if (gated_off(d)) return;
+    }
     __shared__ float park[4][NO][kFewPitch];
     const float* const ins[2] = {lower, upper};
-    const FewRows<RM, 2> rows(ins, weight, d);
+    const FewRows<RM, 2, COLS> rows(ins, weight, d);
     const int wave = threadIdx.x >> 6, lane = rows.lane;
     float lo[NO], up[NO];
 #pragma unroll
     for (int o = 0; o < NO; o++) { lo[o] = 0.f; up[o] = 0.f; }
-    rows.walk([&](const typename FewRows<RM, 2>::Vecs& v, int t) {
+    rows.walk([&](const typename FewRows<RM, 2, COLS>::Vecs& v, int t) {
         // 0 * v is NaN for a NaN or an infinity, and stays in the sum; u - l < 0 betrays l > u
         float zero = 0.f, width = 0.f;
 #pragma unroll
@@ -282,15 +303,15 @@ bound_forward_few_rows_kernel(const float* __restrict__ lower, const float* __re
 
 // p-norm, as norm_forward_quad_kernel: IP = 2, 3, 4, 8 one walk with the powers as they are, again the general way if a
 // sum left [2^-90, 2^100]; IP = 0 a walk for the maxima and one for the sums (the second finds the weights in the caches).
-template <int RM, int IP>
+template <int RM, int IP, int COLS = few_cols(RM)>
 __global__ void __launch_bounds__(256, 3)
 norm_forward_few_rows_kernel(const float* __restrict__ input, const float* __restrict__ weight, float* __restrict__ output,
                              float p, Dims d) {
-    constexpr int kFewCols = few_cols(RM), NO = RM * kFewCols;
+    constexpr int kFewCols = COLS, NO = RM * kFewCols;
     __shared__ float park[4][NO][kFewPitch];
     const float* const ins[1] = {input};
-    const FewRows<RM, 1> rows(ins, weight, d);
-    using Vecs = typename FewRows<RM, 1>::Vecs;
+    const FewRows<RM, 1, COLS> rows(ins, weight, d);
+    using Vecs = typename FewRows<RM, 1, COLS>::Vecs;
     const int wave = threadIdx.x >> 6, lane = rows.lane;
     const float pv = in_vgpr(p);
     auto add = [](float a, float b) { return a + b; };
@@ -370,48 +391,62 @@ norm_forward_few_rows_kernel(const float* __restrict__ input, const float* __res
         output[((size_t)m * d.G + rows.g) * d.NG + n] = shifted_value(d.mean, d.bias, rows.g * d.NG + n, result);
 }
 
-static Dims few_dims(const Problem& pr, int rm) {
+static Dims few_dims(const Problem& pr, int rm, int cols) {
     Dims d = make_dims(pr);
     d.tiles_m = (d.M + rm - 1) / rm;
-    d.tiles_n = (d.NG + 4 * few_cols(rm) - 1) / (4 * few_cols(rm));
+    d.tiles_n = (d.NG + 4 * cols - 1) / (4 * cols);
     return d;
 }
 
-#define FEW_LAUNCH(KERNEL, RM, ...)                                                                                      \
+#define FEW_LAUNCH(KERNEL, RM, COLS, ...)                                                                               \
     do {                                                                                                                \
-        const Dims d = few_dims(pr, RM);                                                                                \
+        const Dims d = few_dims(pr, RM, COLS);                                                                          \
         hipLaunchKernelGGL(KERNEL, dim3((unsigned)d.tiles_m * d.tiles_n * d.G), dim3(256), 0, stream, __VA_ARGS__, d); \
         return hipGetLastError();                                                                                       \
     } while (0)
 
+// ROWS rows with the outputs per wave of cols_of(); LAUNCH(cols) for either.
+#define FEW_EITHER(ROWS, KIND, LAUNCH)                                       \
+    if (pr.B == ROWS) {                                                      \
+        if (cols_of(pr, KIND) == 4) LAUNCH(ROWS, 4); else LAUNCH(ROWS, few_cols(ROWS)); \
+    }
+
 hipError_t inf_forward_few_rows(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr,
                                 hipStream_t stream) {
+#define WITH_POS(RM, COLS) FEW_LAUNCH((inf_forward_few_rows_kernel<RM, true, COLS>), RM, COLS, input, weight, output, pos)
+#define VALUES(RM, COLS) FEW_LAUNCH((inf_forward_few_rows_kernel<RM, false, COLS>), RM, COLS, input, weight, output, pos)
     if (pos) {
-        if (pr.B == 1) FEW_LAUNCH((inf_forward_few_rows_kernel<1, true>), 1, input, weight, output, pos);
-        if (pr.B == 2) FEW_LAUNCH((inf_forward_few_rows_kernel<2, true>), 2, input, weight, output, pos);
-        if (pr.B <= 4) FEW_LAUNCH((inf_forward_few_rows_kernel<4, true>), 4, input, weight, output, pos);
-        FEW_LAUNCH((inf_forward_few_rows_kernel<8, true>), 8, input, weight, output, pos);
+        FEW_EITHER(1, FewKind::kPos, WITH_POS)
+        FEW_EITHER(2, FewKind::kPos, WITH_POS)
+        if (pr.B <= 4) WITH_POS(4, 4);
+        WITH_POS(8, 4);
     }
-    if (pr.B == 1) FEW_LAUNCH((inf_forward_few_rows_kernel<1, false>), 1, input, weight, output, pos);
-    if (pr.B == 2) FEW_LAUNCH((inf_forward_few_rows_kernel<2, false>), 2, input, weight, output, pos);
-    if (pr.B <= 4) FEW_LAUNCH((inf_forward_few_rows_kernel<4, false>), 4, input, weight, output, pos);
-    FEW_LAUNCH((inf_forward_few_rows_kernel<8, false>), 8, input, weight, output, pos);
+    FEW_EITHER(1, FewKind::kValues, VALUES)
+    FEW_EITHER(2, FewKind::kValues, VALUES)
+    if (pr.B <= 4) VALUES(4, 4);
+    VALUES(8, 4);
+#undef WITH_POS
+#undef VALUES
 }
 
 hipError_t bound_forward_few_rows(const float* lower, const float* upper, const float* weight, float* out_lower, float* out_upper,
                                   const Problem& pr, hipStream_t stream) {
-    if (pr.B == 1) FEW_LAUNCH((bound_forward_few_rows_kernel<1>), 1, lower, upper, weight, out_lower, out_upper);
-    if (pr.B == 2) FEW_LAUNCH((bound_forward_few_rows_kernel<2>), 2, lower, upper, weight, out_lower, out_upper);
-    FEW_LAUNCH((bound_forward_few_rows_kernel<4>), 4, lower, upper, weight, out_lower, out_upper);
+#define BOUNDS(RM, COLS) FEW_LAUNCH((bound_forward_few_rows_kernel<RM, COLS>), RM, COLS, lower, upper, weight, out_lower, out_upper)
+    FEW_EITHER(1, FewKind::kBounds, BOUNDS)
+    if (pr.B == 2) BOUNDS(2, 4);
+    BOUNDS(4, 4);
+#undef BOUNDS
 }
 
 template <int IP>
 static hipError_t norm_few_rows(const float* input, const float* weight, float* output, float p, const Problem& pr,
                                 hipStream_t stream) {
-    if (pr.B == 1) FEW_LAUNCH((norm_forward_few_rows_kernel<1, IP>), 1, input, weight, output, p);
-    if (pr.B == 2) FEW_LAUNCH((norm_forward_few_rows_kernel<2, IP>), 2, input, weight, output, p);
-    if (pr.B <= 4) FEW_LAUNCH((norm_forward_few_rows_kernel<4, IP>), 4, input, weight, output, p);
-    FEW_LAUNCH((norm_forward_few_rows_kernel<8, IP>), 8, input, weight, output, p);
+#define NORM(RM, COLS) FEW_LAUNCH((norm_forward_few_rows_kernel<RM, IP, COLS>), RM, COLS, input, weight, output, p)
+    FEW_EITHER(1, FewKind::kNorm, NORM)
+    FEW_EITHER(2, FewKind::kNorm, NORM)
+    if (pr.B <= 4) NORM(4, 4);
+    NORM(8, 4);
+#undef NORM
 }
 
 hipError_t norm_forward_few_rows(const float* input, const float* weight, float* output, float p, const Problem& pr,
