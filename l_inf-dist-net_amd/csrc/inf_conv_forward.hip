@@ -85,7 +85,10 @@ inf_conv_forward_kernel(const float* __restrict__ img, const float* __restrict__
     // directly; with 256 lanes this loop is empty.
     auto wrest = [&](int ch, float* stage) {
         const int kb = ch * kKC;
-        constexpr int REST = POS ? 1 : kRest;   // with pos there are no registers for more
+        // More where there are registers for it: with six the kernel for resident rows, ungrouped, stride 1, takes 178 instead of 167,
+        // two waves per SIMD instead of three (128 images of 128 x 32 x 32 in four groups 185 us, 512 of 64 x 14 x 14 206; 170 and
+        // 194 with one).
+        constexpr int REST = POS || (S == 1 && RESIDENT && !GROUPED) ? 1 : kRest;
         for (int first = tid + kWRegs * NT; first < kKC * a.BN; first += REST * NT) {
             float v[REST];
 #pragma unroll

@@ -12,15 +12,20 @@ from test_shortk_parked_loads import CSRC, library_flags
 pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not on PATH")
 
 
-def scratch_of(source, tmp_path):
-    """Mangled kernel name -> bytes of scratch per lane."""
+def reported(source, tmp_path, what):
+    """Mangled kernel name -> a number that the compiler reports."""
     cmd = ["hipcc"] + library_flags() + ["-Rpass-analysis=kernel-resource-usage", "-c", "--cuda-device-only",
                                          os.path.join(CSRC, source), "-o", str(tmp_path / "out.o")]
     text = subprocess.run(cmd, check=True, capture_output=True, text=True).stderr
     names = re.findall(r"Function Name: (\S+)", text)
-    sizes = re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", text)
+    sizes = re.findall(re.escape(what) + r": (\d+)", text)
     assert names and len(names) == len(sizes)
     return dict(zip(names, map(int, sizes)))
+
+
+def scratch_of(source, tmp_path):
+    """Mangled kernel name -> bytes of scratch per lane."""
+    return reported(source, tmp_path, "ScratchSize [bytes/lane]")
 
 
 def test_one_pass_conv_backward_at_four_waves(tmp_path):
@@ -31,3 +36,10 @@ def test_one_pass_conv_backward_at_four_waves(tmp_path):
     image = [size for name, size in four.items() if "kernelILb1E" in name]
     assert len(columns) == 5 and max(columns) == 0
     assert len(image) == 10 and max(image) <= 72
+
+
+def test_image_forward_without_pos_at_three_waves(tmp_path):
+    """inf_conv_forward_kernel<1, RESIDENT, no POS, not GROUPED>: three waves per SIMD share its 512 registers."""
+    waves = [n for name, n in reported("inf_conv_forward.hip", tmp_path, "Occupancy [waves/SIMD]").items()
+             if "inf_conv_forward_kernelILi1ELb1ELb0ELb0E" in name]
+    assert waves == [3]
