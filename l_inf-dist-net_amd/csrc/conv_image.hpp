@@ -14,7 +14,7 @@ constexpr int kKC = kCC * 9;      // k values per weight stage
 constexpr int kMaxThreads = 256;
 constexpr int kBNP = 68;          // row length of the weight stage: 64 outputs + 4, a constant so that reads take immediate offsets
 constexpr int kWRegs = 9;         // weight words a lane carries from global to LDS per stage (64 outputs x 36 / 256)
-constexpr int kRest = 6;          // weight words a lane has in flight beyond those, where a workgroup has fewer lanes
+constexpr int kRest = 6;          // weight words a lane has in flight beyond those, where a workgroup has fewer lanes (values only)
 // image words a lane carries per stage when the channels are staged (4 channels x rows held x padded width / lanes)
 __host__ __device__ constexpr int x_regs(int S) { return S == 1 ? 7 : 10; }
 
@@ -147,7 +147,7 @@ inline size_t lds_bytes(const ConvFwd& a, int nx) {
 // Clocks of a launch: what the busiest CU's workgroups take, one set of as many as fit after the other.  `one` and `two`: a stage's
 // clocks with one wave per SIMD and with two; `fixed`, `search`: what a workgroup's start and end take, and what the groups
 // divide at the end (the search for the position).
-struct StageClocks { double one, two, fixed, search; int rest; };   // rest: weight words in flight beyond the parked ones
+struct StageClocks { double one, two, fixed, search; int rest; double worth; };   // rest: weight words in flight beyond the parked ones
 inline double launch_clocks(const ConvFwd& a, int nx, int num_cu, const StageClocks& c) {
     const int waves = (a.KG * a.GT + 63) / 64, stages = (a.CGP / kCC + a.KG - 1) / a.KG;
     long at_once = (long)(kLdsLimit / (lds_bytes(a, nx) + (nx > 1 ? 256 : 0)));
@@ -166,13 +166,16 @@ inline double launch_clocks(const ConvFwd& a, int nx, int num_cu, const StageClo
 // outputs are 154 workgroups of four waves then, three tenths of what the device can issue.  Here the tile may be smaller
 // and its channels are shared by up to eight groups of lanes (eight waves in all, two per SIMD), which have stages of their
 // own and meet in LDS at the end.  That layer with 64 channels: bounds 190 -> 117 us, values 85 -> 46; the same images at
-// 28 x 28, 32 channels, 32 outputs: 141 -> 119 and 47 -> 47.  The clocks were fitted to these.  A shape is changed where that gains 7 %,
-// and only below four rounds of workgroups: beyond, the last round's share is small.
+// 28 x 28, 32 channels, 32 outputs: 141 -> 119 and 47 -> 47.  The clocks were fitted to these.  A shape is changed where that gains
+// `worth`, and only below four rounds of workgroups: beyond, the last round's share is small.  Over 134 layers of 1 to 512 images
+// of 7 to 32 pixels, 3 to 128 channels and 8 to 252 outputs the estimate is within a third of the time for values and bounds (7 %
+// asked for); with positions it promises more than there is, 0.68 of the time where 0.89 to 1.09 were measured, 0.88 where 1.28,
+// hence a third.  A smaller tile that is not shared lost as often as it gained (16.2 -> 20.2, 14.8 -> 15.5 us) and is not taken.
 inline void share_channels(const ConvGeom& q, ConvFwd& a, int nx, int num_cu, const StageClocks& clocks_of) {
     if (g_conv_rows_override > 0 && g_conv_groups_override <= 0) return;
     const int forced = g_conv_groups_override;
     const double before = launch_clocks(a, nx, num_cu, clocks_of);
-    double best = forced > 0 ? 1e300 : 0.93 * before;
+    double best = forced > 0 ? 1e300 : clocks_of.worth * before;
     if (forced <= 0 && (double)a.B * a.G * a.tiles_h * a.tiles_n > 4.0 * 2 * num_cu) return;   // at least four rounds
     const int S = q.S, quads = (a.NG + kTN - 1) / kTN, first_tiles = (quads + 15) / 16, nstage = a.CGP / kCC;
     ConvFwd pick = a;
@@ -198,6 +201,7 @@ inline void share_channels(const ConvGeom& q, ConvFwd& a, int nx, int num_cu, co
                 const int per = (nstage + c.KG - 1) / c.KG;
                 if (per == last_per || (forced > 0 && c.KG != forced)) continue;   // a group more than the stages are worth
                 last_per = per;
+                if (c.KG == 1 && forced <= 0) continue;
                 if (lds_bytes(c, nx) > kLdsLimit - (nx > 1 ? 1024 : 0)) break;
                 const double clocks = launch_clocks(c, nx, num_cu, clocks_of);
                 if (clocks < best) { best = clocks; pick = c; }

@@ -49,3 +49,22 @@ def test_few_outputs(case):
         set_tile(-1)
     say("few rows, few outputs", case, f"chosen {chosen:.1f} us, a workgroup per row {row:.1f} us")
     assert chosen < 7 / 6 * row
+
+
+@pytest.mark.parametrize("case", [(31, 110, 28, 176, 2), (44, 7, 16, 159, 1), (31, 20, 32, 52, 4), (33, 48, 15, 62, 2)])
+def test_channels_shared_by_groups_of_lanes(case):
+    """Images with positions: the shape that is chosen is not slower than a tile to a group of lanes."""
+    from gpu_common import DEV, cpp, pkg, say
+    B, C, H, CO, G = case
+    g = torch.Generator(device=DEV).manual_seed(B + C)
+    x, w = torch.rand(B, C, H, H, device=DEV, generator=g), torch.randn(CO, C // G * 9, device=DEV, generator=g)
+    out, pos = torch.empty(B, CO, H * H, device=DEV), torch.empty(B, CO, H * H, device=DEV, dtype=torch.int32)
+    call = lambda: cpp.inf_dist_conv_forward(x, w, out, pos, G, 3, 1, 1)
+    chosen = us(call)
+    pkg._lib.lib().ldist_set_conv_groups_override(1)
+    try:
+        alone = us(call)
+    finally:
+        pkg._lib.lib().ldist_set_conv_groups_override(0)
+    say("groups of lanes", case, f"chosen {chosen:.1f} us, a tile to a group {alone:.1f} us")
+    assert chosen < 1.1 * alone
