@@ -21,6 +21,8 @@
 //
 // 5120 x 5120 with positions, batch 272 / 512: 300 / 470 -> 165 / 205 us; values at 1024 780 -> 155; bounds at 1024 2170 -> 225.
 // Data that the lists cannot help cost 12 to 60 us beside the full walk of 480 to 2170.
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "quad_engine.hpp"
 #include "wave_reduce.hpp"
@@ -979,12 +981,18 @@ int lanes_for(int rows, int strips, int num_cu) {
 // (lists of about 50 and 100 entries per chunk), fitted to eight sizes of weights from 1024 x 784 to 5120 x 5120 at
 // batches of 32 to 1024, against that of the full walk: e.g. 1024 x 3072 at batch 512 (positions) 92 us in full and
 // 80 with lists, at 272 56 and 78; 5120 x 5120 at 64, 128 and 1024 93, 165, 909 and 120, 138, 282 us.
+// Few outputs of a long reduction leave the sample and the scans to few workgroups, which walk all its chunks in turn: the terms
+// beyond one and two chunks, fitted to 552 layers of 600 to 40000 inputs, normal and uniform inputs, of which 66 were slower
+// with lists before (256 x 25088 -> 256 with positions 94 us in full, 174 with lists; 1024 x 25088 -> 64 values 88 and 192), and
+// 3 of the 443 that are left are, by 2 to 11 %.
 // The size alone decides, for the caller asks for the workspace before there is a device to ask.
 static bool lists_pay(const Problem& pr, ForwardKind kind) {
     if (g_tile_override >= 0 || pr.K < 512) return false;
     const double outputs = (double)pr.B * pr.NG, weights = (double)pr.NG * pr.K;
     const bool boxes = kind == ForwardKind::kBounds;
-    const double us = (boxes ? 65 : 55) + 2.1e-6 * weights + (boxes ? 5.3e-5 : 3.5e-5) * outputs;
+    const double beyond_one = std::max(0, pr.K - kMaxChunk), beyond_two = std::max(0, pr.K - 2 * kMaxChunk);
+    const double us = (boxes ? 65 : 55) + 2.1e-6 * weights + (boxes ? 5.3e-5 : 3.5e-5) * outputs +
+                      (boxes ? 3.4e-6 : 1.1e-6) * pr.B * beyond_one + (3.3e-3 + (boxes ? 5.4e-9 : 4.2e-9) * outputs) * beyond_two;
     return 1.1 * us + 5 <= full_walk_us(pr, kind, 256);
 }
 
