@@ -94,6 +94,19 @@ class KernelTimer:
         return n, ms / max(n, 1), flops / max(n, 1)
 
 
+def lists_cover(pkg, batch, what):
+    """Whether every wide layer of the MLP goes through lists of outermost values (csrc/extremes_forward.hip), which leave most
+    differences unevaluated.  what: 0 distances with positions, 1 values, 2 bounds."""
+    import ctypes
+    need = ctypes.c_int64()
+    return all(pkg._lib.lib().ldist_inf_dist_workspace(batch, o, i, 1, 1, what, ctypes.byref(need)) == 0 and need.value > 0
+               for i, o in zip(LAYERS[:-2], LAYERS[1:-1]))
+
+
+LISTS = ("lists of outermost values: sample, lists, two scans and the walk of what they leave (extremes_*_kernel), with the full "
+         "walk's launch, which finds nothing to do")
+
+
 def mnk(x, w):
     return x.size(0) * x.size(2) * w.size(0) * w.size(1)
 
@@ -209,9 +222,10 @@ def workload_c1(pkg, torch, dev):
     return dict(step=step, ops=stack_ops(512), images=512, full_rows=512, cpu=cpu, formula=formula, check=check,
                 name="configs[1]: 5-layer L_inf-dist MLP 3072-5120-5120-5120-5120-10, p=inf, batch 512, "
                      "forward+backward (all grad_x and grad_w), mean shift in training mode",
+                nominal=lists_cover(pkg, 512, 0),
                 kernel=("inf_dist_forward", lambda x_, w_, *_: 2 * mnk(x_, w_),
                         lambda x_, w_, o_, p_, G: w_.size(0) // G > 16,   # the 10-way head runs another kernel
-                        "inf_forward_kernel (tiled L_inf forward)", 2))
+                        LISTS if lists_cover(pkg, 512, 0) else "inf_forward_kernel (tiled L_inf forward)", 2))
 
 
 def workload_c1t(pkg, torch, dev):
@@ -310,9 +324,10 @@ def workload_c3(pkg, torch, dev):
     return dict(step=step, ops=2 * stack_ops(1024), images=1024, full_rows=1024, cpu=cpu, formula=formula, check=check,
                 name="configs[3]: interval-bound certification forward through the MLP, batch 1024, eps=8/255: "
                      "value path + lower/upper bounds + certified margins (bound-ops and dist-ops both counted)",
+                nominal=lists_cover(pkg, 1024, 1) or lists_cover(pkg, 1024, 2),
                 kernel=("inf_dist_bound_forward", lambda l_, u_, w_, *_: 6 * mnk(l_, w_),
                         lambda l_, u_, w_, *_: w_.size(0) > 16,   # the 10-way head runs another kernel
-                        "bound_forward_kernel (tiled interval-bound forward)", 6))
+                        LISTS if lists_cover(pkg, 1024, 2) else "bound_forward_kernel (tiled interval-bound forward)", 6))
 
 
 def workload_c4(pkg, torch, dev):
@@ -702,11 +717,17 @@ def main():
             "traffic": None,
         },
     }
-    # HBM bytes per launch of the roofline kernel (c1: average over the step's four tiled forward launches), from
+    # HBM bytes per launch of the roofline kernel (c1: average over the step's four forward passes of wide layers), from
     # two rocprofv3 --pmc runs of this command: FETCH_SIZE and WRITE_SIZE, each scaled by what the counter reads for
     # a plain copy of known size.  The figure is read from the counter summary kept under profiles/, which names
     # the kernel it was measured on; null when there is no summary for this workload's kernel.
-    out["roofline"]["traffic"], out["roofline"]["traffic_source"] = profile_traffic(args.workload)
+    out["roofline"]["traffic"], out["roofline"]["traffic_source"] = profile_traffic(args.workload, kdesc == LISTS)
+    if wl.get("nominal"):
+        note = ("nominal: every (row, output, input) triple of the pass counts, as a walk of all differences takes them; the lists of "
+                "outermost values settle most outputs without evaluating most of theirs, to the same bits")
+        out["value_note"] = note
+        if kdesc == LISTS:
+            out["roofline"]["rate_note"] = note + ", so the fraction is no utilisation and may exceed what the ALU can do"
     for label, alt in wl.get("step_alt", []):
         for _ in range(args.warmup):
             alt()
@@ -723,8 +744,12 @@ def main():
 
 
 # workload -> (counter summary under profiles/, the roofline kernel's name in it)
-def traffic_profiles():
+def traffic_profiles(lists):
     c2_fused = C2_P != 2.0
+    if lists:
+        return {"c1": ("counters_lists_of_outermost_values.md", "positions, batch 512"),
+                "c1t": ("counters_lists_of_outermost_values.md", "positions, batch 512"),
+                "c3": ("counters_lists_of_outermost_values.md", "bounds, batch 1024")}
     return {"c1": ("counters_c1_mlp_inf.md", "inf_forward_kernel"), "c1t": ("counters_c1t_training_step.md", "inf_forward_kernel"),
             "c0": ("counters_c0_fc_layer.md", "inf_forward_kernel"),
             "c2": (f"counters_c2_mlp_p{C2_P:g}.md", "norm_backward_fused_kernel" if c2_fused else "norm_backward_input_tiled_kernel"),
@@ -734,11 +759,11 @@ def traffic_profiles():
             "c4p": (f"counters_c4p_conv_p{C4_P:g}_from_image.md", "norm_conv_backward_kernel")}
 
 
-def profile_traffic(workload):
+def profile_traffic(workload, lists):
     """(bytes per launch, source file) from the line 'traffic_bytes_per_launch[<kernel>]: <number>' of the
     workload's counter summary under profiles/, or (None, None)."""
     import re
-    name, kernel = traffic_profiles().get(workload, (None, None))
+    name, kernel = traffic_profiles(lists).get(workload, (None, None))
     path = os.path.join(ROOT, "profiles", name) if name else None
     if not path or not os.path.exists(path):
         return None, None

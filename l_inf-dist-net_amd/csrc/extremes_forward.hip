@@ -20,7 +20,10 @@
 // bound: their outputs are walked in full with the comparisons of the other kernels.
 //
 // 5120 x 5120 with positions, batch 272 / 512: 300 / 470 -> 165 / 205 us; values at 1024 780 -> 155; bounds at 1024 2170 -> 225.
-// Data that the lists cannot help cost 12 to 60 us beside the full walk of 480 to 2170.
+// Data that the lists cannot help (two values in both operands) cost the sample and the lists beside the full walk: 15 to 60 us
+// up to 5120 inputs, 75 at 12544, 110 to 140 at 20000.  Weights of a 5 x 5120 net that has been trained through p = 8 ... 1000 and
+// infinity need longer lists than untrained ones: on its own inputs, batch 512, lists / full walk, us, positions 182 / 474, values
+// 162 / 437, bounds 239 / 1125 (untrained 102 / 467, 100 / 429, 121 / 1099).
 #include <algorithm>
 
 #include "kernels.hpp"
