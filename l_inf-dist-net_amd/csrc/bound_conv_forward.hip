@@ -302,7 +302,7 @@ hipError_t bound_conv_forward(const float* lower, const float* upper, const floa
                               const float* bias, hipStream_t stream) {
     ConvFwd a{};
     if (!plan(q, G, CO, a, 2)) return hipErrorInvalidValue;   // the API layer asks bound_conv_forward_supported first
-    share_channels(q, a, 2, num_cu, {27e3, 36e3, 24e3, 0.0, 1, 0.93});
+    share_channels(q, a, 2, num_cu, {27e3, 36e3, 24e3, 0.0, 1});
     a.vec_in = 0;
     a.mean = mean;
     a.bias = bias;

@@ -147,7 +147,7 @@ inline size_t lds_bytes(const ConvFwd& a, int nx) {
 // Clocks of a launch: what the busiest CU's workgroups take, one set of as many as fit after the other.  `one` and `two`: a stage's
 // clocks with one wave per SIMD and with two; `fixed`, `search`: what a workgroup's start and end take, and what the groups
 // divide at the end (the search for the position).
-struct StageClocks { double one, two, fixed, search; int rest; double worth; };   // rest: weight words in flight beyond the parked ones
+struct StageClocks { double one, two, fixed, search; int rest; };   // rest: weight words in flight beyond the parked ones
 inline double launch_clocks(const ConvFwd& a, int nx, int num_cu, const StageClocks& c) {
     const int waves = (a.KG * a.GT + 63) / 64, stages = (a.CGP / kCC + a.KG - 1) / a.KG;
     long at_once = (long)(kLdsLimit / (lds_bytes(a, nx) + (nx > 1 ? 256 : 0)));
@@ -167,17 +167,27 @@ inline double launch_clocks(const ConvFwd& a, int nx, int num_cu, const StageClo
 // and its channels are shared by up to eight groups of lanes (eight waves in all, two per SIMD), which have stages of their
 // own and meet in LDS at the end.  That layer with 64 channels: bounds 190 -> 117 us, values 85 -> 46; the same images at
 // 28 x 28, 32 channels, 32 outputs: 141 -> 119 and 47 -> 47.  The clocks were fitted to these.  A shape is changed where that gains
-// `worth`, and only below four rounds of workgroups: beyond, the last round's share is small.  Over 134 layers of 1 to 512 images
-// of 7 to 32 pixels, 3 to 128 channels and 8 to 252 outputs the estimate is within a third of the time for values and bounds (7 %
-// asked for); with positions it promises more than there is, 0.68 of the time where 0.89 to 1.09 were measured, 0.88 where 1.28,
-// hence a third.  A smaller tile that is not shared lost as often as it gained (16.2 -> 20.2, 14.8 -> 15.5 us) and is not taken.
+// what asked() says, and only below four rounds of workgroups: beyond, the last round's share is small.  Measured over layers of
+// 1 to 512 images of 7 to 32 pixels, 3 to 160 channels and 8 to 256 outputs: for values and bounds (134 layers) the estimate is
+// within a third of the time, and a gain of 7 % is one.  With positions it promises too much: two groups gain from three quarters
+// on where there are stages to share, 59.1 -> 49.7 us for 64 images of 32 x 28 x 28 -> 32 at 0.67 of the clocks, and small ones
+// of a stage each from two thirds on (0.68: 23 -> 25.9); more groups or two large ones of a stage took 1.1 to 1.54 of the time at 0.62
+// to 0.93, and so did launches of more than two workgroups to a CU before (267 images of 74 x 16 x 16 -> 44 in two groups of
+// channels 123 -> 189 us).  A smaller tile that is not shared gains where much is promised (146 images of 3 x 15 x 15 -> 100 at
+// 0.53: 46 -> 33) and not elsewhere (2 of 4 x 20 x 20 -> 222 at 0.75: 16.2 -> 20.2).  194 layers with positions whose shape
+// changes for some rule take 0.785 of their time in all, 5 of them 1.05 to 1.11; with 7 % asked for 0.802, 32 of them up to 1.54.
 inline void share_channels(const ConvGeom& q, ConvFwd& a, int nx, int num_cu, const StageClocks& clocks_of) {
     if (g_conv_rows_override > 0 && g_conv_groups_override <= 0) return;
     const int forced = g_conv_groups_override;
     const double before = launch_clocks(a, nx, num_cu, clocks_of);
-    double best = forced > 0 ? 1e300 : clocks_of.worth * before;
+    double best = forced > 0 ? 1e300 : before;
     if (forced <= 0 && (double)a.B * a.G * a.tiles_h * a.tiles_n > 4.0 * 2 * num_cu) return;   // at least four rounds
     const int S = q.S, quads = (a.NG + kTN - 1) / kTN, first_tiles = (quads + 15) / 16, nstage = a.CGP / kCC;
+    auto asked = [&](const ConvFwd& c) {   // share of the clocks before; with positions there is a search to divide
+        if (c.KG == 1) return 0.62;
+        if (clocks_of.search == 0.0) return 0.93;
+        return (double)a.B * a.G * a.tiles_h * a.tiles_n > 2.0 * num_cu ? 0.0 : c.KG > 2 ? 0.6 : nstage > 3 ? 0.75 : c.GT <= 128 ? 0.65 : 0.6;
+    };
     ConvFwd pick = a;
     int last_nl = 0;
     for (int tiles_n = first_tiles; tiles_n <= quads && tiles_n <= 8 * first_tiles; tiles_n++) {
@@ -201,10 +211,9 @@ inline void share_channels(const ConvGeom& q, ConvFwd& a, int nx, int num_cu, co
                 const int per = (nstage + c.KG - 1) / c.KG;
                 if (per == last_per || (forced > 0 && c.KG != forced)) continue;   // a group more than the stages are worth
                 last_per = per;
-                if (c.KG == 1 && forced <= 0) continue;
                 if (lds_bytes(c, nx) > kLdsLimit - (nx > 1 ? 1024 : 0)) break;
                 const double clocks = launch_clocks(c, nx, num_cu, clocks_of);
-                if (clocks < best) { best = clocks; pick = c; }
+                if (clocks < best && (forced > 0 || clocks < asked(c) * before)) { best = clocks; pick = c; }
             }
         }
     }

@@ -516,7 +516,7 @@ hipError_t inf_conv_forward(const float* img, const float* weight, float* out, i
     ConvFwd a{};
     if (!plan(q, G, CO, a)) return hipErrorInvalidValue;   // the API layer asks inf_conv_forward_supported first
     const bool with_pos = pos != nullptr;
-    share_channels(q, a, 1, num_cu, with_pos ? StageClocks{10e3, 13e3, 14e3, 20e3, 1, 0.66} : StageClocks{9e3, 11.5e3, 14e3, 0.0, kRest, 0.93});
+    share_channels(q, a, 1, num_cu, with_pos ? StageClocks{10e3, 13e3, 14e3, 20e3, 1} : StageClocks{9e3, 11.5e3, 14e3, 0.0, kRest});
     a.mean = mean;
     a.bias = bias;
     a.vec_in = q.W % 4 == 0 && aligned16(img);
