@@ -145,9 +145,9 @@ def _with_workspace(name, what, sizes, dev, args):
     """Calls the form `name` of a forward pass that takes scratch memory, where the library has one for the layer and there is
     memory for it; False elsewhere: the plain entry point is the way.  `args`: pointers before and after the sizes."""
     need = ctypes.c_int64()
+    if _lib.lib().ldist_inf_dist_workspace(*sizes, what, ctypes.byref(need)) != 0 or need.value == 0:   # asks no device
+        return False
     with torch.cuda.device(dev):
-        if _lib.lib().ldist_inf_dist_workspace(*sizes, what, ctypes.byref(need)) != 0 or need.value == 0:
-            return False
         try:
             scratch = torch.empty(need.value, dtype=torch.uint8, device=dev)   # free for later work on the stream on return
         except torch.OutOfMemoryError:
