@@ -131,6 +131,15 @@ LDIST_API int ldist_inf_dist_value_bound_forward(const float* input, const float
                                        const float* bias, float* output, float* output_lower, float* output_upper,
                                        ldist_stream_t stream);
 
+/* The same through lists of outermost values (see ldist_inf_dist_forward_ws): one set of lists and one scan for the points
+ * and their boxes.  Scratch memory as there: 0 bytes where a layer has no such form, and LDIST_EUNSUPPORTED from the pass,
+ * also where input and weight do not allow 128-bit loads; nothing is enqueued then. */
+LDIST_API int ldist_inf_dist_value_bound_workspace(int B, int CO, int CI, int G, int HW, int64_t* bytes);
+LDIST_API int ldist_inf_dist_value_bound_forward_ws(const float* input, const float* input_lower, const float* input_upper,
+                                       const float* weight, int B, int CO, int CI, int G, int HW, const float* mean,
+                                       const float* bias, float* output, float* output_lower, float* output_upper,
+                                       void* workspace, int64_t bytes, ldist_stream_t stream);
+
 /* L_inf backward w.r.t. input.  Replaces inf_dist_backward_input_cuda
  * (model/norm_dist.cpp:17-18, model/inf_dist_cuda.cu:189-196).
  *   grad_input[b, g*K + idx, hw] += (pos >= 0 ? g : -g),  idx = pos & 0x7fffffff

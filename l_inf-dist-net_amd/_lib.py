@@ -25,6 +25,9 @@ SIGNATURES = {
     "ldist_inf_dist_bound_forward_ws": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, ctypes.c_void_p, ctypes.c_int64, _S],
     "ldist_inf_dist_bound_forward": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _S],
     "ldist_inf_dist_value_bound_forward": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _F, _F, _F, _S],
+    "ldist_inf_dist_value_bound_workspace": [_i, _i, _i, _i, _i, ctypes.c_void_p],
+    "ldist_inf_dist_value_bound_forward_ws": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _F, _F, _F, ctypes.c_void_p,
+                                              ctypes.c_int64, _S],
     "ldist_inf_dist_backward_input": [_F, _I, _i, _i, _i, _i, _i, _F, _S],
     "ldist_inf_dist_backward_weight": [_F, _I, _i, _i, _i, _i, _i, _F, _S],
     "ldist_inf_dist_backward_input_overwrite": [_F, _I, _i, _i, _i, _i, _i, _F, _S],

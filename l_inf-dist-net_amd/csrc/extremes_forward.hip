@@ -13,7 +13,14 @@
 //   sample   64 x 64 outputs in full, and for their rows what lists of eight lengths would leave out;
 //   select   the list lengths that cost least by that sample (or none: `dense`, and the kernels of the full walk, which
 //            are launched last and otherwise leave at once, do the work), and every row's list;
-//   scan     first every row's list against all outputs, then every weight row's list against all rows.
+//   scan     first every row's list against all outputs, then every weight row's list against all rows.  Where the weights
+//            need no list (images, or activations spread far wider than the weights) the first scan checks the bounds itself,
+//            and the second leaves at once: 5120 x 5120 with positions at batch 272, 46 + 43 -> 56 + 5 us.
+//
+// Boxes and the points inside them (certification) share sample, lists and first scan: an entry of a row of x is {lower, upper,
+// 32 k, point}.  Where the weights have lists, the second scans of boxes and of values follow it.  Values and bounds of the 5-layer,
+// 5120-wide net at batch 1024: 1450 to 1640 us with passes of their own, 825 together; 5120 x 5120 normal weights and inputs of
+// the same spread, batch 512, 187 + 240 -> 350 us, 1024 256 + 390 -> 580.
 //
 // The reduction is cut into C chunks of at most 2560 k with lists and bounds of their own, so that a chunk of eight rows
 // of the other operand fits half a CU's LDS.  Rows with NaN or infinities (bounds: boxes that are not l <= u) get an infinite
@@ -54,33 +61,36 @@ struct Header {
     int dense;         // the lists are not worth it
     int full;          // the full walk has to do the work: dense, or the lists left too many outputs unsettled
     int failed;        // how many
-    int taken[2][8];   // tiles of a scan that the workgroups of an XCD have taken beyond their first
+    int taken[3][8];   // tiles of a scan (Search::turn) that the workgroups of an XCD have taken beyond their first
 };
 
 // One operand: its rows, their lists in blocks of 16 rows (entry-major, so that 16 neighbouring lanes read 128 bytes)
 // and per chunk and row what the lists left out.
 struct Side {
-    const float *v, *v2;   // v2: the upper ends where v are the lower ends of boxes
+    const float *v, *v2, *v3;   // v2: the upper ends where v are the lower ends of boxes; v3: the points inside them
     int rows, blocks;
-    char* lists;           // [chunk][block][entry][16] of {value, 32 k} or {lower, upper, 32 k, 0}
-    float* rest;           // [chunk][2 or 4][rows]: max, min; boxes: max of the upper ends, min of the lower, max of the lower, min of the upper
+    char* lists;           // [chunk][block][entry][16] of {value, 32 k} or {lower, upper, 32 k, point}
+    float* rest;           // [chunk][rests][rows]: max, min; boxes: max of the upper ends, min of the lower, max of the lower, min of the upper; points: max, min
+    int rests;             // 2, 4 or 6
 };
 
 struct Search {
     Side x, w;
-    float *out, *out2;     // distances, or the lower and upper bounds
+    float *out, *out2, *out3;   // distances, or the lower and upper bounds, and the points' distances
     const float *mean, *bias;   // of Problem
     int32_t* pos;
     Header* head;
     unsigned char* counts; // [workgroup of the sample][combination of lengths]: outputs that would not pass
     float* reach;          // [x, w][length][sampled row]: how far from the center a list of that length begins
     float* partial;        // [row of x][pitch] of the first scan's {value, position}, {upper, lower bound}, or values
+    float* partial3;       // [row of x][pitch] of the points' distances
     int pitch;
+    int turn;              // which of Header::taken a scan counts in
     int* walk;             // [walk_most]: indices of outputs that fail
     int walk_most;
     int K, C, KC;
     int lanes_first, lanes_second;   // rows per workgroup of the two scans
-    float price_x, price_w, price_fail, price_dense;   // of a list entry, of an output that does not pass, of the full walk
+    float price_x, price_w, price_both, price_fail, price_dense;   // of a list entry, of a second scan after the first, of an output that does not pass, of the full walk
 };
 
 __device__ __forceinline__ float wave_max_f(float x) {
@@ -185,9 +195,11 @@ __device__ __forceinline__ void lengths_of(RowChunk<NV>& a, float center, int* h
 }
 
 // A workgroup looks at 4 x 4 outputs: wave i at row i % 8 (four of x, four of w) in every other chunk, then all at the outputs.
-template <int NV, bool PAIR>
+// ENDS: 1 values, 2 boxes, 3 boxes and the points inside them.
+template <int NV, int ENDS>
 __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
-    constexpr int NO = kSampleRows * kSampleRows, NB = PAIR ? 2 : 1, WAVES = 16;
+    constexpr bool PAIR = ENDS >= 2, ALL = ENDS == 3;
+    constexpr int NO = kSampleRows * kSampleRows, NB = ENDS, WAVES = 16;
     __shared__ __align__(16) int hist[WAVES][kBins];
     __shared__ float rest[NB][2 * kSampleRows][8][16];   // [bound][row][length][chunk]: the most that the list leaves out
     __shared__ float reach[2 * kSampleRows][8][16];
@@ -223,14 +235,14 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
     const float center = not_finite(c) ? 0.f : c / 1024.f;
     if (blockIdx.x == 0) {
         if (tid == 0) s.head->center = center;
-        if (tid < 16) s.head->taken[tid >> 3][tid & 7] = 0;
-        if (tid == 16) s.head->failed = 0;
+        if (tid < 24) s.head->taken[tid >> 3][tid & 7] = 0;
+        if (tid == 24) s.head->failed = 0;
     }
 #pragma unroll 1
     for (int ch = first; ch < s.C; ch += WAVES / 8) {
         if (ch != first) load(ch);
         const int kc = min(s.KC, s.K - ch * s.KC);
-        float widest = 0.f, width = 0.f;   // of the boxes, and the mean; half of each
+        float widest = 0.f, width = 0.f, off = 0.f;   // of the boxes, and the mean; half of each; points off the middle
         if constexpr (PAIR) {
             if (of_x) {
 #pragma unroll
@@ -244,6 +256,12 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
 #pragma unroll
                 for (int o = 32; o; o >>= 1) width += __shfl_xor(width, o);
                 width /= kc;
+                if constexpr (ALL) {
+                    b.load(s.x.v3 + (size_t)row * s.K + ch * s.KC, kc, lane);   // both 0 past the end
+#pragma unroll
+                    for (int j = 0; j < NV; j++) off = __builtin_fmaxf(off, __builtin_fabsf(b.v[j] - a.v[j]));
+                    off = wave_max_f(off);
+                }
             }
         }
         a.center_past(kc, lane, center);
@@ -252,28 +270,35 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
                 reach[r][i][ch] = edge;
                 rest[0][r][i][ch] = edge + widest;                    // upper bounds reach further than the middles,
                 if constexpr (PAIR) rest[1][r][i][ch] = edge - width;   // lower bounds less far
+                if constexpr (ALL) rest[2][r][i][ch] = edge + off;
             }
         });
     }
 
-    float up[NO], lo[NO];
+    float up[NO], lo[NO], pt[NO];
 #pragma unroll
-    for (int i = 0; i < NO; i++) up[i] = lo[i] = 0.f;
-    const float *xr[kSampleRows], *ur[kSampleRows], *wr[kSampleRows];
+    for (int i = 0; i < NO; i++) up[i] = lo[i] = pt[i] = 0.f;
+    const float *xr[kSampleRows], *ur[kSampleRows], *pr[kSampleRows], *wr[kSampleRows];
 #pragma unroll
     for (int i = 0; i < kSampleRows; i++) {
         xr[i] = s.x.v + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
         if constexpr (PAIR) ur[i] = s.x.v2 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
+        if constexpr (ALL) pr[i] = s.x.v3 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
         wr[i] = s.w.v + (size_t)sampled(bw * kSampleRows + i, s.w.rows) * s.K;
     }
-    constexpr int AHEAD = PAIR ? 3 : 5;
+    constexpr int AHEAD = ALL ? 2 : PAIR ? 3 : 5;
     for (int kb = 0; kb < s.K; kb += 1024 * AHEAD) {
-        float x[AHEAD][kSampleRows], u[AHEAD][kSampleRows], w[AHEAD][kSampleRows];
+        float x[AHEAD][kSampleRows], u[AHEAD][kSampleRows], p[AHEAD][kSampleRows], w[AHEAD][kSampleRows];
 #pragma unroll
         for (int e = 0; e < AHEAD; e++) {
             const int k = min(kb + e * 1024 + tid, s.K - 1);   // past the end: the last k again
 #pragma unroll
-            for (int i = 0; i < kSampleRows; i++) { x[e][i] = xr[i][k]; w[e][i] = wr[i][k]; if constexpr (PAIR) u[e][i] = ur[i][k]; }
+            for (int i = 0; i < kSampleRows; i++) {
+                x[e][i] = xr[i][k];
+                w[e][i] = wr[i][k];
+                if constexpr (PAIR) u[e][i] = ur[i][k];
+                if constexpr (ALL) p[e][i] = pr[i][k];
+            }
         }
 #pragma unroll
         for (int e = 0; e < AHEAD; e++)
@@ -290,6 +315,7 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
                         U = __builtin_fmaxf(U, __builtin_fabsf(du));
                         L = __builtin_fmaxf(__builtin_fmaxf(L, dl), -du);
                     }
+                    if constexpr (ALL) pt[i * kSampleRows + j] = __builtin_fmaxf(pt[i * kSampleRows + j], __builtin_fabsf(p[e][i] - w[e][j]));
                 }
     }
 #pragma unroll
@@ -299,6 +325,10 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
         if constexpr (PAIR) {
             const float l = wave_max(lo[i]);
             if (lane == 63) outs[wave][NO + i] = l;
+        }
+        if constexpr (ALL) {
+            const float v = wave_max(pt[i]);
+            if (lane == 63) outs[wave][2 * NO + i] = v;
         }
     }
     __syncthreads();
@@ -347,7 +377,7 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
 #pragma unroll
     for (int i = 0; i < 8; i++) fails += sums[i][lane];
     float cost = s.C * (s.price_x * kLengths[lane >> 3] + s.price_w * kLengths[lane & 7]) +
-                 s.price_fail * ((float)fails / (kSampled * kSampled));
+                 (lane > 7 && (lane & 7) ? s.price_both : 0.f) + s.price_fail * ((float)fails / (kSampled * kSampled));
     int pick = lane;
 #pragma unroll
     for (int o = 32; o; o >>= 1) {
@@ -361,184 +391,221 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
     dense = __builtin_amdgcn_readfirstlane(cost > s.price_dense ? 1 : 0);
 }
 
-// A workgroup makes the lists of 16 rows in one chunk, a wave those of two rows: all values beyond `t` from the center,
+// A workgroup makes the lists of eight rows in one chunk, a wave that of a row (with two rows per wave the last workgroups ran
+// alone for half of the time): all values beyond `t` from the center,
 // where t starts as what the sampled rows needed on the average and is moved where the list would overflow or stay half empty
 // (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly,
 // unless more values tie at the outer end than the list has places: such a row's bounds are those of all its values.
 // Bound by reading the operands once.
-template <int NV, bool PAIR>
-__global__ void __launch_bounds__(512, PAIR ? 3 : 5) extremes_select_kernel(Search s) {
-    extern __shared__ __align__(16) char stage[];   // [entry][16] as in Side::lists
+template <int NV, int ENDS>
+__global__ void __launch_bounds__(512, ENDS > 1 ? 4 : 5) extremes_select_kernel(Search s) {
+    extern __shared__ __align__(16) char stage[];   // [entry][8]: half of a block of Side::lists
     __shared__ int sums[8][64];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int per = s.x.blocks + s.w.blocks, ch = blockIdx.x / per;
+    const int per = 2 * (s.x.blocks + s.w.blocks), ch = blockIdx.x / per;
     int block = blockIdx.x % per;
-    const bool of_x = block < s.x.blocks;
+    const bool of_x = block < 2 * s.x.blocks;
     const Side& side = of_x ? s.x : s.w;
-    if (!of_x) block -= s.x.blocks;
-    const int k0 = ch * s.KC;
-    auto row_at = [&](int i) { return __builtin_amdgcn_readfirstlane(min(block * 16 + wave * 2 + i, side.rows - 1)); };
+    if (!of_x) block -= 2 * s.x.blocks;
+    const int k0 = ch * s.KC, r = block * 8 + wave, row = __builtin_amdgcn_readfirstlane(min(r, side.rows - 1));
 
-    auto lists = [&](auto pair) {
-        constexpr bool P = decltype(pair)::value;
-        RowChunk<NV> a, b;
-        int kc = min(s.KC, s.K - k0);
-        auto load = [&](int i, int lane) {
-            const size_t at = (size_t)row_at(i) * s.K + k0;
-            a.load(side.v + at, kc, lane);
-            if constexpr (P) b.load(side.v2 + at, kc, lane);
-        };
-        load(0, tid & 63);
+    auto lists = [&](auto ends) {
+        constexpr bool P = decltype(ends)::value >= 2, ALL = decltype(ends)::value == 3;
+        RowChunk<NV> a;
+        const int kc = min(s.KC, s.K - k0), lane = tid & 63;
+        a.load(side.v + (size_t)row * s.K + k0, kc, lane);
         int ix, iw, dense;
-        choose_lengths(s, sums, wave, tid & 63, ix, iw, dense);
+        choose_lengths(s, sums, wave, lane, ix, iw, dense);
         const int q = kLengths[of_x ? ix : iw];
         if (blockIdx.x == 0 && tid == 0) { s.head->qx = kLengths[ix]; s.head->qw = kLengths[iw]; s.head->dense = s.head->full = dense; }
         if (dense) return;
         const float center = s.head->center;
-        float guess = s.reach[((of_x ? 0 : 1) * 8 + (of_x ? ix : iw)) * kSampled + (tid & 63)];
+        float guess = s.reach[((of_x ? 0 : 1) * 8 + (of_x ? ix : iw)) * kSampled + lane];
 #pragma unroll
         for (int o = 32; o; o >>= 1) guess += __shfl_xor(guess, o);
         guess = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(guess * (1.f / kSampled))));
-#pragma unroll 1
-        for (int i = 0; i < 2; i++) {
-            // what is derived from these is made where it is used, not kept in registers over the loop
-            asm volatile("" : "+s"(kc));
-            int lane = tid & 63;
-            asm volatile("" : "+v"(lane));
-            if (i) load(i, lane);
-            const int row = row_at(i), r = wave * 2 + i;
-            a.center_past(kc, lane, center);
-            if constexpr (P) b.center_past(kc, lane, center);
-            float odd = 0.f;   // NaN if there is a NaN or an infinity
-            bool crossed = false;
+        // twice the middle of a box, where values are compared by themselves
+        constexpr float F = P ? 2.f : 1.f;
+        if constexpr (!P) a.center_past(kc, lane, center);
+        float odd = 0.f;   // NaN if there is a NaN or an infinity
+        bool crossed = false;
 #pragma unroll
-            for (int j = 0; j < NV; j++) {
-                odd = __builtin_fmaf(a.v[j], 0.f, odd);
-                if constexpr (P) { odd = __builtin_fmaf(b.v[j], 0.f, odd); crossed |= a.v[j] > b.v[j]; }
-            }
-            const bool bad = __any(odd != 0.f || crossed);
-            // twice the middle of a box, where values are compared by themselves
-            constexpr float F = P ? 2.f : 1.f;
-            auto key = [&](int j) {
-                if constexpr (P) return a.v[j] + b.v[j];
-                else return a.v[j];
-            };
-            auto count = [&](float t) {
-                const float hi = F * (center + t), lo = F * (center - t);
-                int n = 0;
+        for (int j = 0; j < NV; j++) odd = __builtin_fmaf(a.v[j], 0.f, odd);
+        if constexpr (P) {
+            RowChunk<NV / 2> b;   // half a row at a time: registers
 #pragma unroll
-                for (int j = 0; j < NV; j++) n += __builtin_popcountll(__ballot(key(j) > hi) | __ballot(key(j) < lo));
-                return n;
-            };
-            float hi, lo;
-            if (q == 0) {   // no list: everything is left out
-                hi = -kNever;
-                lo = kNever;
+            for (int h = 0; h < 2; h++) {
+                b.load(side.v2 + (size_t)row * s.K + k0 + h * NV * 32, max(kc - h * NV * 32, 0), lane);
 #pragma unroll
-                for (int j = 0; j < NV; j++) { hi = __builtin_fmaxf(hi, key(j)); lo = __builtin_fminf(lo, key(j)); }
-                hi = wave_max_f(hi);
-                lo = wave_min_f(lo);
-            } else {
-                float t = guess;
-                int n = count(t);
-                if (n > q || n < q / 2) {
-                    float most = 0.f;
-#pragma unroll
-                    for (int j = 0; j < NV; j++) most = __builtin_fmaxf(most, __builtin_fabsf(key(j) - F * center));
-                    // too long a list, and one of no more than what ties at the outer end: center + t, rounded, may lie inside it
-                    float in = 0.f, out = wave_max_f(most) * (1.f / F);
-                    if (n > q) in = t; else out = __builtin_fminf(out, t);
-#pragma unroll 1
-                    for (int step = 0; step < 10; step++) {
-                        t = 0.5f * (in + out);
-                        n = count(t);
-                        if (n > q) { in = t; continue; }
-                        out = t;
-                        if (n >= q - q / 4) break;
-                    }
-                    t = out;
-                }
-                hi = F * (center + t);
-                lo = F * (center - t);
-            }
-            int base = 0;
-            float most = -kNever, least = kNever, most_lower = -kNever, least_upper = kNever;
-#pragma unroll
-            for (int j = 0; j < NV; j++) {
-                const bool in = key(j) > hi || key(j) < lo;
-                const unsigned long long m = __ballot(in);
-                if (m) {
-                    const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-                    if (in && at < q) {
-                        const unsigned k32 = (unsigned)(lane + j * 64) * 32u;
-                        if constexpr (P) reinterpret_cast<uint4*>(stage)[at * 16 + r] = make_uint4(__float_as_uint(a.v[j]), __float_as_uint(b.v[j]), k32, 0u);
-                        else reinterpret_cast<uint2*>(stage)[at * 16 + r] = make_uint2(__float_as_uint(a.v[j]), k32);
-                    }
-                    base += __builtin_popcountll(m);
-                }
-                if constexpr (P) {
-                    most = __builtin_fmaxf(most, in ? -kNever : b.v[j]);
-                    least = __builtin_fminf(least, in ? kNever : a.v[j]);
-                    most_lower = __builtin_fmaxf(most_lower, in ? -kNever : a.v[j]);
-                    least_upper = __builtin_fminf(least_upper, in ? kNever : b.v[j]);
+                for (int j = 0; j < NV / 2; j++) {
+                    float& mid = a.v[h * NV / 2 + j];
+                    odd = __builtin_fmaf(b.v[j], 0.f, odd);
+                    crossed |= mid > b.v[j];
+                    mid += b.v[j];
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (__builtin_expect(base > q, 0)) {   // the list has lost values that no bound above speaks for
+        }
+        if constexpr (P) a.center_past(kc, lane, F * center);
+        bool bad = __any(odd != 0.f || crossed);
+        auto key = [&](int j) { return a.v[j]; };
+        auto count = [&](float t) {
+            const float hi = F * (center + t), lo = F * (center - t);
+            int n = 0;
+#pragma unroll
+            for (int j = 0; j < NV; j++) n += __builtin_popcountll(__ballot(key(j) > hi) | __ballot(key(j) < lo));
+            return n;
+        };
+        float hi, lo;
+        if (q == 0) {   // no list: everything is left out
+            hi = -kNever;
+            lo = kNever;
+#pragma unroll
+            for (int j = 0; j < NV; j++) { hi = __builtin_fmaxf(hi, key(j)); lo = __builtin_fminf(lo, key(j)); }
+            hi = wave_max_f(hi);
+            lo = wave_min_f(lo);
+        } else {
+            float t = guess;
+            int n = count(t);
+            if (n > q || n < q / 2) {
+                float most = 0.f;
+#pragma unroll
+                for (int j = 0; j < NV; j++) most = __builtin_fmaxf(most, __builtin_fabsf(key(j) - F * center));
+                // too long a list, and one of no more than what ties at the outer end: center + t, rounded, may lie inside it
+                float in = 0.f, out = wave_max_f(most) * (1.f / F);
+                if (n > q) in = t; else out = __builtin_fminf(out, t);
+#pragma unroll 1
+                for (int step = 0; step < 10; step++) {
+                    t = 0.5f * (in + out);
+                    n = count(t);
+                    if (n > q) { in = t; continue; }
+                    out = t;
+                    if (n >= q - q / 4) break;
+                }
+                t = out;
+            }
+            hi = F * (center + t);
+            lo = F * (center - t);
+        }
+        struct Ends { float a, b, c; } first = {};
+        int base = 0;
+        float most = -kNever, least = kNever, most_lower = -kNever, least_upper = kNever, most_point = -kNever, least_point = kNever;
+        auto place = [&](bool in, int j, auto&& write) {
+            const unsigned long long m = __ballot(in);
+            if (m) {
+                const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                if (in && at < q) write(at * 8 + wave, (unsigned)(lane + j * 64) * 32u);
+                base += __builtin_popcountll(m);
+            }
+        };
+        if constexpr (P) {
+            // Boxes and points come again, in groups of eight, mostly from the L2: there are no registers for all of them (with
+            // both ends kept 155, which leave a workgroup alone on its CU, with the points 168 and 290 spilled).
+            float odd_point = 0.f;
+            const auto from = [&](const float* v) {
+                return __builtin_amdgcn_make_buffer_rsrc((void*)(v + (size_t)row * s.K + k0), 0, kc * 4, 0x00020000);
+            };
+            const auto ra = from(side.v), rb = from(side.v2), rc = from(ALL ? side.v3 : side.v);
+            auto gather = [&](bool record) {   // else: bounds of all values
+#pragma unroll 1
+                for (int j0 = 0; j0 < NV; j0 += 8) {
+                    Ends e[8];
+                    auto one = [&](auto rsrc, int j) {
+                        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane * 4, (j0 + j) * 256, 0));
+                    };
+#pragma unroll
+                    for (int j = 0; j < 8; j++) e[j] = Ends{one(ra, j), one(rb, j), ALL ? one(rc, j) : 0.f};
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        if (lane >= kc - (j0 + j) * 64) e[j] = Ends{center, center, center};
+                        const float mid = e[j].a + e[j].b;
+                        const bool in = record && (mid > hi || mid < lo);
+                        if (record)
+                            place(in, j0 + j, [&](int to, unsigned k32) {
+                                reinterpret_cast<uint4*>(stage)[to] =
+                                    make_uint4(__float_as_uint(e[j].a), __float_as_uint(e[j].b), k32, __float_as_uint(e[j].c));
+                            });
+                        most = __builtin_fmaxf(most, in ? -kNever : e[j].b);
+                        least = __builtin_fminf(least, in ? kNever : e[j].a);
+                        most_lower = __builtin_fmaxf(most_lower, in ? -kNever : e[j].a);
+                        least_upper = __builtin_fminf(least_upper, in ? kNever : e[j].b);
+                        if constexpr (ALL) {
+                            most_point = __builtin_fmaxf(most_point, in ? -kNever : e[j].c);
+                            least_point = __builtin_fminf(least_point, in ? kNever : e[j].c);
+                            odd_point = __builtin_fmaf(e[j].c, 0.f, odd_point);
+                        }
+                    }
+                    if (j0 == 0) first = e[0];
+                }
+            };
+            gather(true);
+            if (__builtin_expect(base > q, 0)) gather(false);   // the list has lost values that no bound above speaks for
+            if constexpr (ALL) bad |= __any(odd_point != 0.f);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+                place(a.v[j] > hi || a.v[j] < lo, j, [&](int to, unsigned k32) {
+                    reinterpret_cast<uint2*>(stage)[to] = make_uint2(__float_as_uint(a.v[j]), k32);
+                });
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (__builtin_expect(base > q, 0)) {   // as above
 #pragma unroll
                 for (int j = 0; j < NV; j++) {
-                    most = __builtin_fmaxf(most, P ? b.v[j] : a.v[j]);
+                    most = __builtin_fmaxf(most, a.v[j]);
                     least = __builtin_fminf(least, a.v[j]);
-                    if constexpr (P) {
-                        most_lower = __builtin_fmaxf(most_lower, a.v[j]);
-                        least_upper = __builtin_fminf(least_upper, b.v[j]);
-                    }
                 }
-                if constexpr (!P) {
-                    hi = wave_max_f(most);
-                    lo = wave_min_f(least);
-                }
+                hi = wave_max_f(most);
+                lo = wave_min_f(least);
             }
-            // a list that is not full repeats the chunk's first value
-            const unsigned v0 = __builtin_amdgcn_readfirstlane(__float_as_uint(a.v[0]));
-            const unsigned v1 = P ? __builtin_amdgcn_readfirstlane(__float_as_uint(b.v[0])) : 0u;
-            for (int e = base + lane; e < q; e += 64) {
-                if constexpr (P) reinterpret_cast<uint4*>(stage)[e * 16 + r] = make_uint4(v0, v1, 0u, 0u);
-                else reinterpret_cast<uint2*>(stage)[e * 16 + r] = make_uint2(v0, 0u);
+        }
+        // a list that is not full repeats the chunk's first value
+        const auto from_lane_0 = [](float v) { return (unsigned)__builtin_amdgcn_readfirstlane(__float_as_uint(v)); };
+        const unsigned v0 = from_lane_0(P ? first.a : a.v[0]), v1 = from_lane_0(first.b), v2 = from_lane_0(first.c);
+        for (int e = base + lane; e < q; e += 64) {
+            if constexpr (P) reinterpret_cast<uint4*>(stage)[e * 8 + wave] = make_uint4(v0, v1, 0u, v2);
+            else reinterpret_cast<uint2*>(stage)[e * 8 + wave] = make_uint2(v0, 0u);
+        }
+        if constexpr (P) {
+            most = wave_max_f(most);
+            least = wave_min_f(least);
+            most_lower = wave_max_f(most_lower);
+            least_upper = wave_min_f(least_upper);
+            if constexpr (ALL) {
+                most_point = wave_max_f(most_point);
+                least_point = wave_min_f(least_point);
             }
+        } else {
+            most = hi;
+            least = lo;
+        }
+        if (lane == 0 && r < side.rows) {
+            const float inf = __builtin_inff();
+            float* rest = side.rest + (size_t)ch * side.rests * side.rows + row;
+            rest[0] = bad ? inf : most;
+            rest[side.rows] = bad ? -inf : least;
             if constexpr (P) {
-                most = wave_max_f(most);
-                least = wave_min_f(least);
-                most_lower = wave_max_f(most_lower);
-                least_upper = wave_min_f(least_upper);
-            } else {
-                most = hi;
-                least = lo;
+                rest[2 * side.rows] = bad ? inf : most_lower;
+                rest[3 * side.rows] = bad ? -inf : least_upper;
             }
-            if (lane == 0 && block * 16 + r < side.rows) {
-                const float inf = __builtin_inff();
-                float* rest = side.rest + (size_t)ch * (P ? 4 : 2) * side.rows + row;
-                rest[0] = bad ? inf : most;
-                rest[side.rows] = bad ? -inf : least;
-                if constexpr (P) {
-                    rest[2 * side.rows] = bad ? inf : most_lower;
-                    rest[3 * side.rows] = bad ? -inf : least_upper;
-                }
+            if constexpr (ALL) {
+                rest[4 * side.rows] = bad ? inf : most_point;
+                rest[5 * side.rows] = bad ? -inf : least_point;
             }
         }
         __syncthreads();
-        constexpr int E = P ? 16 : 8;   // bytes of an entry
-        uint4* dst = reinterpret_cast<uint4*>(side.lists + ((size_t)ch * side.blocks + block) * q * 16 * E);
-        for (int i = tid; i < q * E; i += 512) dst[i] = reinterpret_cast<const uint4*>(stage)[i];
+        constexpr int E = P ? 16 : 8, S = E / 2;   // bytes of an entry, and 16-byte pieces of the same entry of eight rows
+        uint4* dst = reinterpret_cast<uint4*>(side.lists + ((size_t)ch * side.blocks + block / 2) * q * 16 * E) + (block & 1) * S;
+        for (int i = tid; i < q * S; i += 512) dst[i / S * 2 * S + i % S] = reinterpret_cast<const uint4*>(stage)[i];
     };
-    if constexpr (PAIR) {
-        if (of_x) { lists(std::true_type{}); return; }
+    if constexpr (ENDS > 1) {
+        if (of_x) { lists(std::integral_constant<int, ENDS>{}); return; }
     }
-    lists(std::false_type{});
+    lists(std::integral_constant<int, 1>{});
 }
 
 // ---- scan ------------------------------------------------------------------------------------------------------------
-enum { kWithPos, kOnlyValues, kBoxes };
+enum { kWithPos, kOnlyValues, kBoxes, kBoxesAndPoints };
 __device__ __host__ constexpr int strip_rows(bool pairs) { return pairs ? 4 : 8; }   // 32 bytes per k
 
 // Lanes own rows of one operand (`ln`) and walk their lists; a strip of rows of the other (`sd`) lies in LDS, 32 bytes per
@@ -553,9 +620,19 @@ __device__ __host__ constexpr int strip_rows(bool pairs) { return pairs ? 4 : 8;
 //
 // First pass: lanes are rows of x, results into s.partial.  Second: lanes are rows of w; takes what the first left, checks the
 // bound and notes the outputs that fail it.
+template <class T, int N>
+__device__ __forceinline__ void store_row(T* to, const T (&v)[N]) {   // neighbouring elements, aligned to one
+    static_assert(N % 4 == 0);
+    typedef T Four __attribute__((ext_vector_type(4)));
+    struct __attribute__((packed, aligned(4))) Any { Four v; };
+#pragma unroll
+    for (int j = 0; j < N; j += 4) reinterpret_cast<Any*>(to + j)->v = Four{v[j], v[j + 1], v[j + 2], v[j + 3]};
+}
+
 template <int MODE, bool SECOND>
 __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
-    constexpr bool BOX = MODE == kBoxes, PAIR_ENTRY = BOX && !SECOND, PAIR_STRIP = BOX && SECOND;
+    constexpr bool ALL = MODE == kBoxesAndPoints, BOX = MODE == kBoxes || ALL, PAIR_ENTRY = BOX && !SECOND, PAIR_STRIP = BOX && SECOND;
+    static_assert(!(ALL && SECOND), "the second scans of boxes and points are those of boxes and of values");
     constexpr int RS = strip_rows(PAIR_STRIP), U = kMaxChunk / 512, NT = 512;
     extern __shared__ __align__(16) char lds[];
     if (s.head->dense) return;
@@ -563,7 +640,8 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
     const Side& sd = SECOND ? s.x : s.w;
     const int q = SECOND ? s.head->qw : s.head->qx;
     const bool both = s.head->qx != 0;   // second pass: the first has left something
-    if (!SECOND && !both) return;
+    const bool last = SECOND || s.head->qw == 0;   // no second pass: the first checks the bounds
+    if (SECOND ? q == 0 : !both && !last) return;
     const int K = s.K, KC = s.KC, C = s.C, N = s.w.rows;
     const int LG = SECOND ? s.lanes_second : s.lanes_first, EG = NT / LG;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -585,7 +663,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
     int tile = t_begin + (int)(blockIdx.x / 8);
     if (tile >= t_end) return;
     // The first tile is fixed, the others are taken as workgroups get there; lane 0 has the next one in hand a tile ahead.
-    auto take = [&] { return t_begin + (int)(gridDim.x / 8) + atomicAdd(&s.head->taken[SECOND][xcd], 1); };
+    auto take = [&] { return t_begin + (int)(gridDim.x / 8) + atomicAdd(&s.head->taken[s.turn][xcd], 1); };
     int in_hand = tid == 0 ? take() : 0;
 
     while (true) {
@@ -596,10 +674,10 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
         const bool live = row0 + at < ln.rows;
         const bool wave_live = __builtin_amdgcn_readfirstlane(row0 + (at & ~63)) < ln.rows;
         // values: the difference of the largest magnitude, with its sign, and 32 k; boxes: upper and lower bound
-        float best[RS], low[RS];
+        float best[RS], low[RS], point[RS];
         unsigned key[RS];
 #pragma unroll
-        for (int j = 0; j < RS; j++) { best[j] = low[j] = 0.f; key[j] = 0u; }
+        for (int j = 0; j < RS; j++) { best[j] = low[j] = point[j] = 0.f; key[j] = 0u; }
         int next_tile = t_end;
 #pragma unroll 1
         for (int ch = 0; ch < C; ch++) {
@@ -658,6 +736,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                             const float dl = v - other, du = __uint_as_float(en.y) - other;
                             best[j] = __builtin_fmaxf(__builtin_fmaxf(best[j], __builtin_fabsf(dl)), __builtin_fabsf(du));
                             low[j] = __builtin_fmaxf(__builtin_fmaxf(low[j], dl), -du);
+                            if constexpr (ALL) point[j] = __builtin_fmaxf(point[j], __builtin_fabsf(__uint_as_float(en.w) - other));
                         } else {
                             const float df = SECOND ? other - v : v - other;
                             if constexpr (MODE == kWithPos) {
@@ -698,11 +777,13 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
         for (int j = 0; j < RS / 2; j++) {
             swap(best[j], best[j + RS / 2]);
             if constexpr (BOX) swap(low[j], low[j + RS / 2]);
+            if constexpr (ALL) swap(point[j], point[j + RS / 2]);
             if constexpr (MODE == kWithPos) swap(key[j], key[j + RS / 2]);
         }
         if (EG > 1) {   // the groups of lanes that shared a row's list
             float* pa = reinterpret_cast<float*>(lds);
             unsigned* pb = reinterpret_cast<unsigned*>(lds + NT / 2 * RS * 4);
+            float* pc = reinterpret_cast<float*>(lds + NT * RS * 4);
             for (int half = EG / 2; half > 0; half /= 2) {
                 __syncthreads();
                 if (eg >= half && eg < 2 * half) {
@@ -710,6 +791,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                     for (int j = 0; j < RS; j++) {
                         pa[j * (NT / 2) + tid - half * LG] = best[j];
                         if constexpr (MODE != kOnlyValues) pb[j * (NT / 2) + tid - half * LG] = BOX ? __float_as_uint(low[j]) : key[j];
+                        if constexpr (ALL) pc[j * (NT / 2) + tid - half * LG] = point[j];
                     }
                 }
                 __syncthreads();
@@ -724,6 +806,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                         } else {
                             best[j] = __builtin_fmaxf(best[j], o);
                             if constexpr (BOX) low[j] = __builtin_fmaxf(low[j], __uint_as_float(pb[j * (NT / 2) + tid]));
+                            if constexpr (ALL) point[j] = __builtin_fmaxf(point[j], pc[j * (NT / 2) + tid]);
                         }
                     }
                 }
@@ -731,80 +814,115 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
         }
         auto pos_of = [&](int j) { return best[j] == 0.f ? 0 : (int)((key[j] >> 5) | (__float_as_uint(best[j]) & 0x80000000u)); };
         if (eg == 0 && wave_live) {
-            if constexpr (!SECOND) {
+            if (!last) {
                 if (live) {   // 16 * RS bytes of a row (8 * RS without positions): whole sectors, and all of a lane's in few stores
                     if constexpr (MODE == kOnlyValues) {
-                        float* to = s.partial + (size_t)l * s.pitch + s0;
-#pragma unroll
-                        for (int j = 0; j < RS; j += 4) *reinterpret_cast<F4*>(to + j) = F4{best[j], best[j + 1], best[j + 2], best[j + 3]};
+                        store_row(s.partial + (size_t)l * s.pitch + s0, best);
                     } else {
                         float* to = s.partial + 2 * ((size_t)l * s.pitch + s0);
                         auto second = [&](int j) { return BOX ? low[j] : __int_as_float(pos_of(j)); };
 #pragma unroll
                         for (int j = 0; j < RS; j += 2)
                             *reinterpret_cast<F4*>(to + 2 * j) = F4{__builtin_fabsf(best[j]), second(j), __builtin_fabsf(best[j + 1]), second(j + 1)};
+                        if constexpr (ALL) store_row(s.partial3 + (size_t)l * s.pitch + s0, point);
                     }
                 }
             } else {
-                float limit[RS], limit_low[RS];   // what neither list holds
+                float limit[RS], limit_low[RS], limit_point[RS];   // what neither list holds
 #pragma unroll
-                for (int j = 0; j < RS; j++) limit[j] = limit_low[j] = -kNever;
+                for (int j = 0; j < RS; j++) limit[j] = limit_low[j] = limit_point[j] = -kNever;
                 for (int ch = 0; ch < C; ch++) {
-                    const float* lr = ln.rest + (size_t)ch * 2 * ln.rows + l;
-                    const float lh = lr[0], ll = lr[ln.rows];
+                    const float* lr = ln.rest + (size_t)ch * ln.rests * ln.rows + l;
+                    constexpr int LL = BOX && !SECOND ? 2 : 0, SL = BOX && SECOND ? 2 : 0, LP = ALL ? 4 : 0;   // which of a side's, for lower bounds and points
+                    const float lh = lr[0], ll = lr[ln.rows], lh_low = lr[LL * ln.rows], ll_low = lr[(LL + 1) * ln.rows];
+                    const float lh_point = lr[LP * ln.rows], ll_point = lr[(LP + 1) * ln.rows];
 #pragma unroll
                     for (int j = 0; j < RS; j++) {
-                        const float* sr = sd.rest + (size_t)ch * (BOX ? 4 : 2) * sd.rows + min(s0 + j, sd.rows - 1);
+                        const float* sr = sd.rest + (size_t)ch * sd.rests * sd.rows + min(s0 + j, sd.rows - 1);
                         limit[j] = __builtin_fmaxf(limit[j], __builtin_fmaxf(sr[0] - ll, lh - sr[sd.rows]));
-                        if constexpr (BOX) limit_low[j] = __builtin_fmaxf(limit_low[j], __builtin_fmaxf(sr[2 * sd.rows] - ll, lh - sr[3 * sd.rows]));
+                        if constexpr (BOX) limit_low[j] = __builtin_fmaxf(limit_low[j], __builtin_fmaxf(sr[SL * sd.rows] - ll_low, lh_low - sr[(SL + 1) * sd.rows]));
+                        if constexpr (ALL) limit_point[j] = __builtin_fmaxf(limit_point[j], __builtin_fmaxf(sr[0] - ll_point, lh_point - sr[sd.rows]));
                     }
                 }
-                const float mu = s.mean ? s.mean[l] : 0.f, add = s.bias ? s.bias[l] : 0.f;   // before the stores, which they might alias
-                auto stored = [&](float v) {
-                    if (s.mean) v = v - mu;
-                    if (s.bias) v = v + add;
+                float mu[RS], add[RS];   // before the stores, which they might alias
+#pragma unroll
+                for (int j = 0; j < RS; j++) {
+                    const int n = SECOND ? l : min(s0 + j, N - 1);
+                    mu[j] = s.mean ? s.mean[n] : 0.f;
+                    add[j] = s.bias ? s.bias[n] : 0.f;
+                }
+                auto stored = [&](float v, int j) {
+                    if (s.mean) v = v - mu[j];
+                    if (s.bias) v = v + add[j];
                     return v;
                 };
                 unsigned failed = 0;
+                float got[RS], got_low[RS], got_point[RS];
+                int got_pos[RS];
 #pragma unroll
-                for (int j = 0; j < RS; j++)
-                    if (live && s0 + j < sd.rows) {
-                        const size_t o = (size_t)(s0 + j) * N + l;
-                        const size_t from = (size_t)(s0 + j) * s.pitch + l;   // what the first pass left
-                        float have = 0.f, with = 0.f;
+                for (int j = 0; j < RS; j++) {
+                    const size_t from = SECOND ? (size_t)min(s0 + j, sd.rows - 1) * s.pitch + l : 0;   // what the first pass left
+                    float have = 0.f, with = 0.f;
+                    if constexpr (SECOND) {
                         if constexpr (MODE == kOnlyValues) {
                             if (both) have = s.partial[from];
                         } else if (both) {
-                            const float2 both = reinterpret_cast<const float2*>(s.partial)[from];
-                            have = both.x;
-                            with = both.y;
-                        }
-                        // an infinite limit is a row that the lists cannot speak for, whatever they found
-                        if constexpr (BOX) {
-                            const float lo = __builtin_fmaxf(low[j], with), up = __builtin_fmaxf(best[j], have);
-                            if (up >= limit[j] && lo >= limit_low[j] && limit[j] < __builtin_inff()) {
-                                s.out[o] = stored(lo);
-                                s.out2[o] = stored(up);
-                            } else {
-                                failed |= 1u << j;
-                            }
-                        } else if constexpr (MODE == kOnlyValues) {
-                            const float v = __builtin_fmaxf(best[j], have);
-                            if (v >= limit[j] && limit[j] < __builtin_inff()) s.out[o] = stored(v);
-                            else failed |= 1u << j;
-                        } else {
-                            float v = __builtin_fabsf(best[j]);
-                            int p = pos_of(j);
-                            const int hp = __float_as_int(with);
-                            if (have > v || (have == v && (hp & 0x7fffffff) < (p & 0x7fffffff))) { v = have; p = hp; }
-                            if (v > limit[j]) {   // at the limit a lower k might hold the same value
-                                s.out[o] = stored(v);
-                                s.pos[o] = p;
-                            } else {
-                                failed |= 1u << j;
-                            }
+                            const float2 left = reinterpret_cast<const float2*>(s.partial)[from];
+                            have = left.x;
+                            with = left.y;
                         }
                     }
+                    // an infinite limit is a row that the lists cannot speak for, whatever they found
+                    bool settled;
+                    if constexpr (BOX) {
+                        const float lo = __builtin_fmaxf(low[j], with), up = __builtin_fmaxf(best[j], have);
+                        settled = up >= limit[j] && lo >= limit_low[j] && limit[j] < __builtin_inff();
+                        if constexpr (ALL) settled = settled && point[j] >= limit_point[j];
+                        got_low[j] = stored(lo, j);
+                        got[j] = stored(up, j);
+                        if constexpr (ALL) got_point[j] = stored(point[j], j);
+                    } else if constexpr (MODE == kOnlyValues) {
+                        const float v = __builtin_fmaxf(best[j], have);
+                        settled = v >= limit[j] && limit[j] < __builtin_inff();
+                        got[j] = stored(v, j);
+                    } else {
+                        float v = __builtin_fabsf(best[j]);
+                        int p = pos_of(j);
+                        const int hp = __float_as_int(with);
+                        if (have > v || (have == v && (hp & 0x7fffffff) < (p & 0x7fffffff))) { v = have; p = hp; }
+                        settled = v > limit[j];   // at the limit a lower k might hold the same value
+                        got[j] = stored(v, j);
+                        got_pos[j] = p;
+                    }
+                    if (live && s0 + j < sd.rows && !settled) failed |= 1u << j;
+                }
+                auto index = [&](int j) { return SECOND ? (s0 + j) * N + l : l * N + s0 + j; };
+                // all of them: what has failed is written again by a later launch
+                if (SECOND || s0 + RS > N) {
+#pragma unroll
+                    for (int j = 0; j < RS; j++)
+                        if (live && s0 + j < sd.rows) {
+                            const int o = index(j);
+                            if constexpr (BOX) {
+                                s.out[o] = got_low[j];
+                                s.out2[o] = got[j];
+                                if constexpr (ALL) s.out3[o] = got_point[j];
+                            } else {
+                                s.out[o] = got[j];
+                                if constexpr (MODE == kWithPos) s.pos[o] = got_pos[j];
+                            }
+                        }
+                } else if (live) {
+                    const int o = index(0);
+                    if constexpr (BOX) {
+                        store_row(s.out + o, got_low);
+                        store_row(s.out2 + o, got);
+                        if constexpr (ALL) store_row(s.out3 + o, got_point);
+                    } else {
+                        store_row(s.out + o, got);
+                        if constexpr (MODE == kWithPos) store_row(s.pos + o, got_pos);
+                    }
+                }
                 if (__ballot(failed != 0)) {
                     int n = 0;
 #pragma unroll
@@ -815,7 +933,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                     for (int j = 0; j < RS; j++) {
                         const unsigned long long m = __ballot(failed >> j & 1);
                         const int at = first + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-                        if ((failed >> j & 1) && at < s.walk_most) s.walk[at] = (s0 + j) * N + l;   // more: the full walk follows
+                        if ((failed >> j & 1) && at < s.walk_most) s.walk[at] = index(j);   // more: the full walk follows
                         first += __builtin_popcountll(m);
                     }
                 }
@@ -842,33 +960,43 @@ __global__ void __launch_bounds__(256) extremes_walk_kernel(Search s) {
         const int o = __builtin_amdgcn_readfirstlane(s.walk[i]);
         const float* xr = s.x.v + (size_t)(o / N) * K;
         const float* wr = s.w.v + (size_t)(o % N) * K;
-        if constexpr (MODE == kBoxes) {
+        if constexpr (MODE == kBoxes || MODE == kBoxesAndPoints) {
+            constexpr bool ALL = MODE == kBoxesAndPoints;
             const float* ur = s.x.v2 + (size_t)(o / N) * K;
-            float up = 0.f, lo = 0.f;
+            const float* pr = ALL ? s.x.v3 + (size_t)(o / N) * K : nullptr;
+            float up = 0.f, lo = 0.f, point = 0.f;
             auto one = [&](float x, float u, float w) {
                 const float tl = x - w, tu = u - w, al = __builtin_fabsf(tl), au = __builtin_fabsf(tu);
                 up = __builtin_fmaxf(up, __builtin_fmaxf(al, au));
                 if (!(tl < 0.f && tu > 0.f)) lo = __builtin_fmaxf(lo, __builtin_fminf(al, au));
             };
             for (int kb = 0; kb < K; kb += 256 * 4) {
-                float4_any x[4], u[4], w[4];
+                float4_any x[4], u[4], w[4], p[4];
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
                     const int k = min(kb + c * 256 + lane * 4, K - 4);   // the last vector is moved back, those past the end repeat it
                     x[c] = *reinterpret_cast<const float4_any*>(xr + k);
                     u[c] = *reinterpret_cast<const float4_any*>(ur + k);
+                    if constexpr (ALL) p[c] = *reinterpret_cast<const float4_any*>(pr + k);
                     w[c] = *reinterpret_cast<const float4_any*>(wr + k);
                 }
 #pragma unroll
                 for (int c = 0; c < 4; c++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) one(x[c].v[e], u[c].v[e], w[c].v[e]);
+                    for (int e = 0; e < 4; e++) {
+                        one(x[c].v[e], u[c].v[e], w[c].v[e]);
+                        if constexpr (ALL) point = __builtin_fmaxf(point, __builtin_fabsf(p[c].v[e] - w[c].v[e]));
+                    }
             }
             up = wave_max(up);
             lo = wave_max(lo);
             if (lane == 63) {
                 s.out[o] = shifted_value(s.mean, s.bias, o % N, lo);
                 s.out2[o] = shifted_value(s.mean, s.bias, o % N, up);
+            }
+            if constexpr (ALL) {
+                point = wave_max(point);
+                if (lane == 63) s.out3[o] = shifted_value(s.mean, s.bias, o % N, point);
             }
         } else {
             float v = 0.f;
@@ -908,14 +1036,17 @@ namespace {
 
 struct Layout {
     int C, KC, mb, nb, pitch;
-    size_t counts, reach, partial, walk, x_lists, w_lists, x_rest, w_rest, total;   // byte offsets in the workspace
+    size_t counts, reach, partial, partial3, walk, x_lists, w_lists, x_rest, w_rest, total;   // byte offsets in the workspace
 };
 
 // More outputs than these go to the full walk; forced lists have none after them.
-int walk_most(const Problem& pr) { return g_extremes > 0 ? pr.B * pr.NG : pr.B * pr.NG / 16; }
+size_t walk_most(const Problem& pr, ForwardKind kind) {   // the two second scans of boxes and points may both note an output
+    const size_t outputs = (size_t)pr.B * pr.NG;
+    return g_extremes > 0 ? (kind == ForwardKind::kValueBounds ? 2 : 1) * outputs : outputs / 16;
+}
 
 Layout layout_of(const Problem& pr, ForwardKind kind) {
-    const bool boxes = kind == ForwardKind::kBounds;
+    const bool all = kind == ForwardKind::kValueBounds, boxes = kind == ForwardKind::kBounds || all;
     Layout l{};
     l.C = (pr.K + kMaxChunk - 1) / kMaxChunk;
     l.KC = ((pr.K + l.C - 1) / l.C + 63) / 64 * 64;
@@ -927,11 +1058,12 @@ Layout layout_of(const Problem& pr, ForwardKind kind) {
     l.counts = take((size_t)kSampleGroups * kSampleGroups * 64);
     l.pitch = (pr.NG + 7) / 8 * 8;
     l.partial = take((size_t)pr.B * l.pitch * (kind == ForwardKind::kValues ? 1 : 2) * sizeof(float));
-    l.walk = take((size_t)walk_most(pr) * sizeof(int));
+    l.partial3 = take(all ? (size_t)pr.B * l.pitch * sizeof(float) : 0);
+    l.walk = take(walk_most(pr, kind) * sizeof(int));
     l.reach = take(2 * 8 * kSampled * sizeof(float));
     l.x_lists = take((size_t)l.C * l.mb * kMaxList * 16 * (boxes ? 16 : 8));
     l.w_lists = take((size_t)l.C * l.nb * kMaxList * 16 * 8);
-    l.x_rest = take((size_t)l.C * (boxes ? 4 : 2) * pr.B * sizeof(float));
+    l.x_rest = take((size_t)l.C * (all ? 6 : boxes ? 4 : 2) * pr.B * sizeof(float));
     l.w_rest = take((size_t)l.C * 2 * pr.NG * sizeof(float));
     l.total = at;
     return l;
@@ -941,7 +1073,8 @@ template <int MODE, bool SECOND>
 hipError_t launch_scan(const Search& s, const Problem& pr, hipStream_t stream) {
     auto kern = extremes_scan_kernel<MODE, SECOND>;
     static LdsRecord allowed = {};
-    const size_t strip = (size_t)s.KC * 32, lds = strip > 16384 ? strip : 16384;   // the strip, or what the groups of lanes hand over
+    const size_t strip = (size_t)s.KC * 32, over = MODE == kBoxesAndPoints ? 24576 : 16384;   // the strip, or what the groups of lanes hand over
+    const size_t lds = strip > over ? strip : over;
     if (hipError_t e = allow_lds(kern, (size_t)kMaxChunk * 32, pr.device, allowed); e != hipSuccess) return e;
     const Side &ln = SECOND ? s.w : s.x, &sd = SECOND ? s.x : s.w;
     const int rows = strip_rows(MODE == kBoxes && SECOND), lanes = SECOND ? s.lanes_second : s.lanes_first;
@@ -952,15 +1085,15 @@ hipError_t launch_scan(const Search& s, const Problem& pr, hipStream_t stream) {
     return hipGetLastError();
 }
 
-template <bool PAIR>
+template <int ENDS>
 hipError_t launch_lists(const Search& s, hipStream_t stream) {
-    const unsigned grid = (unsigned)(s.C * (s.x.blocks + s.w.blocks));
-    const size_t stage = (size_t)kMaxList * 16 * (PAIR ? 16 : 8);
+    const unsigned grid = (unsigned)(2 * s.C * (s.x.blocks + s.w.blocks));
+    const size_t stage = (size_t)kMaxList * 8 * (ENDS > 1 ? 16 : 8);
 #define LISTS(NV)                                                                                                                 \
     do {                                                                                                                          \
-        hipLaunchKernelGGL((extremes_sample_kernel<NV, PAIR>), dim3(kSampleGroups * kSampleGroups), dim3(1024), 0, stream, s);     \
+        hipLaunchKernelGGL((extremes_sample_kernel<NV, ENDS>), dim3(kSampleGroups * kSampleGroups), dim3(1024), 0, stream, s);     \
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;                                                          \
-        hipLaunchKernelGGL((extremes_select_kernel<NV, PAIR>), dim3(grid), dim3(512), stage, stream, s);                          \
+        hipLaunchKernelGGL((extremes_select_kernel<NV, ENDS>), dim3(grid), dim3(512), stage, stream, s);                          \
     } while (0)
     if (s.KC <= 1024) LISTS(16);
     else if (s.KC <= 1536) LISTS(24);
@@ -992,7 +1125,8 @@ int lanes_for(int rows, int strips, int num_cu) {
 static bool lists_pay(const Problem& pr, ForwardKind kind) {
     if (g_tile_override >= 0 || pr.K < 512) return false;
     const double outputs = (double)pr.B * pr.NG, weights = (double)pr.NG * pr.K;
-    const bool boxes = kind == ForwardKind::kBounds;
+    const bool boxes = kind != ForwardKind::kInf && kind != ForwardKind::kValues;   // with points: where the boxes alone pay
+    if (boxes) kind = ForwardKind::kBounds;
     const double beyond_one = std::max(0, pr.K - kMaxChunk), beyond_two = std::max(0, pr.K - 2 * kMaxChunk);
     const double us = (boxes ? 65 : 55) + 2.1e-6 * weights + (boxes ? 5.3e-5 : 3.5e-5) * outputs +
                       (boxes ? 3.4e-6 : 1.1e-6) * pr.B * beyond_one + (3.3e-3 + (boxes ? 5.4e-9 : 4.2e-9) * outputs) * beyond_two;
@@ -1006,6 +1140,7 @@ constexpr size_t kScratchMost = (size_t)256 << 20;
 constexpr int kFewestRows = 256;
 static int rows_at_once(const Problem& pr, ForwardKind kind) {
     if (g_extremes == 0 || pr.HW != 1 || pr.G != 1 || pr.NG <= 16 || pr.K < 4 || pr.K > 16 * kMaxChunk) return 0;
+    if (kind == ForwardKind::kValueBounds && pr.K % 4 != 0) return 0;   // no full walk of values to follow
     Problem part = pr;
     for (int shares = 1;; shares++) {
         part.B = shares == 1 ? pr.B : ((pr.B + shares - 1) / shares + 15) / 16 * 16;
@@ -1023,39 +1158,60 @@ size_t extremes_workspace(const Problem& pr, ForwardKind kind, int& rows) {
     return layout_of(part, kind).total;
 }
 
-hipError_t extremes_forward(const float* x, const float* x2, const float* w, float* out, float* out2, int32_t* pos, void* workspace,
-                            const Problem& pr, hipStream_t stream, const int** gate) {
-    const bool boxes = x2 != nullptr;
-    const Layout l = layout_of(pr, boxes ? ForwardKind::kBounds : pos ? ForwardKind::kInf : ForwardKind::kValues);
+hipError_t extremes_forward(const float* x, const float* x2, const float* x3, const float* w, float* out, float* out2, float* out3,
+                            int32_t* pos, void* workspace, const Problem& pr, hipStream_t stream, const int** gate) {
+    const bool all = x3 != nullptr, boxes = x2 != nullptr;
+    const ForwardKind kind = all ? ForwardKind::kValueBounds : boxes ? ForwardKind::kBounds : pos ? ForwardKind::kInf : ForwardKind::kValues;
+    const Layout l = layout_of(pr, kind);
     char* ws = static_cast<char*>(workspace);
     Search s{};
     s.head = reinterpret_cast<Header*>(ws);
     s.counts = reinterpret_cast<unsigned char*>(ws + l.counts);
     s.reach = reinterpret_cast<float*>(ws + l.reach);
     s.partial = reinterpret_cast<float*>(ws + l.partial);
+    s.partial3 = reinterpret_cast<float*>(ws + l.partial3);
     s.pitch = l.pitch;
     s.walk = reinterpret_cast<int*>(ws + l.walk);
-    s.walk_most = walk_most(pr);
-    s.x = Side{x, x2, pr.B, l.mb, ws + l.x_lists, reinterpret_cast<float*>(ws + l.x_rest)};
-    s.w = Side{w, nullptr, pr.NG, l.nb, ws + l.w_lists, reinterpret_cast<float*>(ws + l.w_rest)};
-    s.out = out; s.out2 = out2; s.pos = pos;
+    s.walk_most = (int)std::min<size_t>(walk_most(pr, kind), INT32_MAX);
+    s.x = Side{x, x2, x3, pr.B, l.mb, ws + l.x_lists, reinterpret_cast<float*>(ws + l.x_rest), all ? 6 : boxes ? 4 : 2};
+    s.w = Side{w, nullptr, nullptr, pr.NG, l.nb, ws + l.w_lists, reinterpret_cast<float*>(ws + l.w_rest), 2};
+    s.out = out; s.out2 = out2; s.out3 = out3; s.pos = pos;
     s.mean = pr.mean; s.bias = pr.bias;
     s.K = pr.K; s.C = l.C; s.KC = l.KC;
     s.lanes_first = lanes_for(pr.B, (pr.NG + 7) / 8, pr.num_cu);
     const int second_rows = strip_rows(boxes);
     s.lanes_second = lanes_for(pr.NG, (pr.B + second_rows - 1) / second_rows, pr.num_cu);
     s.price_x = 1.f;
-    s.price_w = boxes ? 2.f : 1.f;
-    s.price_fail = 6.f * pr.K;   // in list entries of one row: a walked output reads two rows, 3 ns with all waves at it, an entry 0.1 ps per output
-    s.price_dense = g_extremes > 0 ? 3e38f : (boxes ? 0.5f : 0.2f) * pr.K;
+    s.price_w = all ? 3.f : boxes ? 2.f : 1.f;
+    s.price_both = all ? 120.f : 60.f;
+    // in list entries of one row: a walked output reads two rows, 3 ns with all waves at it, an entry takes 0.1 ps per output; with
+    // points four rows, mostly twice, 20 ns, and 0.2 ps
+    s.price_fail = (all ? 18.f : boxes ? 9.f : 6.f) * pr.K;
+    s.price_dense = g_extremes > 0 ? 3e38f : (all ? 0.7f : boxes ? 0.5f : 0.2f) * pr.K;
     *gate = &s.head->full;
-    if (hipError_t e = boxes ? launch_lists<true>(s, stream) : launch_lists<false>(s, stream); e != hipSuccess) return e;
+    if (hipError_t e = all ? launch_lists<3>(s, stream) : boxes ? launch_lists<2>(s, stream) : launch_lists<1>(s, stream); e != hipSuccess) return e;
+    auto walk = [&](auto mode) {
+        hipLaunchKernelGGL(extremes_walk_kernel<decltype(mode)::value>, dim3(4 * pr.num_cu), dim3(256), 0, stream, s);
+        return hipGetLastError();
+    };
+    auto second_of = [&](int turn) { Search t = s; t.turn = turn; return t; };
+    if (all) {
+        if (hipError_t e = launch_scan<kBoxesAndPoints, false>(s, pr, stream); e != hipSuccess) return e;
+        if (hipError_t e = launch_scan<kBoxes, true>(second_of(1), pr, stream); e != hipSuccess) return e;
+        Search points = second_of(2);
+        points.x.v = x3;
+        points.x.rest = s.x.rest + (size_t)4 * pr.B;
+        points.out = out3;
+        points.partial = s.partial3;
+        points.lanes_second = lanes_for(pr.NG, (pr.B + 7) / 8, pr.num_cu);
+        if (hipError_t e = launch_scan<kOnlyValues, true>(points, pr, stream); e != hipSuccess) return e;
+        return walk(std::integral_constant<int, kBoxesAndPoints>{});
+    }
 #define SCANS(MODE)                                                                                                       \
     do {                                                                                                                  \
         if (hipError_t e = launch_scan<MODE, false>(s, pr, stream); e != hipSuccess) return e;                   \
-        if (hipError_t e = launch_scan<MODE, true>(s, pr, stream); e != hipSuccess) return e;                    \
-        hipLaunchKernelGGL(extremes_walk_kernel<MODE>, dim3(4 * pr.num_cu), dim3(256), 0, stream, s);                     \
-        return hipGetLastError();                                                                                         \
+        if (hipError_t e = launch_scan<MODE, true>(second_of(1), pr, stream); e != hipSuccess) return e;         \
+        return walk(std::integral_constant<int, MODE>{});                                                                 \
     } while (0)
     if (boxes) SCANS(kBoxes);
     if (pos) SCANS(kWithPos);

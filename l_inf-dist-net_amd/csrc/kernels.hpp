@@ -70,14 +70,15 @@ inline hipError_t allow_lds(Kern kern, size_t bytes, int device, LdsRecord& done
     return e;
 }
 
-enum class ForwardKind { kInf, kValues, kBounds, kNorm };
+enum class ForwardKind { kInf, kValues, kBounds, kNorm, kValueBounds };   // the last: of extremes_workspace only
 // Large fully connected layers: only the differences that can be the maximum (extremes_forward.hip).  The size of its
 // workspace, 0 where the layer is not one of them, and how many rows it is good for: more take several calls.  The launches,
 // for that many rows at most, which leave *gate != 0 on the device where the full walk of them has to follow.  `x2`: the upper
-// ends of boxes, nullptr for distances; pos == nullptr: values only.
+// ends of boxes, nullptr for distances; `x3`, `out3`: points inside the boxes and their distances, or nullptr; pos == nullptr:
+// values only.
 size_t extremes_workspace(const Problem& pr, ForwardKind kind, int& rows);
-hipError_t extremes_forward(const float* x, const float* x2, const float* w, float* out, float* out2, int32_t* pos, void* workspace,
-                            const Problem& pr, hipStream_t stream, const int** gate);
+hipError_t extremes_forward(const float* x, const float* x2, const float* x3, const float* w, float* out, float* out2, float* out3,
+                            int32_t* pos, void* workspace, const Problem& pr, hipStream_t stream, const int** gate);
 hipError_t inf_forward(const float* input, const float* weight, float* output, int32_t* pos, const Problem& pr,
                        hipStream_t stream);
 // Values without pos, for forward passes that no gradient follows (inf_forward.hip); the fc layout with 128-bit loads.

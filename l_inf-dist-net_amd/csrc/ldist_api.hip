@@ -82,8 +82,8 @@ int conv_geometry(int B, int C, int H, int W, int KH, int KW, int stride, int pa
 // The workspace forms of the forward passes: the lists, then the full walk where the lists were not worth it, for as many rows
 // at a time as the workspace is for.  full(part, in, at): the full walk of such a part, whose inputs and outputs begin there.
 template <class FULL>
-int extremes_entry(const float* x, const float* x2, const float* w, const ldist::Problem& pr, ldist::ForwardKind kind,
-                          float* out, float* out2, int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream, FULL&& full) {
+int extremes_entry(const float* x, const float* x2, const float* x3, const float* w, const ldist::Problem& pr, ldist::ForwardKind kind,
+                          float* out, float* out2, float* out3, int32_t* pos, void* workspace, int64_t bytes, ldist_stream_t stream, FULL&& full) {
     int rows;
     const size_t need = ldist::extremes_workspace(pr, kind, rows);
     if (need == 0) return LDIST_EUNSUPPORTED;
@@ -92,8 +92,8 @@ int extremes_entry(const float* x, const float* x2, const float* w, const ldist:
         ldist::Problem part = pr;
         part.B = first + rows < pr.B ? rows : (int)(pr.B - first);
         const size_t in = (size_t)first * pr.K, at = (size_t)first * pr.NG;
-        hipError_t e = ldist::extremes_forward(x + in, x2 ? x2 + in : nullptr, w, out + at, out2 ? out2 + at : nullptr,
-                                               pos ? pos + at : nullptr, workspace, part, (hipStream_t)stream, &part.gate);
+        hipError_t e = ldist::extremes_forward(x + in, x2 ? x2 + in : nullptr, x3 ? x3 + in : nullptr, w, out + at,
+                                               out2 ? out2 + at : nullptr, out3 ? out3 + at : nullptr, pos ? pos + at : nullptr, workspace, part, (hipStream_t)stream, &part.gate);
         if (e == hipSuccess && ldist::g_extremes <= 0) e = full(part, in, at);
         if (int rc = finish(e)) return rc;
     }
@@ -103,7 +103,7 @@ int extremes_entry(const float* x, const float* x2, const float* w, const ldist:
 // Distances, without pos: values only.
 int distances_entry(const float* x, const float* w, const ldist::Problem& pr, float* out, int32_t* pos, void* workspace,
                            int64_t bytes, ldist_stream_t stream) {
-    return extremes_entry(x, nullptr, w, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues, out, nullptr, pos,
+    return extremes_entry(x, nullptr, nullptr, w, pr, pos ? ldist::ForwardKind::kInf : ldist::ForwardKind::kValues, out, nullptr, nullptr, pos,
                           workspace, bytes, stream, [&](const ldist::Problem& part, size_t in, size_t at) {
                               return pos ? ldist::inf_forward(x + in, w, out + at, pos + at, part, (hipStream_t)stream)
                                          : ldist::inf_forward_values(x + in, w, out + at, part, (hipStream_t)stream);
@@ -112,7 +112,7 @@ int distances_entry(const float* x, const float* w, const ldist::Problem& pr, fl
 
 int bounds_entry(const float* lower, const float* upper, const float* w, const ldist::Problem& pr, float* out_lower,
                         float* out_upper, void* workspace, int64_t bytes, ldist_stream_t stream) {
-    return extremes_entry(lower, upper, w, pr, ldist::ForwardKind::kBounds, out_lower, out_upper, nullptr, workspace, bytes, stream,
+    return extremes_entry(lower, upper, nullptr, w, pr, ldist::ForwardKind::kBounds, out_lower, out_upper, nullptr, nullptr, workspace, bytes, stream,
                           [&](const ldist::Problem& part, size_t in, size_t at) {
                               return ldist::bound_forward(lower + in, upper + in, w, out_lower + at, out_upper + at, part,
                                                           (hipStream_t)stream);
@@ -268,6 +268,37 @@ int ldist_inf_dist_value_bound_forward(const float* input, const float* input_lo
     if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
     return finish(ldist::value_bound_forward(input, input_lower, input_upper, weight, mean, bias, output, output_lower,
                                              output_upper, pr, (hipStream_t)stream));
+}
+
+int ldist_inf_dist_value_bound_workspace(int B, int CO, int CI, int G, int HW, int64_t* bytes) {
+    if (!bytes) return LDIST_EINVAL;
+    *bytes = 0;
+    ldist::Problem pr{};
+    if (int rc = check_sizes(B, CO, CI, G, HW, pr)) return rc;
+    int rows;
+    *bytes = (int64_t)ldist::extremes_workspace(pr, ldist::ForwardKind::kValueBounds, rows);
+    return LDIST_OK;
+}
+
+int ldist_inf_dist_value_bound_forward_ws(const float* input, const float* input_lower, const float* input_upper,
+                                          const float* weight, int B, int CO, int CI, int G, int HW, const float* mean,
+                                          const float* bias, float* output, float* output_lower, float* output_upper,
+                                          void* workspace, int64_t bytes, ldist_stream_t stream) {
+    if (!input || !input_lower || !input_upper || !weight || !output || !output_lower || !output_upper || !workspace)
+        return LDIST_EINVAL;
+    ldist::Problem pr{};
+    if (int rc = check_dims(B, CO, CI, G, HW, pr)) return rc;
+    if (HW != 1 || G != 1 || !ldist::inf_forward_values_applicable(pr, input, weight)) return LDIST_EUNSUPPORTED;
+    pr.mean = mean;
+    pr.bias = bias;
+    return extremes_entry(input_lower, input_upper, input, weight, pr, ldist::ForwardKind::kValueBounds, output_lower, output_upper,
+                          output, nullptr, workspace, bytes, stream, [&](const ldist::Problem& part, size_t in, size_t at) {
+                              if (hipError_t e = ldist::bound_forward(input_lower + in, input_upper + in, weight, output_lower + at,
+                                                                      output_upper + at, part, (hipStream_t)stream);
+                                  e != hipSuccess)
+                                  return e;
+                              return ldist::inf_forward_values(input + in, weight, output + at, part, (hipStream_t)stream);
+                          });
 }
 
 static int inf_backward_input_impl(const float* grad_output, const int32_t* pos, int B, int CO, int CI, int G,

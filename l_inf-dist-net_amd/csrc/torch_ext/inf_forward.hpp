@@ -8,15 +8,20 @@
 
 namespace ldist_torch {
 
-// Undefined where the layer has no form with a workspace, and where there is no memory for one: the plain entry points need none.
-inline torch::Tensor workspace(int B, int CO, int CI, int G, int HW, int what, const torch::Tensor& like) {
-    int64_t bytes = 0;
-    if (ldist_inf_dist_workspace(B, CO, CI, G, HW, what, &bytes) != LDIST_OK || bytes == 0) return torch::Tensor();
+// Undefined for no bytes, and where there is no memory for them: the plain entry points need none.
+inline torch::Tensor scratch(int64_t bytes, const torch::Tensor& like) {
+    if (bytes == 0) return torch::Tensor();
     try {
         return torch::empty({bytes}, like.options().dtype(torch::kUInt8).requires_grad(false));
     } catch (const c10::OutOfMemoryError&) {
         return torch::Tensor();
     }
+}
+
+// Undefined also where the layer has no form with a workspace.
+inline torch::Tensor workspace(int B, int CO, int CI, int G, int HW, int what, const torch::Tensor& like) {
+    int64_t bytes = 0;
+    return ldist_inf_dist_workspace(B, CO, CI, G, HW, what, &bytes) == LDIST_OK ? scratch(bytes, like) : torch::Tensor();
 }
 
 // The same with the evaluation-mode shift and bias (either may be null) applied by the forward kernel; fully connected layers.

@@ -10,6 +10,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <climits>
 #include <cmath>
 #include <string>
 #include <tuple>
@@ -586,7 +587,13 @@ std::tuple<Tensor, Tensor, bool> layer_bounds(const Tensor& lower, const Tensor&
     return {as_output(lo, lower, win), as_output(hi, lower, win), from_image};
 }
 
-// Values and bounds in one pass, for layers without a window and with few outputs.
+// Whether `layer_value_bounds` has one pass for a wide layer on B rows: one that the lists of outermost values are for.
+bool value_bounds_pay(int64_t B, int64_t CO, int64_t CI, int64_t G) {
+    int64_t bytes = 0;
+    return B <= INT_MAX && ldist_inf_dist_value_bound_workspace((int)B, (int)CO, (int)CI, (int)G, 1, &bytes) == LDIST_OK && bytes > 0;
+}
+
+// Values and bounds in one pass, for layers without a window: those with few outputs, and those of `value_bounds_pay`.
 std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Tensor& lower, const Tensor& upper,
                                                       const Tensor& weight, const OptTensor& bias, const OptTensor& running,
                                                       int64_t G) {
@@ -601,11 +608,28 @@ std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Ten
     TORCH_CHECK(cl.sizes() == cx.sizes() && cu.sizes() == cx.sizes(), "input_lower and input_upper must match input");
     const On on(cx);
     const Sizes s = sizes_of(cx, w, G);
-    Tensor y = torch::empty(s.output(), cx.options()), lo = torch::empty_like(y), hi = torch::empty_like(y);
-    done("inf_dist_value_bound_forward",
-         ldist_inf_dist_value_bound_forward(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G, s.HW, in(running), in(bias),
-                                            out(y), out(lo), out(hi), on.stream));
     const Window win{1, 1, 0, 1};
+    int64_t bytes = 0;
+    done("inf_dist_value_bound_workspace", ldist_inf_dist_value_bound_workspace(s.B, s.CO, s.CI, (int)G, s.HW, &bytes));
+    Tensor y = torch::empty(s.output(), cx.options()), lo = torch::empty_like(y), hi = torch::empty_like(y);
+    if (bytes == 0) {
+        done("inf_dist_value_bound_forward",
+             ldist_inf_dist_value_bound_forward(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G, s.HW, in(running), in(bias),
+                                                out(y), out(lo), out(hi), on.stream));
+    } else {
+        const Tensor ws = ldist_torch::scratch(bytes, cx);
+        const int rc = !ws.defined() ? LDIST_EUNSUPPORTED
+                                     : ldist_inf_dist_value_bound_forward_ws(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G,
+                                                                             s.HW, in(running), in(bias), out(y), out(lo), out(hi),
+                                                                             ws.data_ptr(), ws.numel(), on.stream);
+        if (rc == LDIST_EUNSUPPORTED) {   // no memory for it, or no 128-bit loads: one pass after the other
+            const Shift shift = make_shift(running, 0.0, false, cx.device());
+            y = distances(on, cx, w, G, INFINITY, bias, shift);
+            std::tie(lo, hi) = bounds_of_columns(cl, cu, w, G, bias, shift);
+        } else {
+            done("inf_dist_value_bound_forward", rc);
+        }
+    }
     return {as_output(y, x, win), as_output(lo, x, win), as_output(hi, x, win)};
 }
 
@@ -688,6 +712,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("layer", &layer, no_lock());
     m.def("layer_bounds", &layer_bounds, no_lock());
     m.def("layer_value_bounds", &layer_value_bounds, no_lock());
+    m.def("value_bounds_pay", &value_bounds_pay, no_lock());
     m.def("margins", &margins, no_lock());
     m.def("pgd_step", &pgd_step, no_lock());
     m.def("adamw_step", &adamw_step, no_lock());

@@ -143,9 +143,14 @@ def norm_dist_backward_ordered(grad_output, input, weight, output, grad_input, g
 
 def _with_workspace(name, what, sizes, dev, args):
     """Calls the form `name` of a forward pass that takes scratch memory, where the library has one for the layer and there is
-    memory for it; False elsewhere: the plain entry point is the way.  `args`: pointers before and after the sizes."""
+    memory for it; False elsewhere: the plain entry point is the way.  `what`: of ldist_inf_dist_workspace, None for values
+    and bounds.  `args`: pointers before and after the sizes."""
     need = ctypes.c_int64()
-    if _lib.lib().ldist_inf_dist_workspace(*sizes, what, ctypes.byref(need)) != 0 or need.value == 0:   # asks no device
+    if what is None:
+        rc = _lib.lib().ldist_inf_dist_value_bound_workspace(*sizes, ctypes.byref(need))
+    else:
+        rc = _lib.lib().ldist_inf_dist_workspace(*sizes, what, ctypes.byref(need))
+    if rc != 0 or need.value == 0:   # asks no device
         return False
     with torch.cuda.device(dev):
         try:
@@ -236,9 +241,11 @@ def inf_dist_value_bound_forward(input, input_lower, input_upper, weight, output
     _expect(weight.size(0) == CO and weight.size(1) * G == CI, "weight must be (CO, CI/G)")
     for t in (output, output_lower, output_upper):
         _expect(tuple(t.shape) == (B, CO, HW), "outputs must be (B, CO, HW)")
-    _call("ldist_inf_dist_value_bound_forward", dev, _p(input), _p(input_lower), _p(input_upper), _p(weight), B, CO, CI,
-          G, HW, _p(mean) if mean is not None else None, _p(bias) if bias is not None else None, _p(output),
-          _p(output_lower), _p(output_upper))
+    before = (_p(input), _p(input_lower), _p(input_upper), _p(weight))
+    after = (_p(mean) if mean is not None else None, _p(bias) if bias is not None else None, _p(output), _p(output_lower),
+             _p(output_upper))
+    if not _with_workspace("ldist_inf_dist_value_bound_forward_ws", None, (B, CO, CI, G, HW), dev, (before, after)):
+        _call("ldist_inf_dist_value_bound_forward", dev, *before, B, CO, CI, G, HW, *after)
 
 
 def _inf_backward_input(name, grad_output, pos, grad_input, G):
