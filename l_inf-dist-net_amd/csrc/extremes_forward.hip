@@ -391,39 +391,37 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
     dense = __builtin_amdgcn_readfirstlane(cost > s.price_dense ? 1 : 0);
 }
 
-// A workgroup makes the lists of eight rows in one chunk, a wave that of a row (with two rows per wave the last workgroups ran
-// alone for half of the time): all values beyond `t` from the center,
+// Resident workgroups take eight rows of a chunk at a time, a wave that of a row: all values beyond `t` from the center,
 // where t starts as what the sampled rows needed on the average and is moved where the list would overflow or stay half empty
 // (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly,
 // unless more values tie at the outer end than the list has places: such a row's bounds are those of all its values.
 // Bound by reading the operands once.
 template <int NV, int ENDS>
-__global__ void __launch_bounds__(512, ENDS > 1 ? 4 : 5) extremes_select_kernel(Search s) {
-    extern __shared__ __align__(16) char stage[];   // [entry][8]: half of a block of Side::lists
+__global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_select_kernel(Search s) {
+    extern __shared__ __align__(16) char stage[];   // [2 kMaxList][8] entries: half of a block of Side::lists, and what `place` finds no place for
     __shared__ int sums[8][64];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int per = 2 * (s.x.blocks + s.w.blocks), ch = blockIdx.x / per;
-    int block = blockIdx.x % per;
-    const bool of_x = block < 2 * s.x.blocks;
-    const Side& side = of_x ? s.x : s.w;
-    if (!of_x) block -= 2 * s.x.blocks;
-    const int k0 = ch * s.KC, r = block * 8 + wave, row = __builtin_amdgcn_readfirstlane(min(r, side.rows - 1));
-
-    auto lists = [&](auto ends) {
-        constexpr bool P = decltype(ends)::value >= 2, ALL = decltype(ends)::value == 3;
-        RowChunk<NV> a;
-        const int kc = min(s.KC, s.K - k0), lane = tid & 63;
-        a.load(side.v + (size_t)row * s.K + k0, kc, lane);
-        int ix, iw, dense;
-        choose_lengths(s, sums, wave, lane, ix, iw, dense);
-        const int q = kLengths[of_x ? ix : iw];
-        if (blockIdx.x == 0 && tid == 0) { s.head->qx = kLengths[ix]; s.head->qw = kLengths[iw]; s.head->dense = s.head->full = dense; }
-        if (dense) return;
-        const float center = s.head->center;
-        float guess = s.reach[((of_x ? 0 : 1) * 8 + (of_x ? ix : iw)) * kSampled + lane];
+    int ix, iw, dense;
+    choose_lengths(s, sums, wave, tid & 63, ix, iw, dense);
+    if (blockIdx.x == 0 && tid == 0) { s.head->qx = kLengths[ix]; s.head->qw = kLengths[iw]; s.head->dense = s.head->full = dense; }
+    if (dense) return;
+    const float center = s.head->center;
+    auto needed = [&](int i) {   // by the sampled rows on the average
+        float sum = s.reach[i * kSampled + (tid & 63)];
 #pragma unroll
-        for (int o = 32; o; o >>= 1) guess += __shfl_xor(guess, o);
-        guess = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(guess * (1.f / kSampled))));
+        for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
+        return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sum * (1.f / kSampled))));
+    };
+    const float guess_x = needed(ix), guess_w = needed(8 + iw);
+
+    auto lists = [&](auto ends, const Side& side, int q, float guess, int ch, int block) {
+        constexpr bool P = decltype(ends)::value >= 2, ALL = decltype(ends)::value == 3;
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));   // what is derived from it is made where it is used, not kept in registers over the loop
+        const int k0 = ch * s.KC, r = block * 8 + wave, row = __builtin_amdgcn_readfirstlane(min(r, side.rows - 1));
+        RowChunk<NV> a;
+        const int kc = min(s.KC, s.K - k0);
+        a.load(side.v + (size_t)row * s.K + k0, kc, lane);
         // twice the middle of a box, where values are compared by themselves
         constexpr float F = P ? 2.f : 1.f;
         if constexpr (!P) a.center_past(kc, lane, center);
@@ -490,11 +488,28 @@ __global__ void __launch_bounds__(512, ENDS > 1 ? 4 : 5) extremes_select_kernel(
         struct Ends { float a, b, c; } first = {};
         int base = 0;
         float most = -kNever, least = kNever, most_lower = -kNever, least_upper = kNever, most_point = -kNever, least_point = kNever;
+        // Without positions the order of a list is free: entry s of row r is one with k = s + r / 2 (mod 8) where the row has such
+        // an entry left, so that 16 neighbouring lanes of a scan read from different banks.
+        const bool spread = s.pos == nullptr;
+        int of_class = 0, over = 0;   // entries with this lane's k mod 8; those beyond an eighth of the list, behind it in `stage`
+        auto before = [](unsigned long long m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0)); };
         auto place = [&](bool in, int j, auto&& write) {
             const unsigned long long m = __ballot(in);
             if (m) {
-                const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-                if (in && at < q) write(at * 8 + wave, (unsigned)(lane + j * 64) * 32u);
+                int at;
+                if (spread) {
+                    const unsigned long long mine = m & (0x0101010101010101ull << (lane & 7));
+                    const int rank = of_class + before(mine);
+                    const unsigned long long beyond = __ballot(in && rank >= q / 8);
+                    at = rank >= q / 8 ? kMaxList + min(over + before(beyond), q) : rank * 8 + ((lane - (r >> 1)) & 7);
+                    in = in && at < kMaxList + q;
+                    over += __builtin_popcountll(beyond);
+                    of_class += __builtin_popcountll(mine);
+                } else {
+                    at = base + before(m);
+                    in = in && at < q;
+                }
+                if (in) write(at * 8 + wave, (unsigned)(lane + j * 64) * 32u);
                 base += __builtin_popcountll(m);
             }
         };
@@ -559,12 +574,28 @@ __global__ void __launch_bounds__(512, ENDS > 1 ? 4 : 5) extremes_select_kernel(
                 lo = wave_min_f(least);
             }
         }
-        // a list that is not full repeats the chunk's first value
-        const auto from_lane_0 = [](float v) { return (unsigned)__builtin_amdgcn_readfirstlane(__float_as_uint(v)); };
-        const unsigned v0 = from_lane_0(P ? first.a : a.v[0]), v1 = from_lane_0(first.b), v2 = from_lane_0(first.c);
-        for (int e = base + lane; e < q; e += 64) {
-            if constexpr (P) reinterpret_cast<uint4*>(stage)[e * 8 + wave] = make_uint4(v0, v1, 0u, v2);
-            else reinterpret_cast<uint2*>(stage)[e * 8 + wave] = make_uint2(v0, 0u);
+        // a list that is not full repeats the chunk's first value, or one of its first eight
+        using Entry = typename std::conditional<P, uint4, uint2>::type;
+        Entry* mine = reinterpret_cast<Entry*>(stage) + wave;
+        auto entry_of = [&](int from) {   // what lane `from` holds of the chunk's first 64
+            const unsigned v0 = __shfl(__float_as_uint(P ? first.a : a.v[0]), from);
+            if constexpr (P) return make_uint4(v0, __shfl(__float_as_uint(first.b), from), (unsigned)from * 32u, __shfl(__float_as_uint(first.c), from));
+            else return make_uint2(v0, (unsigned)from * 32u);
+        };
+        if (spread) {
+            int vacant = 0;
+            for (int e0 = 0; e0 < q; e0 += 64) {
+                const int e = e0 + lane, from = (e + (r >> 1)) & 7;
+                const bool free = e < q && e / 8 >= __shfl(of_class, from);
+                const unsigned long long m = __ballot(free);
+                const int n = vacant + before(m);
+                const Entry pad = entry_of(from < kc ? from : 0);
+                if (free) mine[e * 8] = n < over ? mine[(kMaxList + n) * 8] : pad;
+                vacant += __builtin_popcountll(m);
+            }
+        } else {
+            const Entry pad = entry_of(0);
+            for (int e = base + lane; e < q; e += 64) mine[e * 8] = pad;
         }
         if constexpr (P) {
             most = wave_max_f(most);
@@ -598,10 +629,15 @@ __global__ void __launch_bounds__(512, ENDS > 1 ? 4 : 5) extremes_select_kernel(
         uint4* dst = reinterpret_cast<uint4*>(side.lists + ((size_t)ch * side.blocks + block / 2) * q * 16 * E) + (block & 1) * S;
         for (int i = tid; i < q * S; i += 512) dst[i / S * 2 * S + i % S] = reinterpret_cast<const uint4*>(stage)[i];
     };
-    if constexpr (ENDS > 1) {
-        if (of_x) { lists(std::integral_constant<int, ENDS>{}); return; }
+    const int qx = kLengths[ix], qw = kLengths[iw], of_x = 2 * s.x.blocks;
+    const int per = of_x + (qw ? 2 * s.w.blocks : 0);   // weights without lists: the first scan finds what bounds their rows as it reads them
+#pragma unroll 1
+    for (int unit = blockIdx.x; unit < per * s.C; unit += gridDim.x) {
+        const int ch = unit / per, block = unit - ch * per;
+        if (block < of_x) lists(std::integral_constant<int, ENDS>{}, s.x, qx, guess_x, ch, block);
+        else lists(std::integral_constant<int, 1>{}, s.w, qw, guess_w, ch, block - of_x);
+        __syncthreads();   // `stage` is free again
     }
-    lists(std::integral_constant<int, 1>{});
 }
 
 // ---- scan ------------------------------------------------------------------------------------------------------------
@@ -627,6 +663,32 @@ __device__ __forceinline__ void store_row(T* to, const T (&v)[N]) {   // neighbo
     struct __attribute__((packed, aligned(4))) Any { Four v; };
 #pragma unroll
     for (int j = 0; j < N; j += 4) reinterpret_cast<Any*>(to + j)->v = Four{v[j], v[j + 1], v[j + 2], v[j + 3]};
+}
+
+// The largest of each of 16 values over a wave, NaN where there is one: in lane l that of value l / 4.  Halves, rows of 16, eights
+// and fours of lanes trade the values that the other part goes on with (33 instructions; 16 reductions of their own take 96).
+__device__ __forceinline__ float wave_max_of_16(float (&v)[16], int lane) {
+    auto larger = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
+        v[i] = larger(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 4]), false, false);
+        v[i] = larger(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    constexpr int kHalfMirror = 0x141;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float keep = lane & 8 ? v[i + 2] : v[i], give = lane & 8 ? v[i] : v[i + 2];
+        v[i] = larger(keep, dpp_move<kDppRor8, 0xF>(give, give));
+    }
+    const float keep = lane & 4 ? v[1] : v[0], give = lane & 4 ? v[0] : v[1];
+    float m = larger(keep, dpp_move<kHalfMirror, 0xF>(give, give));
+    m = larger(m, dpp_move<kDppSwap1, 0xF>(m, m));
+    return larger(m, dpp_move<kDppSwap2, 0xF>(m, m));
 }
 
 template <int MODE, bool SECOND>
@@ -696,7 +758,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                 float t[U][8];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    if (u * NT >= kc || q == 0) continue;
+                    if (u * NT >= kc || (q == 0 && !(!SECOND && last))) continue;
                     const unsigned k4 = (unsigned)min(u * NT + tid, kc - 1) * 4u;   // lanes past the chunk store nothing
 #pragma unroll
                     for (int j = 0; j < RS; j++) {
@@ -704,6 +766,33 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                         t[u][PAIR_STRIP ? 2 * j : j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rl, k4, row, 0));
                         if constexpr (PAIR_STRIP) t[u][2 * j + 1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ru, k4, row, 0));
                     }
+                }
+                if (!SECOND && last) {   // weights without lists: what bounds the strip's rows in this chunk is their largest and smallest
+                    float v[16];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) { v[j] = t[0][j]; v[j + 8] = -t[0][j]; }
+#pragma unroll
+                    for (int u = 1; u < U; u++)
+                        if (u * NT < kc) {
+#pragma unroll
+                            for (int j = 0; j < 8; j++) {
+                                v[j] = __builtin_elementwise_maximum(v[j], t[u][j]);
+                                v[j + 8] = __builtin_elementwise_maximum(v[j + 8], -t[u][j]);
+                            }
+                        }
+                    float* part = reinterpret_cast<float*>(lds);   // [wave][16]
+                    const float m = wave_max_of_16(v, lane);
+                    if ((lane & 3) == 0) part[(tid >> 6) * 16 + (lane >> 2)] = m;
+                    __syncthreads();
+                    if (tid < 16) {
+                        float r = part[tid];
+#pragma unroll
+                        for (int i = 1; i < NT / 64; i++) r = __builtin_elementwise_maximum(r, part[i * 16 + tid]);
+                        if (not_finite(r)) r = __builtin_inff();
+                        // workgroups that have this strip under other rows write the same
+                        if (s0 + (tid & 7) < sd.rows) sd.rest[((size_t)ch * 2 + (tid >> 3)) * sd.rows + s0 + (tid & 7)] = tid < 8 ? r : -r;
+                    }
+                    __syncthreads();
                 }
 #pragma unroll
                 for (int u = 0; u < U; u++) {
@@ -750,12 +839,13 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                     }
                 }
             };
-            // entries eg, eg + EG, ... four at a time; a place past the end repeats the last
-            const int quads = ((q - eg + EG - 1) / EG + 3) / 4;
-            Entry en[4], en_next[4];
-            auto read = [&](Entry (&e)[4], int i) {
+            // entries eg, eg + EG, ... four at a time (boxes two: registers); a place past the end repeats the last
+            constexpr int AT = PAIR_ENTRY ? 2 : 4;
+            const int quads = ((q - eg + EG - 1) / EG + AT - 1) / AT;
+            Entry en[AT], en_next[AT];
+            auto read = [&](Entry (&e)[AT], int i) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) e[c] = list[min(eg + (4 * i + c) * EG, q - 1) * 16];
+                for (int c = 0; c < AT; c++) e[c] = list[min(eg + (AT * i + c) * EG, q - 1) * 16];
             };
             if (wave_live && q != 0) read(en, 0);
             __syncthreads();
@@ -764,9 +854,9 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                 for (int i = 0; i < quads; i++) {
                     read(en_next, i + 1);
 #pragma unroll
-                    for (int c = 0; c < 4; c++) entry(en[c]);
+                    for (int c = 0; c < AT; c++) entry(en[c]);
 #pragma unroll
-                    for (int c = 0; c < 4; c++) en[c] = en_next[c];
+                    for (int c = 0; c < AT; c++) en[c] = en_next[c];
                 }
             }
         }
@@ -1086,14 +1176,16 @@ hipError_t launch_scan(const Search& s, const Problem& pr, hipStream_t stream) {
 }
 
 template <int ENDS>
-hipError_t launch_lists(const Search& s, hipStream_t stream) {
-    const unsigned grid = (unsigned)(2 * s.C * (s.x.blocks + s.w.blocks));
-    const size_t stage = (size_t)kMaxList * 8 * (ENDS > 1 ? 16 : 8);
+hipError_t launch_lists(const Search& s, int num_cu, hipStream_t stream) {
+    auto resident = [](int nv) { return nv <= 24 && ENDS == 1 ? 3 : 2; };   // per CU, by registers
+    const int units = 2 * s.C * (s.x.blocks + s.w.blocks);
+    const size_t stage = (size_t)2 * kMaxList * 8 * (ENDS > 1 ? 16 : 8);
 #define LISTS(NV)                                                                                                                 \
     do {                                                                                                                          \
         hipLaunchKernelGGL((extremes_sample_kernel<NV, ENDS>), dim3(kSampleGroups * kSampleGroups), dim3(1024), 0, stream, s);     \
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;                                                          \
-        hipLaunchKernelGGL((extremes_select_kernel<NV, ENDS>), dim3(grid), dim3(512), stage, stream, s);                          \
+        hipLaunchKernelGGL((extremes_select_kernel<NV, ENDS>), dim3((unsigned)std::min(units, resident(NV) * num_cu)), dim3(512), \
+                           stage, stream, s);                                                                                     \
     } while (0)
     if (s.KC <= 1024) LISTS(16);
     else if (s.KC <= 1536) LISTS(24);
@@ -1189,7 +1281,7 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* x3, co
     s.price_fail = (all ? 18.f : boxes ? 9.f : 6.f) * pr.K;
     s.price_dense = g_extremes > 0 ? 3e38f : (all ? 0.7f : boxes ? 0.5f : 0.2f) * pr.K;
     *gate = &s.head->full;
-    if (hipError_t e = all ? launch_lists<3>(s, stream) : boxes ? launch_lists<2>(s, stream) : launch_lists<1>(s, stream); e != hipSuccess) return e;
+    if (hipError_t e = all ? launch_lists<3>(s, pr.num_cu, stream) : boxes ? launch_lists<2>(s, pr.num_cu, stream) : launch_lists<1>(s, pr.num_cu, stream); e != hipSuccess) return e;
     auto walk = [&](auto mode) {
         hipLaunchKernelGGL(extremes_walk_kernel<decltype(mode)::value>, dim3(4 * pr.num_cu), dim3(256), 0, stream, s);
         return hipGetLastError();
