@@ -19,7 +19,7 @@
 // From the image (IMG = true, 3x3 windows) a pixel collects up to nine columns.  Float atomics for that, in memory
 // or in LDS, cost as much as the arithmetic (151 M of them for 128 images of 128 x 32 x 32: 1.2 -> 2.0 ms), so the
 // work is cut such that every pixel has one owner: a tile is 63 columns wide, i.e. seven whole channels, a
-// workgroup takes whole images, and it keeps the image rows of its seven channel planes that its windows are
+// workgroup takes whole images, or bands of one that overlap in the windows they walk, and it keeps the image rows of its seven channel planes that its windows are
 // still adding to in LDS (a ring of rows: a tile of 64 positions covers a few output rows, and everything above
 // the next tile's first window is final).  A tile's sums are parked in LDS by (column, position), over the g and
 // 1/out panels, which are free by then; then every pixel of the ring rows that the tile's windows reach fetches
@@ -53,7 +53,9 @@ constexpr size_t kMaxLds = 159 * 1024;   // all of LDS less the kernel's own sta
 struct ConvBwd {
     int B, G, K, NG, HW, M;          // the unfolded problem: K = 9 channels per group (image) or CI / G
     int tiles_k;                     // column tiles per group
-    int units, units_per_wg;         // what a workgroup walks: tiles of 64 rows (columns), whole images (image)
+    int units, units_per_wg;         // what a workgroup walks: tiles of 64 rows (columns), bands of images (image)
+    int bands, band_rows;            // IMG: bands of an image, and their output rows
+    int halo_rows;                   // IMG: output rows above a band whose windows reach into the band's image rows
     int ring_rows;                   // IMG: image rows per channel plane held in LDS
     int park_extra;                  // IMG: floats between the 1/out panel and the ring that the parked tile runs into
     int slices;                      // workgroups per (group, column tile): units / units_per_wg, rounded up
@@ -178,13 +180,14 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     if (IE == 0 && nb == 0) {
         float top = 0.f, nbot = -__builtin_inff();   // the largest and minus the smallest output of the first tile
         if (u_begin < u_end) {
-            const int rows = IMG ? min(TR, d.HW) : min(TR, d.M - u_begin * TR);
+            const int first_pos = IMG ? u_begin % d.bands * d.band_rows * win.WO : 0;
+            const int rows = IMG ? min(TR, d.HW - first_pos) : min(TR, d.M - u_begin * TR);
             for (int i = tid; i < NG * TR; i += 256) {
                 const int n = i / TR, r = i % TR;
                 if (r < rows) {
                     size_t o;
                     if constexpr (IMG) {
-                        o = ((size_t)(u_begin * d.G + g) * d.NG + n) * d.HW + r;
+                        o = ((size_t)(u_begin / d.bands * d.G + g) * d.NG + n) * d.HW + first_pos + r;
                     } else {
                         const int m = u_begin * TR + r, bi = m / d.HW;
                         o = ((size_t)(bi * d.G + g) * d.NG + n) * d.HW + (m - bi * d.HW);
@@ -234,8 +237,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     __amdgpu_buffer_rsrc_t g_rsrc = x_rsrc, o_rsrc = x_rsrc;
 
     // One tile: rows first_row .. first_row + 63 of the unfolded matrix, of which `rows` exist (IMG: rows of image b
-    // from position pos0).  Leaves the grad_input sums of the lane's patch in acc.
-    auto tile = [&](int first_row, int rows, int b, int pos0, float (&acc)[TI][TJ], WinRow (&wrow)[TI], size_t (&xoff)[TI]) {
+    // from position pos0).  Leaves the grad_input sums of the lane's patch in acc.  `own`: grad_weight gets its sums.
+    auto tile = [&](int first_row, int rows, int b, int pos0, bool own, float (&acc)[TI][TJ], WinRow (&wrow)[TI], size_t (&xoff)[TI]) {
         float q[TI][TJ];
         if constexpr (!IMG) {
 #pragma unroll
@@ -386,7 +389,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 float tot[TJ];
 #pragma unroll
                 for (int j = 0; j < TJ; j++) tot[j] = dpp_lanes_total<TYN>(s[j]);
-                if (ty == TYN - 1) {   // d/dw of |x - w| is minus d/dx
+                if (ty == TYN - 1 && (!IMG || own)) {   // d/dw of |x - w| is minus d/dx
                     float* gp = Gw + (nc + n) * WLD + tx * TJ;
                     if constexpr (TJ == 4) {
                         float4 v = *reinterpret_cast<float4*>(gp);
@@ -432,7 +435,13 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         }
         const float inv_w = 1.0f / (float)W, inv_r = 1.0f / (float)R;
         auto ring_row = [&](int h) { return h - R * (int)(((float)h + 0.5f) * inv_r); };   // h modulo R
-        for (int b = u_begin; b < u_end; b++) {
+        for (int u = u_begin; u < u_end; u++) {
+            const int b = u / d.bands, band = u - b * d.bands;
+            // the band's own positions, and from where its windows reach into the image rows that it owns
+            const int pos_own = band * d.band_rows * win.WO, pos_end = min(d.HW, pos_own + d.band_rows * win.WO);
+            const int pos_first = max(0, pos_own - d.halo_rows * win.WO);
+            const int h_own = band == 0 ? 0 : min(H, max(0, band * d.band_rows * win.S - win.P));
+            const int h_end = pos_end == d.HW ? H : min(H, max(0, (band + 1) * d.band_rows * win.S - win.P));
             float* dst = grad_input + ((size_t)b * win.C + g * win.CG + first_ch) * H * W;
             // Writes image rows h_from .. h_to - 1 of the planes to memory and clears their ring rows.  Rows more than
             // a ring away from h_from have never been touched (the windows reach less far): they are zero.
@@ -459,20 +468,25 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 const_cast<float*>(output + ((size_t)(b * d.G + g) * d.NG + nb) * d.HW), 0, (int)0x80000000u, 0x00020000);
             // the corners of the windows of the lane's positions, moved on by 64 positions per tile (positions past
             // the image's last one are never used: every use asks for i < rows)
+            auto corners = [&](int pos0) {
 #pragma unroll
-            for (int i = 0; i < TI; i++) {
-                const int ho = (ty * TI + i) / win.WO, wo = (ty * TI + i) - ho * win.WO;
-                wrow[i].b = b;
-                wrow[i].h0 = ho * win.S - win.P;
-                wrow[i].w0 = wo * win.S - win.P;
-            }
+                for (int i = 0; i < TI; i++) {
+                    const int pos = pos0 + ty * TI + i, ho = pos / win.WO, wo = pos - ho * win.WO;
+                    wrow[i].b = b;
+                    wrow[i].h0 = ho * win.S - win.P;
+                    wrow[i].w0 = wo * win.S - win.P;
+                }
+            };
+            corners(pos_first);
             const int step_rows = TR / win.WO;
             const int step_h = step_rows * win.S, step_w = (TR - step_rows * win.WO) * win.S;
             const int wrap_w = win.WO * win.S, end_w = wrap_w - win.P;   // a corner's column stays below end_w
-            int flushed = 0;   // image rows below this one are in memory
-            for (int pos0 = 0; pos0 < d.HW; pos0 += TR) {
-                const int rows = min(TR, d.HW - pos0);
-                if (pos0 > 0) {
+            int flushed = h_own;   // of the band's image rows those below this one are in memory
+            int rows = 0;
+            for (int pos0 = pos_first; pos0 < pos_end; pos0 += rows) {
+                if (pos0 == pos_own && pos0 > pos_first) {
+                    corners(pos0);
+                } else if (pos0 > pos_first) {
 #pragma unroll
                     for (int i = 0; i < TI; i++) {
                         wrow[i].h0 += step_h;
@@ -480,9 +494,11 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                         if (wrow[i].w0 >= end_w) { wrow[i].w0 -= wrap_w; wrow[i].h0 += win.S; }
                     }
                 }
-                tile(0, rows, b, pos0, acc, wrow, xoff);
+                const bool own = pos0 >= pos_own;
+                rows = min(TR, (own ? pos_end : pos_own) - pos0);
+                tile(0, rows, b, pos0, own, acc, wrow, xoff);
                 // rows above this tile's first window are final (the last tile's rounds ended with a barrier)
-                const int h_lo = min(H, max(flushed, (pos0 / win.WO) * win.S - win.P));
+                const int h_lo = min(h_end, max(flushed, (pos0 / win.WO) * win.S - win.P));
                 if (h_lo > flushed) flush_rows(flushed, h_lo);
                 flushed = h_lo;
                 __syncthreads();   // ring rows cleared above may be this tile's; every lane is done with the panels
@@ -507,9 +523,9 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                     __syncthreads();
                 }
                 const int last = pos0 + rows - 1;
-                const int h_first = max(0, (pos0 / win.WO) * win.S - win.P);
-                const int h_last = min(H - 1, (last / win.WO) * win.S - win.P + 2 * win.D);
-                const int nrow = h_last - h_first + 1;
+                const int h_first = max(h_own, (pos0 / win.WO) * win.S - win.P);
+                const int h_last = min(h_end - 1, (last / win.WO) * win.S - win.P + 2 * win.D);
+                const int nrow = max(0, h_last - h_first + 1);
                 const float inv_nrow = 1.0f / (float)nrow;
                 for (int i = tid; i < planes * nrow * W; i += 256) {
                     // i = (c * nrow + hr) * W + w; quotients of small numbers through the reciprocal
@@ -535,13 +551,13 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 }
                 __syncthreads();   // the next tile stages over the parked sums; its flush reads the ring
             }
-            flush_rows(flushed, H);
+            flush_rows(flushed, h_end);
             __syncthreads();       // before the ring is used for the next image
         }
     } else {
         for (int t = u_begin; t < u_end; t++) {
             const int m0 = t * TR, rows = min(TR, d.M - m0);
-            tile(m0, rows, 0, 0, acc, wrow, xoff);
+            tile(m0, rows, 0, 0, true, acc, wrow, xoff);
 #pragma unroll
             for (int i = 0; i < TI; i++)
 #pragma unroll
@@ -580,7 +596,7 @@ template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
 hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 const Pieces& pieces, hipStream_t stream) {
-    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, pieces.block, pieces.chunk};
+    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 1, win.HO, 0, 0, 0, 0, pieces.block, pieces.chunk};
     d.tiles_k = IMG ? (win.CG + kPlanes - 1) / kPlanes : (d.K + TCP - 1) / TCP;
     d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
     const long pairs = (long)d.tiles_k * d.G;
@@ -610,6 +626,28 @@ hipError_t launch_conv_backward_blocks(const float* grad_output, const float* in
         if (best < 0 || cost < best_cost) { best = upw; best_cost = cost; }
     }
     d.units_per_wg = (int)best;
+    if constexpr (IMG) {
+        // Few images leave CUs without work, or the last of them without enough.  An image is then cut into bands of output
+        // rows, a workgroup for each: a band owns the image rows that no later window reaches, and walks the windows of
+        // `halo_rows` more output rows above its own, which reach into them, without adding those to grad_weight.  Forward and both
+        // gradients, us, 32 x 32 images, p = 8: 128 of 3 -> 32 channels 226 -> 121 (128 workgroups before), 16 of 32 -> 32 345 -> 151,
+        // 48 465 -> 350, 20 of 64 -> 64 650 -> 467; where three workgroups to the CU come out even anyway (77 of 32 -> 32: 596, 599)
+        // the image stays whole.
+        const int tiles = (pr.HW + TR - 1) / TR, halo = 2 * win.D / win.S;
+        auto banded = [&](int bands, double length) {   // a CU with a single workgroup runs at 0.6 of the rate of several
+            const long on_busiest = ((long)pr.B * bands * pairs + pr.num_cu - 1) / pr.num_cu;
+            return (on_busiest == 1 ? 1.0 / 0.6 : (double)on_busiest) * (length + fixed) + 0.5 * length;
+        };
+        best_cost = banded(1, 1.0);
+        for (int bands = 2; bands <= std::min(16, win.HO) && best == 1; bands++) {
+            const int rows = (win.HO + bands - 1) / bands;
+            if ((win.HO + rows - 1) / rows != bands) continue;
+            const double length = (double)((rows * win.WO + TR - 1) / TR + (halo * win.WO + TR - 1) / TR) / tiles;
+            const double cost = banded(bands, length);
+            if (cost < 0.95 * best_cost) { d.bands = bands; d.band_rows = rows; d.halo_rows = halo; best_cost = cost; }
+        }
+        d.units *= d.bands;
+    }
     const long slices = (d.units + d.units_per_wg - 1) / d.units_per_wg;
     d.slices = (int)slices;
     const long grid = (pairs * slices + 7) / 8 * 8;   // whole rounds of the eight XCDs; the padding exits at once
