@@ -102,7 +102,9 @@ struct NormForward {
 // least; a CU runs one workgroup of eight waves at a time.  32 x 40: 64 x 5120 -> 5120 is 256 tiles instead of 320, 280 ->
 // 189 us at p = 8, 602 -> 386 at p = 37.3.  16 x 32 with two rows per lane: 128 x 12288 -> 512 is 128 tiles instead of 64,
 // 290 -> 184 us and 684 -> 369; 100 x 1024 -> 1024 43 -> 27 and 84 -> 48.  A lane of the latter reads six LDS words for
-// eight differences instead of eight for sixteen, hence the surcharge.
+// eight differences instead of eight for sixteen, hence the surcharge.  16 x 16 with two rows and columns: a wave per k-group, so
+// that two waves per SIMD stay on every CU where 16 x 32 is 128 workgroups: 128 x 16384 -> 512 247 -> 161 us at p = 8, 489 -> 280
+// at p = 37.3, 533 -> 278 at 300; 64 x 3072 -> 1024 53 -> 34; 16 x 784 -> 1024 25 -> 16.
 template <class GEO>
 static hipError_t launch_eight_groups(const Problem& pr, hipStream_t stream, const float* input, const float* weight,
                                       float* output, float p) {
@@ -116,7 +118,8 @@ static hipError_t norm_forward_eight_groups(const float* input, const float* wei
         const long tiles = (long)((pr.B + bm - 1) / bm) * ((pr.NG + bn - 1) / bn) * pr.G;
         return (double)((tiles + pr.num_cu - 1) / pr.num_cu) * bm * bn * price;
     };
-    const double square = cost(32, 32, 1.0), wide = cost(32, 40, 1.0), flat = cost(16, 32, 1.1);
+    const double square = cost(32, 32, 1.0), wide = cost(32, 40, 1.0), flat = cost(16, 32, 1.1), small = cost(16, 16, 1.3);
+    if (small < square && small < wide && small < flat) return launch_eight_groups<Geo<16, 16, 2, 2, 8>>(pr, stream, input, weight, output, p);
     if (wide < square && wide <= flat) return launch_eight_groups<Geo<32, 40, 4, 5, 8>>(pr, stream, input, weight, output, p);
     if (flat < square) return launch_eight_groups<Geo<16, 32, 2, 4, 8>>(pr, stream, input, weight, output, p);
     return launch_eight_groups<Geo<32, 32, 4, 4, 8>>(pr, stream, input, weight, output, p);

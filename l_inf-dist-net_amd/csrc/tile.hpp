@@ -66,7 +66,7 @@ struct Geo {
     static constexpr int XS = KK * SM;           // floats of one x panel
     static constexpr int WS = KK * SN;
     static_assert(TM == 2 || TM == 4 || TM == 8, "TM");
-    static_assert(TN == 4 || TN == 5 || TN == 8, "TN");
+    static_assert(TN == 2 || TN == 4 || TN == 5 || TN == 8, "TN");
     static_assert(BM % TM == 0 && BN % TN == 0, "tile");
     static_assert(NT % 64 == 0, "whole waves");
 
@@ -78,7 +78,7 @@ struct Geo {
     __device__ static constexpr int col(int tx, int j) {
         return TN == 8 ? (j < 4 ? tx * 4 + j : BN / 2 + tx * 4 + (j - 4))
              : TN == 5 ? (j < 4 ? tx * 4 + j : TX * 4 + tx)
-                       : tx * 4 + j;
+                       : tx * TN + j;
     }
 };
 
@@ -94,7 +94,7 @@ struct LanePtr {
     __device__ __forceinline__ void set(const float* xp, const float* wp, int kk, int tx, int ty) {
         const int s = swz(kk);
         x = xp + kk * GEO::SM + ((ty * (GEO::TM == 2 ? 2 : 4)) ^ s);
-        w = wp + kk * GEO::SN + ((tx * 4) ^ s);
+        w = wp + kk * GEO::SN + ((tx * (GEO::TN == 2 ? 2 : 4)) ^ s);
         if constexpr (GEO::TN == 5) w5 = wp + kk * GEO::SN + ((GEO::TX * 4 + tx) ^ s);
     }
 };
@@ -117,6 +117,11 @@ __device__ __forceinline__ void read_x(const float* __restrict__ p, int r, float
 
 template <class GEO>
 __device__ __forceinline__ void read_w(const LanePtr<GEO>& lp, int r, float (&wf)[GEO::TN]) {
+    if constexpr (GEO::TN == 2) {
+        const float2 a = *reinterpret_cast<const float2*>(lp.w + r * GEO::SN);
+        wf[0] = a.x; wf[1] = a.y;
+        return;
+    } else {
     float4 a = *reinterpret_cast<const float4*>(lp.w + r * GEO::SN);
     wf[0] = a.x; wf[1] = a.y; wf[2] = a.z; wf[3] = a.w;
     if constexpr (GEO::TN == 8) {
@@ -124,6 +129,7 @@ __device__ __forceinline__ void read_w(const LanePtr<GEO>& lp, int r, float (&wf
         wf[4] = b.x; wf[5] = b.y; wf[6] = b.z; wf[7] = b.w;
     }
     if constexpr (GEO::TN == 5) wf[4] = lp.w5[r * GEO::SN];
+    }
 }
 
 // Operand registers of KP consecutive k rows (1 or 2): NX x-like panels (1, or 2
