@@ -89,7 +89,7 @@ struct Search {
     int* walk;             // [walk_most]: indices of outputs that fail
     int walk_most;
     int K, C, KC;
-    int lanes_first, lanes_second;   // rows per workgroup of the two scans
+    int lanes_first, lanes_second, lanes_only;   // rows per workgroup of the two scans, and of a first that no second follows
     float price_x, price_w, price_both, price_fail, price_dense;   // of a list entry, of a second scan after the first, of an output that does not pass, of the full walk
 };
 
@@ -705,7 +705,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
     const bool last = SECOND || s.head->qw == 0;   // no second pass: the first checks the bounds
     if (SECOND ? q == 0 : !both && !last) return;
     const int K = s.K, KC = s.KC, C = s.C, N = s.w.rows;
-    const int LG = SECOND ? s.lanes_second : s.lanes_first, EG = NT / LG;
+    const int LG = SECOND ? s.lanes_second : last ? s.lanes_only : s.lanes_first, EG = NT / LG;
     const int tid = threadIdx.x, lane = tid & 63;
     const int eg = __builtin_amdgcn_readfirstlane(tid / LG), at = tid % LG;
     const unsigned odd = (lane & 1) * 16u;   // which half a lane reads first
@@ -1271,6 +1271,12 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* x3, co
     s.mean = pr.mean; s.bias = pr.bias;
     s.K = pr.K; s.C = l.C; s.KC = l.KC;
     s.lanes_first = lanes_for(pr.B, (pr.NG + 7) / 8, pr.num_cu);
+    // Without a list for the weights the lists of x are short, and a strip on its way to LDS costs more than its walk: where two blocks of
+    // rows fit a workgroup with an eighth of its lanes to spare, they share it (200 to 448 rows, 5120 -> 5120, a whole pass 91 -> 83 and
+    // 97 -> 92 us; 3072 -> 4096 76 -> 67).  512 rows of 5120 outputs would leave the last round of strips to a quarter of the
+    // workgroups (64 -> 73 us of the scan), and with both lists two blocks are as fast at best.
+    s.lanes_only = s.lanes_first;
+    while (s.lanes_only < 512 && pr.B > s.lanes_only && pr.B <= s.lanes_only * 7 / 4) s.lanes_only *= 2;
     const int second_rows = strip_rows(boxes);
     s.lanes_second = lanes_for(pr.NG, (pr.B + second_rows - 1) / second_rows, pr.num_cu);
     s.price_x = 1.f;
