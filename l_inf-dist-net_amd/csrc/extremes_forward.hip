@@ -139,6 +139,32 @@ struct RowChunk {
     }
 };
 
+// The largest of each of 16 values over a wave, NaN where there is one: in lane l that of value l / 4.  Halves, rows of 16, eights
+// and fours of lanes trade the values that the other part goes on with (33 instructions; 16 reductions of their own take 96).
+__device__ __forceinline__ float wave_max_of_16(float (&v)[16], int lane) {
+    auto larger = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
+        v[i] = larger(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 4]), false, false);
+        v[i] = larger(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    constexpr int kHalfMirror = 0x141;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float keep = lane & 8 ? v[i + 2] : v[i], give = lane & 8 ? v[i] : v[i + 2];
+        v[i] = larger(keep, dpp_move<kDppRor8, 0xF>(give, give));
+    }
+    const float keep = lane & 4 ? v[1] : v[0], give = lane & 4 ? v[0] : v[1];
+    float m = larger(keep, dpp_move<kHalfMirror, 0xF>(give, give));
+    m = larger(m, dpp_move<kDppSwap1, 0xF>(m, m));
+    return larger(m, dpp_move<kDppSwap2, 0xF>(m, m));
+}
+
 // ---- sample ----------------------------------------------------------------------------------------------------------
 // Distance from the center as a bin of a histogram: 256 to the octave, two octaves below the largest; negative: below.
 struct Bins {
@@ -195,6 +221,8 @@ __device__ __forceinline__ void lengths_of(RowChunk<NV>& a, float center, int* h
 }
 
 // A workgroup looks at 4 x 4 outputs: wave i at row i % 8 (four of x, four of w) in every other chunk, then all at the outputs.
+// Bound by a chain of latencies: the outputs' rows are on their way during the histograms, and their 16 (boxes 32, with points 48)
+// maxima meet 16 at a time: 5120 -> 5120 17.5 -> 15.9 us, boxes with points 29.9 -> 24.7.
 // ENDS: 1 values, 2 boxes, 3 boxes and the points inside them.
 template <int NV, int ENDS>
 __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
@@ -223,8 +251,33 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
     };
     const int first = wave >> 3;
     if (first < s.C) load(first);
+    const float *xr[kSampleRows], *ur[kSampleRows], *pr[kSampleRows], *wr[kSampleRows];   // of the outputs
+#pragma unroll
+    for (int i = 0; i < kSampleRows; i++) {
+        xr[i] = s.x.v + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
+        if constexpr (PAIR) ur[i] = s.x.v2 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
+        if constexpr (ALL) pr[i] = s.x.v3 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
+        wr[i] = s.w.v + (size_t)sampled(bw * kSampleRows + i, s.w.rows) * s.K;
+    }
+    constexpr int AHEAD = ALL ? 2 : PAIR ? 3 : 5;
+    constexpr bool EARLY = ENDS == 1;   // the first of them before the histograms; boxes have no registers for that
+    float x[AHEAD][kSampleRows], u[AHEAD][kSampleRows], p[AHEAD][kSampleRows], w[AHEAD][kSampleRows];
+    auto fetch = [&](int kb) {
+#pragma unroll
+        for (int e = 0; e < AHEAD; e++) {
+            const int k = min(kb + e * 1024 + tid, s.K - 1);   // past the end: the last k again
+#pragma unroll
+            for (int i = 0; i < kSampleRows; i++) {
+                x[e][i] = xr[i][k];
+                w[e][i] = wr[i][k];
+                if constexpr (PAIR) u[e][i] = ur[i][k];
+                if constexpr (ALL) p[e][i] = pr[i][k];
+            }
+        }
+    };
     // a center common to both operands: the mean of 1024 weights; any number is correct
     float c = s.w.v[(size_t)((long long)tid * s.w.rows / 1024) * s.K + (size_t)((long long)tid * 61 % s.K)];
+    if (EARLY) fetch(0);
 #pragma unroll
     for (int o = 32; o; o >>= 1) c += __shfl_xor(c, o);
     if (lane == 0) part[wave] = c;
@@ -278,28 +331,8 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
     float up[NO], lo[NO], pt[NO];
 #pragma unroll
     for (int i = 0; i < NO; i++) up[i] = lo[i] = pt[i] = 0.f;
-    const float *xr[kSampleRows], *ur[kSampleRows], *pr[kSampleRows], *wr[kSampleRows];
-#pragma unroll
-    for (int i = 0; i < kSampleRows; i++) {
-        xr[i] = s.x.v + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
-        if constexpr (PAIR) ur[i] = s.x.v2 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
-        if constexpr (ALL) pr[i] = s.x.v3 + (size_t)sampled(bx * kSampleRows + i, s.x.rows) * s.K;
-        wr[i] = s.w.v + (size_t)sampled(bw * kSampleRows + i, s.w.rows) * s.K;
-    }
-    constexpr int AHEAD = ALL ? 2 : PAIR ? 3 : 5;
     for (int kb = 0; kb < s.K; kb += 1024 * AHEAD) {
-        float x[AHEAD][kSampleRows], u[AHEAD][kSampleRows], p[AHEAD][kSampleRows], w[AHEAD][kSampleRows];
-#pragma unroll
-        for (int e = 0; e < AHEAD; e++) {
-            const int k = min(kb + e * 1024 + tid, s.K - 1);   // past the end: the last k again
-#pragma unroll
-            for (int i = 0; i < kSampleRows; i++) {
-                x[e][i] = xr[i][k];
-                w[e][i] = wr[i][k];
-                if constexpr (PAIR) u[e][i] = ur[i][k];
-                if constexpr (ALL) p[e][i] = pr[i][k];
-            }
-        }
+        if (!EARLY || kb > 0) fetch(kb);
 #pragma unroll
         for (int e = 0; e < AHEAD; e++)
 #pragma unroll
@@ -318,19 +351,13 @@ __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
                     if constexpr (ALL) pt[i * kSampleRows + j] = __builtin_fmaxf(pt[i * kSampleRows + j], __builtin_fabsf(p[e][i] - w[e][j]));
                 }
     }
-#pragma unroll
-    for (int i = 0; i < NO; i++) {
-        const float u = wave_max(up[i]);   // in lane 63
-        if (lane == 63) outs[wave][i] = u;
-        if constexpr (PAIR) {
-            const float l = wave_max(lo[i]);
-            if (lane == 63) outs[wave][NO + i] = l;
-        }
-        if constexpr (ALL) {
-            const float v = wave_max(pt[i]);
-            if (lane == 63) outs[wave][2 * NO + i] = v;
-        }
-    }
+    auto gather = [&](float (&v)[NO], int q) {
+        const float m = wave_max_of_16(v, lane);
+        if ((lane & 3) == 0) outs[wave][q * NO + (lane >> 2)] = m;
+    };
+    gather(up, 0);
+    if constexpr (PAIR) gather(lo, 1);
+    if constexpr (ALL) gather(pt, 2);
     __syncthreads();
     if (tid < NB * NO) {
         float best = outs[0][tid];
@@ -663,32 +690,6 @@ __device__ __forceinline__ void store_row(T* to, const T (&v)[N]) {   // neighbo
     struct __attribute__((packed, aligned(4))) Any { Four v; };
 #pragma unroll
     for (int j = 0; j < N; j += 4) reinterpret_cast<Any*>(to + j)->v = Four{v[j], v[j + 1], v[j + 2], v[j + 3]};
-}
-
-// The largest of each of 16 values over a wave, NaN where there is one: in lane l that of value l / 4.  Halves, rows of 16, eights
-// and fours of lanes trade the values that the other part goes on with (33 instructions; 16 reductions of their own take 96).
-__device__ __forceinline__ float wave_max_of_16(float (&v)[16], int lane) {
-    auto larger = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
-        v[i] = larger(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 4]), false, false);
-        v[i] = larger(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    }
-    constexpr int kHalfMirror = 0x141;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const float keep = lane & 8 ? v[i + 2] : v[i], give = lane & 8 ? v[i] : v[i + 2];
-        v[i] = larger(keep, dpp_move<kDppRor8, 0xF>(give, give));
-    }
-    const float keep = lane & 4 ? v[1] : v[0], give = lane & 4 ? v[0] : v[1];
-    float m = larger(keep, dpp_move<kHalfMirror, 0xF>(give, give));
-    m = larger(m, dpp_move<kDppSwap1, 0xF>(m, m));
-    return larger(m, dpp_move<kDppSwap2, 0xF>(m, m));
 }
 
 template <int MODE, bool SECOND>
