@@ -423,7 +423,8 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
 // (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly,
 // unless more values tie at the outer end than the list has places: such a row's bounds are those of all its values.
 // Bound by reading the operands once.
-template <int NV, int ENDS>
+// SPREAD: no positions follow (its own instantiation: the code of both orders in one made the kernel 43 -> 48 us).
+template <int NV, int ENDS, bool SPREAD>
 __global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_select_kernel(Search s) {
     extern __shared__ __align__(16) char stage[];   // [2 kMaxList][8] entries: half of a block of Side::lists, and what `place` finds no place for
     __shared__ int sums[8][64];
@@ -517,14 +518,14 @@ __global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_sel
         float most = -kNever, least = kNever, most_lower = -kNever, least_upper = kNever, most_point = -kNever, least_point = kNever;
         // Without positions the order of a list is free: entry s of row r is one with k = s + r / 2 (mod 8) where the row has such
         // an entry left, so that 16 neighbouring lanes of a scan read from different banks.
-        const bool spread = s.pos == nullptr;
+        constexpr bool spread = SPREAD;
         int of_class = 0, over = 0;   // entries with this lane's k mod 8; those beyond an eighth of the list, behind it in `stage`
         auto before = [](unsigned long long m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0)); };
         auto place = [&](bool in, int j, auto&& write) {
             const unsigned long long m = __ballot(in);
             if (m) {
                 int at;
-                if (spread) {
+                if constexpr (spread) {
                     const unsigned long long mine = m & (0x0101010101010101ull << (lane & 7));
                     const int rank = of_class + before(mine);
                     const unsigned long long beyond = __ballot(in && rank >= q / 8);
@@ -609,7 +610,7 @@ __global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_sel
             if constexpr (P) return make_uint4(v0, __shfl(__float_as_uint(first.b), from), (unsigned)from * 32u, __shfl(__float_as_uint(first.c), from));
             else return make_uint2(v0, (unsigned)from * 32u);
         };
-        if (spread) {
+        if constexpr (spread) {
             int vacant = 0;
             for (int e0 = 0; e0 < q; e0 += 64) {
                 const int e = e0 + lane, from = (e + (r >> 1)) & 7;
@@ -1185,8 +1186,9 @@ hipError_t launch_lists(const Search& s, int num_cu, hipStream_t stream) {
     do {                                                                                                                          \
         hipLaunchKernelGGL((extremes_sample_kernel<NV, ENDS>), dim3(kSampleGroups * kSampleGroups), dim3(1024), 0, stream, s);     \
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;                                                          \
-        hipLaunchKernelGGL((extremes_select_kernel<NV, ENDS>), dim3((unsigned)std::min(units, resident(NV) * num_cu)), dim3(512), \
-                           stage, stream, s);                                                                                     \
+        const dim3 grid((unsigned)std::min(units, resident(NV) * num_cu));                                                        \
+        if (ENDS == 1 && s.pos) hipLaunchKernelGGL((extremes_select_kernel<NV, ENDS, ENDS != 1>), grid, dim3(512), stage, stream, s); \
+        else hipLaunchKernelGGL((extremes_select_kernel<NV, ENDS, true>), grid, dim3(512), stage, stream, s);                      \
     } while (0)
     if (s.KC <= 1024) LISTS(16);
     else if (s.KC <= 1536) LISTS(24);
