@@ -15,11 +15,11 @@
 //            are launched last and otherwise leave at once, do the work), and every row's list;
 //   scan     first every row's list against all outputs, then every weight row's list against all rows.  Where the weights
 //            need no list (images, or activations spread far wider than the weights) the first scan checks the bounds itself,
-//            and the second leaves at once: 5120 x 5120 with positions at batch 272, 46 + 43 -> 56 + 5 us.
+//            and the second leaves at once: 5120 x 5120 with positions at batch 272, 46 + 43 -> 50 + 5 us.
 //
 // Boxes and the points inside them (certification) share sample, lists and first scan: an entry of a row of x is {lower, upper,
 // 32 k, point}.  Where the weights have lists, the second scans of boxes and of values follow it.  Values and bounds of the 5-layer,
-// 5120-wide net at batch 1024: 1450 to 1640 us with passes of their own, 825 together; 5120 x 5120 normal weights and inputs of
+// 5120-wide net at batch 1024: 1450 to 1640 us with passes of their own, 745 together; 5120 x 5120 normal weights and inputs of
 // the same spread, batch 512, 187 + 240 -> 350 us, 1024 256 + 390 -> 580.
 //
 // The reduction is cut into C chunks of at most 2560 k with lists and bounds of their own, so that a chunk of eight rows
