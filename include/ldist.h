@@ -169,6 +169,11 @@ LDIST_API int ldist_norm_dist_forward_values(const float* input, const float* we
                                              float* output, float p, ldist_stream_t stream);
 
 
+/* Which tile ldist_norm_dist_forward takes on a device of `num_cu` compute units for a fully connected layer on 16-byte aligned
+ * tensors: 1000 rows + outputs where it is one of the tiles with eight k-groups, 0 for another kernel, negative for arguments that
+ * the pass refuses.  For tests of the rule: asks no device, no counterpart in the reference. */
+LDIST_API int ldist_which_forward_tile(int B, int CO, int CI, int G, float p, int num_cu);
+
 /* p-norm backward w.r.t. input.  Replaces norm_dist_backward_input_cuda
  * (model/norm_dist.cpp:9-10, model/norm_dist_cuda.cu:438-448).
  *   grad_input[m,k] = sum_n g[m,n] * (|x-w| / output[m,n])^(p-1) * (x-w > 0 ? 1 : -1)

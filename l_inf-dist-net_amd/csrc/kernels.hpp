@@ -199,6 +199,9 @@ hipError_t norm_conv_backward_weight(const float* grad_output, const float* img,
 extern int g_conv_rows_override;
 extern int g_conv_groups_override;
 extern int g_conv_staging_override;
+// The tile that norm_forward takes before a gradient, as 1000 rows + outputs, where it is one of those with eight k-groups, else
+// 0; on the host alone, for aligned tensors.
+int norm_forward_tile(const Problem& pr, float p);
 // Whether norm_forward without gradients applies Problem::mean and bias.
 bool norm_forward_shifts(const Problem& pr, float p);
 bool inf_conv_forward_supported(const ConvGeom& q, int G, int CO);

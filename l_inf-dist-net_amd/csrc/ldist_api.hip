@@ -150,6 +150,14 @@ int ldist_set_tile_override(int choice) {
     return LDIST_OK;
 }
 
+int ldist_which_forward_tile(int B, int CO, int CI, int G, float p, int num_cu) {
+    ldist::Problem pr{};
+    if (!valid_p(p) || num_cu <= 0) return LDIST_EINVAL;
+    if (int rc = check_sizes(B, CO, CI, G, 1, pr)) return rc;
+    pr.num_cu = num_cu;
+    return ldist::norm_forward_tile(pr, p);
+}
+
 int ldist_set_extremes(int choice) {
     if (choice < -1 || choice > 1) return LDIST_EINVAL;
     ldist::g_extremes = choice;

@@ -103,8 +103,13 @@ struct NormForward {
 // 189 us at p = 8, 602 -> 386 at p = 37.3.  16 x 32 with two rows per lane: 128 x 12288 -> 512 is 128 tiles instead of 64,
 // 290 -> 184 us and 684 -> 369; 100 x 1024 -> 1024 43 -> 27 and 84 -> 48.  A lane of the latter reads six LDS words for
 // eight differences instead of eight for sixteen, hence the surcharge.  16 x 16 with two rows and columns: a wave per k-group, so
-// that two waves per SIMD stay on every CU where 16 x 32 is 128 workgroups: 128 x 16384 -> 512 247 -> 161 us at p = 8, 489 -> 280
-// at p = 37.3, 533 -> 278 at 300; 64 x 3072 -> 1024 53 -> 34; 16 x 784 -> 1024 25 -> 16.
+// that two waves per SIMD stay on every CU where 16 x 32 is 128 workgroups: 128 x 16384 -> 512 237 -> 142 us at p = 8, 489 -> 279
+// at p = 37.3, 533 -> 278 at 300; 64 x 3072 -> 1024 54 -> 33; 16 x 784 -> 1024 25 -> 16.  It reads four LDS words for four
+// differences, which shows in several rounds of tiles: three of them against one of 32 x 32, 64 x 5120 -> 3072, 134 -> 147 us at
+// p = 8, 87 -> 105 at 2, but 303 -> 281 at 37.3 and 404 -> 388 at 300; five against three of 16 x 32, 80 x 4096 -> 4096, 200 -> 202 at
+// p = 8, 399 -> 384 at 37.3.  So its price depends on what a difference costs: 1.5 where a power is a few multiplications, 1.3
+// where it is a logarithm and an exponential, unless the reduction is short or its loads are single words (64 x 511 -> 3072, p = 37.3,
+// three rounds 3 % slower).
 template <class GEO>
 static hipError_t launch_eight_groups(const Problem& pr, hipStream_t stream, const float* input, const float* weight,
                                       float* output, float p) {
@@ -112,17 +117,39 @@ static hipError_t launch_eight_groups(const Problem& pr, hipStream_t stream, con
                                                    weight, output, p);
 }
 
-static hipError_t norm_forward_eight_groups(const float* input, const float* weight, float* output, float p, const Problem& pr,
-                                            hipStream_t stream) {
+enum class EightGroups { k32x32, k32x40, k16x32, k16x16 };
+static EightGroups eight_groups_tile(const Problem& pr, float p, bool vec) {
     auto cost = [&](int bm, int bn, double price) {
         const long tiles = (long)((pr.B + bm - 1) / bm) * ((pr.NG + bn - 1) / bn) * pr.G;
         return (double)((tiles + pr.num_cu - 1) / pr.num_cu) * bm * bn * price;
     };
-    const double square = cost(32, 32, 1.0), wide = cost(32, 40, 1.0), flat = cost(16, 32, 1.1), small = cost(16, 16, 1.3);
-    if (small < square && small < wide && small < flat) return launch_eight_groups<Geo<16, 16, 2, 2, 8>>(pr, stream, input, weight, output, p);
-    if (wide < square && wide <= flat) return launch_eight_groups<Geo<32, 40, 4, 5, 8>>(pr, stream, input, weight, output, p);
-    if (flat < square) return launch_eight_groups<Geo<16, 32, 2, 4, 8>>(pr, stream, input, weight, output, p);
-    return launch_eight_groups<Geo<32, 32, 4, 4, 8>>(pr, stream, input, weight, output, p);
+    const bool dear = small_int_power(p) == 0 || small_int_power(p) == 7;   // the exponents without an instantiation of their own
+    const double square = cost(32, 32, 1.0), wide = cost(32, 40, 1.0), flat = cost(16, 32, 1.1);
+    const double small = cost(16, 16, dear && vec && pr.K >= 512 ? 1.3 : 1.5);
+    if (small < square && small < wide && small < flat) return EightGroups::k16x16;
+    if (wide < square && wide <= flat) return EightGroups::k32x40;
+    return flat < square ? EightGroups::k16x32 : EightGroups::k32x32;
+}
+
+static hipError_t norm_forward_eight_groups(const float* input, const float* weight, float* output, float p, const Problem& pr,
+                                            hipStream_t stream) {
+    switch (eight_groups_tile(pr, p, can_vec4(pr, input, weight))) {
+        case EightGroups::k16x16: return launch_eight_groups<Geo<16, 16, 2, 2, 8>>(pr, stream, input, weight, output, p);
+        case EightGroups::k32x40: return launch_eight_groups<Geo<32, 40, 4, 5, 8>>(pr, stream, input, weight, output, p);
+        case EightGroups::k16x32: return launch_eight_groups<Geo<16, 32, 2, 4, 8>>(pr, stream, input, weight, output, p);
+        default: return launch_eight_groups<Geo<32, 32, 4, 4, 8>>(pr, stream, input, weight, output, p);
+    }
+}
+
+int norm_forward_tile(const Problem& pr, float p) {
+    if (pr.NG <= kSkinnyMaxNG || pr.HW != 1 || g_tile_override >= 0) return 0;
+    if (choose_tile(pr.B, pr.NG, pr.G, pr.num_cu) != TileChoice::M32N32K8) return 0;
+    switch (eight_groups_tile(pr, p, pr.K % 4 == 0)) {
+        case EightGroups::k16x16: return 16016;
+        case EightGroups::k32x40: return 32040;
+        case EightGroups::k16x32: return 16032;
+        default: return 32032;
+    }
 }
 
 bool norm_forward_shifts(const Problem& pr, float p) {
