@@ -360,6 +360,11 @@ LDIST_API int ldist_norm_dist_conv_backward(const float* grad_output, const floa
                                             const float* output, int B, int C, int H, int W, int CO, int G, int KH, int KW,
                                             int stride, int padding, int dilation, float* grad_img, float* grad_weight,
                                             float p, ldist_stream_t stream);
+/* Into how many bands of output rows ldist_norm_dist_conv_backward cuts an image on a device of `num_cu` compute units (3x3
+ * window): 1 whole images, 0 where its one kernel does not cover the layer, negative for arguments that the pass refuses.  For
+ * tests of the rule: asks no device, no counterpart in the reference. */
+LDIST_API int ldist_which_conv_bands(int B, int C, int H, int W, int CO, int G, int stride, int padding, int dilation, float p,
+                                     int num_cu);
 /* The forward passes with the evaluation-mode shift and bias of the layer in the same launch: what is stored for channel c
  * is (v - mean[c]) + bias[c], either of which may be null; otherwise as the entry point without `_shifted`.  Fully
  * connected layers (HW = 1) and 3x3 image layers.  pos may be null: values only (LDIST_EUNSUPPORTED where there is no

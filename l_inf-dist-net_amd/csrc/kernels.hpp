@@ -179,6 +179,7 @@ hipError_t norm_backward_fused(const float* grad_output, const float* input, con
 // input or from the image.
 bool norm_conv_backward_fused_applicable(const Problem& pr, float p);
 bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO, float p, int num_cu);
+int norm_conv_backward_bands(const ConvGeom& q, int G, int CO, float p, int num_cu);   // into how many bands that cuts an image; 0: not applicable
 hipError_t norm_conv_backward_fused_columns(const float* grad_output, const float* input, const float* weight,
                                             const float* output, float* grad_input, float* grad_weight, float p,
                                             const Problem& pr, hipStream_t stream);

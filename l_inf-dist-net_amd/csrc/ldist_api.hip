@@ -641,6 +641,14 @@ int ldist_norm_dist_conv_backward(const float* grad_output, const float* img, co
                                                    pr.device, (hipStream_t)stream));
 }
 
+int ldist_which_conv_bands(int B, int C, int H, int W, int CO, int G, int stride, int padding, int dilation, float p, int num_cu) {
+    if (CO <= 0 || G <= 0 || !valid_p(p) || num_cu <= 0) return LDIST_EINVAL;
+    ldist::ConvGeom q{};
+    if (int rc = conv_geometry(B, C, H, W, 3, 3, stride, padding, dilation, q)) return rc;
+    if (C % G != 0 || CO % G != 0) return LDIST_EINVAL;
+    return ldist::norm_conv_supported(q, G, CO) ? ldist::norm_conv_backward_bands(q, G, CO, p, num_cu) : 0;
+}
+
 int ldist_set_conv_staging_override(int mode) {
     if (mode < 0 || mode > 3) return LDIST_EINVAL;
     ldist::g_conv_staging_override = mode;

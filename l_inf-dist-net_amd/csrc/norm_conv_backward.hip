@@ -580,7 +580,8 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
 namespace {
 
 // Image rows per plane the ring must hold: the most that the windows of one tile of 64 positions cover (tiles start
-// at multiples of 64 inside an image).  Not more: 32 -> 64 channels at stride 2 on 32 x 32 need nine rows, and with
+// at multiples of 64 inside an image; in a band, whose own positions and whose halo begin with an output row, the i-th tile of
+// either begins as far into a row as the image's i-th, and is no longer).  Not more: 32 -> 64 channels at stride 2 on 32 x 32 need nine rows, and with
 // sixteen (the next power of two) a CU held one workgroup instead of two (128 images, p = 8: 386 -> 270 us).
 int ring_rows_for(const ImgWin& win, int HW) {
     int out_rows = 1;
@@ -592,19 +593,36 @@ int ring_rows_for(const ImgWin& win, int HW) {
     return (out_rows - 1) * win.S + 2 * win.D + 1;
 }
 
-template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
-hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
-                                float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
-                                const Pieces& pieces, hipStream_t stream) {
-    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 1, win.HO, 0, 0, 0, 0, pieces.block, pieces.chunk};
-    d.tiles_k = IMG ? (win.CG + kPlanes - 1) / kPlanes : (d.K + TCP - 1) / TCP;
-    d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
-    const long pairs = (long)d.tiles_k * d.G;
-    if constexpr (IMG) {
-        d.ring_rows = ring_rows_for(win, pr.HW);
-        d.park_extra = park_extra(d.chunk);
-    }
-    const size_t lds = lds_bytes(pieces, IMG ? image_floats(d.chunk, d.ring_rows, win.H, win.W) : 0);
+size_t lds_of(const Pieces& pieces, const ImgWin& win, int HW, bool img) {
+    return lds_bytes(pieces, img ? image_floats(pieces.chunk, ring_rows_for(win, HW), win.H, win.W) : 0);
+}
+
+int tiles_of(const Problem& pr, const ImgWin& win, bool img) {   // column tiles per group
+    return img ? (win.CG + kPlanes - 1) / kPlanes : (pr.K + TCP - 1) / TCP;
+}
+
+// The fewest pieces with which a CU still holds as many workgroups as the launch has for it (three at most).  Pieces buy
+// room for more of them and cost a barrier per chunk and a walk over the rows per block; where the launch cannot use the
+// room they only cost: 44 images of 28 x 25 x 32 to 67 outputs, p = 20.5 (176 workgroups), 568 us in two blocks, 472 whole;
+// 41 of 9 x 30 x 31 to 78, p = 1.5, 768 and 607; 79 of 12 x 7 x 31 to 33, p = 20.5, 88 and 84.
+Pieces pieces_of(const Problem& pr, const ImgWin& win, bool img) {
+    const long units = img ? pr.B : ((long)pr.B * pr.HW + TR - 1) / TR;
+    const long wgs = units * tiles_of(pr, win, img) * pr.G;
+    const long wanted = std::min(3L, (wgs + pr.num_cu - 1) / pr.num_cu);
+    for (const Pieces& c : {Pieces{pr.NG, pr.NG}, Pieces{pr.NG, outputs_staged(pr.NG)}})
+        if (lds_of(c, win, pr.HW, img) <= kMaxLds && on_a_cu(lds_of(c, win, pr.HW, img)) >= wanted) return c;
+    return least_pieces(pr.NG);
+}
+
+// Waves per SIMD of the instantiation, hence workgroups per CU that its registers admit.
+int waves_of(const Pieces& pieces, const Problem& pr, const ImgWin& win, bool img) {
+    return pieces.chunk == pr.NG && on_a_cu(lds_of(pieces, win, pr.HW, img)) >= 4 ? 4 : 3;
+}
+
+struct Share { int units_per_wg, bands, band_rows, halo_rows; };   // of a launch: units per workgroup, and ConvBwd's bands
+
+Share share_of(const Problem& pr, const ImgWin& win, bool img, long pairs, size_t lds, int waves) {
+    const long units = img ? pr.B : ((long)pr.B * pr.HW + TR - 1) / TR;
     // Units per workgroup.  A CU issues at the same rate whether two, three or four workgroups share it, so what a
     // launch takes is what the busiest CU has to work through: workgroups per CU (dealt round robin) times units per
     // workgroup.  With few long workgroups that is uneven -- 860 workgroups of three images on 256 CUs leave twelve
@@ -618,34 +636,62 @@ hipError_t launch_conv_backward_blocks(const float* grad_output, const float* in
     const long resident = per_cu * pr.num_cu;
     long best = -1;
     double best_cost = 0;
-    const double fixed = IMG ? 0.3 / std::max(1, (pr.HW + TR - 1) / TR) : 0.3;   // in units: an image is HW / 64 tiles
-    const long lo = std::max(1L, ((long)d.units * pairs + 16 * resident - 1) / (16 * resident));
-    for (long upw = lo; upw <= d.units && upw < lo + 4096; upw++) {
-        const long wgs = pairs * ((d.units + upw - 1) / upw);
+    const double fixed = img ? 0.3 / std::max(1, (pr.HW + TR - 1) / TR) : 0.3;   // in units: an image is HW / 64 tiles
+    const long lo = std::max(1L, (units * pairs + 16 * resident - 1) / (16 * resident));
+    for (long upw = lo; upw <= units && upw < lo + 4096; upw++) {
+        const long wgs = pairs * ((units + upw - 1) / upw);
         const double cost = (double)((wgs + pr.num_cu - 1) / pr.num_cu) * ((double)upw + fixed) + 0.5 * (double)upw;
         if (best < 0 || cost < best_cost) { best = upw; best_cost = cost; }
     }
-    d.units_per_wg = (int)best;
+    Share share{(int)best, 1, win.HO, 0};
+    if (!img || best > 1) return share;
+    // Few images leave CUs without work, or the last of them without enough.  An image is then cut into bands of output
+    // rows, a workgroup for each: a band owns the image rows that no later window reaches, and walks the windows of
+    // `halo_rows` more output rows above its own, which reach into them, without adding those to grad_weight.  Both gradients,
+    // us, 32 x 32 images, p = 8: 128 of 3 -> 32 channels 187 -> 76 (128 workgroups before), 16 of 32 -> 32 277 -> 73, 48 277 -> 160,
+    // 20 of 64 -> 64 452 -> 269; where three workgroups to the CU come out even anyway (77 of 32 -> 32) the image stays whole.
+    // A CU with a single workgroup runs at 0.6 of the rate of several.  Where LDS admits only one (the tiles of 65 and more
+    // outputs) the bands of a CU run in turn at that rate, each with its halo: 64 images of 3 -> 128 take 4 bands (166 us), not 8 (204),
+    // and 20 of 64 -> 128 none (841, two bands 907).  Where it admits two, an odd one comes last and alone (64 of 32 -> 128 in two
+    // groups 480, two bands 511).
+    const int tiles = (pr.HW + TR - 1) / TR, halo = 2 * win.D / win.S;
+    const long at_once = std::min((long)waves, on_a_cu(lds));
+    auto banded = [&](int bands, double length) {
+        const long on_busiest = ((long)pr.B * bands * pairs + pr.num_cu - 1) / pr.num_cu;
+        if (at_once == 1) return (double)on_busiest / 0.6 * (length + fixed);
+        if (at_once == 2) return ((double)(on_busiest / 2 * 2) + (double)(on_busiest % 2) / 0.6) * (length + fixed);
+        return (on_busiest == 1 ? 1.0 / 0.6 : (double)on_busiest) * (length + fixed) + 0.5 * length;
+    };
+    best_cost = banded(1, 1.0);
+    for (int bands = 2; bands <= std::min(16, win.HO); bands++) {
+        const int rows = (win.HO + bands - 1) / bands;
+        if ((win.HO + rows - 1) / rows != bands) continue;
+        const double length = (double)((rows * win.WO + TR - 1) / TR + (halo * win.WO + TR - 1) / TR) / tiles;
+        const double cost = banded(bands, length);
+        if (cost < 0.95 * best_cost) { share = Share{1, bands, rows, halo}; best_cost = cost; }
+    }
+    return share;
+}
+
+template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
+hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
+                                float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
+                                const Pieces& pieces, hipStream_t stream) {
+    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 1, win.HO, 0, 0, 0, 0, pieces.block, pieces.chunk};
+    d.tiles_k = tiles_of(pr, win, IMG);
+    d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
+    const long pairs = (long)d.tiles_k * d.G;
     if constexpr (IMG) {
-        // Few images leave CUs without work, or the last of them without enough.  An image is then cut into bands of output
-        // rows, a workgroup for each: a band owns the image rows that no later window reaches, and walks the windows of
-        // `halo_rows` more output rows above its own, which reach into them, without adding those to grad_weight.  Forward and both
-        // gradients, us, 32 x 32 images, p = 8: 128 of 3 -> 32 channels 226 -> 121 (128 workgroups before), 16 of 32 -> 32 345 -> 151,
-        // 48 465 -> 350, 20 of 64 -> 64 650 -> 467; where three workgroups to the CU come out even anyway (77 of 32 -> 32: 596, 599)
-        // the image stays whole.
-        const int tiles = (pr.HW + TR - 1) / TR, halo = 2 * win.D / win.S;
-        auto banded = [&](int bands, double length) {   // a CU with a single workgroup runs at 0.6 of the rate of several
-            const long on_busiest = ((long)pr.B * bands * pairs + pr.num_cu - 1) / pr.num_cu;
-            return (on_busiest == 1 ? 1.0 / 0.6 : (double)on_busiest) * (length + fixed) + 0.5 * length;
-        };
-        best_cost = banded(1, 1.0);
-        for (int bands = 2; bands <= std::min(16, win.HO) && best == 1; bands++) {
-            const int rows = (win.HO + bands - 1) / bands;
-            if ((win.HO + rows - 1) / rows != bands) continue;
-            const double length = (double)((rows * win.WO + TR - 1) / TR + (halo * win.WO + TR - 1) / TR) / tiles;
-            const double cost = banded(bands, length);
-            if (cost < 0.95 * best_cost) { d.bands = bands; d.band_rows = rows; d.halo_rows = halo; best_cost = cost; }
-        }
+        d.ring_rows = ring_rows_for(win, pr.HW);
+        d.park_extra = park_extra(d.chunk);
+    }
+    const size_t lds = lds_of(pieces, win, pr.HW, IMG);
+    const Share share = share_of(pr, win, IMG, (long)d.tiles_k * d.G, lds, WAVES);
+    d.units_per_wg = share.units_per_wg;
+    if constexpr (IMG) {
+        d.bands = share.bands;
+        d.band_rows = share.band_rows;
+        d.halo_rows = share.halo_rows;
         d.units *= d.bands;
     }
     const long slices = (d.units + d.units_per_wg - 1) / d.units_per_wg;
@@ -664,22 +710,12 @@ template <bool IMG, int IE>
 hipError_t launch_conv_backward(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 hipStream_t stream) {
-    // The fewest pieces with which a CU still holds as many workgroups as the launch has for it (three at most).  Pieces buy
-    // room for more of them and cost a barrier per chunk and a walk over the rows per block; where the launch cannot use the
-    // room they only cost: 44 images of 28 x 25 x 32 to 67 outputs, p = 20.5 (176 workgroups), 568 us in two blocks, 472 whole;
-    // 41 of 9 x 30 x 31 to 78, p = 1.5, 768 and 607; 79 of 12 x 7 x 31 to 33, p = 20.5, 88 and 84.
-    const long units = IMG ? pr.B : ((long)pr.B * pr.HW + TR - 1) / TR;
-    const long wgs = units * (IMG ? (win.CG + kPlanes - 1) / kPlanes : (pr.K + TCP - 1) / TCP) * pr.G;
-    const long wanted = std::min(3L, (wgs + pr.num_cu - 1) / pr.num_cu);
-    const int ring_rows = IMG ? ring_rows_for(win, pr.HW) : 0;
-    Pieces pieces = least_pieces(pr.NG);
-    auto lds_of = [&](const Pieces& c) { return lds_bytes(c, IMG ? image_floats(c.chunk, ring_rows, win.H, win.W) : 0); };
-    for (const Pieces& c : {Pieces{pr.NG, pr.NG}, Pieces{pr.NG, outputs_staged(pr.NG)}})
-        if (lds_of(c) <= kMaxLds && on_a_cu(lds_of(c)) >= wanted) { pieces = c; break; }
+    const Pieces pieces = pieces_of(pr, win, IMG);
+    const bool four = waves_of(pieces, pr, win, IMG) == 4;
 #define LDIST_LAUNCH(BLOCKS, WAVES, HALF) \
     launch_conv_backward_blocks<IMG, IE, BLOCKS, WAVES, HALF>(grad_output, input, weight, output, grad_input, grad_weight, p, pr, win, pieces, stream)
     if (pieces.block < pr.NG) return LDIST_LAUNCH(true, 3, IMG);
-    if (pieces.chunk < pr.NG || on_a_cu(lds_of(pieces)) < 4) return LDIST_LAUNCH(false, 3, IMG);
+    if (!four) return LDIST_LAUNCH(false, 3, IMG);
     // Halving shortens the launch where every column tile is halved; beside whole tiles, which take as long as before, it only
     // costs its registers (6 % of four-output layers, nothing gained by any with 2 to 17 column tiles).
     if (IMG && win.CG * 9 <= TCP / 2) return LDIST_LAUNCH(false, 4, IMG);
@@ -752,6 +788,14 @@ bool norm_conv_backward_fused_image_applicable(const ConvGeom& q, int G, int CO,
     const int tiles_k = (win.CG + kPlanes - 1) / kPlanes, last = win.CG - kPlanes * (tiles_k - 1), L = q.HO * q.WO;
     const double here = (tiles_k - 1) * TCP + (last * 9 <= TCP / 2 ? TCP / 2 : TCP), there = (win.CG * 9 + 63) / 64 * 64;
     return blocks_pay(q.B, tiles_k, G, there / here * L / ((L + TR - 1) / TR * TR), p, num_cu);
+}
+
+int norm_conv_backward_bands(const ConvGeom& q, int G, int CO, float p, int num_cu) {
+    if (!norm_conv_backward_fused_image_applicable(q, G, CO, p, num_cu)) return 0;
+    const Problem pr{q.B, G, q.C / G * 9, CO / G, q.HO * q.WO, num_cu, 0};
+    const ImgWin win{q.C, q.C / G, q.H, q.W, q.HO, q.WO, q.S, q.P, q.D};
+    const Pieces pieces = pieces_of(pr, win, true);
+    return share_of(pr, win, true, (long)tiles_of(pr, win, true) * G, lds_of(pieces, win, pr.HW, true), waves_of(pieces, pr, win, true)).bands;
 }
 
 // From the unfolded input (B, CI, HW): every element of grad_input is written, grad_weight is added to.
