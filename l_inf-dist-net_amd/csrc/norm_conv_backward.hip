@@ -38,6 +38,7 @@
 #include "wave_reduce.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ldist {
 
@@ -49,19 +50,24 @@ constexpr int WLD = TCP;            // row length of the weight and grad_weight 
 constexpr int TI = 8, TJ = 2;       // a lane's patch: rows x columns; 64 / TI lanes share a column pair, inside one DPP row
 constexpr int kPlanes = 7;          // IMG: channels per tile (63 columns)
 constexpr size_t kMaxLds = 159 * 1024;   // all of LDS less the kernel's own static words
+constexpr int kInBands = 16;        // POWER below
 
 struct ConvBwd {
     int B, G, K, NG, HW, M;          // the unfolded problem: K = 9 channels per group (image) or CI / G
     int tiles_k;                     // column tiles per group
     int units, units_per_wg;         // what a workgroup walks: tiles of 64 rows (columns), bands of images (image)
-    int bands, band_rows;            // IMG: bands of an image, and their output rows
-    int halo_rows;                   // IMG: output rows above a band whose windows reach into the band's image rows
     int ring_rows;                   // IMG: image rows per channel plane held in LDS
     int park_extra;                  // IMG: floats between the 1/out panel and the ring that the parked tile runs into
     int slices;                      // workgroups per (group, column tile): units / units_per_wg, rounded up
     int block;                       // outputs whose weights and grad_weight sums are in LDS at a time
     int chunk;                       // of which g and 1/out are staged at a time
 };
+
+// Images in bands: how many, their output rows, and the output rows above a band whose windows reach into its image rows.
+struct Bands { int bands, band_rows, halo_rows; };
+struct ConvBwdInBands : ConvBwd, Bands {};
+__device__ __forceinline__ Bands bands_of(const ConvBwd&) { return {1, 0, 0}; }
+__device__ __forceinline__ Bands bands_of(const ConvBwdInBands& d) { return d; }
 
 // A group's outputs are taken in equal blocks of up to 64, one after the other over the same units, where the device has
 // workgroups for the room this makes: the two tiles of 128 outputs leave room for one per CU.  grad_input has one owner all
@@ -114,12 +120,18 @@ inline long on_a_cu(size_t lds) { return (long)(160 * 1024 / ((lds + 256 + 1279)
 // 1024 positions to 20 outputs, p = 4, 61 us against 50, 46 images of 14 x 29 x 21 to 6 outputs, p = 62, 90 against 77),
 // and there is no halving where not every tile can be halved.
 // HALF: column tiles of at most half the width are shared by two halves of the workgroup (below).
-template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
+// POWER: IE, plus kInBands where images are cut into bands of output rows (an instantiation of its own: what bands need took 1 to
+// 8 % of the time of launches without any; 179 images of 65 x 23 x 20 to 8 outputs, p = 8, 163 -> 175 us, 128 of 64 x 16 x 16 to 64,
+// p = 37.3, 426 -> 444).
+template <bool IMG, int POWER, bool BLOCKS, int WAVES, bool HALF>
 __global__ void __launch_bounds__(256, WAVES)
 norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __restrict__ input,
                           const float* __restrict__ weight, const float* __restrict__ output,
-                          float* __restrict__ grad_input, float* __restrict__ grad_weight, float e, ConvBwd d,
-                          ImgWin win) {
+                          float* __restrict__ grad_input, float* __restrict__ grad_weight, float e,
+                          typename std::conditional<(POWER >= kInBands), ConvBwdInBands, ConvBwd>::type d, ImgWin win) {
+    constexpr bool BANDS = POWER >= kInBands;
+    constexpr int IE = BANDS ? POWER - kInBands : POWER;
+    const Bands cut = bands_of(d);
     constexpr int TC = IMG ? 9 * kPlanes : TCP;   // columns per tile
     constexpr bool ONE_CHUNK = WAVES == 4;        // the whole group is staged at once
     extern __shared__ __align__(16) float lds[];
@@ -180,14 +192,14 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
     if (IE == 0 && nb == 0) {
         float top = 0.f, nbot = -__builtin_inff();   // the largest and minus the smallest output of the first tile
         if (u_begin < u_end) {
-            const int first_pos = IMG ? u_begin % d.bands * d.band_rows * win.WO : 0;
+            const int first_pos = BANDS ? u_begin % cut.bands * cut.band_rows * win.WO : 0;
             const int rows = IMG ? min(TR, d.HW - first_pos) : min(TR, d.M - u_begin * TR);
             for (int i = tid; i < NG * TR; i += 256) {
                 const int n = i / TR, r = i % TR;
                 if (r < rows) {
                     size_t o;
                     if constexpr (IMG) {
-                        o = ((size_t)(u_begin / d.bands * d.G + g) * d.NG + n) * d.HW + first_pos + r;
+                        o = ((size_t)((BANDS ? u_begin / cut.bands : u_begin) * d.G + g) * d.NG + n) * d.HW + first_pos + r;
                     } else {
                         const int m = u_begin * TR + r, bi = m / d.HW;
                         o = ((size_t)(bi * d.G + g) * d.NG + n) * d.HW + (m - bi * d.HW);
@@ -389,7 +401,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 float tot[TJ];
 #pragma unroll
                 for (int j = 0; j < TJ; j++) tot[j] = dpp_lanes_total<TYN>(s[j]);
-                if (ty == TYN - 1 && (!IMG || own)) {   // d/dw of |x - w| is minus d/dx
+                if (ty == TYN - 1 && (!BANDS || own)) {   // d/dw of |x - w| is minus d/dx
                     float* gp = Gw + (nc + n) * WLD + tx * TJ;
                     if constexpr (TJ == 4) {
                         float4 v = *reinterpret_cast<float4*>(gp);
@@ -436,12 +448,12 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
         const float inv_w = 1.0f / (float)W, inv_r = 1.0f / (float)R;
         auto ring_row = [&](int h) { return h - R * (int)(((float)h + 0.5f) * inv_r); };   // h modulo R
         for (int u = u_begin; u < u_end; u++) {
-            const int b = u / d.bands, band = u - b * d.bands;
+            const int b = BANDS ? u / cut.bands : u, band = BANDS ? u - b * cut.bands : 0;
             // the band's own positions, and from where its windows reach into the image rows that it owns
-            const int pos_own = band * d.band_rows * win.WO, pos_end = min(d.HW, pos_own + d.band_rows * win.WO);
-            const int pos_first = max(0, pos_own - d.halo_rows * win.WO);
-            const int h_own = band == 0 ? 0 : min(H, max(0, band * d.band_rows * win.S - win.P));
-            const int h_end = pos_end == d.HW ? H : min(H, max(0, (band + 1) * d.band_rows * win.S - win.P));
+            const int pos_own = BANDS ? band * cut.band_rows * win.WO : 0, pos_end = BANDS ? min(d.HW, pos_own + cut.band_rows * win.WO) : d.HW;
+            const int pos_first = BANDS ? max(0, pos_own - cut.halo_rows * win.WO) : 0;
+            const int h_own = band == 0 ? 0 : min(H, max(0, band * cut.band_rows * win.S - win.P));
+            const int h_end = !BANDS || pos_end == d.HW ? H : min(H, max(0, (band + 1) * cut.band_rows * win.S - win.P));
             float* dst = grad_input + ((size_t)b * win.C + g * win.CG + first_ch) * H * W;
             // Writes image rows h_from .. h_to - 1 of the planes to memory and clears their ring rows.  Rows more than
             // a ring away from h_from have never been touched (the windows reach less far): they are zero.
@@ -477,14 +489,24 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                     wrow[i].w0 = wo * win.S - win.P;
                 }
             };
-            corners(pos_first);
+            if constexpr (BANDS) {
+                corners(pos_first);
+            } else {   // not corners(0), for which the compiler orders the whole kernel otherwise: 2 % slower in blocks and at general exponents
+#pragma unroll
+                for (int i = 0; i < TI; i++) {
+                    const int ho = (ty * TI + i) / win.WO, wo = (ty * TI + i) - ho * win.WO;
+                    wrow[i].b = b;
+                    wrow[i].h0 = ho * win.S - win.P;
+                    wrow[i].w0 = wo * win.S - win.P;
+                }
+            }
             const int step_rows = TR / win.WO;
             const int step_h = step_rows * win.S, step_w = (TR - step_rows * win.WO) * win.S;
             const int wrap_w = win.WO * win.S, end_w = wrap_w - win.P;   // a corner's column stays below end_w
             int flushed = h_own;   // of the band's image rows those below this one are in memory
-            int rows = 0;
-            for (int pos0 = pos_first; pos0 < pos_end; pos0 += rows) {
-                if (pos0 == pos_own && pos0 > pos_first) {
+            int step = TR;   // a band's halo ends with a shorter tile
+            for (int pos0 = pos_first; pos0 < pos_end; pos0 += BANDS ? step : TR) {
+                if (BANDS && pos0 == pos_own && pos0 > pos_first) {
                     corners(pos0);
                 } else if (pos0 > pos_first) {
 #pragma unroll
@@ -494,8 +516,9 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                         if (wrow[i].w0 >= end_w) { wrow[i].w0 -= wrap_w; wrow[i].h0 += win.S; }
                     }
                 }
-                const bool own = pos0 >= pos_own;
-                rows = min(TR, (own ? pos_end : pos_own) - pos0);
+                const bool own = !BANDS || pos0 >= pos_own;
+                const int rows = min(TR, (own ? pos_end : pos_own) - pos0);
+                if (BANDS) step = rows;
                 tile(0, rows, b, pos0, own, acc, wrow, xoff);
                 // rows above this tile's first window are final (the last tile's rounds ended with a barrier)
                 const int h_lo = min(h_end, max(flushed, (pos0 / win.WO) * win.S - win.P));
@@ -525,7 +548,7 @@ norm_conv_backward_kernel(const float* __restrict__ grad_output, const float* __
                 const int last = pos0 + rows - 1;
                 const int h_first = max(h_own, (pos0 / win.WO) * win.S - win.P);
                 const int h_last = min(h_end - 1, (last / win.WO) * win.S - win.P + 2 * win.D);
-                const int nrow = max(0, h_last - h_first + 1);
+                const int nrow = BANDS ? max(0, h_last - h_first + 1) : h_last - h_first + 1;
                 const float inv_nrow = 1.0f / (float)nrow;
                 for (int i = tid; i < planes * nrow * W; i += 256) {
                     // i = (c * nrow + hr) * W + w; quotients of small numbers through the reciprocal
@@ -619,7 +642,7 @@ int waves_of(const Pieces& pieces, const Problem& pr, const ImgWin& win, bool im
     return pieces.chunk == pr.NG && on_a_cu(lds_of(pieces, win, pr.HW, img)) >= 4 ? 4 : 3;
 }
 
-struct Share { int units_per_wg, bands, band_rows, halo_rows; };   // of a launch: units per workgroup, and ConvBwd's bands
+struct Share { int units_per_wg; Bands cut; };   // of a launch
 
 Share share_of(const Problem& pr, const ImgWin& win, bool img, long pairs, size_t lds, int waves) {
     const long units = img ? pr.B : ((long)pr.B * pr.HW + TR - 1) / TR;
@@ -643,7 +666,7 @@ Share share_of(const Problem& pr, const ImgWin& win, bool img, long pairs, size_
         const double cost = (double)((wgs + pr.num_cu - 1) / pr.num_cu) * ((double)upw + fixed) + 0.5 * (double)upw;
         if (best < 0 || cost < best_cost) { best = upw; best_cost = cost; }
     }
-    Share share{(int)best, 1, win.HO, 0};
+    Share share{(int)best, {1, win.HO, 0}};
     if (!img || best > 1) return share;
     // Few images leave CUs without work, or the last of them without enough.  An image is then cut into bands of output
     // rows, a workgroup for each: a band owns the image rows that no later window reaches, and walks the windows of
@@ -668,7 +691,7 @@ Share share_of(const Problem& pr, const ImgWin& win, bool img, long pairs, size_
         if ((win.HO + rows - 1) / rows != bands) continue;
         const double length = (double)((rows * win.WO + TR - 1) / TR + (halo * win.WO + TR - 1) / TR) / tiles;
         const double cost = banded(bands, length);
-        if (cost < 0.95 * best_cost) { share = Share{1, bands, rows, halo}; best_cost = cost; }
+        if (cost < 0.95 * best_cost) { share.cut = Bands{bands, rows, halo}; best_cost = cost; }
     }
     return share;
 }
@@ -677,7 +700,7 @@ template <bool IMG, int IE, bool BLOCKS, int WAVES, bool HALF>
 hipError_t launch_conv_backward_blocks(const float* grad_output, const float* input, const float* weight, const float* output,
                                 float* grad_input, float* grad_weight, float p, const Problem& pr, const ImgWin& win,
                                 const Pieces& pieces, hipStream_t stream) {
-    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 1, win.HO, 0, 0, 0, 0, pieces.block, pieces.chunk};
+    ConvBwd d{pr.B, pr.G, pr.K, pr.NG, pr.HW, pr.B * pr.HW, 0, 0, 0, 0, 0, 0, pieces.block, pieces.chunk};
     d.tiles_k = tiles_of(pr, win, IMG);
     d.units = IMG ? pr.B : (d.M + TR - 1) / TR;
     const long pairs = (long)d.tiles_k * d.G;
@@ -688,22 +711,22 @@ hipError_t launch_conv_backward_blocks(const float* grad_output, const float* in
     const size_t lds = lds_of(pieces, win, pr.HW, IMG);
     const Share share = share_of(pr, win, IMG, (long)d.tiles_k * d.G, lds, WAVES);
     d.units_per_wg = share.units_per_wg;
-    if constexpr (IMG) {
-        d.bands = share.bands;
-        d.band_rows = share.band_rows;
-        d.halo_rows = share.halo_rows;
-        d.units *= d.bands;
-    }
+    d.units *= share.cut.bands;
     const long slices = (d.units + d.units_per_wg - 1) / d.units_per_wg;
     d.slices = (int)slices;
     const long grid = (pairs * slices + 7) / 8 * 8;   // whole rounds of the eight XCDs; the padding exits at once
-    auto kern = norm_conv_backward_kernel<IMG, IE, BLOCKS, WAVES, HALF>;
-    static LdsRecord lds_allowed = {};
-    // the limit is raised once, to the most any layer may ask for
-    if (hipError_t e = allow_lds(kern, kMaxLds, pr.device, lds_allowed); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, grad_output, input, weight,
-                       output, grad_input, grad_weight, p - 1.0f, d, win);
-    return hipGetLastError();
+    auto launch = [&](auto kern, LdsRecord& lds_allowed, const auto& args) {
+        // the limit is raised once, to the most any layer may ask for
+        if (hipError_t e = allow_lds(kern, kMaxLds, pr.device, lds_allowed); e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, grad_output, input, weight,
+                           output, grad_input, grad_weight, p - 1.0f, args, win);
+        return hipGetLastError();
+    };
+    static LdsRecord whole = {}, bands = {};
+    if constexpr (IMG)
+        if (share.cut.bands > 1)
+            return launch(norm_conv_backward_kernel<true, IE + kInBands, BLOCKS, WAVES, HALF>, bands, ConvBwdInBands{d, share.cut});
+    return launch(norm_conv_backward_kernel<IMG, IE, BLOCKS, WAVES, HALF>, whole, d);
 }
 
 template <bool IMG, int IE>
@@ -795,7 +818,7 @@ int norm_conv_backward_bands(const ConvGeom& q, int G, int CO, float p, int num_
     const Problem pr{q.B, G, q.C / G * 9, CO / G, q.HO * q.WO, num_cu, 0};
     const ImgWin win{q.C, q.C / G, q.H, q.W, q.HO, q.WO, q.S, q.P, q.D};
     const Pieces pieces = pieces_of(pr, win, true);
-    return share_of(pr, win, true, (long)tiles_of(pr, win, true) * G, lds_of(pieces, win, pr.HW, true), waves_of(pieces, pr, win, true)).bands;
+    return share_of(pr, win, true, (long)tiles_of(pr, win, true) * G, lds_of(pieces, win, pr.HW, true), waves_of(pieces, pr, win, true)).cut.bands;
 }
 
 // From the unfolded input (B, CI, HW): every element of grad_input is written, grad_weight is added to.

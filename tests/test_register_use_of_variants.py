@@ -1,0 +1,19 @@
+"""Scratch memory of instantiations that stand beside others of the same kernel, as the compiler reports it for the library's own
+flags (no GPU needed): what a rarer form needs must not cost the usual one its registers."""
+import re
+import shutil
+
+import pytest
+
+from test_register_use import scratch_of
+
+pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not on PATH")
+
+
+def test_conv_backward_of_whole_images_beside_bands(tmp_path):
+    """Four waves per SIMD, multiply-only exponents: 60 bytes without bands of images, 72 in the one form that has them."""
+    sizes = scratch_of("norm_conv_backward.hip", tmp_path)
+    whole = [size for name, size in sizes.items() if re.search(r"norm_conv_backward_kernelILb1ELi[1-9]ELb0ELi4E", name)]
+    bands = [size for name, size in sizes.items() if re.search(r"norm_conv_backward_kernelILb1ELi(?:16|17|18|19|23)ELb0ELi4E", name)]
+    assert len(whole) == 8 and max(whole) <= 60
+    assert len(bands) == 10 and max(bands) <= 72
