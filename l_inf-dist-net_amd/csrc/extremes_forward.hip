@@ -423,10 +423,11 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
 // (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly,
 // unless more values tie at the outer end than the list has places: such a row's bounds are those of all its values.
 // Bound by reading the operands once.
-// SPREAD: no positions follow (its own instantiation: the code of both orders in one made the kernel 43 -> 48 us).
+// SPREAD: no positions follow, and the order of a list is free (its own instantiation: the code of both orders in one made the
+// kernel 43 -> 48 us).
 template <int NV, int ENDS, bool SPREAD>
 __global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_select_kernel(Search s) {
-    extern __shared__ __align__(16) char stage[];   // [2 kMaxList][8] entries: half of a block of Side::lists, and what `place` finds no place for
+    extern __shared__ __align__(16) char stage[];   // [2 kMaxList][8] entries: half of a block of Side::lists, and what finds no place in its order
     __shared__ int sums[8][64];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int ix, iw, dense;
@@ -516,28 +517,12 @@ __global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_sel
         struct Ends { float a, b, c; } first = {};
         int base = 0;
         float most = -kNever, least = kNever, most_lower = -kNever, least_upper = kNever, most_point = -kNever, least_point = kNever;
-        // Without positions the order of a list is free: entry s of row r is one with k = s + r / 2 (mod 8) where the row has such
-        // an entry left, so that 16 neighbouring lanes of a scan read from different banks.
-        constexpr bool spread = SPREAD;
-        int of_class = 0, over = 0;   // entries with this lane's k mod 8; those beyond an eighth of the list, behind it in `stage`
         auto before = [](unsigned long long m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0)); };
         auto place = [&](bool in, int j, auto&& write) {
             const unsigned long long m = __ballot(in);
             if (m) {
-                int at;
-                if constexpr (spread) {
-                    const unsigned long long mine = m & (0x0101010101010101ull << (lane & 7));
-                    const int rank = of_class + before(mine);
-                    const unsigned long long beyond = __ballot(in && rank >= q / 8);
-                    at = rank >= q / 8 ? kMaxList + min(over + before(beyond), q) : rank * 8 + ((lane - (r >> 1)) & 7);
-                    in = in && at < kMaxList + q;
-                    over += __builtin_popcountll(beyond);
-                    of_class += __builtin_popcountll(mine);
-                } else {
-                    at = base + before(m);
-                    in = in && at < q;
-                }
-                if (in) write(at * 8 + wave, (unsigned)(lane + j * 64) * 32u);
+                const int at = base + before(m);
+                if (in && at < q) write(at * 8 + wave, (unsigned)(lane + j * 64) * 32u);
                 base += __builtin_popcountll(m);
             }
         };
@@ -610,15 +595,50 @@ __global__ void __launch_bounds__(512, ENDS > 1 || NV > 24 ? 4 : 6) extremes_sel
             if constexpr (P) return make_uint4(v0, __shfl(__float_as_uint(first.b), from), (unsigned)from * 32u, __shfl(__float_as_uint(first.c), from));
             else return make_uint2(v0, (unsigned)from * 32u);
         };
-        if constexpr (spread) {
-            int vacant = 0;
+        if constexpr (SPREAD) {
+            // Entry s of row r becomes one with k = s + r / 2 (mod 8) where the row has such an entry left, so that 16 neighbouring lanes
+            // of a scan read from different banks.  Done on the finished list, 64 entries at a time: where every 64 values were put in
+            // order as they were found, with lists for both operands the kernel took 28 instead of 24 us of 512 x 3072 -> 5120, 44 instead
+            // of 37 with 5120 inputs, 59 instead of 51 for boxes at batch 1024 (20, 35 and 56 in the order of k).
+            const int n = min(base, q);
+            int of_class = 0, over = 0, vacant = 0;   // entries with this lane's k mod 8; those beyond an eighth of the list, kept behind it
+            Entry own[kMaxList / 64];
+#pragma unroll
+            for (int i = 0; i < kMaxList / 64; i++) own[i] = i * 64 + lane < n ? mine[(i * 64 + lane) * 8] : Entry{};
+            __builtin_amdgcn_wave_barrier();   // all of them, before the first is overwritten
+#pragma unroll
+            for (int i = 0; i < kMaxList / 64; i++) {
+                if (i * 64 >= n) break;
+                unsigned k32;
+                if constexpr (P) k32 = own[i].z;
+                else k32 = own[i].y;
+                const unsigned long long all = __ballot(i * 64 + lane < n);
+                unsigned long long bit[3];
+#pragma unroll
+                for (int b = 0; b < 3; b++) bit[b] = __ballot(k32 >> (5 + b) & 1u);
+                auto of = [&](unsigned c) {   // which of the 64 have k mod 8 = c
+                    unsigned long long m = all;
+#pragma unroll
+                    for (int b = 0; b < 3; b++) m &= c >> b & 1u ? bit[b] : ~bit[b];
+                    return m;
+                };
+                const unsigned c = k32 >> 5 & 7u;
+                const int rank = __shfl(of_class, (int)c) + before(of(c));
+                const bool in = i * 64 + lane < n;
+                const unsigned long long beyond = __ballot(in && rank >= q / 8);
+                if (in) mine[(rank >= q / 8 ? kMaxList + over + before(beyond) : rank * 8 + (((int)c - (r >> 1)) & 7)) * 8] = own[i];
+                over += __builtin_popcountll(beyond);
+                of_class += __builtin_popcountll(of(lane & 7u));
+            }
+            __builtin_amdgcn_wave_barrier();
             for (int e0 = 0; e0 < q; e0 += 64) {
                 const int e = e0 + lane, from = (e + (r >> 1)) & 7;
                 const bool free = e < q && e / 8 >= __shfl(of_class, from);
                 const unsigned long long m = __ballot(free);
-                const int n = vacant + before(m);
-                const Entry pad = entry_of(from < kc ? from : 0);
-                if (free) mine[e * 8] = n < over ? mine[(kMaxList + n) * 8] : pad;
+                const int nth = vacant + before(m);
+                Entry put = entry_of(from < kc ? from : 0);
+                if (free && nth < over) put = mine[(kMaxList + nth) * 8];   // a conditional expression would choose between their addresses: the pad in memory
+                if (free) mine[e * 8] = put;
                 vacant += __builtin_popcountll(m);
             }
         } else {

@@ -17,3 +17,10 @@ def test_conv_backward_of_whole_images_beside_bands(tmp_path):
     bands = [size for name, size in sizes.items() if re.search(r"norm_conv_backward_kernelILb1ELi(?:16|17|18|19|23)ELb0ELi4E", name)]
     assert len(whole) == 8 and max(whole) <= 60
     assert len(bands) == 10 and max(bands) <= 72
+
+
+def test_lists_of_outermost_values(tmp_path):
+    """extremes_select_kernel<NV, ENDS, SPREAD> of up to 32 values per lane: no scratch memory in any form."""
+    sizes = {name: size for name, size in scratch_of("extremes_forward.hip", tmp_path).items()
+             if re.search(r"extremes_select_kernelILi(?:16|24|32)E", name)}
+    assert len(sizes) == 12 and max(sizes.values()) == 0
