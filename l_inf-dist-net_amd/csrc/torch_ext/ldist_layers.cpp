@@ -593,10 +593,11 @@ bool value_bounds_pay(int64_t B, int64_t CO, int64_t CI, int64_t G) {
     return B <= INT_MAX && ldist_inf_dist_value_bound_workspace((int)B, (int)CO, (int)CI, (int)G, 1, &bytes) == LDIST_OK && bytes > 0;
 }
 
-// Values and bounds in one pass, for layers without a window: those with few outputs, and those of `value_bounds_pay`.
-std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Tensor& lower, const Tensor& upper,
-                                                      const Tensor& weight, const OptTensor& bias, const OptTensor& running,
-                                                      int64_t G) {
+// Values and bounds in one pass, for layers without a window: those with few outputs, and those of `value_bounds_pay`.  And
+// whether it was one pass.
+std::tuple<Tensor, Tensor, Tensor, bool> layer_value_bounds(const Tensor& x, const Tensor& lower, const Tensor& upper,
+                                                            const Tensor& weight, const OptTensor& bias, const OptTensor& running,
+                                                            int64_t G) {
     at::NoGradGuard no_grad;
     const Tensor w = weight.contiguous(), cx = as_columns(x), cl = as_columns(lower), cu = as_columns(upper);
     check(cx, "input", w.device());
@@ -612,6 +613,7 @@ std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Ten
     int64_t bytes = 0;
     done("inf_dist_value_bound_workspace", ldist_inf_dist_value_bound_workspace(s.B, s.CO, s.CI, (int)G, s.HW, &bytes));
     Tensor y = torch::empty(s.output(), cx.options()), lo = torch::empty_like(y), hi = torch::empty_like(y);
+    bool together = true;
     if (bytes == 0) {
         done("inf_dist_value_bound_forward",
              ldist_inf_dist_value_bound_forward(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G, s.HW, in(running), in(bias),
@@ -622,7 +624,8 @@ std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Ten
                                      : ldist_inf_dist_value_bound_forward_ws(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G,
                                                                              s.HW, in(running), in(bias), out(y), out(lo), out(hi),
                                                                              ws.data_ptr(), ws.numel(), on.stream);
-        if (rc == LDIST_EUNSUPPORTED) {   // no memory for it, or no 128-bit loads: one pass after the other
+        together = rc != LDIST_EUNSUPPORTED;
+        if (!together) {   // no memory for it, or no 128-bit loads: one pass after the other
             const Shift shift = make_shift(running, 0.0, false, cx.device());
             y = distances(on, cx, w, G, INFINITY, bias, shift);
             std::tie(lo, hi) = bounds_of_columns(cl, cu, w, G, bias, shift);
@@ -630,7 +633,7 @@ std::tuple<Tensor, Tensor, Tensor> layer_value_bounds(const Tensor& x, const Ten
             done("inf_dist_value_bound_forward", rc);
         }
     }
-    return {as_output(y, x, win), as_output(lo, x, win), as_output(hi, x, win)};
+    return {as_output(y, x, win), as_output(lo, x, win), as_output(hi, x, win), together};
 }
 
 // Certified margins (BoundFinalIdentity) with gradients to both bounds.
