@@ -619,13 +619,14 @@ std::tuple<Tensor, Tensor, Tensor, bool> layer_value_bounds(const Tensor& x, con
              ldist_inf_dist_value_bound_forward(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G, s.HW, in(running), in(bias),
                                                 out(y), out(lo), out(hi), on.stream));
     } else {
-        const Tensor ws = ldist_torch::scratch(bytes, cx);
+        Tensor ws = ldist_torch::scratch(bytes, cx);
         const int rc = !ws.defined() ? LDIST_EUNSUPPORTED
                                      : ldist_inf_dist_value_bound_forward_ws(in(cx), in(cl), in(cu), in(w), s.B, s.CO, s.CI, (int)G,
                                                                              s.HW, in(running), in(bias), out(y), out(lo), out(hi),
                                                                              ws.data_ptr(), ws.numel(), on.stream);
         together = rc != LDIST_EUNSUPPORTED;
-        if (!together) {   // no memory for it, or no 128-bit loads: one pass after the other
+        if (!together) {   // no memory for it, or no 128-bit loads: one pass after the other, in the memory that they need by themselves
+            ws = y = lo = hi = Tensor();
             const Shift shift = make_shift(running, 0.0, false, cx.device());
             y = distances(on, cx, w, G, INFINITY, bias, shift);
             std::tie(lo, hi) = bounds_of_columns(cl, cu, w, G, bias, shift);

@@ -1,5 +1,5 @@
 """Values and bounds of a wide layer where the one pass through lists of outermost values (csrc/extremes_forward.hip) cannot be
-taken, or is taken in parts: the same results, bit for bit, as without lists."""
+taken, or is taken in parts: the same results, bit for bit, as without lists, and in no more memory than two passes need."""
 import ctypes
 
 import pytest
@@ -96,3 +96,33 @@ def test_tensors_that_128_bit_loads_do_not_reach(which):
     assert layer.last_route == (TWO if which in (0, 3) else ONE_PASS)   # the boxes are read in single words
     for a, b in zip(got, in_full(layer, *tensors[:3])):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_no_memory_for_the_scratch():
+    """An allocator that has room for three results, and neither for the lists beside them nor for a fourth."""
+    from gpu_common import DEV, say
+    B, CO, CI = 1024, 5120, 5120
+    result = B * CO * 4
+    say("values and bounds without memory")
+    layer, x = layer_and_inputs(B, CO, CI)
+    triple = (x, x - 0.1, x + 0.1)
+    want = [t.cpu() for t in layer(*triple)]
+    assert layer.last_route == ONE_PASS and workspace(B, CO, CI) > 2 * result
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 3 * result + (16 << 20)) / total)
+    try:
+        held = []                      # what the allocator has free inside its segments, and what was put aside for the results
+        with pytest.raises(torch.OutOfMemoryError):
+            while len(held) < 1000:
+                held.append(torch.empty(result, dtype=torch.uint8, device=DEV))
+        del held[-3:]
+        got = layer(*triple)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert layer.last_route == TWO
+    for a, b in zip(got, want):
+        assert torch.equal(a.cpu(), b)
