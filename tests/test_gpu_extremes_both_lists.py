@@ -1,0 +1,79 @@
+"""Lists of outermost values (csrc/extremes_forward.hip) where both operands have them, so that what the first scan leaves is taken
+up by the second ones, and where the weights have none, so that the first scan checks the bounds: which of the two it was is read
+back from the header of the workspace.  Forced onto layers at the edges of strips, list blocks, lane groups and chunks; bit for
+bit."""
+import ctypes
+
+import pytest
+import torch
+
+import oracle
+from helpers import gen
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(70, 100, 2560), (33, 81, 2564), (65, 41, 1540), (17, 257, 1028), (260, 48, 5200), (515, 23, 1300), (20, 530, 5124)]
+FORMS = ["positions", "values", "bounds", "values and bounds"]
+
+
+@pytest.fixture(autouse=True)
+def _reset():
+    from gpu_common import pkg
+    yield
+    pkg._lib.lib().ldist_set_extremes(-1)
+
+
+def run(form, x, lo, up, w):
+    """Results, and the lengths of the two operands' lists."""
+    from gpu_common import DEV, pkg
+    lib = pkg._lib.lib()
+    B, K, CO = x.size(0), x.size(1), w.size(0)
+    x, lo, up, w = (t.contiguous().to(DEV) for t in (x, lo, up, w))
+    at = lambda t: ctypes.c_void_p(t.data_ptr())
+    need, sizes = ctypes.c_int64(), (B, CO, K, 1, 1)
+    if form == "values and bounds":
+        assert lib.ldist_inf_dist_value_bound_workspace(*sizes, ctypes.byref(need)) == 0
+    else:
+        assert lib.ldist_inf_dist_workspace(*sizes, FORMS.index(form), ctypes.byref(need)) == 0
+    assert need.value > 0
+    space = torch.empty(need.value, dtype=torch.uint8, device=DEV)
+    out = [torch.full((B, CO), float("nan"), device=DEV) for _ in range(3)]
+    pos = torch.full((B, CO), -7, dtype=torch.int32, device=DEV)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    last = (at(space), need.value, stream)
+    if form == "values and bounds":
+        rc = lib.ldist_inf_dist_value_bound_forward_ws(at(x), at(lo), at(up), at(w), *sizes, None, None, at(out[0]), at(out[1]),
+                                                       at(out[2]), *last)
+    elif form == "bounds":
+        rc = lib.ldist_inf_dist_bound_forward_ws(at(lo), at(up), at(w), *sizes, at(out[0]), at(out[1]), *last)
+    else:
+        rc = lib.ldist_inf_dist_forward_ws(at(x), at(w), *sizes, at(out[0]), at(pos) if form == "positions" else None, *last)
+    assert rc == 0
+    _, qx, qw = space[:12].view(torch.int32).tolist()   # Header: center, qx, qw
+    return [t.cpu() for t in out], pos.cpu(), qx, qw
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("lists", ["both", "x alone"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_forced_lists(shape, lists, form):
+    from gpu_common import pkg, say
+    B, CO, K = shape
+    say("extremes, lists of", lists, form, shape)
+    x, w = torch.randn(B, K, generator=gen(1)), torch.randn(CO, K, generator=gen(2)) * (1.0 if lists == "both" else 0.01)
+    lo, up = x - 0.05, x + 0.05
+    assert pkg._lib.lib().ldist_set_extremes(1) == 0
+    (a, b, c), pos, qx, qw = run(form, x, lo, up, w)
+    assert qx > 0 and (qw > 0) == (lists == "both")
+    columns = lambda t: t.view(B, K, 1).contiguous()
+    values, at = oracle.inf_dist_forward(columns(x), w, 1)
+    lower, upper = oracle.inf_dist_bound_forward(columns(lo), columns(up), w, 1)
+    same = lambda got, want: torch.equal(got, want.view(B, CO))
+    if form == "bounds":
+        assert same(a, lower) and same(b, upper)
+    else:
+        assert same(a, values)
+    if form == "positions":
+        assert same(pos, at)
+    if form == "values and bounds":
+        assert same(b, lower) and same(c, upper)
