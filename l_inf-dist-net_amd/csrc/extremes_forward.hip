@@ -50,6 +50,7 @@ constexpr int kBinShift = 15;
 constexpr int kSampled = 64;                 // rows of either operand that the sample looks at
 constexpr int kSampleRows = 4;               // of them in one workgroup
 constexpr int kSampleGroups = kSampled / kSampleRows;
+constexpr int kBoxFails = 1 << 29, kPointFails = 1 << 30;   // beside an index of Search::walk (boxes and points have scratch memory for 2^24 outputs)
 constexpr float kNever = 3.402823466e38f;    // bound of an empty remainder; finite, so that infinite bounds stay infinite beside it
 
 // How many entries of a list are meant to be taken, so that those of rows with a few more still fit.
@@ -86,8 +87,9 @@ struct Search {
     float* partial3;       // [row of x][pitch] of the points' distances
     int pitch;
     int turn;              // which of Header::taken a scan counts in
-    int* walk;             // [walk_most]: indices of outputs that fail
+    int* walk;             // [walk_most]: indices of outputs that fail; boxes and points: with what of them fails
     int walk_most;
+    int note;              // boxes and points: what a scan notes as failing, of its boxes, of its points or both
     int K, C, KC;
     int lanes_first, lanes_second, lanes_only;   // rows per workgroup of the two scans, and of a first that no second follows
     float price_x, price_w, price_both, price_fail, price_dense;   // of a list entry, of a second scan after the first, of an output that does not pass, of the full walk
@@ -1045,7 +1047,7 @@ __global__ void __launch_bounds__(512, 4) extremes_scan_kernel(Search s) {
                     for (int j = 0; j < RS; j++) {
                         const unsigned long long m = __ballot(failed >> j & 1);
                         const int at = first + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-                        if ((failed >> j & 1) && at < s.walk_most) s.walk[at] = index(j);   // more: the full walk follows
+                        if ((failed >> j & 1) && at < s.walk_most) s.walk[at] = index(j) | s.note;   // more: the full walk follows
                         first += __builtin_popcountll(m);
                     }
                 }
@@ -1069,47 +1071,58 @@ __global__ void __launch_bounds__(256) extremes_walk_kernel(Search s) {
     }
     const int lane = threadIdx.x & 63, K = s.K, N = s.w.rows;
     for (int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); i < failed; i += gridDim.x * 4) {
-        const int o = __builtin_amdgcn_readfirstlane(s.walk[i]);
+        const int note = __builtin_amdgcn_readfirstlane(s.walk[i]), o = note & (kBoxFails - 1);
         const float* xr = s.x.v + (size_t)(o / N) * K;
         const float* wr = s.w.v + (size_t)(o % N) * K;
         if constexpr (MODE == kBoxes || MODE == kBoxesAndPoints) {
-            constexpr bool ALL = MODE == kBoxesAndPoints;
-            const float* ur = s.x.v2 + (size_t)(o / N) * K;
-            const float* pr = ALL ? s.x.v3 + (size_t)(o / N) * K : nullptr;
-            float up = 0.f, lo = 0.f, point = 0.f;
-            auto one = [&](float x, float u, float w) {
-                const float tl = x - w, tu = u - w, al = __builtin_fabsf(tl), au = __builtin_fabsf(tu);
-                up = __builtin_fmaxf(up, __builtin_fmaxf(al, au));
-                if (!(tl < 0.f && tu > 0.f)) lo = __builtin_fmaxf(lo, __builtin_fminf(al, au));
-            };
-            for (int kb = 0; kb < K; kb += 256 * 4) {
-                float4_any x[4], u[4], w[4], p[4];
+            auto walk = [&](auto box, auto points) {
+                constexpr bool BOX = decltype(box)::value, POINT = decltype(points)::value;
+                const float* ur = s.x.v2 + (size_t)(o / N) * K;
+                const float* pr = POINT ? s.x.v3 + (size_t)(o / N) * K : nullptr;
+                float up = 0.f, lo = 0.f, point = 0.f;
+                auto one = [&](float x, float u, float w) {
+                    const float tl = x - w, tu = u - w, al = __builtin_fabsf(tl), au = __builtin_fabsf(tu);
+                    up = __builtin_fmaxf(up, __builtin_fmaxf(al, au));
+                    if (!(tl < 0.f && tu > 0.f)) lo = __builtin_fmaxf(lo, __builtin_fminf(al, au));
+                };
+                for (int kb = 0; kb < K; kb += 256 * 4) {
+                    float4_any x[4], u[4], w[4], p[4];
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int k = min(kb + c * 256 + lane * 4, K - 4);   // the last vector is moved back, those past the end repeat it
-                    x[c] = *reinterpret_cast<const float4_any*>(xr + k);
-                    u[c] = *reinterpret_cast<const float4_any*>(ur + k);
-                    if constexpr (ALL) p[c] = *reinterpret_cast<const float4_any*>(pr + k);
-                    w[c] = *reinterpret_cast<const float4_any*>(wr + k);
-                }
-#pragma unroll
-                for (int c = 0; c < 4; c++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        one(x[c].v[e], u[c].v[e], w[c].v[e]);
-                        if constexpr (ALL) point = __builtin_fmaxf(point, __builtin_fabsf(p[c].v[e] - w[c].v[e]));
+                    for (int c = 0; c < 4; c++) {
+                        const int k = min(kb + c * 256 + lane * 4, K - 4);   // the last vector is moved back, those past the end repeat it
+                        if constexpr (BOX) x[c] = *reinterpret_cast<const float4_any*>(xr + k);
+                        if constexpr (BOX) u[c] = *reinterpret_cast<const float4_any*>(ur + k);
+                        if constexpr (POINT) p[c] = *reinterpret_cast<const float4_any*>(pr + k);
+                        w[c] = *reinterpret_cast<const float4_any*>(wr + k);
                     }
-            }
-            up = wave_max(up);
-            lo = wave_max(lo);
-            if (lane == 63) {
-                s.out[o] = shifted_value(s.mean, s.bias, o % N, lo);
-                s.out2[o] = shifted_value(s.mean, s.bias, o % N, up);
-            }
-            if constexpr (ALL) {
-                point = wave_max(point);
-                if (lane == 63) s.out3[o] = shifted_value(s.mean, s.bias, o % N, point);
-            }
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            if constexpr (BOX) one(x[c].v[e], u[c].v[e], w[c].v[e]);
+                            if constexpr (POINT) point = __builtin_fmaxf(point, __builtin_fabsf(p[c].v[e] - w[c].v[e]));
+                        }
+                }
+                if constexpr (BOX) {
+                    up = wave_max(up);
+                    lo = wave_max(lo);
+                    if (lane == 63) {
+                        s.out[o] = shifted_value(s.mean, s.bias, o % N, lo);
+                        s.out2[o] = shifted_value(s.mean, s.bias, o % N, up);
+                    }
+                }
+                if constexpr (POINT) {
+                    point = wave_max(point);
+                    if (lane == 63) s.out3[o] = shifted_value(s.mean, s.bias, o % N, point);
+                }
+            };
+            // The second scans of boxes and of points note an output each, for what it is that fails there: the 23933 outputs of a
+            // trained 1024 x 3072 -> 5120 layer, all of them noted twice, took 228 us with both walked for either note, 119 now.
+            using Yes = std::true_type;
+            using No = std::false_type;
+            if (MODE == kBoxes || (note & (kBoxFails | kPointFails)) == kBoxFails) walk(Yes{}, No{});
+            else if (note & kBoxFails) walk(Yes{}, Yes{});
+            else walk(No{}, Yes{});
         } else {
             float v = 0.f;
             int p = 0;   // k with the sign of the difference
@@ -1153,8 +1166,8 @@ struct Layout {
 
 // More outputs than these go to the full walk; forced lists have none after them.
 size_t walk_most(const Problem& pr, ForwardKind kind) {   // the two second scans of boxes and points may both note an output
-    const size_t outputs = (size_t)pr.B * pr.NG;
-    return g_extremes > 0 ? (kind == ForwardKind::kValueBounds ? 2 : 1) * outputs : outputs / 16;
+    const size_t outputs = (size_t)pr.B * pr.NG * (kind == ForwardKind::kValueBounds ? 2 : 1);
+    return g_extremes > 0 ? outputs : outputs / 16;
 }
 
 Layout layout_of(const Problem& pr, ForwardKind kind) {
@@ -1293,6 +1306,7 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* x3, co
     s.out = out; s.out2 = out2; s.out3 = out3; s.pos = pos;
     s.mean = pr.mean; s.bias = pr.bias;
     s.K = pr.K; s.C = l.C; s.KC = l.KC;
+    s.note = all ? kBoxFails | kPointFails : 0;
     s.lanes_first = lanes_for(pr.B, (pr.NG + 7) / 8, pr.num_cu);
     // Without a list for the weights the lists of x are short, and a strip on its way to LDS costs more than its walk: where two blocks of
     // rows fit a workgroup with an eighth of its lanes to spare, they share it (200 to 448 rows, 5120 -> 5120, a whole pass 91 -> 83 and
@@ -1306,7 +1320,9 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* x3, co
     s.price_w = all ? 3.f : boxes ? 2.f : 1.f;
     s.price_both = all ? 120.f : 60.f;
     // in list entries of one row: a walked output reads two rows, 3 ns with all waves at it, an entry takes 0.1 ps per output; with
-    // points four rows, mostly twice, 20 ns, and 0.2 ps
+    // points five rows in two walks, 10 ns, and 0.2 ps.  The price there is higher than that, for what a sample of 64 x 64 outputs
+    // does not see: with 12 instead of 18 1024 x 3072 -> 5120 normal values take 533 instead of 437 us, 512 x 4096 -> 4096 291 and 254,
+    // and nothing is faster by more than 1 %.
     s.price_fail = (all ? 18.f : boxes ? 9.f : 6.f) * pr.K;
     s.price_dense = g_extremes > 0 ? 3e38f : (all ? 0.7f : boxes ? 0.5f : 0.2f) * pr.K;
     *gate = &s.head->full;
@@ -1315,11 +1331,11 @@ hipError_t extremes_forward(const float* x, const float* x2, const float* x3, co
         hipLaunchKernelGGL(extremes_walk_kernel<decltype(mode)::value>, dim3(4 * pr.num_cu), dim3(256), 0, stream, s);
         return hipGetLastError();
     };
-    auto second_of = [&](int turn) { Search t = s; t.turn = turn; return t; };
+    auto second_of = [&](int turn, int note = 0) { Search t = s; t.turn = turn; t.note = note; return t; };
     if (all) {
         if (hipError_t e = launch_scan<kBoxesAndPoints, false>(s, pr, stream); e != hipSuccess) return e;
-        if (hipError_t e = launch_scan<kBoxes, true>(second_of(1), pr, stream); e != hipSuccess) return e;
-        Search points = second_of(2);
+        if (hipError_t e = launch_scan<kBoxes, true>(second_of(1, kBoxFails), pr, stream); e != hipSuccess) return e;
+        Search points = second_of(2, kPointFails);
         points.x.v = x3;
         points.x.rest = s.x.rest + (size_t)4 * pr.B;
         points.out = out3;
