@@ -18,19 +18,19 @@
 //            and the second leaves at once: 5120 x 5120 with positions at batch 272, 46 + 43 -> 50 + 5 us.
 //
 // Boxes and the points inside them (certification) share sample, lists and first scan: an entry of a row of x is {lower, upper,
-// 32 k, point}.  Where the weights have lists, the second scans of boxes and of values follow it.  Values and bounds of the 5-layer,
-// 5120-wide net at batch 1024: 1450 to 1640 us with passes of their own, 745 together; 5120 x 5120 normal weights and inputs of
-// the same spread, batch 512, 187 + 240 -> 350 us, 1024 256 + 390 -> 580.
+// 32 k, point}.  Where the weights have lists, the second scans of boxes and of values follow it.  Certification of the 5-layer,
+// 5120-wide net at batch 1024: 1500 us with passes of their own, 820 together; 5120 x 5120 normal weights and inputs of the same
+// spread, batch 512, 171 + 229 -> 330 us, 1024 235 + 385 -> 548.
 //
 // The reduction is cut into C chunks of at most 2560 k with lists and bounds of their own, so that a chunk of eight rows
 // of the other operand fits half a CU's LDS.  Rows with NaN or infinities (bounds: boxes that are not l <= u) get an infinite
 // bound: their outputs are walked in full with the comparisons of the other kernels.
 //
-// 5120 x 5120 with positions, batch 272 / 512: 300 / 470 -> 165 / 205 us; values at 1024 780 -> 155; bounds at 1024 2170 -> 225.
-// Data that the lists cannot help (two values in both operands) cost the sample and the lists beside the full walk: 15 to 60 us
+// 5120 x 5120, full walk -> lists, us: layers of an untrained net on its own inputs, positions at batch 512 445 -> 102, values at 1024
+// 780 -> 100, bounds at 1024 2170 -> 142; normal weights and inputs of the same spread 215, 235 and 385.  Data that the lists cannot help (two values in both operands) cost the sample and the lists beside the full walk: 15 to 60 us
 // up to 5120 inputs, 75 at 12544, 110 to 140 at 20000.  Weights of a 5 x 5120 net that has been trained through p = 8 ... 1000 and
-// infinity need longer lists than untrained ones: on its own inputs, batch 512, lists / full walk, us, positions 182 / 474, values
-// 162 / 437, bounds 239 / 1125 (untrained 102 / 467, 100 / 429, 121 / 1099).
+// infinity need lists of their own, and leave more outputs to be walked: on its own inputs at batch 1024 positions 155 to 169, values 135
+// to 160, bounds 211 to 223, values with bounds 297 to 342.
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -225,7 +225,8 @@ __device__ __forceinline__ void lengths_of(RowChunk<NV>& a, float center, int* h
 // A workgroup looks at 4 x 4 outputs: wave i at row i % 8 (four of x, four of w) in every other chunk, then all at the outputs.
 // Bound by a chain of latencies: the outputs' rows are on their way during the histograms, and their 16 (boxes 32, with points 48)
 // maxima meet 16 at a time: 5120 -> 5120 17.5 -> 15.9 us, boxes with points 29.9 -> 24.7.
-// ENDS: 1 values, 2 boxes, 3 boxes and the points inside them.
+// ENDS: 1 values, 2 boxes, 3 boxes and the points inside them.  Of 40 values per lane 1 is spilled without boxes, and 31 registers with
+// points, outside of the loops over the outputs.
 template <int NV, int ENDS>
 __global__ void __launch_bounds__(1024) extremes_sample_kernel(Search s) {
     constexpr bool PAIR = ENDS >= 2, ALL = ENDS == 3;
@@ -425,6 +426,7 @@ __device__ __forceinline__ void choose_lengths(const Search& s, int (&sums)[8][6
 // (rows of weights are alike: most pass at once).  What the list leaves out lies in [center - t, center + t] then, exactly,
 // unless more values tie at the outer end than the list has places: such a row's bounds are those of all its values.
 // Bound by reading the operands once.
+// Boxes of 40 values per lane spill 18 registers of what all of a workgroup's rows share.
 // SPREAD: no positions follow, and the order of a list is free (its own instantiation: the code of both orders in one made the
 // kernel 43 -> 48 us).
 template <int NV, int ENDS, bool SPREAD>
@@ -698,14 +700,19 @@ __device__ __host__ constexpr int strip_rows(bool pairs) { return pairs ? 4 : 8;
 // k, so that an entry costs two 128-bit reads at a place of its own for eight differences (boxes in the strip: four rows,
 // lower and upper end).  Odd lanes read the second half first: two lanes at the same k mod 8 then miss each other's banks.
 //
-// Bound by the vector unit (3.5 instructions per difference with the position) beside those reads, 60 % of whose cycles are
-// bank conflicts of random places: 5120 x 5120 at batch 512, 96 + 128 entries per row: 59 + 70 us, of which 25 are w from
-// memory.  Four rows per strip with four workgroups per CU read the lists twice as often: 92 + 105 us before, and 73 + 91 with
-// eight rows, both with the first pass's results stored one by one to 64 rows at a time (35 us of that pass); a strip's next chunk fetched between the
-// entries made their loads wait for it (they return in order): 82 us.
+// Bound by neither unit but by phases that take turns: the hand-out and the heads of the lists, a strip on its way to LDS, the
+// walk.  5120 x 5120 with positions, at 2.7 clocks per instruction: batch 272, weights without lists, 50 us, the vector unit 22 % and
+// LDS 13 % busy; batch 512 with both lists 65 + 68 us, 42 % and 37 %, 58 % of the latter bank conflicts of places in the order of k
+// (where the order of a list is free, 34 to 42 %).  Boxes and points at batch 1024 136 us, the vector unit 49 %.  Four rows per
+// strip with four workgroups per CU read the lists twice as often: 92 + 105 us before, and 73 + 91 with eight rows, both with the first
+// pass's results stored one by one to 64 rows at a time (35 us of that pass); a strip's next chunk fetched between the entries made
+// their loads wait for it (they return in order): 82 us.
 //
-// First pass: lanes are rows of x, results into s.partial.  Second: lanes are rows of w; takes what the first left, checks the
-// bound and notes the outputs that fail it.
+// First pass: lanes are rows of x.  Where the weights have lists, its results go into s.partial, and the second pass, whose lanes are
+// rows of w, takes them up; whichever is the last checks the bound, stores every output and notes those that fail it.
+//
+// Two workgroups of eight waves to a CU leave a lane 128 registers, which the first pass of boxes (3 spilled) and that of boxes and
+// points (13) exceed: numbers of a tile, stored and fetched once per tile, none of them in the walk.
 template <class T, int N>
 __device__ __forceinline__ void store_row(T* to, const T (&v)[N]) {   // neighbouring elements, aligned to one
     static_assert(N % 4 == 0);
@@ -1248,7 +1255,9 @@ int lanes_for(int rows, int strips, int num_cu) {
 // Few outputs of a long reduction leave the sample and the scans to few workgroups, which walk all its chunks in turn: the terms
 // beyond one and two chunks, fitted to 552 layers of 600 to 40000 inputs, normal and uniform inputs, of which 66 were slower
 // with lists before (256 x 25088 -> 256 with positions 94 us in full, 174 with lists; 1024 x 25088 -> 64 values 88 and 192), and
-// 3 of the 443 that are left are, by 2 to 11 %.
+// 3 of the 443 that are left are, by 2 to 11 %.  Sample, lists and first scan have become faster since, and points share those of the
+// boxes, so that layers stay in full which lists would serve: values and bounds of 256 x 2048 -> 2048 159 us, 60 to 109 with lists,
+// 32 x 5120 -> 5120 167, 85 to 142.
 // The size alone decides, for the caller asks for the workspace before there is a device to ask.
 static bool lists_pay(const Problem& pr, ForwardKind kind) {
     if (g_tile_override >= 0 || pr.K < 512) return false;

@@ -160,7 +160,8 @@ bool norm_forward_shifts(const Problem& pr, float p) {
 // size.  A forward pass that trains keeps the order of summation it has always had (chunks of 32 k, alternating between
 // the k-groups of the tile that fits the size): the batch-mean shift behind a layer of nearly equal distances leaves small
 // differences of large numbers, and one unit in the last place of the distances was seen a thousand times as large in the
-// gradients of a five-layer net.
+// gradients of a five-layer net.  The bits of general exponents below 128 depend on the tile all the same: its first stage gives the
+// unit that its logarithms are taken in.
 hipError_t norm_forward(const float* input, const float* weight, float* output, float p, const Problem& pr,
                         bool values_only, hipStream_t stream) {
     if (pr.NG <= kSkinnyMaxNG && values_only && few_rows_of_few_outputs(pr, true, small_int_power(p) < 2 || small_int_power(p) == 7))

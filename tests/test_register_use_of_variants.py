@@ -24,3 +24,14 @@ def test_lists_of_outermost_values(tmp_path):
     sizes = {name: size for name, size in scratch_of("extremes_forward.hip", tmp_path).items()
              if re.search(r"extremes_select_kernelILi(?:16|24|32)E", name)}
     assert len(sizes) == 12 and max(sizes.values()) == 0
+
+
+def test_scans_and_samples_of_lists(tmp_path):
+    """What the first scans of boxes, and the longest rows of the sample and list kernels, spill outside of their loops; no more, and
+    nothing in any other form."""
+    allowed = {"scan_kernelILi3ELb0E": 40, "scan_kernelILi2ELb0E": 16, "sample_kernelILi40ELi3E": 68, "sample_kernelILi40ELi1E": 8,
+               "select_kernelILi40ELi2E": 76, "select_kernelILi40ELi3E": 76}
+    sizes = {name: size for name, size in scratch_of("extremes_forward.hip", tmp_path).items() if "extremes_" in name}
+    assert sum(any(form in name for name in sizes) for form in allowed) == len(allowed)
+    for name, size in sizes.items():
+        assert size <= max((most for form, most in allowed.items() if form in name), default=0), name
